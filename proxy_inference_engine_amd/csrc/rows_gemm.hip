@@ -7,7 +7,7 @@
 // which costs nothing: the matrix cores are idle either way.  The K-split partial sums meet in LDS.
 //
 // The same kernel runs batched over heads (per-head up- / down-projections), over a list of unlike matrices, grouped over the active experts of a mixture (row lists), and for
-// any M (blockIdx.z walks 16 * NT rows at a time).
+// any M (blockIdx.z walks 16 * NT rows at a time).  Long rows of x that several rows share a pass with go through LDS instead (k_rows_lds).
 #include <algorithm>
 
 #include "stack_types.hpp"
@@ -15,6 +15,7 @@
 size_t w16m_size(int N, int K);
 
 typedef __attribute__((ext_vector_type(8))) __bf16 mf_bf16x8;
+typedef __attribute__((ext_vector_type(8))) _Float16 mf_f16x8;
 typedef __attribute__((ext_vector_type(4))) float mf_f32x4;
 typedef __attribute__((ext_vector_type(4))) u32 mf_u32x4;
 
@@ -29,16 +30,16 @@ struct RowsWork {
     const int *rows;  // x row of local row i (nullptr: row0 + i)
     int xoff, yoff;
 };
-__device__ __forceinline__ bool rows_select(const RowsArgs &a, RowsWork &k) {
+// b: blockIdx.y; last: the shared expert's
+__device__ __forceinline__ bool rows_select(const RowsArgs &a, RowsWork &k, int b, int last) {
     k.w = a.m.w, k.x = a.m.x, k.y = a.m.y, k.N = a.m.N, k.K = a.m.K, k.ldx = a.m.ldx, k.ldy = a.m.ldy;
     k.count = a.M, k.row0 = 0, k.rows = a.rows, k.xoff = k.yoff = 0;
-    const int b = blockIdx.y;
     if (a.n_mats) {
         const RowsMat &m = a.mats[b];
         k.w = m.w, k.x = m.x, k.y = m.y, k.N = m.N, k.K = m.K, k.ldx = m.ldx, k.ldy = m.ldy;
         return true;
     }
-    if (a.shared.w && b == (int)gridDim.y - 1) {
+    if (a.shared.w && b == last) {
         k.w = a.shared.w, k.x = a.shared.x, k.y = a.shared.y, k.N = a.shared.N, k.K = a.shared.K, k.ldx = a.shared.ldx, k.ldy = a.shared.ldy;
         return true;
     }
@@ -54,7 +55,14 @@ __device__ __forceinline__ bool rows_select(const RowsArgs &a, RowsWork &k) {
     return true;
 }
 
-// One finished value (m: result row inside the group, n: feature); pair: the value of feature n + 1 (ROWS_SILU_MUL, ROWS_CLIP_MUL, ROWS_GELU_MUL)
+template <class E>
+__device__ __forceinline__ mf_f32x4 rows_mfma(mf_u32x4 w, mf_u32x4 x, mf_f32x4 acc) {
+    if constexpr (__is_same(E, ElemF16)) return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(mf_f16x8, w), __builtin_bit_cast(mf_f16x8, x), acc, 0, 0, 0);
+    else return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(mf_bf16x8, w), __builtin_bit_cast(mf_bf16x8, x), acc, 0, 0, 0);
+}
+__host__ __device__ __forceinline__ bool rows_paired(int epi) { return epi == ROWS_SILU_MUL || epi == ROWS_CLIP_MUL || epi == ROWS_GELU_MUL || epi == ROWS_SWIGLU; }
+
+// One finished value (m: result row inside the group, n: feature); pair: the value of feature n + 1 (rows_paired)
 template <class E>
 __device__ __forceinline__ void rows_finish(const RowsArgs &a, const RowsWork &k, int m, int n, float v, float pair) {
     typedef typename E::type T;
@@ -82,6 +90,22 @@ __device__ __forceinline__ void rows_finish(const RowsArgs &a, const RowsWork &k
             break;
         case ROWS_GELU_SIDE: ((T *)k.y)[row * k.ldy + n] = E::pack(gelu_tanh<sizeof(T) == 4>(v) * BF16::to_f32(token_vector(a.side, row)[n])); break;
         case ROWS_SOFTCAP: ((float *)k.y)[row * k.ldy + n] = a.act_limit * stack_tanh<sizeof(T) == 4>(v * a.scale / a.act_limit); break;
+        case ROWS_LINEAR:
+        case ROWS_SWIGLU:
+            if constexpr (sizeof(T) == 2) {  // (the Llama's Linears: 16-bit stacks only)
+                auto once = [&](float z, int at) {
+                    const T r = E::pack(z);
+                    return a.bias ? E::pack(E::load(&r) + E::load((const T *)a.bias + at)) : r;
+                };
+                const T g = once(v, n);
+                if (a.epi == ROWS_LINEAR) ((T *)k.y)[row * k.ldy + n] = g;
+                else if (!(n & 1)) {
+                    const float z = E::load(&g);
+                    const T s = E::pack(z / (1.0f + expf(-z))), u = once(pair, n + 1);
+                    ((T *)k.y)[row * k.ldy + (n >> 1)] = E::pack(E::load(&s) * E::load(&u));
+                }
+            }
+            break;
         case ROWS_SPLIT:
             if (n < a.split) ((T *)k.y)[row * k.ldy + n] = E::pack(v);
             else a.y2[row * a.ldy2 + n - a.split] = v;
@@ -118,7 +142,7 @@ __device__ __forceinline__ bool rows_ride(const RowsArgs &a, float *red) {
 
 // NT: blocks of 16 rows of x; KW: waves along K; NN: blocks of 16 features per wave (two share the x operands); MERGE: x = the merged key splits of head
 // blockIdx.y (RowsArgs::merge), put together in LDS by every workgroup of the head; NORM: RowsArgs::x_norm (every workgroup sees its rows whole)
-template <int NT, int KW, int NN, bool MERGE = false, bool NORM = false>
+template <class E, int NT, int KW, int NN, bool MERGE = false, bool NORM = false>
 __global__ void __launch_bounds__(512) k_rows_w16m(const RowsArgs a) {
     constexpr int NW = 8 / KW, U = NT >= 4 ? 2 : 4;
     constexpr int ST = 20;  // floats per (row, 16 features) line of the reduction image
@@ -143,7 +167,7 @@ __global__ void __launch_bounds__(512) k_rows_w16m(const RowsArgs a) {
         __syncthreads();
     }
     RowsWork k;
-    if (!rows_select(a, k)) return;
+    if (!rows_select(a, k, blockIdx.y, (int)gridDim.y - 1)) return;
     const int i0 = blockIdx.z * 16 * NT;
     if (i0 >= k.count) return;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -192,8 +216,7 @@ __global__ void __launch_bounds__(512) k_rows_w16m(const RowsArgs a) {
 #pragma unroll
                             for (int i = 0; i < 4; ++i) ss = fmaf(lo_f32<BF16>(xv[u][0][i]), lo_f32<BF16>(xv[u][0][i]), fmaf(hi_f32<BF16>(xv[u][0][i]), hi_f32<BF16>(xv[u][0][i]), ss));
 #pragma unroll
-                    for (int t = 0; t < NT; ++t)
-                        acc[n][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(mf_bf16x8, w), __builtin_bit_cast(mf_bf16x8, xv[u][t]), acc[n][t], 0, 0, 0);
+                    for (int t = 0; t < NT; ++t) acc[n][t] = rows_mfma<E>(w, xv[u][t], acc[n][t]);
                 }
         };
         mf_u32x4 w0[U][NN], w1[U][NN], x0[U][NT], x1[U][NT];
@@ -215,7 +238,7 @@ __global__ void __launch_bounds__(512) k_rows_w16m(const RowsArgs a) {
 #pragma unroll
         for (int t = 0; t < NT; ++t) *(mf_f32x4 *)(s_red + (((wave * NN + n) * NT + t) * 16 + c) * ST + 4 * kq) = acc[n][t];
     __syncthreads();
-    const bool paired = a.epi == ROWS_SILU_MUL || a.epi == ROWS_CLIP_MUL || a.epi == ROWS_GELU_MUL;
+    const bool paired = rows_paired(a.epi);
     for (int id = threadIdx.x; id < NW * NN * NT * 256; id += 512) {
         const int nl = id & 15, ml = (id >> 4) % (16 * NT), wn2 = id / (256 * NT), w = wn2 / NN, nn = wn2 % NN;
         const int n = ((int)blockIdx.x * NW * NN + wn2) * 16 + nl, m = i0 + ml;
@@ -234,7 +257,133 @@ __global__ void __launch_bounds__(512) k_rows_w16m(const RowsArgs a) {
             for (int q = 0; q < KW; ++q) sum += s_ss[w * KW + q][ml];
             v *= 1.0f / sqrtf(sum / (float)k.K + a.x_eps);
         }
-        rows_finish<ElemBF16>(a, k, m, n, v, p);
+        rows_finish<E>(a, k, m, n, v, p);
+    }
+}
+
+// Rows that share a pass, x through LDS.  k_rows_w16m fetches every 16 B of x into the lanes that multiply it, 16 scattered runs of 64 B per instruction, for every 16 or 32 features
+// again: from 8 rows on that, and no longer the weights, is what the time goes to ([28672, 4096]: 37 us with 1 row, 41 / 52 / 58 / 88 with 8 / 16 / 32 / 64; profile and counts agree, the
+// matrix cores idle).  Here a workgroup of eight waves takes 16 NN features and all of K in chunks of 256 U columns: the chunk's rows come in as whole lines, once per workgroup
+// (registers, then one of two LDS buffers; rows padded by 16 B, conflict-free both ways), each wave multiplies every eighth 32-column step by weights that it streams two chunks ahead.
+// Loads go by descriptors whose bounds drop what lies behind a row, a matrix or K (zeros), so no load has a branch around it.  Two workgroups share a CU (launch bounds: 128 registers),
+// one loads while the other finishes.  Sixteen features per wave and step re-read x most (NN = 1), four blocks least: NN follows from how many workgroups are left (rows_gemm_launch).
+// [28672, 4096] with 8 / 16 / 32 / 64 rows: 39 / 40 / 42 / 64 us = 6.0 / 5.8 / 5.6 / 3.7 TB/s; 60 active experts of [2816, 2048] with 3 rows each: 131 -> 110 us (6.3 TB/s).
+template <class E, int NT, int NN, int U>
+__global__ void __launch_bounds__(512, 4) k_rows_lds(const RowsArgs a) {
+    constexpr int C = 256 * U, LD = C + 8, ST = 20;                // columns of x per chunk; u16 per LDS row; floats per line of the reduction image
+    constexpr int PR = C / 8, RP = 512 / PR, XJ = 16 * NT / RP;    // 16-byte pieces per row of a chunk; rows that 512 threads fetch at once; pieces per thread
+    constexpr size_t X_BYTES = (size_t)2 * 16 * NT * LD * 2, RED_BYTES = (size_t)8 * NN * NT * 16 * ST * 4;
+    static_assert(512 % PR == 0 && 16 * NT % RP == 0, "whole rows per round of loads");
+    __shared__ __attribute__((aligned(16))) char s_mem[X_BYTES > RED_BYTES ? X_BYTES : RED_BYTES];
+    u16 *s_x = (u16 *)s_mem;
+    float *s_red = (float *)s_mem;
+    if constexpr (__is_same(E, ElemBF16))
+        if (rows_ride<ElemBF16, 512>(a, s_red)) return;
+    int bx = blockIdx.x, by = blockIdx.y;
+    if (a.flat_tiles < 0) {  // a list, workgroup after workgroup
+        for (by = 0;; ++by) {
+            const int t = (a.mats[by].N + 16 * NN - 1) / (16 * NN);
+            if (bx < t) break;
+            bx -= t;
+        }
+    } else if (a.flat_tiles > 0) {  // experts, then the shared one
+        by = min(bx / a.flat_tiles, a.flat_batches), bx -= by * a.flat_tiles;
+    }
+    RowsWork k;
+    if (!rows_select(a, k, by, a.flat_tiles > 0 ? a.flat_batches : (int)gridDim.y - 1)) return;
+    if (bx * NN * 16 >= k.N) return;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), c = lane & 15, kq = lane >> 4;
+    const int t16 = bx * NN, groups = (k.K + 63) >> 6, steps = 2 * groups, K8 = (k.K + 7) & ~7, iters = (steps + 8 * U - 1) / (8 * U);
+    const int w_tiles = min(((k.N + 31) >> 5) - (t16 >> 1), (NN + 1) / 2);  // 32-row tiles of this workgroup: a matrix ends with a whole tile
+    const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>(k.w + (size_t)(t16 >> 1) * groups * 4096), 0, w_tiles * groups * 4096, 0x00020000);
+    const unsigned wlane = (kq >> 1) * 1024 + ((kq & 1) * 32 + c) * 16 + (t16 & 1) * 256;
+    const int xc = threadIdx.x % PR * 8, xr0 = threadIdx.x / PR;  // this thread's columns and rows of a chunk
+    for (int i0 = blockIdx.z * 16 * NT; i0 < k.count; i0 += gridDim.z * 16 * NT) {
+        const u16 *x0 = (const u16 *)k.x + (k.rows ? 0 : (size_t)(k.row0 + i0) * k.ldx) + k.xoff;
+        const __amdgpu_buffer_rsrc_t xs = __builtin_amdgcn_make_buffer_rsrc(const_cast<u16 *>(x0), 0, 0x7FFFFFF0, 0x00020000);
+        constexpr unsigned NOWHERE = 0x80000000u;  // behind every descriptor's end
+        unsigned xo[XJ];
+#pragma unroll
+        for (int j = 0; j < XJ; ++j) {
+            const int r = xr0 + RP * j;
+            const bool in = i0 + r < k.count;
+            const int xr = k.rows ? k.rows[in ? i0 + r : i0] : r;
+            xo[j] = in ? (unsigned)(xr * k.ldx + xc) * 2u : NOWHERE;
+        }
+        auto load_x = [&](int it, mf_u32x4(&xv)[XJ]) {
+            const unsigned at = xc + it * C < K8 ? (unsigned)(it * C * 2) : NOWHERE;
+#pragma unroll
+            for (int j = 0; j < XJ; ++j) xv[j] = __builtin_amdgcn_raw_buffer_load_b128(xs, (int)(xo[j] | at) < 0 ? NOWHERE : xo[j] + at, 0, 0);
+        };
+        auto store_x = [&](int buf, const mf_u32x4(&xv)[XJ]) {
+#pragma unroll
+            for (int j = 0; j < XJ; ++j) *(mf_u32x4 *)(s_x + (buf * 16 * NT + xr0 + RP * j) * LD + xc) = xv[j];
+        };
+        auto load_w = [&](int it, mf_u32x4(&wv)[U][NN]) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int s = (it * U + u) * 8 + wave;
+#pragma unroll
+                for (int n = 0; n < NN; ++n)  // non-temporal: a pass reads a weight once
+                    wv[u][n] = __builtin_amdgcn_raw_buffer_load_b128(wr, s < steps ? wlane + (unsigned)((n >> 1) * groups * 4096 + s * 2048 + (n & 1) * 256) : NOWHERE, 0, 2);
+            }
+        };
+        mf_f32x4 acc[NN][NT];
+#pragma unroll
+        for (int n = 0; n < NN; ++n)
+#pragma unroll
+            for (int t = 0; t < NT; ++t) acc[n][t] = (mf_f32x4){0.0f, 0.0f, 0.0f, 0.0f};
+        auto multiply = [&](int buf, const mf_u32x4(&wv)[U][NN]) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                mf_u32x4 xv[NT];
+#pragma unroll
+                for (int t = 0; t < NT; ++t) xv[t] = *(const mf_u32x4 *)(s_x + (buf * 16 * NT + 16 * t + c) * LD + (8 * u + wave) * 32 + 8 * kq);
+#pragma unroll
+                for (int n = 0; n < NN; ++n)
+#pragma unroll
+                    for (int t = 0; t < NT; ++t) acc[n][t] = rows_mfma<E>(wv[u][n], xv[t], acc[n][t]);
+            }
+        };
+        // (x before w: waiting for the next chunk's x must not wait for the weights behind it)
+        mf_u32x4 w[2][U][NN], xv[XJ];
+        load_x(0, xv);
+        load_w(0, w[0]);
+        store_x(0, xv);
+        load_x(1, xv);
+        load_w(1, w[1]);
+        __syncthreads();
+        for (int it = 0; it < iters; it += 2) {
+#pragma unroll
+            for (int d = 0; d < 2; ++d) {
+                if (it + d >= iters) break;
+                multiply(d, w[d]);
+                store_x(d ^ 1, xv);
+                load_x(it + d + 2, xv);
+                load_w(it + d + 2, w[d]);
+                __syncthreads();
+            }
+        }
+        // lane (kq, c) holds features 4 kq .. + 3 of row c
+#pragma unroll
+        for (int n = 0; n < NN; ++n)
+#pragma unroll
+            for (int t = 0; t < NT; ++t) *(mf_f32x4 *)(s_red + (((wave * NN + n) * NT + t) * 16 + c) * ST + 4 * kq) = acc[n][t];
+        __syncthreads();
+        const bool paired = rows_paired(a.epi);
+        for (int id = threadIdx.x; id < NN * NT * 256; id += 512) {
+            const int nl = id & 15, ml = (id >> 4) % (16 * NT), nn = id / (256 * NT), n = (t16 + nn) * 16 + nl, m = i0 + ml;
+            if (n >= k.N || m >= k.count || (paired && (nl & 1))) continue;
+            const float *r = s_red + ((nn * NT + (ml >> 4)) * 16 + (ml & 15)) * ST + nl;
+            float v = 0.0f, p = 0.0f;
+#pragma unroll
+            for (int q = 0; q < 8; ++q) v += r[q * NN * NT * 16 * ST];
+            if (paired)
+#pragma unroll
+                for (int q = 0; q < 8; ++q) p += r[q * NN * NT * 16 * ST + 1];
+            rows_finish<E>(a, k, m, n, v, p);
+        }
+        __syncthreads();
     }
 }
 
@@ -243,7 +392,7 @@ __global__ void __launch_bounds__(256) k_rows_f32(const RowsArgs a) {
     __shared__ float s_w[16][65], s_x[16][65], s_v[16][17];
     if (rows_ride<ElemF32, 256>(a, s_v[0])) return;
     RowsWork k;
-    if (!rows_select(a, k)) return;
+    if (!rows_select(a, k, blockIdx.y, (int)gridDim.y - 1)) return;
     const int i0 = blockIdx.z * 16, n0 = blockIdx.x * 16;
     if (i0 >= k.count || n0 >= k.N) return;
     const int tn = threadIdx.x & 15, tm = threadIdx.x >> 4;
@@ -269,7 +418,37 @@ __global__ void __launch_bounds__(256) k_rows_f32(const RowsArgs a) {
     if (n < k.N && m < k.count) rows_finish<ElemF32>(a, k, m, n, acc, s_v[tm][tn < 15 ? tn + 1 : 15]);
 }
 
-template <int NT, int NN>
+template <class E, int NT, int NN, int U>
+int rows_lds_go(RowsArgs a, int n_max, int batches, hipStream_t st) {
+    auto tiles = [](int n) { return (unsigned)((n + 16 * NN - 1) / (16 * NN)); };
+    dim3 grid(tiles(n_max), (unsigned)(batches + rows_riders(a)), (unsigned)((a.M + 16 * NT - 1) / (16 * NT)));
+    if (a.active) {  // one workgroup per tile of every expert, and it goes through all the expert's rows: most experts have few
+        a.flat_batches = a.shared.w ? batches - 1 : batches, a.flat_tiles = (int)tiles(a.m.N);
+        grid = dim3(a.flat_batches * a.flat_tiles + (a.shared.w ? tiles(a.shared.N) : 0));
+    } else if (a.n_mats) {
+        a.flat_tiles = -1, grid.x = 0, grid.y = 1;
+        for (int i = 0; i < a.n_mats; ++i) grid.x += tiles(a.mats[i].N);
+    }
+    hipLaunchKernelGGL((k_rows_lds<E, NT, NN, U>), grid, dim3(512), 0, st, a);
+    PIE_LAUNCH_CHECK();
+    return PIE_OK;
+}
+
+// Which of the two, and how many features a workgroup of k_rows_lds takes; blocks: 16-feature blocks of the whole launch.  Measured, us (k_rows_w16m / NN = 1 / 2 / 4; x in LDS wins from
+// about 5 rows on, where the rows are long enough for eight waves to share them):
+//   [28672, 4096]: 8 rows 41 / 43 / 39 / 39, 32 rows 58 / 59 / 48 / 42    [11264, 2048]: 8 rows 11.1 / 14.1 / 12.8 / 12.1, 32 rows 17.5 / 17.2 / 15.9 / 13.9
+//   [6144, 4096]: 8 rows 13.6 / 14.6 / 12.3 / 17.5, 32 rows 17.0 / 19.1 / 15.2 / 20.3    [4096, 14336]: 8 rows 23.6 / 22.3 / 27.9 / 46.9, 32 rows 41 / 30 / 37 / 54
+// Fewer blocks than that leave CUs without a workgroup; more than 32 rows of x per CU take the room of the fourth block.
+template <class E>
+int rows_lds_pick(const RowsArgs &a, int n_max, long blocks, int batches, hipStream_t st) {
+    if (a.M <= 16 || a.active)
+        return blocks < 320 ? rows_lds_go<E, 1, 1, 4>(a, n_max, batches, st) : a.active ? rows_lds_go<E, 1, 4, 1>(a, n_max, batches, st) : rows_lds_go<E, 1, 2, 2>(a, n_max, batches, st);
+    if (a.M <= 32)
+        return blocks < 320 ? rows_lds_go<E, 2, 1, 2>(a, n_max, batches, st) : blocks < 640 ? rows_lds_go<E, 2, 2, 2>(a, n_max, batches, st) : rows_lds_go<E, 2, 4, 1>(a, n_max, batches, st);
+    return blocks < 320 ? rows_lds_go<E, 4, 1, 1>(a, n_max, batches, st) : rows_lds_go<E, 4, 2, 1>(a, n_max, batches, st);
+}
+
+template <class E, int NT, int NN>
 int rows_go(const RowsArgs &a, int n_max, int k_max, int batches, hipStream_t st) {
     const int steps = 2 * ((k_max + 63) / 64), tiles = (n_max + 16 * NN - 1) / (16 * NN);
     const int z = (a.M + 16 * NT - 1) / (16 * NT);  // (grouped: most experts have few rows, their later z leave at once)
@@ -277,20 +456,12 @@ int rows_go(const RowsArgs &a, int n_max, int k_max, int batches, hipStream_t st
     int kw = steps >= 32 ? 8 : steps >= 16 ? 4 : steps >= 8 ? 2 : 1;
     while (kw < 8 && steps >= 2 * kw && (size_t)((tiles + 8 / kw - 1) / (8 / kw)) * batches * z < 256) kw *= 2;
     const dim3 grid((unsigned)((tiles + 8 / kw - 1) / (8 / kw)), (unsigned)(batches + rows_riders(a)), (unsigned)z);
-    if (a.x_norm) {
-        if (kw == 8) hipLaunchKernelGGL((k_rows_w16m<1, 8, 1, false, true>), grid, dim3(512), 0, st, a);
-        else if (kw == 4) hipLaunchKernelGGL((k_rows_w16m<1, 4, 1, false, true>), grid, dim3(512), 0, st, a);
-        else if (kw == 2) hipLaunchKernelGGL((k_rows_w16m<1, 2, 1, false, true>), grid, dim3(512), 0, st, a);
-        else hipLaunchKernelGGL((k_rows_w16m<1, 1, 1, false, true>), grid, dim3(512), 0, st, a);
-    } else if (a.merge.splits > 0) {
-        if (kw == 8) hipLaunchKernelGGL((k_rows_w16m<1, 8, 1, true>), grid, dim3(512), 0, st, a);
-        else if (kw == 4) hipLaunchKernelGGL((k_rows_w16m<1, 4, 1, true>), grid, dim3(512), 0, st, a);
-        else if (kw == 2) hipLaunchKernelGGL((k_rows_w16m<1, 2, 1, true>), grid, dim3(512), 0, st, a);
-        else hipLaunchKernelGGL((k_rows_w16m<1, 1, 1, true>), grid, dim3(512), 0, st, a);
-    } else if (kw == 8) hipLaunchKernelGGL((k_rows_w16m<NT, 8, NN>), grid, dim3(512), 0, st, a);
-    else if (kw == 4) hipLaunchKernelGGL((k_rows_w16m<NT, 4, NN>), grid, dim3(512), 0, st, a);
-    else if (kw == 2) hipLaunchKernelGGL((k_rows_w16m<NT, 2, NN>), grid, dim3(512), 0, st, a);
-    else hipLaunchKernelGGL((k_rows_w16m<NT, 1, NN>), grid, dim3(512), 0, st, a);
+    auto go = [&](auto k8, auto k4, auto k2, auto k1) { hipLaunchKernelGGL((kw == 8 ? k8 : kw == 4 ? k4 : kw == 2 ? k2 : k1), grid, dim3(512), 0, st, a); };
+    if constexpr (__is_same(E, ElemBF16)) {
+        if (a.x_norm) go(&k_rows_w16m<E, 1, 8, 1, false, true>, &k_rows_w16m<E, 1, 4, 1, false, true>, &k_rows_w16m<E, 1, 2, 1, false, true>, &k_rows_w16m<E, 1, 1, 1, false, true>);
+        else if (a.merge.splits > 0) go(&k_rows_w16m<E, 1, 8, 1, true>, &k_rows_w16m<E, 1, 4, 1, true>, &k_rows_w16m<E, 1, 2, 1, true>, &k_rows_w16m<E, 1, 1, 1, true>);
+    }
+    if (!a.x_norm && a.merge.splits <= 0) go(&k_rows_w16m<E, NT, 8, NN>, &k_rows_w16m<E, NT, 4, NN>, &k_rows_w16m<E, NT, 2, NN>, &k_rows_w16m<E, NT, 1, NN>);
     PIE_LAUNCH_CHECK();
     return PIE_OK;
 }
@@ -333,10 +504,31 @@ int rows_gemm_launch(int dtype, const RowsArgs &a, int batches, hipStream_t st) 
     int n_all = batches == 1 ? n_max : 0;
     for (int i = 0; i < a.n_mats; ++i) n_all += a.mats[i].N;
     const bool narrow = (long)batches * n_max <= 16 * 64 && !a.merge.splits;  // so few workgroups that they should not all read all rows
-    if (a.M <= 16 || a.active || narrow) return rows_go<1, 1>(a, n_max, k_max, batches, st);
+    long blocks = 0;  // of 16 features, over the whole launch
+    for (int i = 0; i < a.n_mats; ++i) blocks += (a.mats[i].N + 15) / 16;
+    if (!a.n_mats) blocks = (long)batches * ((a.m.N + 15) / 16);
+    const bool within = (size_t)(a.rows || a.gather ? a.M : 64) * (size_t)a.m.ldx * 2 < (1u << 31);  // k_rows_lds counts an operand's bytes in 31 bits
+    if (a.M > 4 && k_max >= 1024 && !narrow && !a.x_norm && a.merge.splits <= 0 && within) return rows_lds_pick<ElemBF16>(a, n_max, blocks, batches, st);
+    if (a.M <= 16 || a.active || narrow) return rows_go<ElemBF16, 1, 1>(a, n_max, k_max, batches, st);
     const bool wide = n_all >= 32 * 140;  // two feature blocks per wave where half as many workgroups still fill most of the chip
-    if (a.M <= 32) return wide ? rows_go<2, 2>(a, n_max, k_max, batches, st) : rows_go<2, 1>(a, n_max, k_max, batches, st);
-    return wide ? rows_go<4, 2>(a, n_max, k_max, batches, st) : rows_go<4, 1>(a, n_max, k_max, batches, st);
+    if (a.M <= 32) return wide ? rows_go<ElemBF16, 2, 2>(a, n_max, k_max, batches, st) : rows_go<ElemBF16, 2, 1>(a, n_max, k_max, batches, st);
+    return wide ? rows_go<ElemBF16, 4, 2>(a, n_max, k_max, batches, st) : rows_go<ElemBF16, 4, 1>(a, n_max, k_max, batches, st);
+}
+
+template <class E>
+static int rows_w16_go(const RowsArgs &a, hipStream_t st) {
+    return a.M > 4 && a.m.K >= 1024 ? rows_lds_pick<E>(a, a.m.N, (a.m.N + 15) / 16, 1, st) : rows_go<E, 1, 1>(a, a.m.N, a.m.K, 1, st);
+}
+
+int rows_w16_launch(int dtype, const void *w16m, const void *x, int M, int N, int K, void *y, const void *bias, bool swiglu, hipStream_t st) {
+    PIE_REQUIRE(M >= 1 && M <= ROWS_W16_MAX && N > 0 && K > 0 && K % 64 == 0, PIE_E_SHAPE, "few-row 16-bit Linear: 1 to 32 rows, in_features % 64 == 0");
+    PIE_REQUIRE(dtype == PIE_BF16 || dtype == PIE_F16, PIE_E_ARG, "few-row 16-bit Linear: dtype must be PIE_BF16 or PIE_F16");
+    PIE_REQUIRE(pie_aligned(x, 16) && pie_aligned(w16m, 16), PIE_E_ALIGN, "few-row 16-bit Linear: 16-byte alignment required");
+    PIE_REQUIRE(!swiglu || N % 2 == 0, PIE_E_SHAPE, "few-row 16-bit Linear: the fused activation pairs columns");
+    RowsArgs a = {};
+    a.m = {(const char *)w16m, N, K, x, K, y, swiglu ? N / 2 : N};
+    a.M = M, a.epi = swiglu ? ROWS_SWIGLU : ROWS_LINEAR, a.bias = (const u16 *)bias;
+    return dtype == PIE_F16 ? rows_w16_go<ElemF16>(a, st) : rows_w16_go<ElemBF16>(a, st);
 }
 
 extern "C" {

@@ -18,6 +18,11 @@ struct ElemBF16 {
     static __device__ __forceinline__ float load(const u16 *p) { return BF16::to_f32(*p); }
     static __device__ __forceinline__ u16 pack(float v) { return BF16::from_f32(v); }
 };
+struct ElemF16 {
+    typedef u16 type;
+    static __device__ __forceinline__ float load(const u16 *p) { return F16::to_f32(*p); }
+    static __device__ __forceinline__ u16 pack(float v) { return F16::from_f32(v); }
+};
 struct ElemF32 {
     typedef float type;
     static __device__ __forceinline__ float load(const float *p) { return *p; }
@@ -292,6 +297,8 @@ enum RowsEpi {
     ROWS_GELU_MUL = 8,   // rows (2 i, 2 i + 1) = (gate_i, up_i), plus the bias: y[m][i] = T(gelu_tanh(gate) * up)
     ROWS_GELU_SIDE = 9,  // y[m][n] = T(gelu_tanh(v) * the row's token's side vector[n])
     ROWS_SOFTCAP = 10,   // y[m][n] = act_limit tanh(v * scale / act_limit), fp32 (capped logits)
+    ROWS_LINEAR = 11,    // y[m][n] = T(T(v) + bias), bias in T
+    ROWS_SWIGLU = 12,    // rows (2 i, 2 i + 1) = (gate_i, up_i), each rounded as by ROWS_LINEAR: y[m][i] = T(T(silu(gate)) * up)
 };
 // g sigmoid(alpha g) (u + 1) with g = min(gate, limit), u = clamp(up, -limit, limit)
 __device__ __forceinline__ float clipped_glu(float gate, float up, float alpha, float limit) {
@@ -329,7 +336,8 @@ struct RowsArgs {
     const int *rows;       // ungrouped, nullable: x row of result row i
     RowsMat mats[ROWS_LIST];  // n_mats > 0: blockIdx.y picks one of these instead of m, each with its own sizes and operands
     int n_mats;
-    const u16 *bias;       // ROWS_GELU_MUL: bf16 [N], nullable
+    int flat_tiles, flat_batches;  // set by the launcher (k_rows_lds): workgroups of one expert's matrix, experts; or -1: a list, workgroup after workgroup
+    const u16 *bias;       // ROWS_GELU_MUL (bf16), ROWS_LINEAR, ROWS_SWIGLU: [N], nullable
     TokenVectors side;     // ROWS_GELU_SIDE
     int epi;
     float scale;
@@ -353,6 +361,9 @@ struct RowsArgs {
 };
 // batches: blockIdx.y extent (1 for a plain Linear; heads; active experts (+ 1 with a shared expert))
 int rows_gemm_launch(int dtype, const RowsArgs &a, int batches, hipStream_t st);
+// y [M, N] = T(x W^T) (+ bias), or (swiglu) the MLP activation [M, N / 2] of a packed gate|up matrix, for few rows; W: W16M tiles in bf16 or f16, x [M][K] packed, K % 64 == 0
+constexpr int ROWS_W16_MAX = 32;
+int rows_w16_launch(int dtype, const void *w16m, const void *x, int M, int N, int K, void *y, const void *bias, bool swiglu, hipStream_t st);
 // bytes of a packed [N, K] weight of the stack's dtype, and the repack from row-major bf16
 size_t rows_weight_bytes(int dtype, int N, int K);
 

@@ -1,0 +1,62 @@
+"""The Linear of 5 to 64 rows whose operand goes through LDS (k_rows_lds), where it can go wrong: a last chunk of K that is not whole, row blocks that are not full, experts with more rows
+than a block, output widths on both sides of every choice of features per workgroup, float16, biases."""
+import numpy as np
+import pytest
+import torch
+
+import taduzen_util as tu
+from oracle import taduzen_oracle as orc
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("vocab", [331, 5203, 10259])   # 21, 326 and 642 blocks of 16 features: one, two and four per workgroup
+def test_stack_linears_against_the_oracle(vocab):
+    """K = 1096 and 1100 (chunks of 256, 512 or 1024 columns), experts with 2 / 3 of the rows each beside a shared one, every wanted row through the head.  bfloat16 storage everywhere: two layers'
+    roundings of 2^-9 stay below 0.04 of a row (the bound of the other tests of this design); a dropped or doubled chunk is a quarter of a product and more."""
+    from proxy_inference_engine_amd.models.taduzen import Model, ModelArgs
+    cfg = tu.config([(tu.latent(heads=9, dim=120, vdim=116, rank=72, window=40), tu.dense(1100)), (tu.latent(heads=2, rank=40), tu.moe(ff=1100, experts=3, top=2, shared=1300))], width=1096, vocab=vocab)
+    w = tu.weights(cfg, seed=8)
+    m = Model(ModelArgs(**cfg), {k: v.cuda() for k, v in w.items()}, dtype=torch.bfloat16)
+    m.enable_paged_kv(num_pages=8)
+    wn = tu.as_numpy(w)
+    for n in (4, 5, 16, 17, 32, 33, 60):
+        ids, c = tu.tokens(cfg, n, seed=n), m.make_cache()
+        got = m.step_portions([(ids, c)], [list(range(n))]).cpu().numpy()
+        c[0].page_manager.release()
+        assert tu.err(got, orc.forward(cfg, wn, ids)) < 0.04, n
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("vocab", [330, 5210, 10260])
+def test_dense_llama_step_of_several_rows(dtype, vocab):
+    """A step of B sequences against the same tokens fed to single sequences (another kernel: the GEMV).  Two layers, both sides accumulate in fp32 and round to T at the same places: four ulps of the largest
+    logit, rms four ulps, as everywhere in this suite."""
+    from _util import assert_vec_close
+    from proxy_inference_engine_amd.models.llama import Model, ModelArgs
+    from proxy_inference_engine_amd.models.utils import synthetic_checkpoint
+    cfg = {"model_type": "llama", "hidden_size": 1088, "num_hidden_layers": 2, "intermediate_size": 1472, "num_attention_heads": 16, "num_key_value_heads": 4, "head_dim": 64,
+           "vocab_size": vocab, "rms_norm_eps": 1e-5, "tie_word_embeddings": False, "attention_bias": True, "mlp_bias": True, "quantization": None}
+    m = Model(ModelArgs(**cfg), synthetic_checkpoint(cfg, seed=2, dtype=dtype))
+    m.enable_paged_kv(num_pages=96, max_blocks=2)
+    rng = np.random.default_rng(3)
+    prompts = [rng.integers(0, vocab, 7 + i % 5).astype(np.int32) for i in range(32)]
+    feed = torch.from_numpy(rng.integers(0, vocab, 32).astype(np.int32)).cuda()
+    want = []
+    for i, p in enumerate(prompts):
+        c = m.make_cache()
+        m.step(torch.from_numpy(p).cuda(), c)
+        want.append(m.step(feed[i:i + 1], c)[2].float().cpu().numpy().reshape(-1))
+        c[0].page_manager.release()
+    for B in (1, 2, 5, 6, 16, 17, 32):
+        caches = [m.make_cache() for _ in range(B)]
+        for p, c in zip(prompts, caches):
+            m.step(torch.from_numpy(p).cuda(), c)
+        for step in range(4):   # eager, captured, replayed; the same position again after every step
+            got = m.step_batch(feed[:B], caches)[2].float().cpu().numpy()
+            for i in range(B):
+                assert_vec_close(got[i], want[i], "bfloat16" if dtype == torch.bfloat16 else "float16", what=f"B {B} row {i} step {step}")
+                for layer in caches[i]:
+                    layer.trim(1)
+        for c in caches:
+            c[0].page_manager.release()
