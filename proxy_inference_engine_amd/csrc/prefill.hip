@@ -19,6 +19,7 @@
 
 #include "decoder.hpp"
 #include "prefill_attn.hpp"
+#include "stack_types.hpp"  // rows_w16_launch
 
 int embedding_launch(const int32_t *ids, int L, const uint32_t *codes, const void *scales, const void *biases, int V, int H, int dtype,
                      void *out, const float *freqs, const DecState *state, float *rope_cs, int half, hipStream_t st, int bits);
@@ -711,17 +712,22 @@ static int linear_rows(pie_decoder *d, const void *packed, int N, int K, const u
     PIE_REQUIRE(K % 64 == 0, PIE_E_SHAPE, "prefill: a many-row Linear needs in_features % 64 == 0 (pie_set_knob(PIE_KNOB_PREFILL_MIN, 1000000) processes prompts as iterated decode steps)");
     u16 *wM = s->wM;
     bool ready = false;
-    if (keep) {
+    auto it = s->resident.find(packed);
+    if (it != s->resident.end()) wM = it->second, ready = true;
+    else if (keep && resident_budget(d) >= w16m_size(N, K)) {
         const size_t bytes = w16m_size(N, K);
-        auto it = s->resident.find(packed);
-        if (it != s->resident.end()) wM = it->second, ready = true;
-        else if (resident_budget(d) >= bytes) {
-            if (hipMalloc((void **)&wM, bytes) == hipSuccess) s->resident[packed] = wM, s->resident_left -= bytes, ++s->alloc_gen;
-            else (void)hipGetLastError(), wM = s->wM, s->resident_left = 0;  // out of memory: scratch from here on
-        }
+        if (hipMalloc((void **)&wM, bytes) == hipSuccess) s->resident[packed] = wM, s->resident_left -= bytes, ++s->alloc_gen;
+        else (void)hipGetLastError(), wM = s->wM, s->resident_left = 0;  // out of memory: scratch from here on
     }
     int rc = PIE_OK;
     if (!ready && (rc = expand_weights<T>(d, packed, N, K, wM, s->wT, st))) return rc;
+    // A few sequences' step, a few prompt rows: the streaming form, one launch without slabs or a reduce behind it, up to the rows where k_w16l_gemm's tiles are full enough.  8B layer
+    // with 8 rows, k_w16l_gemm (+ reduce) / streaming, us: q|k|v, o_proj and down 58 + 14 / 43, gate|up 55 / 39; with 32 rows 58 + 14 / 57, 55 / 42.
+    if (M <= ROWS_W16_MAX) {
+        const bool sg = act && used_act;
+        if (sg) *used_act = true;
+        return rows_w16_launch(d->cfg.dtype, wM, x, M, N, K, sg ? act : y, bias, sg, st);
+    }
     if ((rc = w4l_reserve(w16l_workspace_bytes(M, N, K)))) return rc;  // fp32 slabs of a K-split shape (few rows, narrow matrices)
     bool fused = false;  // gate|up: bias and SwiGLU in the GEMM's epilogue where the shape does not split K
     rc = w16l_gemm_launch(d->cfg.dtype, wM, x, 0, M, N, K, y, s->w4l_ws, st, bias, (act && used_act) ? act : nullptr, &fused, 0);
@@ -982,7 +988,9 @@ static int decode_batch_t(pie_decoder *d, const int32_t *tokens, const int32_t *
         if ((rc = add_rms_norm_rows<T>(s->x, s->r, next_norm, c.rms_eps, B, H, c.dtype, s->xn, st, sd.S > 1 ? w.bdown : nullptr, &sd)))
             return rc;
     }
-    if ((rc = linear_rows<T>(d, d->glob.lm_head, c.vocab, H, s->xn, B, logits, st, false, nullptr, true))) return rc;
+    // the head's 16-bit tiles stay, like the layers' (int4: its W4M tiles do): laid out anew for every step they cost more than the product (268 MB: 115 us beside 42)
+    const bool keep_head = d->mat_fmt(d->glob.lm_head) != PIE_W_INT4_G64;
+    if ((rc = linear_rows<T>(d, d->glob.lm_head, c.vocab, H, s->xn, B, logits, st, keep_head, nullptr, true))) return rc;
     return logits_tail_rows_launch(c.dtype, logits, c.vocab, B, s->tail_stats, logprobs, next_tokens, st);
 }
 
@@ -1081,7 +1089,8 @@ static int prefill_varlen_t(pie_decoder *d, const int32_t *ids, const int32_t *r
     // the normalised last row of every prompt -> lm_head -> tail
     hipLaunchKernelGGL(k_gather_rows, dim3(S), dim3(256), 0, st, (const uint4 *)s->xn, last_rows, H / 8, (uint4 *)s->r);
     PIE_LAUNCH_CHECK();
-    if ((rc = linear_rows<T>(d, d->glob.lm_head, c.vocab, H, s->r, S, logits, st, false, nullptr, true))) return rc;
+    const bool keep_head = d->mat_fmt(d->glob.lm_head) != PIE_W_INT4_G64;  // (as in a step)
+    if ((rc = linear_rows<T>(d, d->glob.lm_head, c.vocab, H, s->r, S, logits, st, keep_head, nullptr, true))) return rc;
     return logits_tail_rows_launch(c.dtype, logits, c.vocab, S, s->tail_stats, logprobs, next_tokens, st);
 }
 
