@@ -443,6 +443,7 @@ int pie_decoder_set_state(pie_decoder *d, int offset, int token, void *stream) {
     PIE_REQUIRE(token < d->embed_vocab(), PIE_E_ARG, "pie_decoder_set_state: token id out of range");
     hipLaunchKernelGGL(k_set_state, dim3(1), dim3(1), 0, (hipStream_t)stream, d->state, offset, token, -1);
     PIE_LAUNCH_CHECK();
+    d->pos_hint = offset;
     return PIE_OK;
 }
 
@@ -459,6 +460,7 @@ int pie_decoder_step(pie_decoder *d, int flags, void *stream) {
     if (rc) return rc;
     hipStream_t st = (hipStream_t)stream;
     const bool with_logits = (flags & PIE_STEP_LOGITS) != 0;
+    ++d->pos_hint;
     if (!(flags & PIE_STEP_GRAPH)) return enqueue_step(d, &d->state->token, with_logits, d->logits, st);
     const int gi = with_logits ? 1 : 0;
     if (d->graph[gi] && d->graph_fused[gi] && !fuse_attn(d, 0)) drop_graphs(d);  // fusion was withdrawn (knob, a third live decoder): capture the two-launch form
@@ -525,6 +527,7 @@ int pie_decoder_prefill(pie_decoder *d, const int32_t *ids, int L, void *logits_
     // int8 pages: the batched prompt path of ONE sequence reads and writes T pages; such prompts run as decode steps here (fresh prompts go
     // through pie_decoder_prefill_batch, which the Python host does)
     if (L >= prefill_min_rows() && !d->tp() && !(d->kv_i8 && d->block_table)) return prefill_batched(d, ids, nullptr, L, logits_all, st);  // MLX's qmm regime
+    d->pos_hint += L;
     for (int l = 0; l < L; ++l) {
         const bool last = l == L - 1;
         u16 *dst = logits_all ? (u16 *)logits_all + (size_t)l * d->cfg.vocab : d->logits;
@@ -548,6 +551,7 @@ int pie_decoder_prefill_embeds(pie_decoder *d, const void *embeds, int L, void *
     // run as decode steps, each with its row copied into the residual stream instead of an embedding launch (no RoPE table either: the
     // q|k|v epilogue computes its own angles).  The greedy token the tail leaves in the device-side state is that of the last row.
     const size_t row_bytes = 2 * (size_t)d->cfg.hidden;
+    d->pos_hint += L;
     d->row_is_h = true;
     for (int l = 0; l < L && !rc; ++l) {
         u16 *dst = logits_all ? (u16 *)logits_all + (size_t)l * d->cfg.vocab : d->logits;

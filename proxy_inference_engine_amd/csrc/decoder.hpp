@@ -37,6 +37,7 @@ struct pie_decoder {
     // prologue merges (one launch less); long ones spread up to 32 splits per kv-head over the chip and merge them with
     // k_attn_combine -- the scoring loop is VALU work, 4 splits leave it on 32 CUs (83 us per layer at T = 8k, measured).
     bool combine = false;
+    int pos_hint = 0;  // what the caller last set state.pos to plus the tokens forwarded since (the device's number decides; this one plans launches)
     int merge_max_cap = 1024, kv_cap = 0;  // measured: merged wins at capacities 512 and 1024, the combine launch from 2048
     bool kv_i8 = false;  // PIE_OPT_KV_I8: the page slabs hold int8 pages (paged_i8.hip)
     bool row_is_h = false;  // the step's input row already sits in `h` (a row of caller-made embeddings): no embedding launch, no RoPE table

@@ -383,6 +383,8 @@ struct PrefillScratch {
     unsigned batch_gen = 0, warm_gen = 0;
     void *w4l_ws = nullptr;   // fp32 partial tiles of the K-split prompt GEMM (w4m_gemm.hip)
     size_t w4l_ws_bytes = 0;
+    float *attn_part = nullptr;  // sums of prompt attention split along the keys (prefill_attn.hpp)
+    size_t attn_part_bytes = 0;
     int resident_mode = -1;   // -1: budget not fixed yet
     size_t resident_left = 0; // bytes still available for resident copies
 };
@@ -412,8 +414,10 @@ static void scratch_release(PrefillScratch *s) {  // the chunk buffers; resident
     const size_t left = s->resident_left;
     void *keep_ws = s->w4l_ws;
     const size_t keep_wsb = s->w4l_ws_bytes;
+    float *keep_part = s->attn_part;
+    const size_t keep_pb = s->attn_part_bytes;
     *s = PrefillScratch();
-    s->w4l_ws = keep_ws, s->w4l_ws_bytes = keep_wsb;
+    s->w4l_ws = keep_ws, s->w4l_ws_bytes = keep_wsb, s->attn_part = keep_part, s->attn_part_bytes = keep_pb;
     s->resident = std::move(keep), s->resident_w4m = std::move(keep_m), s->resident_mode = mode, s->resident_left = left;
     s->tail_stats = keep_ts, s->tail_entries = keep_tr, s->alloc_gen = gen;
 }
@@ -425,6 +429,7 @@ void prefill_free(pie_decoder *d) {
     for (auto &kv : d->prefill->resident_w4m) (void)hipFree(kv.second);
     if (d->prefill->tail_stats) (void)hipFree(d->prefill->tail_stats);
     if (d->prefill->w4l_ws) (void)hipFree(d->prefill->w4l_ws);
+    if (d->prefill->attn_part) (void)hipFree(d->prefill->attn_part);
     if (d->prefill->batch_graph) (void)hipGraphExecDestroy(d->prefill->batch_graph);
     delete d->prefill;
     d->prefill = nullptr;
@@ -479,6 +484,23 @@ static int scratch_reserve(pie_decoder *d, int rows, size_t w_elems, int splits)
     }
 #undef PF_ALLOC
     return PIE_OK;
+}
+
+// A prompt's attention split along the keys where that pays and its sums have room (before: keys cached in front of the first row)
+static void split_attn(pie_decoder *d, PrefillAttnArgs &a, int before) {
+    PrefillScratch *s = d->prefill;
+    const int splits = prefill_attn_splits(a.M, before, a.Hkv);
+    const size_t need = prefill_attn_part_bytes(a.M, a.Hq, d->cfg.head_dim, splits);
+    if (need > s->attn_part_bytes) {
+        if (s->attn_part) (void)hipFree(s->attn_part);
+        s->attn_part = nullptr, s->attn_part_bytes = 0, ++s->alloc_gen;
+        if (hipMalloc((void **)&s->attn_part, need) != hipSuccess) {
+            (void)hipGetLastError();
+            return;
+        }
+        s->attn_part_bytes = need;
+    }
+    if (splits > 1) a.splits = splits, a.part = s->attn_part;
 }
 
 // ---------------------------------------------------------------- the batched forward
@@ -774,7 +796,7 @@ static int prefill_t(pie_decoder *d, const int32_t *ids, const void *embeds, int
             if ((rc = linear_rows<T>(d, w.wqkv, NQKV, H, s->xn, M, s->qkv, st, true, w.bqkv, false, nullptr, &roped, &re, w.bqkv ? nullptr : &sq)))
                 return rc;
             if (!roped) {
-                const unsigned row_wgs = sq.S > 1 ? (M < 512 ? 4u : 1u) : 1u;  // few rows of slabs: four workgroups per row (256 tokens: 6.03 vs 6.20 ms; from 512 rows no difference)
+                const unsigned row_wgs = M < (sq.S > 1 ? 512 : 128) ? 4u : 1u;  // few rows: four workgroups per row (slabs, 256 tokens: 6.03 vs 6.20 ms; from 512 rows no difference)
                 decltype(&k_rope_append_rows<T, false, false>) rope_k = &k_rope_append_rows<T, false, false>;
                 if (sq.S > 1) rope_k = &k_rope_append_rows<T, true, false>;
                 hipLaunchKernelGGL(rope_k, dim3(M, row_wgs), dim3(256), 0, st, s->qkv, NQKV, d->glob.rope_freqs, d->state, d->kv_table, li,
@@ -787,6 +809,7 @@ static int prefill_t(pie_decoder *d, const int32_t *ids, const void *embeds, int
                 pa.q = s->q, pa.kv_table = d->kv_table, pa.layer = li, pa.n_layers = c.n_layers, pa.state = d->state;
                 pa.block_table = d->block_table, pa.n_pages = d->n_pages;
                 pa.M = M, pa.Hq = c.n_heads, pa.Hkv = c.n_kv_heads, pa.scale = 1.0f / sqrtf((float)D), pa.out = s->attn;
+                split_attn(d, pa, d->pos_hint + c0);
                 if ((rc = prefill_attn_launch_t<T>(pa, D, st))) return rc;
             } else {  // PIE_KNOB_PREFILL_ATTN_VALU = 1: the VALU decode kernel, one query row per blockIdx.z (cross-check for the tests)
                 AttnArgs a = {};
@@ -957,7 +980,7 @@ static int decode_batch_t(pie_decoder *d, const int32_t *tokens, const int32_t *
             decltype(&k_rope_append_rows<T, false, false>) rope_k = &k_rope_append_rows<T, false, false>;
             if (sq.S > 1) rope_k = d->kv_i8 ? &k_rope_append_rows<T, true, true> : &k_rope_append_rows<T, true, false>;
             else if (d->kv_i8) rope_k = &k_rope_append_rows<T, false, true>;
-            hipLaunchKernelGGL(rope_k, dim3(B, sq.S > 1 ? 4u : 1u), dim3(256), 0, st, s->qkv, NQKV, d->glob.rope_freqs, nullptr, nullptr, li, c.n_layers,
+            hipLaunchKernelGGL(rope_k, dim3(B, sq.S > 1 || B < 128 ? 4u : 1u), dim3(256), 0, st, s->qkv, NQKV, d->glob.rope_freqs, nullptr, nullptr, li, c.n_layers,
                                c.n_heads, c.n_kv_heads, D, c.rope_traditional, s->q, block_tables, n_pages, s->rope_cs, ctx_len, max_blocks, (u16 *)slabs[li],
                                (const int *)nullptr, (u16 *)nullptr, (u16 *)nullptr, sq.part, sq.S, sq.MN, i8pb);
             PIE_LAUNCH_CHECK();
@@ -1064,6 +1087,7 @@ static int prefill_varlen_t(pie_decoder *d, const int32_t *ids, const int32_t *r
             ca.k = (const u16 *)slabs[li], ca.v = (const u16 *)slabs[li] + (size_t)c.n_kv_heads * PIE_PAGE_TOKENS * D;
             ca.offset = ch[2], ca.cap = PIE_PAGE_TOKENS, ca.block_table = block_tables + (size_t)ch[3] * max_blocks, ca.n_pages = n_pages;
             ca.M = ch[1], ca.Hq = c.n_heads, ca.Hkv = c.n_kv_heads, ca.scale = pa.scale;
+            split_attn(d, ca, ch[2]);
             if ((rc = prefill_attn_launch_t<T>(ca, D, st))) return rc;
         }
         W4lSlabs so, sd;  // K-split products handed to their consumers as fp32 slabs (as in the single-prompt path)
@@ -1218,5 +1242,7 @@ extern "C" int pie_decoder_step_batch(pie_decoder *d, const int32_t *tokens, con
 int prefill_batched(pie_decoder *d, const int32_t *ids, const void *embeds, int L, void *logits_all, hipStream_t st) {
     const int rep = d->cfg.n_heads / d->cfg.n_kv_heads;
     PIE_REQUIRE(rep >= 1 && rep <= 8, PIE_E_SHAPE, "prefill: n_heads / n_kv_heads must be between 1 and 8");
-    return d->cfg.dtype == PIE_BF16 ? prefill_t<BF16>(d, ids, embeds, L, logits_all, st) : prefill_t<F16>(d, ids, embeds, L, logits_all, st);
+    const int rc = d->cfg.dtype == PIE_BF16 ? prefill_t<BF16>(d, ids, embeds, L, logits_all, st) : prefill_t<F16>(d, ids, embeds, L, logits_all, st);
+    d->pos_hint += L;
+    return rc;
 }

@@ -6,16 +6,20 @@
 // whole prefill beyond ~1k tokens.  Here one workgroup owns (32 query rows) x (one kv-head group); wave w owns q-head
 // g*REP + w, so a staged K/V block serves all q-heads of the group.
 //
-// Per 32-key block, per wave (v_mfma_f32_32x32x16, fp32 accumulators):
-//   S^T[key, row]  = K . Q^T        8 MFMAs;  A = K rows from the LDS image (ds_read_b128), B = Q fragments kept in VGPRs.
+// Per block of 64 keys (32 where fewer than four waves share it), per wave (v_mfma_f32_32x32x16, fp32 accumulators):
+//   S^T[key, row]  = K . Q^T        2 x 8 MFMAs, two chains side by side;  A = K rows from the LDS image (ds_read_b128), B = Q fragments kept in VGPRs.
 //                                   Orientation chosen so the softmax reduction runs over REGISTERS (keys), not lanes,
 //                                   and so P^T is directly the B operand of the next product (no lane movement);
-//   online softmax in fp32, base 2 (one v_exp_f32 per score), running max / sum per query row = per lane pair;
+//   online softmax in fp32, base 2 (one fma and one v_exp_f32 per score; a block that every row sees whole -- all but a tile's last ones -- takes no mask),
+//                                   running max / sum per query row = per lane pair;
 //   O^T[dim, row] += V^T . P^T      A = V^T via ds_read_b64_tr_b16 (hardware transpose of the row-major V image),
-//                                   B = P^T split into hi + lo halves of T (2 x 8 MFMAs): P keeps ~16 mantissa bits, the
+//                                   B = P^T split into hi + lo halves of T (2 x 16 MFMAs, four chains): P keeps ~16 mantissa bits, the
 //                                   "fp32 until one rounding" contract of the fused kernel within 2^-17.
-// K/V blocks are fetched to registers one block ahead and written to a 16 KB swizzled LDS image (the guide's dual-use
-// layout (b): conflict-free for both the row reads and the transposed reads).
+// K/V blocks are fetched to registers one block ahead and written to one of two swizzled LDS images (the guide's dual-use
+// layout (b): conflict-free for both the row reads and the transposed reads): one barrier per block.
+// What bounds it: the vector instructions between the products, and, while few workgroups run, one block's chain of latencies.  Blocks of 32 keys masked element by element, two barriers
+// and 25 instead of 12 instructions per pair of scores took, for 32 / 8 heads of 128: 4096 rows 303 us (now 227 = 0.9 PFLOP/s with the split P), 1024 rows 60 (38), 509 rows 30 (22),
+// 37 rows behind 900 cached ones 54 (35; with the keys split 18).
 #pragma once
 #include "attention.hpp"
 #include "common.hpp"
@@ -42,6 +46,8 @@ struct PrefillAttnArgs {
     const int *seg_lo, *seg_hi;
     const int *block_table;              // paged KV (nullable, decoder only): kv_table holds the layers' slab K / V bases; key t
     int n_pages;                         //   lives in page block_table[t / 64] (each [Hkv, 64, D]) at row t % 64
+    int splits;                          // SPLIT instantiation: workgroups along the keys (gridDim.y); their partial sums meet in k_prefill_combine
+    float *part;                         //   [M, Hq, splits] x {[D] weighted sums}, then [M, Hq, splits] x {running max, sum}
 };
 
 template <class T> struct MfmaT;
@@ -55,6 +61,15 @@ template <> struct MfmaT<F16> {
         return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b), c, 0, 0, 0);
     }
 };
+
+// two fp32 -> one packed pair of T in a single v_cvt_pk
+template <class T>
+__device__ __forceinline__ u32 pa_pack2(float lo, float hi) {
+    typedef float f2_t __attribute__((ext_vector_type(2)));
+    typedef typename std::conditional<std::is_same<T, F16>::value, _Float16, __bf16>::type e_t;
+    typedef e_t e2_t __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(u32, __builtin_convertvector((f2_t){lo, hi}, e2_t));
+}
 
 // byte offset of 16-byte chunk `ch` (0 .. D/8-1) of row `row` (0..31) in a [32][D x 16-bit] LDS tile: the guide's dual-use
 // swizzle (b) for 256-byte rows; for D = 64 the same XOR folded to the row's 8 chunks (a bijection inside the row, which is
@@ -75,12 +90,14 @@ __device__ __forceinline__ int pa_off(int row, int ch) {
 // QT: 32-row query tiles per workgroup (1 or 2).  With QT = 2 the workgroup has 2*REP waves -- waves [0, REP) own the first
 // tile, [REP, 2 REP) the second -- and one staged K/V block serves 64 query rows: half the L2 -> LDS traffic and barriers per
 // unit of work, at the same number of waves per CU (one 8-wave workgroup instead of two 4-wave ones for REP = 4).
-template <class T, int D, int REP, int QT, bool SEG = false>
-__global__ void __launch_bounds__(REP * QT * 64) k_prefill_attn(const PrefillAttnArgs a) {
-    constexpr int BK = 32, NT = REP * QT * 64, CH = D / 8, KS = D / 16, DT = D / 32;  // chunks per row, k-steps of Q.K^T, 32-dim output tiles
+// SPLIT: blockIdx.y takes its share of the tile's key blocks and leaves its sums to k_prefill_combine (prefill_attn_splits says when).
+template <class T, int D, int REP, int QT, bool SEG = false, bool SPLIT = false>
+__global__ void __launch_bounds__(REP * QT * 64, 2) k_prefill_attn(const PrefillAttnArgs a) {
+    constexpr int NT = REP * QT * 64, NB = NT >= 256 ? 2 : 1, BK = 32 * NB;  // keys per block: 64 where enough threads share their loads
+    constexpr int CH = D / 8, KS = D / 16, DT = D / 32;                      // chunks per row, k-steps of Q.K^T, 32-dim output tiles
     constexpr int BM = 32 * QT;
     constexpr int CPT = (BK * CH + NT - 1) / NT;                                   // 16-byte chunks per thread and tile
-    __shared__ __attribute__((aligned(16))) char k_lds[BK * 2 * D], v_lds[BK * 2 * D];
+    __shared__ __attribute__((aligned(16))) char kv_lds[2][2][BK * 2 * D];         // [block parity][K, V]
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int c = lane & 31, h = lane >> 5;
     // XCD-aware tile mapping: workgroups go round-robin over the 8 XCDs by linear id, so the kv-head group is the FASTEST
@@ -89,7 +106,7 @@ __global__ void __launch_bounds__(REP * QT * 64) k_prefill_attn(const PrefillAtt
     const int g = (int)blockIdx.x % a.Hkv, tile = (int)blockIdx.x / a.Hkv;
     const int wg_r0 = ((a.M + BM - 1) / BM - 1 - tile) * BM;                  // first query row of the workgroup
     const int r0 = wg_r0 + 32 * (wave / REP), hq = g * REP + wave % REP;     // this wave's 32-row tile and q-head
-    // paged KV: a key block (BK = 32 rows) never straddles a 64-row page, so its page is one scalar table lookup per fetch;
+    // paged KV: a key block (BK = 32 or 64 rows) never straddles a 64-row page, so its page is one scalar table lookup per fetch;
     // the contiguous case is the same code with one "page" of `cap` rows (mask keeps every row bit, page offset 0)
     const bool paged = a.block_table != nullptr;
     const int pos0 = a.state ? a.state->pos : a.offset, cap = paged ? 64 : a.state ? a.state->cap : a.cap;
@@ -99,8 +116,17 @@ __global__ void __launch_bounds__(REP * QT * 64) k_prefill_attn(const PrefillAtt
     // last / first key any row of this tile attends (segment bounds are non-decreasing in the row index)
     // (bounds clamped to the buffer: a bad segment table must not become a wild address)
     const int t_last = SEG ? max(min(a.seg_hi[r_last], a.cap), 1) - 1 : pos0 + r_last;
-    const int b_first = SEG ? min(max(a.seg_lo[wg_r0], 0), t_last) / BK : 0;
-    const int n_blocks = t_last / BK + 1;
+    const int n_all = t_last / BK + 1, share = SPLIT ? (n_all + a.splits - 1) / a.splits : n_all;  // (key blocks of the tile, and of this workgroup)
+    const int b_first = SEG ? min(max(a.seg_lo[wg_r0], 0), t_last) / BK : SPLIT ? (int)blockIdx.y * share : 0;
+    const int n_blocks = SPLIT ? min(b_first + share, n_all) : n_all;
+    if constexpr (SPLIT)
+        if (b_first >= n_blocks) {  // fewer blocks than workgroups: an empty share weighs nothing
+            if (h == 0 && r0 + c < a.M) {
+                float *ml = a.part + (size_t)a.M * a.Hq * a.splits * D + (((size_t)(r0 + c) * a.Hq + hq) * a.splits + blockIdx.y) * 2;
+                ml[0] = ATTN_NEG, ml[1] = 0.0f;
+            }
+            return;
+        }
     const u16 *kbase = (a.state ? reinterpret_cast<const u16 *>(a.kv_table[a.layer]) : a.k) + (size_t)g * cap * D;
     const u16 *vbase = (a.state ? reinterpret_cast<const u16 *>(a.kv_table[a.n_layers + a.layer]) : a.v) + (size_t)g * cap * D;
 
@@ -121,8 +147,8 @@ __global__ void __launch_bounds__(REP * QT * 64) k_prefill_attn(const PrefillAtt
     if constexpr (i < CPT) {                                                                     \
         const int x = threadIdx.x + i * NT;                                                      \
         if (x < BK * CH) {                                                                       \
-            *reinterpret_cast<uint4 *>(k_lds + pa_off<D>(x / CH, x % CH)) = kr;                  \
-            *reinterpret_cast<uint4 *>(v_lds + pa_off<D>(x / CH, x % CH)) = vr;                  \
+            *reinterpret_cast<uint4 *>(kv_lds[buf][0] + pa_off<D>(x / CH, x % CH)) = kr;                  \
+            *reinterpret_cast<uint4 *>(kv_lds[buf][1] + pa_off<D>(x / CH, x % CH)) = vr;                  \
         }                                                                                        \
     }
     auto fetch = [&](int b) {
@@ -130,7 +156,7 @@ __global__ void __launch_bounds__(REP * QT * 64) k_prefill_attn(const PrefillAtt
         PA_FETCH1(0, k0, v0) PA_FETCH1(1, k1, v1) PA_FETCH1(2, k2, v2) PA_FETCH1(3, k3, v3)
         PA_FETCH1(4, k4, v4) PA_FETCH1(5, k5, v5) PA_FETCH1(6, k6, v6) PA_FETCH1(7, k7, v7)
     };
-    auto publish = [&]() {
+    auto publish = [&](int buf) {
         PA_PUBLISH1(0, k0, v0) PA_PUBLISH1(1, k1, v1) PA_PUBLISH1(2, k2, v2) PA_PUBLISH1(3, k3, v3)
         PA_PUBLISH1(4, k4, v4) PA_PUBLISH1(5, k5, v5) PA_PUBLISH1(6, k6, v6) PA_PUBLISH1(7, k7, v7)
     };
@@ -147,7 +173,13 @@ __global__ void __launch_bounds__(REP * QT * 64) k_prefill_attn(const PrefillAtt
     // last (and, SEG, first) key this lane's query row attends (rows past M are padding: never stored)
     const int t_row = SEG ? a.seg_hi[qrow] - 1 : pos0 + r0 + c;
     const int t_lo = SEG ? a.seg_lo[qrow] : 0;
-    const float sl2 = a.scale * ATTN_LOG2E;
+    const float sl2 = fabsf(a.scale) * ATTN_LOG2E;  // (a negative scale turns the sign of the queries: the largest score is the largest product)
+    if (a.scale < 0.0f)
+#pragma unroll
+        for (int s = 0; s < KS; ++s) qf[s].x ^= 0x80008000u, qf[s].y ^= 0x80008000u, qf[s].z ^= 0x80008000u, qf[s].w ^= 0x80008000u;
+    // keys that every row of this wave sees: such blocks need no mask (bounds are non-decreasing in the row)
+    const int wr0 = r0 < a.M ? r0 : a.M - 1, wr1 = r0 + 31 < a.M ? r0 + 31 : a.M - 1;
+    const int all_hi = SEG ? a.seg_hi[wr0] - 1 : pos0 + wr0, all_lo = SEG ? a.seg_lo[wr1] : 0;
 
     f32x16_t oacc[DT];
 #pragma unroll
@@ -160,31 +192,44 @@ __global__ void __launch_bounds__(REP * QT * 64) k_prefill_attn(const PrefillAtt
     // 4-row x 16-column block; lane i of the group receives column i, row q in element q
     const int grp = lane >> 4, tq = (lane & 15) >> 2, tp = lane & 3;
 
+    publish(0);
+    __syncthreads();
     for (int b = b_first; b < n_blocks; ++b) {
-        __syncthreads();  // every wave is done reading the previous block's image
-        publish();
-        __syncthreads();
+        const int buf = (b - b_first) & 1;
+        const char *k_lds = kv_lds[buf][0], *v_lds = kv_lds[buf][1];
         if (b + 1 < n_blocks) fetch(b + 1);
 
-        // S^T = K . Q^T : rows = keys (registers), cols = query rows (lanes)
-        f32x16_t sacc;
+        // S^T = K . Q^T : rows = keys (registers), cols = query rows (lanes); the blocks of 32 keys are independent chains
+        f32x16_t sc[NB];
 #pragma unroll
-        for (int i = 0; i < 16; ++i) sacc[i] = 0.0f;
+        for (int n = 0; n < NB; ++n)
 #pragma unroll
-        for (int s = 0; s < KS; ++s) {
-            const uint4 kf = *reinterpret_cast<const uint4 *>(k_lds + pa_off<D>(c, 2 * s + h));
-            sacc = MfmaT<T>::run(kf, qf[s], sacc);
-        }
-        // online softmax over keys: register i <-> key t0 + (i & 3) + 8 (i >> 2) + 4 h
+            for (int i = 0; i < 16; ++i) sc[n][i] = 0.0f;
+#pragma unroll
+        for (int s = 0; s < KS; ++s)
+#pragma unroll
+            for (int n = 0; n < NB; ++n) {
+                const uint4 kf = *reinterpret_cast<const uint4 *>(k_lds + pa_off<D>(32 * n + c, 2 * s + h));
+                sc[n] = MfmaT<T>::run(kf, qf[s], sc[n]);
+            }
+        // online softmax over keys: register i of block n <-> key t0 + 32 n + (i & 3) + 8 (i >> 2) + 4 h
         const int t0 = b * BK;
-        float sc[16], mloc = ATTN_NEG;
+        const bool masked = t0 + BK - 1 > all_hi || (SEG && t0 < all_lo);  // uniform for the wave
+        auto sees = [&](int n, int i) {
+            const int t = t0 + 32 * n + (i & 3) + 8 * (i >> 2) + 4 * h;
+            return t <= t_row && (!SEG || t >= t_lo);
+        };
+        if (masked)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const int t = t0 + (i & 3) + 8 * (i >> 2) + 4 * h;
-            sc[i] = (t <= t_row && (!SEG || t >= t_lo)) ? sacc[i] * sl2 : ATTN_NEG;
-            mloc = fmaxf(mloc, sc[i]);
-        }
-        mloc = xor32_max(mloc);  // the other 16 keys of the block live in the partner lane
+            for (int n = 0; n < NB; ++n)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) sc[n][i] = sees(n, i) ? sc[n][i] : ATTN_NEG;
+        float mloc = ATTN_NEG;
+#pragma unroll
+        for (int n = 0; n < NB; ++n)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) mloc = fmaxf(mloc, sc[n][i]);
+        mloc = xor32_max(mloc) * sl2;  // the other half of the block's keys lives in the partner lane
         const float m_new = fmaxf(m_run, mloc);
         if (m_new > m_run) {  // rare after the first blocks
             const float alpha = attn_exp2(m_run - m_new);
@@ -195,22 +240,25 @@ __global__ void __launch_bounds__(REP * QT * 64) k_prefill_attn(const PrefillAtt
                 for (int i = 0; i < 16; ++i) oacc[dt][i] *= alpha;
             m_run = m_new;
         }
-        u32 phi[8], plo[8];
+        u32 phi[NB][8], plo[NB][8];
 #pragma unroll
-        for (int i = 0; i < 16; i += 2) {
-            const int ta = t0 + (i & 3) + 8 * (i >> 2) + 4 * h;
-            const float pa = (ta <= t_row && (!SEG || ta >= t_lo)) ? attn_exp2(sc[i] - m_run) : 0.0f;
-            const float pb = (ta + 1 <= t_row && (!SEG || ta + 1 >= t_lo)) ? attn_exp2(sc[i + 1] - m_run) : 0.0f;
-            l_run += pa + pb;
-            const float ha = round_T<T>(pa), hb = round_T<T>(pb);
-            phi[i >> 1] = pack2<T>(ha, hb);
-            plo[i >> 1] = pack2<T>(pa - ha, pb - hb);
-        }
+        for (int n = 0; n < NB; ++n)
+#pragma unroll
+            for (int i = 0; i < 16; i += 2) {
+                float pa = attn_exp2(fmaf(sc[n][i], sl2, -m_run)), pb = attn_exp2(fmaf(sc[n][i + 1], sl2, -m_run));
+                if (masked) pa = sees(n, i) ? pa : 0.0f, pb = sees(n, i + 1) ? pb : 0.0f;
+                l_run += pa + pb;
+                const u32 hi = pa_pack2<T>(pa, pb);
+                phi[n][i >> 1] = hi;
+                plo[n][i >> 1] = pa_pack2<T>(pa - lo_f32<T>(hi), pb - hi_f32<T>(hi));
+            }
         // O^T += V^T . P^T : k-step s covers keys 16 s .. 16 s + 15 in the operand order 16 s + 8 (j >> 2) + 4 h + (j & 3)
 #pragma unroll
-        for (int s = 0; s < 2; ++s) {
-            const uint4 bh = make_uint4(phi[4 * s], phi[4 * s + 1], phi[4 * s + 2], phi[4 * s + 3]);
-            const uint4 bl = make_uint4(plo[4 * s], plo[4 * s + 1], plo[4 * s + 2], plo[4 * s + 3]);
+        for (int s = 0; s < 2 * NB; ++s) {
+            const int n = s >> 1, e = 4 * (s & 1);
+            const uint4 bh = make_uint4(phi[n][e], phi[n][e + 1], phi[n][e + 2], phi[n][e + 3]);
+            const uint4 bl = make_uint4(plo[n][e], plo[n][e + 1], plo[n][e + 2], plo[n][e + 3]);
+            uint4 vf[DT];
 #pragma unroll
             for (int dt = 0; dt < DT; ++dt) {
                 const int ch = 4 * dt + 2 * (grp & 1) + (tp >> 1);
@@ -219,11 +267,31 @@ __global__ void __launch_bounds__(REP * QT * 64) k_prefill_attn(const PrefillAtt
                 const v4i16_t hi4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
                     (__attribute__((address_space(3))) v4i16_t *)(v_lds + pa_off<D>(16 * s + 8 + 4 * h + tq, ch) + 8 * (tp & 1)));
                 const uint2 a0 = __builtin_bit_cast(uint2, lo4), a1 = __builtin_bit_cast(uint2, hi4);
-                const uint4 vf = make_uint4(a0.x, a0.y, a1.x, a1.y);
-                oacc[dt] = MfmaT<T>::run(vf, bh, oacc[dt]);
-                oacc[dt] = MfmaT<T>::run(vf, bl, oacc[dt]);
+                vf[dt] = make_uint4(a0.x, a0.y, a1.x, a1.y);
             }
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt) oacc[dt] = MfmaT<T>::run(vf[dt], bh, oacc[dt]);
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt) oacc[dt] = MfmaT<T>::run(vf[dt], bl, oacc[dt]);
         }
+        if (b + 1 < n_blocks) {  // (the other image: its last readers passed the barrier in front of this block)
+            publish(buf ^ 1);
+            __syncthreads();
+        }
+    }
+    if constexpr (SPLIT) {
+        const float l = xor32_sum(l_run);
+        if (r0 + c < a.M) {
+            const size_t at = ((size_t)(r0 + c) * a.Hq + hq) * a.splits + blockIdx.y;
+            float *acc = a.part + at * D, *ml = a.part + (size_t)a.M * a.Hq * a.splits * D + at * 2;
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+                    *reinterpret_cast<float4 *>(acc + 32 * dt + 8 * k + 4 * h) = make_float4(oacc[dt][4 * k], oacc[dt][4 * k + 1], oacc[dt][4 * k + 2], oacc[dt][4 * k + 3]);
+            if (h == 0) ml[0] = m_run, ml[1] = l;
+        }
+        return;
     }
     // normalise: the pair (lane, lane ^ 32) shares the query row and holds the two halves of the row sum
     const float inv = 1.0f / xor32_sum(l_run);
@@ -240,9 +308,61 @@ __global__ void __launch_bounds__(REP * QT * 64) k_prefill_attn(const PrefillAtt
     }
 }
 
+// The shares of a (row, head) merged in their order, one thread per four numbers: sum_z w_z acc_z / sum_z w_z l_z, w_z = exp2(m_z - max m).
+template <class T, int D>
+__global__ void __launch_bounds__(256) k_prefill_combine(const float *part, int splits, int pairs, u16 *out) {
+    const int i = blockIdx.x * 256 + threadIdx.x, pair = i / (D / 4), d = i % (D / 4) * 4;
+    if (pair >= pairs) return;
+    const float *acc = part + (size_t)pair * splits * D + d, *ml = part + (size_t)pairs * splits * D + (size_t)pair * splits * 2;
+    float m = ATTN_NEG, l = 0.0f;
+    for (int z = 0; z < splits; ++z) m = fmaxf(m, ml[2 * z]);
+    float4 o = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+#pragma unroll 4
+    for (int z = 0; z < splits; ++z) {
+        const float w = attn_exp2(ml[2 * z] - m), lz = ml[2 * z + 1];
+        if (lz == 0.0f) continue;  // nothing seen: its sums were never written
+        const float4 v = *reinterpret_cast<const float4 *>(acc + (size_t)z * D);
+        l = fmaf(w, lz, l), o.x = fmaf(w, v.x, o.x), o.y = fmaf(w, v.y, o.y), o.z = fmaf(w, v.z, o.z), o.w = fmaf(w, v.w, o.w);
+    }
+    const float inv = 1.0f / l;
+    *reinterpret_cast<uint2 *>(out + (size_t)pair * D + d) = make_uint2(pack2<T>(o.x * inv, o.y * inv), pack2<T>(o.z * inv, o.w * inv));
+}
+
+// Workgroups along the keys: rows behind a long cached prefix are few tiles with many blocks each (37 rows: 16 workgroups of 30 blocks).  `before`: keys in front of the first row.  Every
+// share costs its sums (4 D bytes per row and head, twice): at least two blocks of 64 keys per share up to 64 rows, three beyond, up to two workgroups per CU.  us, 1 / 2 / 4 / 8 shares:
+// 8 rows behind 500: 20 / 14 / 12 / 12; 37 behind 900: 35 / 24 / 18 / 17; 100: 38 / 26 / 21 / 23; 200: 41 / 30 / 26 / 30; 509: 53 / 42 / 40 / 46; 32 behind 4000: 131 / 73 / 42 / 29 (16: 28).
+// Rows of a fresh prompt see half of the blocks on average and gain nothing (509 rows: 22 / 26).
+static inline int prefill_attn_splits(int M, int before, int Hkv) {
+    const int shares = before / 64 / (M <= 64 ? 2 : 3), room = 512 / ((M + 31) / 32 * Hkv);
+    const int s = shares < room ? shares : room;
+    return s < 2 ? 1 : s > 16 ? 16 : s;
+}
+static inline size_t prefill_attn_part_bytes(int M, int Hq, int D, int splits) { return splits > 1 ? (size_t)M * Hq * splits * (D + 2) * sizeof(float) : 0; }
+
 template <class T, int D>
 static int prefill_attn_launch_d(const PrefillAttnArgs &a, hipStream_t st) {
     const int rep = a.Hq / a.Hkv;
+    if (a.splits > 1) {
+        const dim3 grid((a.M + 31) / 32 * a.Hkv, a.splits);
+#define PA_SPLIT(R) hipLaunchKernelGGL((k_prefill_attn<T, D, R, 1, false, true>), grid, dim3(R * 64), 0, st, a); break
+        switch (rep) {
+            case 1: PA_SPLIT(1);
+            case 2: PA_SPLIT(2);
+            case 3: PA_SPLIT(3);
+            case 4: PA_SPLIT(4);
+            case 5: PA_SPLIT(5);
+            case 6: PA_SPLIT(6);
+            case 7: PA_SPLIT(7);
+            case 8: PA_SPLIT(8);
+            default: return pie::fail(PIE_E_SHAPE, "prefill attention: n_heads / n_kv_heads must be between 1 and 8");
+        }
+#undef PA_SPLIT
+        PIE_LAUNCH_CHECK();
+        const int pairs = a.M * a.Hq;
+        hipLaunchKernelGGL((k_prefill_combine<T, D>), dim3((unsigned)(((size_t)pairs * (D / 4) + 255) / 256)), dim3(256), 0, st, a.part, a.splits, pairs, a.out);
+        PIE_LAUNCH_CHECK();
+        return PIE_OK;
+    }
     const int qt = pie_knob(PIE_KNOB_PREFILL_QT);  // test knob: 1 forces one 32-row query tile per workgroup, 2 forces two wherever they fit
     // 2 tiles need 2*rep <= 8 waves of up to 256 registers, and only pay while the halved grid still fills the 256 CUs
     // (8B model: 4096 tokens 54.9 -> 53.9 ms, 8000 tokens 126.3 -> 125.0 ms; at 1024 tokens it would idle half the chip)

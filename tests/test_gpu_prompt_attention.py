@@ -1,0 +1,63 @@
+"""Prompt attention: the op at the edges of its blocks and masks against float64, and the form split along the keys (rows behind a cached prefix) against the row-by-row kernel."""
+import numpy as np
+import pytest
+import torch
+
+from proxy_inference_engine_amd import _ffi, hip_ops as ops
+
+pytestmark = pytest.mark.gpu
+EPS = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("heads", [(2, 2), (3, 1), (4, 2), (8, 2), (5, 1), (8, 1)], ids=str)
+@pytest.mark.parametrize("D", [64, 128])
+def test_causal_rows_against_float64(heads, D, dtype):
+    """Lengths and offsets around the blocks of 32 and 64 keys and the tiles of 32 rows; a scale of either sign, and zero (plain means).  The result is rounded once: one ulp of the largest
+    output (values are at most about 4, sums of weights 1, P is split to 16 bits)."""
+    Hq, Hkv = heads
+    g = torch.Generator().manual_seed(D + Hq)
+    for L, off, scale in ((2, 0, 0.3), (31, 1, 0.3), (32, 32, -0.3), (33, 63, 0.3), (64, 0, 0.0), (65, 64, -0.2), (97, 130, 0.3), (150, 7, 0.2)):
+        T = off + L
+        q, k, v = (torch.randn(1, n, m, D, generator=g).to(dtype) for n, m in ((Hq, L), (Hkv, T), (Hkv, T)))
+        got = ops.scaled_dot_product_attention(q.cuda(), k.cuda(), v.cuda(), scale, mask="causal").double().cpu()
+        r = Hq // Hkv
+        s = q.double() @ k.double().repeat_interleave(r, 1).transpose(-1, -2).contiguous() * scale
+        s = s.masked_fill(torch.arange(T)[None] > torch.arange(L)[:, None] + off, -torch.inf)
+        want = torch.softmax(s, -1) @ v.double().repeat_interleave(r, 1)
+        assert (got - want).abs().max() <= EPS[dtype] * want.abs().max(), (L, off, scale)
+
+
+@pytest.mark.parametrize("paged", [False, True], ids=["contiguous", "paged"])
+@pytest.mark.parametrize("geometry", [(8, 2, 64), (8, 1, 128), (2, 2, 128)], ids=str)
+def test_rows_behind_a_prefix_split_along_the_keys(geometry, paged):
+    """700 cached tokens: 2 to 5 shares, the last ones empty or partly masked.  Two layers against the kernel that takes one query row at a time: both keep fp32 until one rounding, so four ulps of the
+    largest logit as everywhere in this suite."""
+    from _util import assert_vec_close
+    from proxy_inference_engine_amd.models.llama import Model, ModelArgs
+    from proxy_inference_engine_amd.models.utils import synthetic_checkpoint
+    Hq, Hkv, D = geometry
+    cfg = {"model_type": "llama", "hidden_size": 256, "num_hidden_layers": 2, "intermediate_size": 512, "num_attention_heads": Hq, "num_key_value_heads": Hkv, "head_dim": D, "vocab_size": 320,
+           "rms_norm_eps": 1e-5, "tie_word_embeddings": False, "quantization": None}
+    w = synthetic_checkpoint(cfg, seed=5)
+    for n in list(w):
+        if "q_proj" in n or "k_proj" in n:
+            w[n] = w[n] * 6   # sharp attention: single keys decide
+    m = Model(ModelArgs(**cfg), w)
+    if paged:
+        m.enable_paged_kv(num_pages=40, max_blocks=20)
+    ids = torch.from_numpy(np.random.default_rng(1).integers(0, 320, 920).astype(np.int32)).cuda()
+    cache = m.make_cache()
+    m.step(ids[:700], cache)
+    for n in (6, 32, 33, 65, 130, 200):
+        got = []
+        for valu in (1, None):
+            _ffi.set_knob("prefill_attn_valu", valu)
+            try:
+                got.append(m(ids[None, 700:700 + n], cache=cache).float().cpu().numpy()[0])
+            finally:
+                _ffi.set_knob("prefill_attn_valu", None)
+            for layer in cache:
+                layer.trim(n)
+        for i in range(n):
+            assert_vec_close(got[1][i], got[0][i], "bfloat16", what=f"{n} rows, row {i}")
