@@ -263,22 +263,23 @@ __global__ void __launch_bounds__(512) k_rows_w16m(const RowsArgs a) {
 
 // Rows that share a pass, x through LDS.  k_rows_w16m fetches every 16 B of x into the lanes that multiply it, 16 scattered runs of 64 B per instruction, for every 16 or 32 features
 // again: from 8 rows on that, and no longer the weights, is what the time goes to ([28672, 4096]: 37 us with 1 row, 41 / 52 / 58 / 88 with 8 / 16 / 32 / 64; profile and counts agree, the
-// matrix cores idle).  Here a workgroup of eight waves takes 16 NN features and all of K in chunks of 256 U columns: the chunk's rows come in as whole lines, once per workgroup
-// (registers, then one of two LDS buffers; rows padded by 16 B, conflict-free both ways), each wave multiplies every eighth 32-column step by weights that it streams two chunks ahead.
-// Loads go by descriptors whose bounds drop what lies behind a row, a matrix or K (zeros), so no load has a branch around it.  Two workgroups share a CU (launch bounds: 128 registers),
+// matrix cores idle).  Here a workgroup of WV (eight) waves takes 16 NN features and all of K in chunks of 32 WV U columns: the chunk's rows come in as whole lines, once per workgroup
+// (registers, then one of two LDS buffers; rows padded by 16 B, conflict-free both ways), each wave multiplies every WV-th 32-column step by weights that it streams two chunks ahead.
+// Loads go by descriptors whose bounds drop what lies behind a row, a matrix or K (zeros), so no load has a branch around it.  Two workgroups of eight waves share a CU (launch bounds: 128 registers),
 // one loads while the other finishes.  Sixteen features per wave and step re-read x most (NN = 1), four blocks least: NN follows from how many workgroups are left (rows_gemm_launch).
-// [28672, 4096] with 8 / 16 / 32 / 64 rows: 39 / 40 / 42 / 64 us = 6.0 / 5.8 / 5.6 / 3.7 TB/s; 60 active experts of [2816, 2048] with 3 rows each: 131 -> 110 us (6.3 TB/s).
-template <class E, int NT, int NN, int U>
-__global__ void __launch_bounds__(512, 4) k_rows_lds(const RowsArgs a) {
-    constexpr int C = 256 * U, LD = C + 8, ST = 20;                // columns of x per chunk; u16 per LDS row; floats per line of the reduction image
-    constexpr int PR = C / 8, RP = 512 / PR, XJ = 16 * NT / RP;    // 16-byte pieces per row of a chunk; rows that 512 threads fetch at once; pieces per thread
-    constexpr size_t X_BYTES = (size_t)2 * 16 * NT * LD * 2, RED_BYTES = (size_t)8 * NN * NT * 16 * ST * 4;
-    static_assert(512 % PR == 0 && 16 * NT % RP == 0, "whole rows per round of loads");
+// [28672, 4096] with 8 / 16 / 32 / 64 rows: 39 / 40 / 42 / 64 us = 6.0 / 5.8 / 5.6 / 3.7 TB/s.  Experts have fewer bytes per workgroup, and workgroups of four waves (WV) fill the gaps that
+// others leave better: 60 active ones of [2816, 2048] with 3 rows each 131 (k_rows_w16m) -> 110 (eight waves) -> 103 us (6.7 TB/s), of [2048, 1408] 90 -> 58 -> 53 us.
+template <class E, int NT, int NN, int U, int WV = 8>
+__global__ void __launch_bounds__(64 * WV, 4) k_rows_lds(const RowsArgs a) {
+    constexpr int C = 32 * WV * U, LD = C + 8, ST = 20;            // columns of x per chunk; u16 per LDS row; floats per line of the reduction image
+    constexpr int PR = C / 8, RP = 64 * WV / PR, XJ = 16 * NT / RP;  // 16-byte pieces per row of a chunk; rows that all threads fetch at once; pieces per thread
+    constexpr size_t X_BYTES = (size_t)2 * 16 * NT * LD * 2, RED_BYTES = (size_t)WV * NN * NT * 16 * ST * 4;
+    static_assert(64 * WV % PR == 0 && 16 * NT % RP == 0, "whole rows per round of loads");
     __shared__ __attribute__((aligned(16))) char s_mem[X_BYTES > RED_BYTES ? X_BYTES : RED_BYTES];
     u16 *s_x = (u16 *)s_mem;
     float *s_red = (float *)s_mem;
     if constexpr (__is_same(E, ElemBF16))
-        if (rows_ride<ElemBF16, 512>(a, s_red)) return;
+        if (rows_ride<ElemBF16, 64 * WV>(a, s_red)) return;
     int bx = blockIdx.x, by = blockIdx.y;
     if (a.flat_tiles < 0) {  // a list, workgroup after workgroup
         for (by = 0;; ++by) {
@@ -286,14 +287,16 @@ __global__ void __launch_bounds__(512, 4) k_rows_lds(const RowsArgs a) {
             if (bx < t) break;
             bx -= t;
         }
-    } else if (a.flat_tiles > 0) {  // experts, then the shared one
-        by = min(bx / a.flat_tiles, a.flat_batches), bx -= by * a.flat_tiles;
+    } else if (a.flat_tiles > 0) {  // the shared expert (it has all rows, and the longest workgroups), then the others
+        const int first = a.shared.w ? (a.shared.N + 16 * NN - 1) / (16 * NN) : 0;
+        if (bx < first) by = a.flat_batches;
+        else by = (bx - first) / a.flat_tiles, bx = (bx - first) % a.flat_tiles;
     }
     RowsWork k;
     if (!rows_select(a, k, by, a.flat_tiles > 0 ? a.flat_batches : (int)gridDim.y - 1)) return;
     if (bx * NN * 16 >= k.N) return;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), c = lane & 15, kq = lane >> 4;
-    const int t16 = bx * NN, groups = (k.K + 63) >> 6, steps = 2 * groups, K8 = (k.K + 7) & ~7, iters = (steps + 8 * U - 1) / (8 * U);
+    const int t16 = bx * NN, groups = (k.K + 63) >> 6, steps = 2 * groups, K8 = (k.K + 7) & ~7, iters = (steps + WV * U - 1) / (WV * U);
     const int w_tiles = min(((k.N + 31) >> 5) - (t16 >> 1), (NN + 1) / 2);  // 32-row tiles of this workgroup: a matrix ends with a whole tile
     const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>(k.w + (size_t)(t16 >> 1) * groups * 4096), 0, w_tiles * groups * 4096, 0x00020000);
     const unsigned wlane = (kq >> 1) * 1024 + ((kq & 1) * 32 + c) * 16 + (t16 & 1) * 256;
@@ -322,7 +325,7 @@ __global__ void __launch_bounds__(512, 4) k_rows_lds(const RowsArgs a) {
         auto load_w = [&](int it, mf_u32x4(&wv)[U][NN]) {
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                const int s = (it * U + u) * 8 + wave;
+                const int s = (it * U + u) * WV + wave;
 #pragma unroll
                 for (int n = 0; n < NN; ++n)  // non-temporal: a pass reads a weight once
                     wv[u][n] = __builtin_amdgcn_raw_buffer_load_b128(wr, s < steps ? wlane + (unsigned)((n >> 1) * groups * 4096 + s * 2048 + (n & 1) * 256) : NOWHERE, 0, 2);
@@ -338,7 +341,7 @@ __global__ void __launch_bounds__(512, 4) k_rows_lds(const RowsArgs a) {
             for (int u = 0; u < U; ++u) {
                 mf_u32x4 xv[NT];
 #pragma unroll
-                for (int t = 0; t < NT; ++t) xv[t] = *(const mf_u32x4 *)(s_x + (buf * 16 * NT + 16 * t + c) * LD + (8 * u + wave) * 32 + 8 * kq);
+                for (int t = 0; t < NT; ++t) xv[t] = *(const mf_u32x4 *)(s_x + (buf * 16 * NT + 16 * t + c) * LD + (WV * u + wave) * 32 + 8 * kq);
 #pragma unroll
                 for (int n = 0; n < NN; ++n)
 #pragma unroll
@@ -371,16 +374,16 @@ __global__ void __launch_bounds__(512, 4) k_rows_lds(const RowsArgs a) {
             for (int t = 0; t < NT; ++t) *(mf_f32x4 *)(s_red + (((wave * NN + n) * NT + t) * 16 + c) * ST + 4 * kq) = acc[n][t];
         __syncthreads();
         const bool paired = rows_paired(a.epi);
-        for (int id = threadIdx.x; id < NN * NT * 256; id += 512) {
+        for (int id = threadIdx.x; id < NN * NT * 256; id += 64 * WV) {
             const int nl = id & 15, ml = (id >> 4) % (16 * NT), nn = id / (256 * NT), n = (t16 + nn) * 16 + nl, m = i0 + ml;
             if (n >= k.N || m >= k.count || (paired && (nl & 1))) continue;
             const float *r = s_red + ((nn * NT + (ml >> 4)) * 16 + (ml & 15)) * ST + nl;
             float v = 0.0f, p = 0.0f;
 #pragma unroll
-            for (int q = 0; q < 8; ++q) v += r[q * NN * NT * 16 * ST];
+            for (int q = 0; q < WV; ++q) v += r[q * NN * NT * 16 * ST];
             if (paired)
 #pragma unroll
-                for (int q = 0; q < 8; ++q) p += r[q * NN * NT * 16 * ST + 1];
+                for (int q = 0; q < WV; ++q) p += r[q * NN * NT * 16 * ST + 1];
             rows_finish<E>(a, k, m, n, v, p);
         }
         __syncthreads();
@@ -418,7 +421,7 @@ __global__ void __launch_bounds__(256) k_rows_f32(const RowsArgs a) {
     if (n < k.N && m < k.count) rows_finish<ElemF32>(a, k, m, n, acc, s_v[tm][tn < 15 ? tn + 1 : 15]);
 }
 
-template <class E, int NT, int NN, int U>
+template <class E, int NT, int NN, int U, int WV = 8>
 int rows_lds_go(RowsArgs a, int n_max, int batches, hipStream_t st) {
     auto tiles = [](int n) { return (unsigned)((n + 16 * NN - 1) / (16 * NN)); };
     dim3 grid(tiles(n_max), (unsigned)(batches + rows_riders(a)), (unsigned)((a.M + 16 * NT - 1) / (16 * NT)));
@@ -429,20 +432,20 @@ int rows_lds_go(RowsArgs a, int n_max, int batches, hipStream_t st) {
         a.flat_tiles = -1, grid.x = 0, grid.y = 1;
         for (int i = 0; i < a.n_mats; ++i) grid.x += tiles(a.mats[i].N);
     }
-    hipLaunchKernelGGL((k_rows_lds<E, NT, NN, U>), grid, dim3(512), 0, st, a);
+    hipLaunchKernelGGL((k_rows_lds<E, NT, NN, U, WV>), grid, dim3(64 * WV), 0, st, a);
     PIE_LAUNCH_CHECK();
     return PIE_OK;
 }
 
 // Which of the two, and how many features a workgroup of k_rows_lds takes; blocks: 16-feature blocks of the whole launch.  Measured, us (k_rows_w16m / NN = 1 / 2 / 4; x in LDS wins from
 // about 5 rows on, where the rows are long enough for eight waves to share them):
-//   [28672, 4096]: 8 rows 41 / 43 / 39 / 39, 32 rows 58 / 59 / 48 / 42    [11264, 2048]: 8 rows 11.1 / 14.1 / 12.8 / 12.1, 32 rows 17.5 / 17.2 / 15.9 / 13.9
+//   [28672, 4096]: 8 rows 41 / 43 / 39 / 39, 32 rows 58 / 59 / 48 / 42    [11264, 2048]: 8 rows 11.1 / 14.1 / 13.1 / 11.4, 32 rows 17.5 / 17.2 / 15.9 / 13.9    [32768, 4096]: 8 rows 47 / 49 / 42 / 45
 //   [6144, 4096]: 8 rows 13.6 / 14.6 / 12.3 / 17.5, 32 rows 17.0 / 19.1 / 15.2 / 20.3    [4096, 14336]: 8 rows 23.6 / 22.3 / 27.9 / 46.9, 32 rows 41 / 30 / 37 / 54
 // Fewer blocks than that leave CUs without a workgroup; more than 32 rows of x per CU take the room of the fourth block.
 template <class E>
 int rows_lds_pick(const RowsArgs &a, int n_max, long blocks, int batches, hipStream_t st) {
-    if (a.M <= 16 || a.active)
-        return blocks < 320 ? rows_lds_go<E, 1, 1, 4>(a, n_max, batches, st) : a.active ? rows_lds_go<E, 1, 4, 1>(a, n_max, batches, st) : rows_lds_go<E, 1, 2, 2>(a, n_max, batches, st);
+    if (a.active) return rows_lds_go<E, 1, 2, 2, 4>(a, n_max, batches, st);
+    if (a.M <= 16) return blocks < 320 ? rows_lds_go<E, 1, 1, 4>(a, n_max, batches, st) : rows_lds_go<E, 1, 2, 2>(a, n_max, batches, st);
     if (a.M <= 32)
         return blocks < 320 ? rows_lds_go<E, 2, 1, 2>(a, n_max, batches, st) : blocks < 640 ? rows_lds_go<E, 2, 2, 2>(a, n_max, batches, st) : rows_lds_go<E, 2, 4, 1>(a, n_max, batches, st);
     return blocks < 320 ? rows_lds_go<E, 4, 1, 1>(a, n_max, batches, st) : rows_lds_go<E, 4, 2, 1>(a, n_max, batches, st);
