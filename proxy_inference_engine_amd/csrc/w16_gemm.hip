@@ -67,12 +67,12 @@ int w16m_from_w16s_launch(const void *w16s, int N, int K, void *w16m, hipStream_
     return PIE_OK;
 }
 
-// Decomposition: row tile (64 / 128 / 256 rows), strips per wave (workgroup = 128 or 256 columns) and K split, by a small cost model
-// calibrated on tools/w16_bench sweep (8B and vision-tower shapes, 64 .. 4096 rows): a K step of a (32 mb) x (128 sw) tile costs
-// t(mb, sw) us -- larger tiles are cheaper per MFMA (0.125 us per 32 x 32 block pair for 64 x 128, 0.09 for 256 x 256) but quantise worse --
-// less when part of the chip idles (the large tiles are power-bound: the clock rises); workgroups run in rounds of 256; few rows
-// are bound by the weight stream (~5.5 TB/s); a launch costs ~4 us of ramp, prologue and epilogue; a K split writes and re-reads its fp32
-// slabs and launches the reduce.
+// Decomposition: row tile (64 / 128 / 256 rows), strips per wave (workgroup = 128 or 256 columns) and K split, by a small cost model fitted to every such choice on 143 products of 40 to
+// 3000 rows (8B, 1B and vision-tower widths, weights from HBM: a model's other matrices have passed through the caches since a matrix was last used; fitted to weights that still lie in
+// the 256 MB behind the L2s it preferred plans up to 1.4 times slower).  A K step of a (32 mb) x (128 sw) tile costs t(mb, sw) us -- larger tiles are cheaper per MFMA but quantise worse --
+// and no less than its weights take from beyond the caches, which the row tiles of a column share; workgroups run in rounds of 256, counted on the XCD that has most; all weights come
+// once through HBM (5.6 TB/s); a launch costs 5.8 us of ramp, prologue and epilogue; a K split writes and re-reads its fp32 slabs and launches the reduce.  Over those products its choices
+// take 1.4 % longer than the best ones (those of the model before: 6.2 %); [4096, 14336]: 64 / 128 / 509 / 1024 rows 40 / 40 / 91 / 123 -> 34 / 34 / 67 / 113 us.
 struct W16Plan {
     int mb, sw, S;
 };
@@ -88,29 +88,31 @@ static int w16_even_splits(int groups, int S) {  // the largest split count <= S
         S = s2;
     }
 }
-static W16Plan w16_plan(int M, int N, int K, bool no_split = false) {
+static bool w16_narrow(int tn, int tm) { return tn < 8 && tm >= 8; }  // column tiles that would leave XCDs without work: row tiles go over the XCDs instead
+// no_split: one pass over K; two: two strips per wave
+static W16Plan w16_plan(int M, int N, int K, bool no_split = false, bool two = false) {
     const int groups = (K + 63) / 64;
     if (g_w16_plan_override[0]) return {g_w16_plan_override[0], g_w16_plan_override[1], w16_even_splits(groups, g_w16_plan_override[2])};
     const int mb_max = M <= 64 ? 2 : (M <= 128 ? 4 : 8);
     W16Plan best = {mb_max, 2, 1};
     double best_us = 1e30;
-    // t(mb, sw) = light + (full - light) * load: one partial round of workgroups runs at a higher clock than sustained full rounds
-    static const double t_light[4][3] = {{0, 0, 0}, {0, 0.25, 0.42}, {0, 0.31, 0.60}, {0, 0.50, 1.45}};  // [log2 mb][sw]
-    static const double t_rows[4][3] = {{0, 0, 0}, {0, 0.25, 0.45}, {0, 0.48, 0.80}, {0, 0.83, 1.45}};
-    static const double t_tall[4][3] = {{0, 0, 0}, {0, 0.31, 0.53}, {0, 0.46, 0.84}, {0, 0.90, 1.45}};  // many row tiles: small tiles re-read the weights from beyond their XCD's L2
-    const double (&t_full)[4][3] = M > 512 ? t_tall : t_rows;
-    const double stream_us = 2.0 * N * (64.0 * groups) / 5.5e6;
+    // t(mb, sw) = light + (full - light) * load: one partial round of workgroups runs at a higher clock than full rounds, but waits longer for each step's loads
+    static const double t_light[4][3] = {{0, 0, 0}, {0, 0.30, 0.63}, {0, 0.43, 0.78}, {0, 0.61, 1.05}};  // [log2 mb][sw]
+    static const double t_full[4][3] = {{0, 0, 0}, {0, 0.30, 0.52}, {0, 0.45, 0.82}, {0, 0.83, 1.45}};
+    const double stream_us = 2.0 * N * (64.0 * groups) / 5.6e6;
     for (int S = 1; S <= (no_split ? 1 : 16) && (S == 1 || 8 * S <= groups); ++S)
         for (int mb = mb_max; mb >= 2; mb >>= 1)
-            for (int sw = 2; sw >= (no_split ? 2 : 1); --sw) {
-                const int wgs = ((N + 128 * sw - 1) / (128 * sw)) * ((M + 32 * mb - 1) / (32 * mb)) * S;
+            for (int sw = 2; sw >= (two ? 2 : 1); --sw) {
+                const int tn = (N + 128 * sw - 1) / (128 * sw), tm = (M + 32 * mb - 1) / (32 * mb), wgs = tn * tm * S;
+                const int most = (w16_narrow(tn, tm) ? (tm + 7) / 8 * tn : (tn + 7) / 8 * tm) * S;  // workgroups of the XCD that has most: 32 run at once
                 const int steps = ((groups + S - 1) / S + 3) & ~3;
-                const int rounds = (wgs + 255) / 256;
-                const double load = rounds > 1 ? 1.0 : (double)wgs / 256.0;
+                const double load = wgs < 256 ? (double)wgs / 256.0 : 1.0;
+                const double cold = tm < 22 ? 0.36 * sw * (1.0 - 0.047 * (tm - 1)) : 0.0;
                 const int mi = mb == 8 ? 3 : (mb == 4 ? 2 : 1);
-                double us = rounds * steps * (t_light[mi][sw] + (t_full[mi][sw] - t_light[mi][sw]) * load);
-                us = (us > stream_us ? us : stream_us) + 4.0;
-                if (S > 1) us += (double)M * N * 4.0 * (2 * S + 0.5) / 4.0e6 + 2.0;
+                const double t = t_light[mi][sw] + (t_full[mi][sw] - t_light[mi][sw]) * load;
+                double us = (most + 31) / 32 * steps * (t > cold ? t : cold);
+                us = (us > stream_us ? us : stream_us) + 5.8;
+                if (S > 1) us += (double)M * N * 4.0 * (2 * S + 0.5) / 5.1e6 + 0.6;
                 if (us < best_us) best_us = us, best = {mb, sw, S};
             }
     best.S = w16_even_splits(groups, best.S);
@@ -138,10 +140,13 @@ int w16l_gemm_launch(int dtype, const void *w16m, const void *x, int ldx, int M,
     PIE_REQUIRE(M >= 1 && N > 0 && K > 0, PIE_E_SHAPE, "16-bit GEMM: empty operand");
     PIE_REQUIRE(pie_aligned(w16m, 16) && pie_aligned(x, 16) && pie_aligned(y, 8) && (!bias || pie_aligned(bias, (N & 3) ? 2 : 8)), PIE_E_ALIGN, "16-bit GEMM: 16-byte alignment required");
     PIE_REQUIRE(dtype == PIE_BF16 || dtype == PIE_F16, PIE_E_ARG, "16-bit GEMM: dtype must be PIE_BF16 or PIE_F16");
-    // swiglu_act without `fused`: the caller has no fallback (the C ABI's fused MLP): plan without a K split, two strips per wave
-    W16Plan plan = w16_plan(M, N, K, (swiglu_act && !fused) || (N & 3));  // (the fp32 slabs of a K split are written 16 bytes at a time)
+    // One pass over K where the slabs do not fit the output: rows that are not a multiple of 16 bytes, a row stride of the caller's; and where swiglu_act comes without `fused`: the caller
+    // has no fallback (the C ABI's fused MLP).  The fused activation is built for two strips per wave: the best tile among those.
+    const bool one_pass = (swiglu_act && !fused) || (N & 3) || (!swiglu_act && ldy && ldy != N);
+    W16Plan plan = w16_plan(M, N, K, one_pass);
+    if (swiglu_act && plan.S == 1) plan = w16_plan(M, N, K, true, true);
     const bool sg = swiglu_act && plan.S == 1;
-    if (sg) plan.sw = 2;  // (the fused activation is built for two strips per wave)
+    if (sg) plan.sw = 2;  // (a developer's override)
     PIE_REQUIRE(plan.S == 1 || workspace, PIE_E_ARG, "16-bit GEMM: this shape splits K and needs its workspace");
     W16Args a = {};
     int rc = w16_zero_block(&a.zero);
@@ -150,7 +155,6 @@ int w16l_gemm_launch(int dtype, const void *w16m, const void *x, int ldx, int M,
     const int out_cols = sg ? N / 2 : N;
     if (ldy == 0 || (swiglu_act && !sg)) ldy = out_cols;  // (a declined fusion writes the packed y)
     PIE_REQUIRE(ldy >= out_cols, PIE_E_SHAPE, "16-bit GEMM: output row stride must cover the row");
-    PIE_REQUIRE(plan.S == 1 || ldy == N, PIE_E_SHAPE, "16-bit GEMM: a K-split shape writes packed rows");
     a.w16m = (const char *)w16m, a.x = (const u16 *)x, a.M = M, a.N = N, a.K = Kx, a.ldx = ldx, a.ldy = ldy;
     a.y = (u16 *)(sg ? swiglu_act : y), a.part = plan.S > 1 ? (float *)workspace : nullptr;
     a.bias = plan.S > 1 ? nullptr : (const u16 *)bias;
@@ -159,7 +163,7 @@ int w16l_gemm_launch(int dtype, const void *w16m, const void *x, int ldx, int M,
 #ifdef W16L_PROF
     a.prof = g_w16_prof;
 #endif
-    a.narrow = a.tn < 8 && a.tm >= 8;
+    a.narrow = w16_narrow(a.tn, a.tm);
     const dim3 grid((unsigned)(a.narrow ? 8 * ((a.tm + 7) / 8) * a.tn : 8 * ((a.tn + 7) / 8) * a.tm), (unsigned)plan.S);
 #define W16_GO(TT, MB_, SW_, SG_) hipLaunchKernelGGL((k_w16l_gemm<TT, MB_, SW_, SG_>), grid, dim3(256), 0, st, a)
 #define W16_SW(TT, MB_) \
@@ -209,7 +213,7 @@ int pie_linear_w16m(const void *x, int ldx, const void *w16m, const void *bias, 
     PIE_REQUIRE(dtype == PIE_BF16 || dtype == PIE_F16, PIE_E_ARG, "pie_linear_w16m: dtype must be PIE_BF16 or PIE_F16");
     PIE_REQUIRE(pie_aligned(x, 16) && pie_aligned(w16m, 16) && pie_aligned(y, 16) && (!bias || pie_aligned(bias, (N & 3) ? 2 : 8)), PIE_E_ALIGN,
                 "pie_linear_w16m: 16-byte alignment required");
-    const size_t need = swiglu ? 0 : w16l_workspace_bytes(M, N, K);
+    const size_t need = swiglu || (ldy && ldy != N) ? 0 : w16l_workspace_bytes(M, N, K);
     PIE_REQUIRE(need == 0 || (workspace && workspace_bytes >= need), PIE_E_ARG, "pie_linear_w16m: workspace smaller than pie_linear_w16m_workspace(M, N, K)");
     return w16l_gemm_launch(dtype, w16m, x, ldx, M, N, K, swiglu ? nullptr : y, workspace, (hipStream_t)stream, bias, swiglu ? y : nullptr, nullptr, ldy);
 }
