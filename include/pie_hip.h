@@ -454,6 +454,8 @@ int pie_page_add_ref(pie_page_pool *pool, uint32_t page_id);
 int pie_page_ref_count(const pie_page_pool *pool, uint32_t page_id, uint32_t *count);
 int pie_page_num_tokens(const pie_page_pool *pool, uint32_t page_id, size_t *n);
 int pie_page_set_num_tokens(pie_page_pool *pool, uint32_t page_id, size_t n);
+/* The counts of a sequence's n pages in order, `tokens` in all: 64 each, then the rest, then 0. */
+int pie_page_mark_tokens(pie_page_pool *pool, const uint32_t *page_ids, size_t n, size_t tokens);
 int pie_page_ptrs(const pie_page_pool *pool, uint32_t page_id, void **k, void **v);
 size_t pie_page_i8_bytes(int n_kv_heads, int head_dim);
 int pie_page_scale_ptrs(const pie_page_pool *pool, uint32_t page_id, void **k_scale, void **v_scale);

@@ -25,7 +25,7 @@ KERNELS = {"embed": 0, "qkv": 1, "attn": 2, "o_proj": 3, "gate_up": 4, "down": 5
 BASE_EXPORTS = [
     "pie_hello", "pie_version", "pie_last_error", "pie_device_info", "pie_set_knob", "pie_get_knob",
     "pie_page_pool_slab_bytes", "pie_page_pool_create", "pie_page_pool_destroy", "pie_page_pool_size", "pie_page_pool_num_free",
-    "pie_page_alloc", "pie_page_free", "pie_page_add_ref", "pie_page_ref_count", "pie_page_num_tokens", "pie_page_set_num_tokens",
+    "pie_page_alloc", "pie_page_free", "pie_page_add_ref", "pie_page_ref_count", "pie_page_num_tokens", "pie_page_set_num_tokens", "pie_page_mark_tokens",
     "pie_page_ptrs", "pie_page_i8_bytes", "pie_page_scale_ptrs",
     "pie_w16m_bytes", "pie_repack_w16m", "pie_linear_w16m_workspace", "pie_linear_w16m",
     "pie_stack_weight_bytes", "pie_stack_pack_weight", "pie_stack_create", "pie_stack_destroy", "pie_stack_set_layer", "pie_stack_page_row",
@@ -158,6 +158,7 @@ def base() -> C.CDLL:
     lib.pie_page_ref_count.argtypes = [C.c_void_p, C.c_uint32, C.POINTER(C.c_uint32)]
     lib.pie_page_num_tokens.argtypes = [C.c_void_p, C.c_uint32, C.POINTER(C.c_size_t)]
     lib.pie_page_set_num_tokens.argtypes = [C.c_void_p, C.c_uint32, C.c_size_t]
+    lib.pie_page_mark_tokens.argtypes = [C.c_void_p, C.POINTER(C.c_uint32), C.c_size_t, C.c_size_t]
     lib.pie_stack_weight_bytes.argtypes = [C.c_int, C.c_int, C.c_int]
     lib.pie_stack_pack_weight.argtypes = [C.c_void_p, C.c_int, C.c_int, C.c_int, C.c_void_p, C.c_void_p]
     lib.pie_stack_create.argtypes = [C.POINTER(pie_stack_config), C.POINTER(C.c_void_p)]
@@ -214,6 +215,7 @@ def load() -> C.CDLL:
     lib.pie_page_ref_count.argtypes = [C.c_void_p, C.c_uint32, C.POINTER(C.c_uint32)]
     lib.pie_page_num_tokens.argtypes = [C.c_void_p, C.c_uint32, C.POINTER(C.c_size_t)]
     lib.pie_page_set_num_tokens.argtypes = [C.c_void_p, C.c_uint32, C.c_size_t]
+    lib.pie_page_mark_tokens.argtypes = [C.c_void_p, C.POINTER(C.c_uint32), C.c_size_t, C.c_size_t]
     lib.pie_paged_attn_workspace_bytes.restype = C.c_size_t
     lib.pie_paged_attn_decode.argtypes = [C.c_void_p, C.c_void_p, C.c_size_t, C.c_void_p, C.c_int, C.c_void_p] + [C.c_int] * 4 + [
         C.c_float, C.c_int, C.c_void_p, C.c_void_p, C.c_void_p]

@@ -203,8 +203,8 @@ class PagedSequence:
         self._mark_tokens()
 
     def _mark_tokens(self) -> None:
-        for j, pid in enumerate(self.pages):  # KVPage.num_tokens (page.hpp:69,100-103)
-            self.allocator.get_page(pid).set_num_tokens(max(0, min(TOKEN_CAPACITY_PER_PAGE, self.offset - j * TOKEN_CAPACITY_PER_PAGE)))
+        n = len(self.pages)  # KVPage.num_tokens (page.hpp:69,100-103), all pages in one native call: every step of every sequence comes through here
+        _f.check(_f.base().pie_page_mark_tokens(self.allocator._h, (C.c_uint32 * n)(*self.pages), n, self.offset))
 
     def truncate(self, length: int) -> None:
         """Keeps the first `length` positions and returns the pages behind them to the pool."""

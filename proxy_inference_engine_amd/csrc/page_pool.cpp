@@ -177,6 +177,16 @@ int pie_page_set_num_tokens(pie_page_pool *p, uint32_t id, size_t n) {
     return PIE_OK;
 }
 
+int pie_page_mark_tokens(pie_page_pool *p, const uint32_t *ids, size_t n, size_t tokens) {
+    POOL_REQUIRE(p && (ids || n == 0), PIE_E_ARG, "pie_page_mark_tokens: null pointer");
+    for (size_t j = 0; j < n; ++j) {
+        if (int rc = check_id(p, ids[j], "pie_page_mark_tokens")) return rc;
+        const size_t before = j * PIE_PAGE_TOKENS;
+        p->pages[ids[j]].num_tokens.store(tokens <= before ? 0 : tokens - before < PIE_PAGE_TOKENS ? tokens - before : PIE_PAGE_TOKENS, std::memory_order_release);
+    }
+    return PIE_OK;
+}
+
 int pie_page_ptrs(const pie_page_pool *p, uint32_t id, void **k, void **v) {
     if (int rc = check_id(p, id, "pie_page_ptrs")) return rc;
     POOL_REQUIRE(k && v, PIE_E_ARG, "pie_page_ptrs: null pointer");

@@ -572,7 +572,7 @@ class Model:
                    "tokens": torch.empty(B, dtype=torch.int32, device=self.device), "ctx": torch.empty(B, dtype=torch.int32, device=self.device),
                    "logits": torch.empty((B, V), dtype=self.dtype, device=self.device),
                    "logprobs": torch.empty((B, V), dtype=torch.float32, device=self.device),
-                   "next": torch.empty(B, dtype=torch.int32, device=self.device), "key": None}
+                   "next": torch.empty(B, dtype=torch.int32, device=self.device), "key": None, "at": None}
             self._batch_bufs.pop(B, None)
             while len(self._batch_bufs) >= 4:  # a serving loop revisits few batch sizes: keep the 4 most recent sets (each [B, V] fp32 + T)
                 self._batch_bufs.pop(next(iter(self._batch_bufs)))
@@ -585,7 +585,13 @@ class Model:
             buf["table"].copy_(table)
             buf["key"] = key
         buf["tokens"].copy_(tokens)
-        buf["ctx"].copy_(torch.tensor([s.offset + 1 for s in seqs], dtype=torch.int32))
+        # the lengths stay on the device from step to step: a copy from the host would wait until the previous step is done and leave the GPU idle while this one is prepared
+        at = [s.offset + 1 for s in seqs]
+        if buf["at"] == [n - 1 for n in at]:
+            buf["ctx"].add_(1)
+        elif buf["at"] != at:
+            buf["ctx"].copy_(torch.tensor(at, dtype=torch.int32))
+        buf["at"] = at
         n = len(self.layers)
         slabs = (C.c_void_p * n)(*[a.slab[i].data_ptr() for i in range(n)])
         self._match_page_format(a)

@@ -303,3 +303,21 @@ def test_int8_page_geometry_and_oracle_quantiser():
     s = np.full((7, 3), 1 / 32, np.float16)
     err = np.abs(po.kv_i8_dequantize(po.kv_i8_quantize(y, s), s) - y)
     assert err[np.abs(y) <= 127 / 32].max() <= 0.5 / 32 + 1e-7                                                          # half a step inside the range
+
+
+def test_marking_a_sequence_of_pages_in_one_call():
+    """pie_page_mark_tokens: whole pages first, then the rest, then nothing; an id beyond the pool is refused."""
+    import ctypes as C
+
+    from proxy_inference_engine_amd import _ffi
+    alloc = make_allocator(5)
+    ids = [alloc.allocate_page() for _ in range(4)]
+
+    def mark(pages, tokens):
+        _ffi.check(_ffi.base().pie_page_mark_tokens(alloc._h, (C.c_uint32 * len(pages))(*pages), len(pages), tokens))
+    for tokens in (0, 1, 63, 64, 65, 128, 200, 255, 256, 300):
+        mark(ids, tokens)
+        assert [alloc.get_page(p).num_tokens() for p in ids] == [max(0, min(64, tokens - 64 * j)) for j in range(4)]
+    mark([], 7)
+    with pytest.raises(IndexError):
+        mark([ids[0], 5], 70)
