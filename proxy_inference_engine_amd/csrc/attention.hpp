@@ -66,11 +66,9 @@ struct AttnArgs {
     const int *block_table, *ctx_len;
     int bt_stride, n_pages;
     unsigned *prof;   // developer build (-DPIE_ATTN_PROF): stamps of workgroup (0, 0, 0), words 2..9 of the decoder's scratch; nullptr otherwise
-    // Infinity-Cache warm-up riding on the CUs this launch leaves idle (decoder only): workgroups with blockIdx.y >= splits stream o_proj's
-    // weights with plain coalesced loads and discard them, so that launch's 9.4 MB then come from the cache.  Re-decided in round 4
-    // ("x 18.7 attention traffic for 0.3 %"): same box, three alternating repetitions -- with it 1.198-1.201 ms per 8B step,
-    // without it 1.211-1.217 (+1.3 %), with an XCD-matched one-dword-per-line L2 touch instead 1.222-1.245.  The bytes leave HBM once either
-    // way (FETCH_SIZE counts Infinity-Cache hits: o_proj's own fetch is then served on-die); what moves is WHEN they leave it.
+    // Infinity-Cache warm-up riding on the CUs this launch leaves idle (decoder only, PIE_KNOB_ATTN_WARM_MAX_MB; off by default, the figures
+    // are at ATTN_WARM_DEFAULT_MB): workgroups with blockIdx.y >= splits stream o_proj's weights with plain coalesced loads and discard them,
+    // so that launch's bytes then come from the cache.  They leave HBM once either way; what moves is WHEN they leave it.
     const char *pf_ptr;
     unsigned long long pf_bytes;
     int pf_rows;      // extra blockIdx.y rows doing this (0 = none)

@@ -68,10 +68,12 @@ static void drop_graphs(pie_decoder *d) {
         }
 }
 
-// The attention launch's idle CUs warm at most this much of o_proj's stream: 9.4 MB (the 8B int4 matrix, all of it) is what the launch's ~5 us
-// can carry; uncapped, the 33.5 MB of the dense 8B o_proj stretched the launch itself: dense 2.81 -> 3.00 ms per step, int8 (17.8 MB) 1.74 -> 1.81
-// (cap 10: 2.81 / 1.75; off: 2.81 / 1.74; int4: 1.186-1.191 with, 1.190 without)
-constexpr int ATTN_WARM_DEFAULT_MB = 10;
+// The attention launch's idle CUs can warm the Infinity Cache with this much of o_proj's stream (attention.hpp); none by default.  The reads compete
+// with q|k|v's own last units when attention runs behind the seam of that launch, and hold the launch's end where it does not.  ms per step
+// with 10 MB / 3 MB / none -- 32 / 8 heads of 128, 32 layers: int4 1.175 / 1.138 / 1.140, int4 pages 1.178 / 1.151 / 1.153, int8 1.729 / 1.669 / 1.673,
+// dense 2.786 / 2.720 / 2.729; four int4 layers 0.348 / 0.334 / 0.329; attention launched alone: Llama-3.2-3B 0.826 / 0.814 / 0.808, 28 heads of 128
+// 1.239 / 1.251 / 1.243, four dense f16 layers of 32 heads of 64 0.350 / 0.351 / 0.343.
+constexpr int ATTN_WARM_DEFAULT_MB = 0;
 // Workgroups with equal blockIdx.x % 8 share an XCD (tools/pilot_probe, every grid size and history): what the fused q|k|v + attention launch
 // relies on, so it is checked once per process on the real dispatcher (a partitioned device with one XCD passes trivially).
 __global__ void k_xcc_probe(unsigned *out) {
@@ -121,7 +123,7 @@ static AttnArgs attn_args(pie_decoder *d, int li) {
     a.block_table = d->block_table, a.n_pages = d->n_pages, a.bt_stride = 0;
     a.nt_kv = d->combine;  // long-context plan (capacity > 1024): the cache no longer survives in the Infinity Cache between steps
     a.prof = d->pf_sink;
-    // the CUs this launch leaves idle warm the Infinity Cache with o_proj's weights (attention.hpp: +1.3 % on the step)
+    // PIE_KNOB_ATTN_WARM_MAX_MB: the CUs this launch leaves idle warm the Infinity Cache with o_proj's weights
     if (!d->combine) {
         const int f = d->mat_fmt(w.wo);
         a.pf_rows = (256 - c.n_kv_heads * d->splits) / c.n_kv_heads;

@@ -276,8 +276,8 @@ __device__ __forceinline__ float lane_value(float v, int lane) {  // wave-unifor
 // L2, every workgroup adds 1 to its XCD's counter (an atomic performed AT that L2: no release fence; the counter only grows, 32 per
 // launch), and the group's attention workgroups poll it with sc1 loads and then run k_attn_decode's body (no acquire fence: the CU's L1
 // was invalidated at launch and has not seen these lines).  tools/seam_probe: 0.12 us from the last arrival to the release, 0.96 us until 32 KB
-// of the group's fresh data are read -- against 3.9 us for a dependent launch.  The other 28 workgroups of the XCD warm the Infinity Cache
-// with o_proj's weights (what the attention launch's idle workgroups did).  Same rows, same units, same order: bit-identical to two launches.
+// of the group's fresh data are read -- against 3.9 us for a dependent launch.  The other workgroups of the XCD leave (or, under
+// PIE_KNOB_ATTN_WARM_MAX_MB, warm the Infinity Cache with o_proj's weights).  Same rows, same units, same order: bit-identical to two launches.
 template <class T, int PRO, int EPI, int NPT, int ABL = 0, int FMT = FMT_W4S, int FUSE = 0>
 __global__ void __launch_bounds__(GEMV_WAVES * 64, 4) k_w4s_gemv(const GemvArgs a) {
 #if defined(PIE_GEMV_PROF) && PIE_GEMV_PROF == 3
