@@ -111,6 +111,8 @@ __device__ __forceinline__ uint4 attn_load_row(const u16 *p) {
 struct AttnNoSeam {
     __device__ __forceinline__ void operator()() const {}
 };
+template <class SEAM>
+struct attn_seam_gives_rows : std::false_type {};  // the seam leaves q (s_q [REP][D]) and the new position's K and V rows (s_kv [2][D]) in LDS
 // q0: the first of the REP query heads scored here (the kernel: g * REP, all heads of the kv group; the fused caller: ONE head of group g per
 // workgroup -- a head's online softmax never looks at another head, so the grouping does not change a bit).
 template <class T, int D, int REP, bool PAGED, bool NTKV, int WAVES, class SEAM = AttnNoSeam>
@@ -215,7 +217,9 @@ __device__ __forceinline__ void attn_decode_body(const AttnArgs &a, const int g,
         for (int d = 0; d < DA; ++d) {
             const int t = first + d * NSUB * TPW + ts;
             if (on && t == Ttot - 1 && t < t_end) {
-                if constexpr (PAGED) {
+                if constexpr (attn_seam_gives_rows<SEAM>::value) {
+                    kq[d] = *reinterpret_cast<const uint4 *>(seam.s_kv + dc * 8), vq[d] = *reinterpret_cast<const uint4 *>(seam.s_kv + D + dc * 8);
+                } else if constexpr (PAGED) {
                     const size_t off = (size_t)page_of(d) * page_elems + (size_t)(t & 63) * D;
                     kq[d] = attn_load_row<NTKV>(kbase + off), vq[d] = attn_load_row<NTKV>(vbase + off);
                 } else {
@@ -228,7 +232,9 @@ __device__ __forceinline__ void attn_decode_body(const AttnArgs &a, const int g,
     u32 qr[REP][4];
 #pragma unroll
     for (int h = 0; h < REP; ++h) {
-        uint4 qv = *reinterpret_cast<const uint4 *>(a.q + ((size_t)row * a.Hq + q0 + h) * D + dc * 8);
+        uint4 qv;
+        if constexpr (attn_seam_gives_rows<SEAM>::value) qv = *reinterpret_cast<const uint4 *>(seam.s_q + h * D + dc * 8);
+        else qv = *reinterpret_cast<const uint4 *>(a.q + ((size_t)row * a.Hq + q0 + h) * D + dc * 8);
         qr[h][0] = qv.x, qr[h][1] = qv.y, qr[h][2] = qv.z, qr[h][3] = qv.w;
     }
     float m[REP], l[REP], acc[REP][8];
@@ -404,6 +410,94 @@ __global__ void __launch_bounds__(WAVES * 64) k_attn_decode(const AttnArgs a) {
     attn_decode_body<T, D, REP, PAGED, NTKV, WAVES>(a, g, split, (int)blockIdx.z, g * REP);
 }
 
+// V = float2 / float4: one thread's NV vectors at element offsets off[]; the slabs are fetched BATCH at a time (all BATCH x NV loads in flight
+// before the first add -- a plain loop over the slabs waits out one memory latency per slab: 15 us instead of 5 for a 64-row o_proj
+// consumer) and added strictly in slab order.
+template <class V, int NV, int BATCH = 4>
+__device__ __forceinline__ void slab_sum(const float *part, int S, size_t MN, const size_t (&off)[NV], V (&acc)[NV]) {
+#pragma unroll
+    for (int v = 0; v < NV; ++v) acc[v] = *reinterpret_cast<const V *>(part + off[v]);
+    for (int z = 1; z < S; z += BATCH) {
+        V b[BATCH][NV];
+#pragma unroll
+        for (int u = 0; u < BATCH; ++u) {
+            const size_t zz = (size_t)(z + u < S ? z + u : S - 1) * MN;  // clamp, never branch around a load
+#pragma unroll
+            for (int v = 0; v < NV; ++v) b[u][v] = *reinterpret_cast<const V *>(part + zz + off[v]);
+        }
+#pragma unroll
+        for (int u = 0; u < BATCH; ++u)
+            if (z + u < S) {
+#pragma unroll
+                for (int v = 0; v < NV; ++v) {
+                    acc[v].x += b[u][v].x, acc[v].y += b[u][v].y;
+                    if constexpr (sizeof(V) == 16) acc[v].z += b[u][v].z, acc[v].w += b[u][v].w;
+                }
+            }
+    }
+}
+
+// A batch's step (one row per sequence, T pages): RoPE and the append of the new K / V row inside the attention launch.  The launch they had to themselves
+// moves 12 KB a row in the 4.8 - 5.5 us any dependent launch takes; here a workgroup rotates its kv group's q heads under the latency of its first K / V
+// rows -- every split its own copy, a few KB from L2 -- and the split that ends with the new position also rotates k, stores k and v to the page and scores
+// them from LDS.  The arithmetic is k_rope_append_rows', term for term.  Rows are distinct sequences: no other row reads the position stored here.
+// Llama-3-8B int4, q|k|v as fp32 slabs, rope + attention of a layer, us: 8 rows at 200 cached positions
+// 5.5 + 9.6 -> 10.6, 32 rows at 1000 5.5 + 31.1 -> 30.9; dense, T rows, 8 rows at 1000 4.8 + 12.5 -> 14.9.
+struct AttnRopeArgs : AttnArgs {
+    const u16 *qkv;         // [rows, n_cols], packed columns (2 i, 2 i + 1) of a q / k head = its dims (i, i + D / 2) ...
+    const float *part;      // ... or the S fp32 slabs of a K-split product, MN elements apart (S > 1)
+    int S, n_cols, traditional;
+    size_t MN;
+    const float *rope_cs;   // [rows][D / 2] (cos, sin)
+    u16 *pages;             // = slab
+};
+template <class T, int D, int REP, int NT>
+struct AttnRopeSeam {
+    const AttnRopeArgs &a;
+    int g, split, row;
+    u16 *s_q, *s_kv;
+    __device__ __forceinline__ void operator()() const {
+        constexpr int half = D / 2;
+        const int Ttot = a.ctx_len[row], pos = Ttot - 1;  // >= 0: an idle slot has left
+        const bool newest = split == attn_split(Ttot, a.splits).active - 1;
+        const unsigned pg = min((unsigned)a.block_table[(size_t)row * a.bt_stride + (pos >> 6)], (unsigned)a.n_pages - 1u);
+        u16 *kdst = a.pages + (size_t)pg * 2 * 64 * a.Hkv * D + ((size_t)g * 64 + (pos & 63)) * D, *vdst = kdst + (size_t)a.Hkv * 64 * D;
+        for (int p = threadIdx.x; p < (newest ? REP + 2 : REP) * half; p += NT) {
+            const int h = p / half, ii = p % half;  // h: REP q heads, k, v
+            const size_t at = (size_t)row * a.n_cols + (h < REP ? g * REP + h : a.Hq + (h == REP ? g : a.Hkv + g)) * D + 2 * ii;
+            u32 pr;
+            if (a.S > 1) {
+                const size_t i[1] = {at};
+                float2 v[1];
+                slab_sum<float2, 1>(a.part, a.S, a.MN, i, v);
+                pr = pack2<T>(v[0].x, v[0].y);
+            } else pr = *reinterpret_cast<const u32 *>(a.qkv + at);
+            if (h == REP + 1) {
+                *reinterpret_cast<u32 *>(vdst + 2 * ii) = pr, *reinterpret_cast<u32 *>(s_kv + D + 2 * ii) = pr;
+                continue;
+            }
+            const float ra = lo_f32<T>(pr), rb = hi_f32<T>(pr);
+            const float2 cs = *reinterpret_cast<const float2 *>(a.rope_cs + ((size_t)row * half + ii) * 2);
+            const int i0 = a.traditional ? 2 * ii : ii, i1 = a.traditional ? 2 * ii + 1 : ii + half;
+            const u16 o0 = T::from_f32(__fsub_rn(__fmul_rn(ra, cs.x), __fmul_rn(rb, cs.y))), o1 = T::from_f32(__fadd_rn(__fmul_rn(ra, cs.y), __fmul_rn(rb, cs.x)));
+            u16 *dst = h < REP ? s_q + h * D : s_kv;
+            dst[i0] = o0, dst[i1] = o1;
+            if (h == REP) kdst[i0] = o0, kdst[i1] = o1;
+        }
+        __syncthreads();  // (a newest row beyond the ring is read from its page, by this workgroup only)
+    }
+};
+template <class T, int D, int REP, int NT>
+struct attn_seam_gives_rows<AttnRopeSeam<T, D, REP, NT>> : std::true_type {};
+
+template <class T, int D, int REP, bool NTKV>
+__global__ void __launch_bounds__(ATTN_WAVES * 64) k_attn_rope_decode(const AttnRopeArgs a) {
+    constexpr int NT = ATTN_WAVES * 64;
+    __shared__ __attribute__((aligned(16))) u16 s_q[REP * D], s_kv[2 * D];
+    const int g = blockIdx.x, split = blockIdx.y, row = blockIdx.z;
+    attn_decode_body<T, D, REP, true, NTKV, ATTN_WAVES>(a, g, split, row, g * REP, AttnRopeSeam<T, D, REP, NT>{a, g, split, row, s_q, s_kv});
+}
+
 // Merge of the active splits for 8 consecutive dims [d0, d0+8) of q-head h (fp32):
 // out[d] = sum_j w_j acc_j[d] / sum_j w_j l_j,  w_j = exp(m_j - max m).  Split in a load half and a math half so a
 // caller can put other loads in flight between them.  Loads are issued for all MAXS slots (clamped to an active
@@ -494,3 +588,4 @@ __global__ void __launch_bounds__(256) k_attn_combine(const AttnArgs a, int D) {
 
 // combine = false: leave the partials for the consumer's prologue (decoder: o_proj GEMV, PRO_ATTN).
 int attn_decode_launch(int dtype, int D, AttnArgs &a, bool combine, hipStream_t stream);
+int attn_rope_decode_launch(int dtype, int D, const AttnRopeArgs &a, hipStream_t stream);

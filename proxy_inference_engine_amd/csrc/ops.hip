@@ -55,6 +55,44 @@ int attn_decode_launch(int dtype, int D, AttnArgs &a, bool combine, hipStream_t 
     return pie::fail(PIE_E_SHAPE, "sdpa_decode: head_dim must be 64 or 128 and dtype bf16/f16");
 }
 
+// the step of a batch over T pages, RoPE and append inside (k_attn_rope_decode)
+template <class T, int D, bool NT>
+static int attn_rope_launch_rep(int rep, const AttnRopeArgs &a, hipStream_t st) {
+    const dim3 grid(a.Hkv, a.splits, a.rows), block(ATTN_WAVES * 64);
+#define ATTN_GO(R) \
+    case R: hipLaunchKernelGGL((k_attn_rope_decode<T, D, R, NT>), grid, block, 0, st, a); break
+    switch (rep) {
+        ATTN_GO(1);
+        ATTN_GO(2);
+        ATTN_GO(3);
+        ATTN_GO(4);
+        ATTN_GO(5);
+        ATTN_GO(6);
+        ATTN_GO(7);
+        ATTN_GO(8);
+        default: return pie::fail(PIE_E_SHAPE, "sdpa_decode: n_heads / n_kv_heads must be between 1 and 8");
+    }
+#undef ATTN_GO
+    PIE_LAUNCH_CHECK();
+    if (a.splits > 1) {
+        hipLaunchKernelGGL(k_attn_combine<T>, dim3(a.Hq, a.rows), dim3(256), 0, st, a, D);
+        PIE_LAUNCH_CHECK();
+    }
+    return PIE_OK;
+}
+int attn_rope_decode_launch(int dtype, int D, const AttnRopeArgs &a, hipStream_t st) {
+    PIE_REQUIRE(a.Hkv > 0 && a.Hq % a.Hkv == 0, PIE_E_SHAPE, "sdpa_decode: Hq must be a multiple of Hkv");
+    PIE_REQUIRE(a.splits >= 1 && a.splits <= ATTN_MAX_SPLITS, PIE_E_ARG, "sdpa_decode: bad split count");
+    const int rep = a.Hq / a.Hkv;
+#define ATTN_D(T_, D_) return a.nt_kv ? attn_rope_launch_rep<T_, D_, true>(rep, a, st) : attn_rope_launch_rep<T_, D_, false>(rep, a, st)
+    if (dtype == PIE_BF16 && D == 128) ATTN_D(BF16, 128);
+    if (dtype == PIE_BF16 && D == 64) ATTN_D(BF16, 64);
+    if (dtype == PIE_F16 && D == 128) ATTN_D(F16, 128);
+    if (dtype == PIE_F16 && D == 64) ATTN_D(F16, 64);
+#undef ATTN_D
+    return pie::fail(PIE_E_SHAPE, "sdpa_decode: head_dim must be 64 or 128 and dtype bf16/f16");
+}
+
 // ---------------------------------------------------------------- mx.fast.rms_norm: one workgroup per row
 template <class T>
 __global__ void __launch_bounds__(256) k_rms_norm(const u16 *x, const u16 *w, float eps, int H, u16 *y) {

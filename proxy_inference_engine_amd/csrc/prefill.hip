@@ -130,33 +130,6 @@ struct W4lSlabs {
 #ifndef SLAB_BATCH
 #define SLAB_BATCH 4
 #endif
-// V = float2 / float4: one thread's NV vectors at element offsets off[]; the slabs are fetched BATCH at a time (all BATCH x NV loads in flight
-// before the first add -- a plain loop over the slabs waits out one memory latency per slab: 15 us instead of 5 for a 64-row o_proj
-// consumer) and added strictly in slab order.
-template <class V, int NV, int BATCH = 4>
-__device__ __forceinline__ void slab_sum(const float *part, int S, size_t MN, const size_t (&off)[NV], V (&acc)[NV]) {
-#pragma unroll
-    for (int v = 0; v < NV; ++v) acc[v] = *reinterpret_cast<const V *>(part + off[v]);
-    for (int z = 1; z < S; z += BATCH) {
-        V b[BATCH][NV];
-#pragma unroll
-        for (int u = 0; u < BATCH; ++u) {
-            const size_t zz = (size_t)(z + u < S ? z + u : S - 1) * MN;  // clamp, never branch around a load
-#pragma unroll
-            for (int v = 0; v < NV; ++v) b[u][v] = *reinterpret_cast<const V *>(part + zz + off[v]);
-        }
-#pragma unroll
-        for (int u = 0; u < BATCH; ++u)
-            if (z + u < S) {
-#pragma unroll
-                for (int v = 0; v < NV; ++v) {
-                    acc[v].x += b[u][v].x, acc[v].y += b[u][v].y;
-                    if constexpr (sizeof(V) == 16) acc[v].z += b[u][v].z, acc[v].w += b[u][v].w;
-                }
-            }
-    }
-}
-
 // RoPE (llama/utils.py:42-50, offset = cache.offset) + cache append (reusable.py:134-137) for M rows of the packed
 // q|k|v projection: packed columns (2i, 2i+1) of a q/k head are its dims (i, i + D/2); v columns are natural.
 // grid M, one thread per packed column pair.
@@ -976,21 +949,23 @@ static int decode_batch_t(pie_decoder *d, const int32_t *tokens, const int32_t *
         W4lSlabs sq;  // q|k|v as the fp32 slabs of a K-split product (no Linear bias: RoPE takes T(x W^T + b))
         if ((rc = linear_rows<T>(d, w.wqkv, NQKV, H, s->xn, B, s->qkv, st, true, w.bqkv, false, nullptr, &roped, &re, w.bqkv ? nullptr : &sq)))
             return rc;
-        if (!roped) {
-            decltype(&k_rope_append_rows<T, false, false>) rope_k = &k_rope_append_rows<T, false, false>;
-            if (sq.S > 1) rope_k = d->kv_i8 ? &k_rope_append_rows<T, true, true> : &k_rope_append_rows<T, true, false>;
-            else if (d->kv_i8) rope_k = &k_rope_append_rows<T, false, true>;
+        const bool rope_in_attn = !roped && !d->kv_i8;  // T pages: inside the attention launch (k_attn_rope_decode)
+        if (!roped && d->kv_i8) {
+            decltype(&k_rope_append_rows<T, false, false>) rope_k = &k_rope_append_rows<T, false, true>;
+            if (sq.S > 1) rope_k = &k_rope_append_rows<T, true, true>;
             hipLaunchKernelGGL(rope_k, dim3(B, sq.S > 1 || B < 128 ? 4u : 1u), dim3(256), 0, st, s->qkv, NQKV, d->glob.rope_freqs, nullptr, nullptr, li, c.n_layers,
                                c.n_heads, c.n_kv_heads, D, c.rope_traditional, s->q, block_tables, n_pages, s->rope_cs, ctx_len, max_blocks, (u16 *)slabs[li],
                                (const int *)nullptr, (u16 *)nullptr, (u16 *)nullptr, sq.part, sq.S, sq.MN, i8pb);
             PIE_LAUNCH_CHECK();
         }
-        AttnArgs a = {};
+        AttnRopeArgs a = {};
         a.q = s->q, a.slab = (const u16 *)slabs[li], a.block_table = block_tables, a.ctx_len = ctx_len, a.bt_stride = max_blocks, a.n_pages = n_pages;
         a.rows = B, a.Hq = c.n_heads, a.Hkv = c.n_kv_heads, a.splits = splits, a.scale = 1.0f / sqrtf((float)D);
         a.nt_kv = (size_t)B * max_blocks * 64 >= 2048;
         a.part_acc = s->part_acc, a.part_ml = s->part_ml, a.out = s->attn;
-        if ((rc = d->kv_i8 ? paged_attn_i8_launch(c.dtype, D, a, st) : attn_decode_launch(c.dtype, D, a, true, st))) return rc;
+        a.qkv = s->qkv, a.part = sq.part, a.S = sq.S, a.MN = sq.MN, a.n_cols = NQKV, a.rope_cs = s->rope_cs, a.traditional = c.rope_traditional, a.pages = (u16 *)slabs[li];
+        rc = d->kv_i8 ? paged_attn_i8_launch(c.dtype, D, a, st) : rope_in_attn ? attn_rope_decode_launch(c.dtype, D, a, st) : attn_decode_launch(c.dtype, D, a, true, st);
+        if (rc) return rc;
         W4lSlabs so, sd;  // o_proj / down handed over as K-split fp32 slabs where the shape qualifies
         if ((rc = linear_rows<T>(d, w.wo, H, QD, s->attn, B, s->r, st, true, w.bo, false, nullptr, nullptr, nullptr,
                                  H <= 8192 ? &so : nullptr)))

@@ -1,0 +1,57 @@
+"""RoPE and the K / V append inside the attention launch of a batch's step (k_attn_rope_decode): the new position at every edge of its page and of the split that
+ends with it, one split and several, the group sizes in use, both rotary conventions, the projection as T rows (dense, biased) and as K-split slabs
+(int4 from six rows).  The reference is each sequence served alone: other kernels append its row and score its cache."""
+import numpy as np
+import pytest
+import torch
+
+from tests._util import assert_vec_close
+
+pytestmark = pytest.mark.gpu
+
+LENS = [1, 2, 31, 63, 64, 65, 128, 257, 520]  # positions cached before the step: the new row opens a page at 64 and 128, lies beyond the first loads in flight at 257 and 520
+
+
+def _model(hidden, Hq, Hkv, D, traditional, quant, bias):
+    from proxy_inference_engine_amd.models.llama import Model, ModelArgs
+    from proxy_inference_engine_amd.models.utils import synthetic_checkpoint
+    cfg = {"model_type": "llama", "hidden_size": hidden, "num_hidden_layers": 2, "intermediate_size": 512, "num_attention_heads": Hq, "num_key_value_heads": Hkv, "head_dim": D,
+           "rms_norm_eps": 1e-5, "vocab_size": 512, "rope_theta": 10000.0, "max_position_embeddings": 2048, "tie_word_embeddings": False, "rope_traditional": traditional,
+           "attention_bias": bias}
+    if quant:
+        cfg["quantization"] = {"group_size": 64, "bits": 4}
+    return Model(ModelArgs(**cfg), synthetic_checkpoint(cfg, seed=11, lm_head_gain=4.0))
+
+
+@pytest.mark.parametrize("hidden,Hq,Hkv,D,traditional,quant,bias", [
+    (512, 8, 2, 64, False, False, False), (512, 4, 4, 128, True, False, False), (896, 7, 1, 128, False, False, True),
+    (1024, 8, 2, 128, False, True, False), (1024, 16, 2, 64, True, True, False), (768, 6, 2, 128, False, True, True)])
+@pytest.mark.parametrize("rows", [9, 2])
+def test_batch_step_appends_and_attends_like_each_sequence_alone(hidden, Hq, Hkv, D, traditional, quant, bias, rows):
+    model = _model(hidden, Hq, Hkv, D, traditional, quant, bias)
+    lens = LENS if rows == len(LENS) else [64, 520]
+    rng = np.random.default_rng(rows)
+    prompts = [rng.integers(0, 512, n).astype(np.int32) for n in lens]
+    pool = model.enable_paged_kv(num_pages=2 * sum(n // 64 + 2 for n in lens), max_blocks=16)
+    feed, both = [7 + i for i in range(len(lens))], []
+    for batch in (False, True):
+        caches = [model.make_cache() for _ in lens]
+        for p, c in zip(prompts, caches):
+            model.step(torch.from_numpy(p).cuda(), c)
+        if batch:
+            got = model.step_batch(torch.tensor(feed, dtype=torch.int32, device="cuda"), caches, graph=False)[2].float().cpu().numpy()
+        else:
+            got = np.stack([model.step(torch.tensor([t], dtype=torch.int32, device="cuda"), c)[2].float().cpu().numpy().reshape(-1) for t, c in zip(feed, caches)])
+        rows_of = []
+        for c, n in zip(caches, lens):
+            page = pool.slab[0].view(torch.bfloat16).view(-1, 2, Hkv, 64, D)[c[0].page_manager.pages[n // 64]]
+            rows_of.append(page[:, :, n % 64].clone())
+        both.append((got, torch.stack(rows_of)))
+    (alone, row_alone), (batched, row_batched) = both
+    for i, n in enumerate(lens):
+        assert_vec_close(batched[i], alone[i], "bfloat16", what=f"row {i}, {n} positions cached")
+        # layer 0's new K / V row, whose inputs are equal.  Per side half an ulp (2^-9) for T(x W^T), for the bias added to it, both up to sqrt 2 larger after the rotation of a
+        # pair, and for the rotation: 3.8 x 2^-9; both sides 2^-6.06 of the largest element.  int4 from six rows: weights rounded to T, 2^-9 of each product more, ~2^-9 of an
+        # element in the mean.  Under 2^-5 together; another position's row or angle is off by the element itself.
+        a, b = row_alone[i].float(), row_batched[i].float()
+        assert float((a - b).abs().max()) <= float(a.abs().max()) * 2 ** -5, (i, n)
