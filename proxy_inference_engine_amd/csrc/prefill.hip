@@ -563,11 +563,9 @@ int w4r_gemm_launch(int dtype, const void *w4m, const void *x, int M, int N, int
                     const W4mRope *rope, int *slabs, bool *bias_done, bool wide_scales);
 
 // int4 checkpoints: prompts beyond small_rows() rows run the hand-written many-row W4 MFMA GEMM on the same W4M tiles -- no 16-bit
-// copy of the weights, no hipBLASLt (which remains the path of shapes the tile kernels do not take: N not a multiple of 32).
+// copy of the weights (shapes the tile kernels do not take, N not a multiple of 32, go through the T copy and k_w16l_gemm).
 static bool w4l_enabled() { return true; }
-// Dense (16-bit) modules keep the library GEMM: for 16-bit weights hipBLASLt is a plain GEMM done well.  The hand-written 16-bit kernel of
-// rounds 2-3 (k_w16l_gemm: 0-20 % slower on prompts, 15-38 % on the vision tower's small shapes) was deleted in round 4 (EXPERIMENTS.md).
-// Rows up to which an int4 Linear runs on the W4M kernel instead of the T copy + hipBLASLt (PIE_KNOB_SMALL_M: 0 disables, max 32).
+// Rows up to which an int4 Linear runs on the W4M kernel instead of the T copy + k_w16l_gemm (PIE_KNOB_SMALL_M: 0 disables, max 32).
 static int small_rows() {
     const int k = pie_knob(PIE_KNOB_SMALL_M);
     const int v = k >= 0 ? k : 32;
@@ -865,8 +863,8 @@ static int batch_attn_splits(const pie_decoder *d, int B, int max_blocks) {
 }
 
 // ---------------------------------------------------------------- one decode step for B sequences (continuous batching)
-// The weights stream once for all B rows (few-row int4 GEMM for B <= 32, the T copy + hipBLASLt beyond); each row is its own
-// sequence: RoPE at its own position, K/V appended to its own page, attention over its own block table (k_attn_decode PAGED,
+// The weights stream once for all B rows (few-row int4 GEMM for B <= 32, the T copy + k_w16l_gemm beyond); each row is its own
+// sequence: RoPE at its own position, K/V appended to its own page, attention over its own block table (k_attn_rope_decode,
 // one sequence per blockIdx.z), lm_head + tail on every row.  What the reference's Scheduler / BatchDetails / PagedAttention
 // skeleton (src/pie_core/include/engine/batch_details.hpp:10-88, scheduler.hpp) describes for decode-state sequences.
 template <class T>
