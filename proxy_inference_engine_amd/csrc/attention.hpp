@@ -187,9 +187,8 @@ __device__ __forceinline__ void attn_decode_body(const AttnArgs &a, const int g,
         int t = first + b * NSUB * TPW + ts;
         t = t < t_end ? t : t_end - 1;  // clamp, never branch around a load
         // Before the seam NO lane may touch the row this launch writes (position Ttot - 1) -- not even a clamped, discarded load: it would park a
-        // stale line of that row in this CU's L1, and the real load after the seam would hit it.  Such lanes read the row before it (an empty
-        // cache: the buffer's last row); the one valid lane is loaded again behind the seam.
-        // (PAGED: the page id stays the clamped row's -- any row of any of the sequence's pages will do, as long as it is not row (Ttot - 1) % 64 of its page)
+        // stale line of that row in this CU's L1, and the real load after the seam would hit it.  Such lanes read another row of its page (of an empty
+        // cache: the buffer's last), which the sequence may never have written; all of them are loaded again behind the seam.
         if (HAS_SEAM && before_seam && t >= Ttot - 1) t = Ttot >= 2 ? Ttot - 2 : cap - 1;
         if constexpr (PAGED) {
             const size_t off = (size_t)pgq[d] * page_elems + (size_t)(t & 63) * D;
@@ -209,14 +208,15 @@ __device__ __forceinline__ void attn_decode_body(const AttnArgs &a, const int g,
     for (int d = 0; d < DA; ++d) issue(d, d);
     if constexpr (HAS_SEAM) {
         // the rows cached by earlier steps are on their way; now wait for this step's q / k / v, then fetch the one row of the ring that was
-        // written in this launch (position Ttot - 1, if this split holds it and it sits in the first DA blocks)
+        // written in this launch (position Ttot - 1, if this split holds it and it sits in the first DA blocks) -- for the lanes past it in the
+        // block as well: their weight is 0, but 0 times what lies in a row that nobody wrote may be NaN
         seam();
         before_seam = false;
         ATTN_STAMP(7);  // released
 #pragma unroll
         for (int d = 0; d < DA; ++d) {
-            const int t = first + d * NSUB * TPW + ts;
-            if (on && t == Ttot - 1 && t < t_end) {
+            const int t = Ttot - 1;
+            if (d < n_blk && t_end == Ttot && first + d * NSUB * TPW + ts >= t) {
                 if constexpr (attn_seam_gives_rows<SEAM>::value) {
                     kq[d] = *reinterpret_cast<const uint4 *>(seam.s_kv + dc * 8), vq[d] = *reinterpret_cast<const uint4 *>(seam.s_kv + D + dc * 8);
                 } else if constexpr (PAGED) {

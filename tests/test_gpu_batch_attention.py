@@ -55,3 +55,37 @@ def test_batch_step_appends_and_attends_like_each_sequence_alone(hidden, Hq, Hkv
         # element in the mean.  Under 2^-5 together; another position's row or angle is off by the element itself.
         a, b = row_alone[i].float(), row_batched[i].float()
         assert float((a - b).abs().max()) <= float(a.abs().max()) * 2 ** -5, (i, n)
+
+
+def _poison(pool, value):
+    for slab in pool.slab:
+        slab.view(torch.bfloat16).fill_(value)
+
+
+@pytest.mark.parametrize("hidden,Hq,Hkv,D,quant,rows", [
+    (512, 8, 2, 64, False, 3), (512, 8, 2, 64, False, 6), (512, 4, 4, 128, False, 3), (512, 4, 4, 128, False, 6), (1024, 8, 2, 128, True, 6),
+    (512, 32, 8, 128, False, 1), (512, 32, 8, 128, True, 1)])
+def test_a_step_that_opens_a_page_reads_no_row_that_nobody_wrote(hidden, Hq, Hkv, D, quant, rows):
+    """The new position is row 0 of a fresh page (0, 64 and 128 cached): what else lies in the pool -- a recycled page's rows, memory never written -- may be NaN or infinite
+    and must not count, not even with weight 0.  The same pool filled with zeros gives the same bits.  Three rows: one split; six: several; one row (32 / 8 heads of 128): the
+    attention behind the q|k|v launch."""
+    model = _model(hidden, Hq, Hkv, D, False, quant, False)
+    cached = [0, 64, 128] * (rows // 3) if rows > 1 else [0, 64, 128]
+    prompts = [np.random.default_rng(i).integers(0, 512, n).astype(np.int32) for i, n in enumerate(cached)]
+    pool = model.enable_paged_kv(num_pages=2 * sum(n // 64 + 1 for n in cached), max_blocks=4)
+    feed = torch.arange(7, 7 + len(cached), dtype=torch.int32, device="cuda")
+    got = []
+    for fill in (0.0, float("nan"), float("inf")):
+        _poison(pool, fill)
+        caches = [model.make_cache() for _ in cached]
+        for p, c in zip(prompts, caches):
+            if len(p):
+                model.step(torch.from_numpy(p).cuda(), c)
+        if rows > 1:
+            got.append(model.step_batch(feed, caches, graph=False)[2].clone())
+        else:
+            got.append(torch.stack([model.step(feed[i:i + 1], c)[2].clone().reshape(-1) for i, c in enumerate(caches)]))
+        for c in caches:
+            c[0].page_manager.release()
+    assert not torch.isnan(got[0]).any()
+    assert torch.equal(got[0], got[1]) and torch.equal(got[0], got[2])
