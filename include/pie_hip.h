@@ -559,6 +559,9 @@ typedef struct pie_stack pie_stack;
 /* packed weight of a Linear [N, K] in the stack's dtype: W16M tiles, or fp32 rows of 64 ceil(K / 64).  w: row-major bf16 [N][K] on the device. */
 size_t pie_stack_weight_bytes(int dtype, int N, int K);
 int pie_stack_pack_weight(const void *w, int N, int K, int dtype, void *packed, void *stream);
+/* Which kernel a plain bf16 Linear [N, K] of M rows takes (host only): 0 the one that fetches both operands itself, 1 the one that brings x through LDS.
+ * ldx: elements from one row of x to the next; x_rows: how many rows x holds where a list picks the M from them (0: they follow one another). */
+int pie_stack_linear_kernel(int M, int N, int K, int ldx, int x_rows);
 
 /* A norm.  NONE: the identity.  DYN_TANH: w * tanh(param x) + b, element by element.  RMS: x / sqrt(mean(x^2) + param) * w.
  * w, b: fp32 [width rounded up to 8, zeros past it] on the device, 16-byte aligned (b: DYN_TANH only). */

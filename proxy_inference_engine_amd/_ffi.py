@@ -28,7 +28,7 @@ BASE_EXPORTS = [
     "pie_page_alloc", "pie_page_free", "pie_page_add_ref", "pie_page_ref_count", "pie_page_num_tokens", "pie_page_set_num_tokens", "pie_page_mark_tokens",
     "pie_page_ptrs", "pie_page_i8_bytes", "pie_page_scale_ptrs",
     "pie_w16m_bytes", "pie_repack_w16m", "pie_linear_w16m_workspace", "pie_linear_w16m",
-    "pie_stack_weight_bytes", "pie_stack_pack_weight", "pie_stack_create", "pie_stack_destroy", "pie_stack_set_layer", "pie_stack_page_row",
+    "pie_stack_weight_bytes", "pie_stack_pack_weight", "pie_stack_linear_kernel", "pie_stack_create", "pie_stack_destroy", "pie_stack_set_layer", "pie_stack_page_row",
     "pie_stack_page_bytes", "pie_stack_state_floats", "pie_stack_forward", "pie_stack_launches", "pie_logprobs_argmax_f32", "pie_logprobs_argmax_f32_workspace",
 ]
 EXPORTS = BASE_EXPORTS + [
@@ -160,6 +160,7 @@ def base() -> C.CDLL:
     lib.pie_page_set_num_tokens.argtypes = [C.c_void_p, C.c_uint32, C.c_size_t]
     lib.pie_page_mark_tokens.argtypes = [C.c_void_p, C.POINTER(C.c_uint32), C.c_size_t, C.c_size_t]
     lib.pie_stack_weight_bytes.argtypes = [C.c_int, C.c_int, C.c_int]
+    lib.pie_stack_linear_kernel.argtypes = [C.c_int] * 5
     lib.pie_stack_pack_weight.argtypes = [C.c_void_p, C.c_int, C.c_int, C.c_int, C.c_void_p, C.c_void_p]
     lib.pie_stack_create.argtypes = [C.POINTER(pie_stack_config), C.POINTER(C.c_void_p)]
     lib.pie_stack_destroy.argtypes = lib.pie_stack_launches.argtypes = [C.c_void_p]

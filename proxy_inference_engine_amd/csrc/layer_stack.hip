@@ -1164,7 +1164,7 @@ int stack_enqueue(pie_stack *s, const pie_stack_batch &b, const Plan &plan, hipS
     if (b.n_want > 0) {
         RowsArgs a = {};
         a.m = {(const char *)s->cfg.head, V, W, s->h.p, WA, b.logits, V};
-        a.M = b.n_want, a.epi = s->cfg.logit_cap > 0.0f ? ROWS_SOFTCAP : ROWS_SCALE_F32, a.scale = s->cfg.logit_scale, a.act_limit = s->cfg.logit_cap, a.rows = b.want;
+        a.M = b.n_want, a.epi = s->cfg.logit_cap > 0.0f ? ROWS_SOFTCAP : ROWS_SCALE_F32, a.scale = s->cfg.logit_scale, a.act_limit = s->cfg.logit_cap, a.rows = b.want, a.x_rows = M;
         p.linear(a);
         if (!p.rc && b.next) {
             hipLaunchKernelGGL(k_f32_stats, dim3(ST_TILES, (unsigned)b.n_want), dim3(256), 0, st, b.logits, V, s->stats.p);

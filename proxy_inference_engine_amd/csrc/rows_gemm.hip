@@ -478,6 +478,16 @@ __global__ void __launch_bounds__(256) k_pack_f32(const u16 *w, int N, int K, in
 
 }  // namespace
 
+static bool rows_narrow(const RowsArgs &a, int n_max, int batches) { return (long)batches * n_max <= 16 * 64 && !a.merge.splits; }  // so few workgroups that they should not all read all rows
+// k_rows_lds counts the bytes behind its first row of x in 31 bits: all of x where a list picks rows from it, 64 rows otherwise
+static bool rows_lds_reaches(const RowsArgs &a) {
+    const size_t rows = a.rows ? (size_t)a.x_rows : a.gather ? (size_t)a.M : 64;
+    return rows * (size_t)a.m.ldx * 2 < (1u << 31);
+}
+static bool rows_lds_serves(const RowsArgs &a, int n_max, int k_max, int batches) {
+    return a.M > 4 && k_max >= 1024 && !rows_narrow(a, n_max, batches) && !a.x_norm && a.merge.splits <= 0 && rows_lds_reaches(a);
+}
+
 size_t rows_weight_bytes(int dtype, int N, int K) {
     return dtype == PIE_F32 ? (size_t)N * ((K + 63) & ~63) * 4 : w16m_size(N, K);
 }
@@ -506,13 +516,11 @@ int rows_gemm_launch(int dtype, const RowsArgs &a, int batches, hipStream_t st) 
     PIE_REQUIRE(a.m.ldx % 8 == 0 && a.x_batch % 8 == 0 && pie_aligned(a.m.x, 16) && pie_aligned(a.m.w, 16), PIE_E_ALIGN, "row-wise Linear: 16-byte alignment required");
     int n_all = batches == 1 ? n_max : 0;
     for (int i = 0; i < a.n_mats; ++i) n_all += a.mats[i].N;
-    const bool narrow = (long)batches * n_max <= 16 * 64 && !a.merge.splits;  // so few workgroups that they should not all read all rows
     long blocks = 0;  // of 16 features, over the whole launch
     for (int i = 0; i < a.n_mats; ++i) blocks += (a.mats[i].N + 15) / 16;
     if (!a.n_mats) blocks = (long)batches * ((a.m.N + 15) / 16);
-    const bool within = (size_t)(a.rows || a.gather ? a.M : 64) * (size_t)a.m.ldx * 2 < (1u << 31);  // k_rows_lds counts an operand's bytes in 31 bits
-    if (a.M > 4 && k_max >= 1024 && !narrow && !a.x_norm && a.merge.splits <= 0 && within) return rows_lds_pick<ElemBF16>(a, n_max, blocks, batches, st);
-    if (a.M <= 16 || a.active || narrow) return rows_go<ElemBF16, 1, 1>(a, n_max, k_max, batches, st);
+    if (rows_lds_serves(a, n_max, k_max, batches)) return rows_lds_pick<ElemBF16>(a, n_max, blocks, batches, st);
+    if (a.M <= 16 || a.active || rows_narrow(a, n_max, batches)) return rows_go<ElemBF16, 1, 1>(a, n_max, k_max, batches, st);
     const bool wide = n_all >= 32 * 140;  // two feature blocks per wave where half as many workgroups still fill most of the chip
     if (a.M <= 32) return wide ? rows_go<ElemBF16, 2, 2>(a, n_max, k_max, batches, st) : rows_go<ElemBF16, 2, 1>(a, n_max, k_max, batches, st);
     return wide ? rows_go<ElemBF16, 4, 2>(a, n_max, k_max, batches, st) : rows_go<ElemBF16, 4, 1>(a, n_max, k_max, batches, st);
@@ -538,6 +546,14 @@ extern "C" {
 
 size_t pie_stack_weight_bytes(int dtype, int N, int K) {
     return N > 0 && K > 0 && (dtype == PIE_BF16 || dtype == PIE_F32) ? rows_weight_bytes(dtype, N, K) : 0;
+}
+
+int pie_stack_linear_kernel(int M, int N, int K, int ldx, int x_rows) {
+    PIE_REQUIRE(M > 0 && N > 0 && K > 0 && ldx >= K && x_rows >= 0, -1, "pie_stack_linear_kernel: bad sizes");
+    RowsArgs a = {};
+    const int any = 0;
+    a.m.N = N, a.m.K = K, a.m.ldx = ldx, a.M = M, a.rows = x_rows ? &any : nullptr, a.x_rows = x_rows;
+    return rows_lds_serves(a, N, K, 1);
 }
 
 int pie_stack_pack_weight(const void *w, int N, int K, int dtype, void *packed, void *stream) {

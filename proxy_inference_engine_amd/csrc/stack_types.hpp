@@ -334,6 +334,7 @@ struct RowsArgs {
     bool gather;           // grouped: x row = list[position] (else x row = position); y row = position always
     RowsMat shared;        // blockIdx.y == batches - 1 when shared.w: all M rows, this matrix (the expert every token takes)
     const int *rows;       // ungrouped, nullable: x row of result row i
+    int x_rows;            // with rows: how many rows x holds
     RowsMat mats[ROWS_LIST];  // n_mats > 0: blockIdx.y picks one of these instead of m, each with its own sizes and operands
     int n_mats;
     int flat_tiles, flat_batches;  // set by the launcher (k_rows_lds): workgroups of one expert's matrix, experts; or -1: a list, workgroup after workgroup

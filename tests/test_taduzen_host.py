@@ -111,3 +111,16 @@ def test_oracle_mistakes_show(mistake, monkeypatch):
     elif mistake == "act":
         monkeypatch.setattr(orc, "relu2", lambda z: np.maximum(z, 0.0))
     assert tu.err(orc.forward(cfg, w, ids), want) > 0.05
+
+
+def test_rows_picked_from_more_than_2_gib_take_the_kernel_with_64_bit_addresses():
+    """The head multiplies a few wanted rows of a pass of up to 65535: what counts is where those may lie, not how many they are.  Widths to 32768 are accepted."""
+    from proxy_inference_engine_amd import _ffi
+
+    def lds(M, K, ldx, x_rows):
+        return _ffi.base().pie_stack_linear_kernel(M, 4000, K, ldx, x_rows)
+    for M in (5, 16, 64):
+        assert lds(M, 32768, 32768, 0) == 1 and lds(M, 32768, 32768, M) == 1 and lds(M, 32768, 32768, 32767) == 1
+        assert lds(M, 32768, 32768, 32768) == 0 and lds(M, 32768, 32896, 32650) == 0 and lds(M, 32768, 32768, 65535) == 0
+        assert lds(M, 16384, 16384, 65535) == 1 and lds(M, 16384, 16400, 65535) == 0
+    assert _ffi.base().pie_stack_linear_kernel(0, 1, 1, 1, 0) < 0
