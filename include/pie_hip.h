@@ -506,7 +506,7 @@ int pie_paged_attn_decode_i8(const void *q, const void *slab, size_t n_pages, co
  *   and 3420, are padded by the host); y: rows of ldy elements (0 = packed).  swiglu != 0: the weight's rows interleave (gate_i, up_i),
  *   bias likewise, and y [M, N / 2] = T(T(silu(g)) * u) with g, u the rounded, biased Linear outputs (MLP, vision.py:196-197: the values
  *   of the GEMM followed by pie_bias_silu_mul).  workspace: pie_linear_w16m_workspace(M, N, K) bytes of device scratch for the
- *   shapes that split K (few rows, narrow matrices; 0 for most and for swiglu).  Any N (16-byte stores when N and ldy are multiples
+ *   shapes that split K (few rows, narrow matrices; 0 for most; none is needed for swiglu or with ldy != N, which take one pass over K).  Any N (16-byte stores when N and ldy are multiples
  *   of 8); swiglu needs N % 8 == 0.
  * pie_gelu: nn.GELU() exact form, fp32 inside, one rounding.
  * pie_vision_qkv_rope: qkv T [N, 3, H, D] (+ optional bias T [3 * H * D], the qkv Linear's) -> q T [N, H, DP], k, v T [H, N, DP] with rotate-half rotary on q and k

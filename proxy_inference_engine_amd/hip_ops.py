@@ -585,9 +585,7 @@ def linear_rows(x: torch.Tensor, weight, bias: torch.Tensor | None = None, *, sw
     ldy = -(-cols // pad_to) * pad_to if pad_to else cols
     y = (torch.zeros if ldy != cols else torch.empty)((M, ldy), dtype=x.dtype, device=x.device)
     lib = _ffi.load()
-    wsb = 0 if swiglu else int(lib.pie_linear_w16m_workspace(M, N, K))
-    if wsb and ldy != cols:
-        raise ValueError("linear_rows: pad_to is not available for shapes that split K")
+    wsb = 0 if swiglu or ldy != cols else int(lib.pie_linear_w16m_workspace(M, N, K))  # (padded rows take one pass over K)
     ws = torch.empty(wsb, dtype=torch.uint8, device=x.device) if wsb else None
     _ffi.check(lib.pie_linear_w16m(_ffi.p(x), x.stride(0), _ffi.p(pk.tiles), _ffi.p(bias.contiguous() if bias is not None else None), M, N, K,
                                    _ffi.dtype_code(x.dtype), _ffi.p(y), ldy, int(swiglu), _ffi.p(ws), wsb, _ffi.stream()))

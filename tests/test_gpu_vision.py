@@ -106,6 +106,19 @@ def test_fused_gate_up_linear_is_the_gemm_followed_by_bias_silu_mul(ops, dt, M, 
     assert torch.equal(ops.linear_rows(padded, ops.pack_linear(dw)), ops.linear_rows(got, dw))
 
 
+@pytest.mark.parametrize("M,N,K,pad", [(40, 1000, 1152, 64), (300, 1000, 1152, 64), (129, 1176, 1280, 32), (509, 36, 4096, 64), (33, 1000, 1152, 1000)])
+def test_padded_rows_of_shapes_that_would_split_k(ops, M, N, K, pad):
+    """linear_rows(..., pad_to=...): rows wider than the matrix take one pass over K, whatever the plan for packed rows is.  One rounding of a sum of K products that is good to
+    K 2^-24 of its terms: half an ulp of the largest result, under 2^-8 of it."""
+    rng = np.random.default_rng(M + N)
+    x, w = dev(po.round_T(rng.standard_normal((M, K)), "bfloat16"), "bfloat16"), dev(po.round_T(rng.standard_normal((N, K)) / np.sqrt(K), "bfloat16"), "bfloat16")
+    got = ops.linear_rows(x, w, pad_to=pad)
+    cols = -(-N // pad) * pad
+    assert got.shape == (M, cols) and not got[:, N:].any()
+    want = x.double().cpu() @ w.double().cpu().T
+    assert float((got[:, :N].double().cpu() - want).abs().max()) <= 2.0 ** -8 * float(want.abs().max())
+
+
 def test_linear_w16m_refuses_what_it_cannot_do(ops):
     """pie_linear_w16m through the C ABI: a K-split shape without its workspace, a fused SiLU * up on an odd column count, an x row stride shorter
     than the padded K, and a host tensor are errors (status + pie_last_error), not silent fallbacks."""
