@@ -282,6 +282,8 @@ int pie_gateup_row_map(int inter, int32_t *map /* [2*inter], source rows of cat(
 
 int pie_decoder_create(const pie_decoder_config *cfg, pie_decoder **out);
 int pie_decoder_destroy(pie_decoder *d);
+/* The decoder keeps copies of the matrices in other layouts (the batched paths' operands).  Weights changed in place, or others behind the same pointers: call
+ * again what set them; it drops the copies and the captured graphs. */
 int pie_decoder_set_layer(pie_decoder *d, int layer, const pie_layer_weights *w);
 int pie_decoder_set_globals(pie_decoder *d, const pie_global_weights *w);
 /* Per-layer cache buffers [n_kv_heads, capacity, head_dim] T (ReusableKVCache.keys/values with B=1);

@@ -357,6 +357,7 @@ int pie_decoder_set_globals(pie_decoder *d, const pie_global_weights *w) {
     else if (w->lm_head != w->embed_codes) d->fmt_map.erase(w->lm_head);
     PIE_REQUIRE(pie_aligned(w->lm_head, 256) && pie_aligned(w->final_norm, 16) && pie_aligned(w->embed_codes, 16), PIE_E_ALIGN,
                 "pie_decoder_set_globals: misaligned weight");
+    prefill_globals_changed(d, w->lm_head);
     d->glob = *w;
     d->glob_set = true;
     drop_graphs(d);

@@ -93,4 +93,5 @@ int paged_attn_i8_launch(int dtype, int D, const AttnArgs &a, hipStream_t st);
 int prefill_min_rows();
 int prefill_batched(pie_decoder *d, const int32_t *ids, const void *embeds, int L, void *logits_all, hipStream_t st);
 void prefill_free(pie_decoder *d);
+void prefill_globals_changed(pie_decoder *d, const void *new_head);  // (before d->glob changes)
 int enqueue_kernel(pie_decoder *d, int which, int li, const int *token_ptr, u16 *logits_dst, hipStream_t st, bool embed_here = false);  // embed_here: PIE_K_QKV of layer 0 also embeds the token

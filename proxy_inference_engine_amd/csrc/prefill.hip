@@ -21,6 +21,8 @@
 #include "prefill_attn.hpp"
 #include "stack_types.hpp"  // rows_w16_launch
 
+size_t w16m_size(int N, int K);  // bytes of a matrix as W16M and as W4M tiles
+size_t w4m_bytes(int N, int K);
 int embedding_launch(const int32_t *ids, int L, const uint32_t *codes, const void *scales, const void *biases, int V, int H, int dtype,
                      void *out, const float *freqs, const DecState *state, float *rope_cs, int half, hipStream_t st, int bits);
 
@@ -408,6 +410,19 @@ void prefill_free(pie_decoder *d) {
     d->prefill = nullptr;
 }
 
+// The embedding, the final norm and the head are others from here on, perhaps behind the same pointers: the old and the new head's copies and the captured
+// step go, the layers' copies stay
+void prefill_globals_changed(pie_decoder *d, const void *new_head) {
+    PrefillScratch *s = d->prefill;
+    if (!s) return;
+    ++s->alloc_gen;
+    for (const void *head : {(const void *)d->glob.lm_head, new_head}) {
+        const int N = d->cfg.vocab, K = d->cfg.hidden;
+        if (auto it = s->resident.find(head); it != s->resident.end()) (void)hipFree(it->second), s->resident.erase(it), s->resident_left += w16m_size(N, K);
+        if (auto it = s->resident_w4m.find(head); it != s->resident_w4m.end()) (void)hipFree(it->second), s->resident_w4m.erase(it), s->resident_left += w4m_bytes(N, K);
+    }
+}
+
 int prefill_min_rows() {  // read per call (not cached): tests and tools switch regimes inside one process
     const int k = pie_knob(PIE_KNOB_PREFILL_MIN);  // prompts shorter than this run as iterated decode steps (MLX's qmv regime)
     const int n = k >= 0 ? k : 6;  // MLX's own qmv limit is 6..32 rows by device and shape; 5 ms batched vs 1.35 ms per iterated row
@@ -494,7 +509,6 @@ static size_t resident_budget(pie_decoder *d) {
 }
 
 // w16_gemm.hpp / w4m_gemm.hip: the 16-bit many-row MFMA GEMM on W16M tiles (weights in MFMA A-fragment order)
-size_t w16m_size(int N, int K);
 int w16m_from_rows_launch(const void *w, int N, int K, void *w16m, hipStream_t st);
 int w16m_from_w16s_launch(const void *w16s, int N, int K, void *w16m, hipStream_t st);
 size_t w16l_workspace_bytes(int M, int N, int K);
@@ -533,10 +547,9 @@ static int expand_weights(pie_decoder *d, const void *packed, int N, int K, void
     return w16m_from_rows_launch(staging, N, K, w16m, st);
 }
 
-// y[M, N] = x[M, K] . W^T for one streaming-layout matrix.  keep: a layer matrix (eligible for the resident copy); the
-// lm_head of a logits-on-every-position call always goes through the scratch.
+// y[M, N] = x[M, K] . W^T for one streaming-layout matrix.  keep: a resident copy may be made (layer matrices, the head of batch steps); the
+// lm_head of a logits-on-every-position call uses one that is there, and goes through the scratch otherwise.
 // w4m_gemm.hip: the few-row int4 GEMM on W4M tiles
-size_t w4m_bytes(int N, int K);
 int w4m_repack_launch(const void *w4s, int N, int K, void *w4m, hipStream_t st);
 struct W4mRope {  // q|k|v epilogue arguments (defined identically in w4m_gemm.hip)
     const float *rope_cs;

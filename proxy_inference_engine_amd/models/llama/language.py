@@ -285,6 +285,7 @@ class Model:
         gw = _ffi.pie_global_weights(self.embed_tokens[0].data_ptr(), *(t.data_ptr() if t is not None else None for t in self.embed_tokens[1:]),
                                      self.norm.data_ptr(), self.lm_head.packed.data_ptr(), self.rope.freqs.data_ptr(), f_embed, f_head)
         _ffi.check(lib.pie_decoder_set_globals(self._dec, C.byref(gw)))
+        self._globals = gw  # (given again after a change in place)
         # device-side token history: history[p] = greedy token chosen for position p (written by the tail kernel)
         self.history = torch.zeros(1 << 20, dtype=torch.int32, device=device)
         _ffi.check(lib.pie_decoder_bind_outputs(self._dec, _ffi.p(self.logits), _ffi.p(self.logprobs), _ffi.p(self.token), _ffi.p(self.hidden),

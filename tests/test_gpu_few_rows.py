@@ -60,3 +60,46 @@ def test_dense_llama_step_of_several_rows(dtype, vocab):
                     layer.trim(1)
         for c in caches:
             c[0].page_manager.release()
+
+
+@pytest.mark.parametrize("bits", [None, 8, 4], ids=["dense", "int8", "int4"])
+def test_a_head_changed_in_place_is_seen_after_set_globals(bits):
+    """The head's tiles stay with the decoder; pie_decoder_set_globals says that the weights behind its pointers are others.  Batch steps, eager and replayed, and prompts with logits
+    everywhere, against a decoder that was made with the new head."""
+    import ctypes as C
+
+    from proxy_inference_engine_amd import _ffi
+    from proxy_inference_engine_amd.models.llama import Model, ModelArgs
+    from proxy_inference_engine_amd.models.utils import synthetic_checkpoint
+    cfg = {"model_type": "llama", "hidden_size": 512, "num_hidden_layers": 2, "intermediate_size": 512, "num_attention_heads": 8, "num_key_value_heads": 2, "head_dim": 64, "vocab_size": 1024,
+           "rms_norm_eps": 1e-5, "tie_word_embeddings": False, "quantization": {"group_size": 64, "bits": bits} if bits else None}
+    w = synthetic_checkpoint(cfg, seed=3)
+    others = synthetic_checkpoint(cfg, seed=4)
+    a, b = Model(ModelArgs(**cfg), dict(w)), Model(ModelArgs(**cfg), dict(w, **{k: v for k, v in others.items() if k.startswith("lm_head")}))
+    feed, ids = torch.arange(8, dtype=torch.int32, device="cuda"), torch.arange(40, dtype=torch.int32, device="cuda")
+    caches = {}
+    for m in (a, b):
+        m.enable_paged_kv(num_pages=32, max_blocks=4)
+        caches[m] = [m.make_cache() for _ in range(8)]
+        for i, c in enumerate(caches[m]):
+            m.step(ids[:9 + i], c)
+
+    def steps(m, graph):
+        out = []
+        for _ in range(3):
+            out.append(m.step_batch(feed, caches[m], graph=graph)[2].clone())
+            for c in caches[m]:
+                for layer in c:
+                    layer.trim(1)
+        c = m.make_cache()
+        out.append(m(ids[None], cache=c).clone())
+        c[0].page_manager.release()
+        return out
+    before = steps(a, True)
+    want = steps(b, True)
+    assert not torch.equal(before[0], want[0])
+    a.lm_head.packed.copy_(b.lm_head.packed)
+    _ffi.check(_ffi.load().pie_decoder_set_globals(a._dec, C.byref(a._globals)))
+    for graph in (False, True):
+        for got, ref in zip(steps(a, graph), want):
+            assert torch.equal(got, ref)
