@@ -358,8 +358,7 @@ struct PrefillScratch {
     unsigned batch_gen = 0, warm_gen = 0;
     void *w4l_ws = nullptr;   // fp32 partial tiles of the K-split prompt GEMM (w4m_gemm.hip)
     size_t w4l_ws_bytes = 0;
-    float *attn_part = nullptr;  // sums of prompt attention split along the keys (prefill_attn.hpp)
-    size_t attn_part_bytes = 0;
+    float *attn_part = nullptr;  // sums of prompt attention split along the keys (reserve_attn_part)
     int resident_mode = -1;   // -1: budget not fixed yet
     size_t resident_left = 0; // bytes still available for resident copies
 };
@@ -390,9 +389,8 @@ static void scratch_release(PrefillScratch *s) {  // the chunk buffers; resident
     void *keep_ws = s->w4l_ws;
     const size_t keep_wsb = s->w4l_ws_bytes;
     float *keep_part = s->attn_part;
-    const size_t keep_pb = s->attn_part_bytes;
     *s = PrefillScratch();
-    s->w4l_ws = keep_ws, s->w4l_ws_bytes = keep_wsb, s->attn_part = keep_part, s->attn_part_bytes = keep_pb;
+    s->w4l_ws = keep_ws, s->w4l_ws_bytes = keep_wsb, s->attn_part = keep_part;
     s->resident = std::move(keep), s->resident_w4m = std::move(keep_m), s->resident_mode = mode, s->resident_left = left;
     s->tail_stats = keep_ts, s->tail_entries = keep_tr, s->alloc_gen = gen;
 }
@@ -474,21 +472,17 @@ static int scratch_reserve(pie_decoder *d, int rows, size_t w_elems, int splits)
     return PIE_OK;
 }
 
-// A prompt's attention split along the keys where that pays and its sums have room (before: keys cached in front of the first row)
+// Room for the sums of prompt attention split along the keys: the most that any split takes (34 MB at 32 / 8 heads of 128), once, with the first prompt's buffers -- no captured launch
+// holds it, and a serving loop's longer and longer prefixes must neither allocate nor invalidate the captured batch step.  No room: prompts are not split.
+static void reserve_attn_part(pie_decoder *d) {
+    const pie_decoder_config &c = d->cfg;
+    if (d->prefill->attn_part || 512 / c.n_kv_heads < 2) return;
+    if (hipMalloc((void **)&d->prefill->attn_part, prefill_attn_part_bytes(c.n_heads, c.n_kv_heads, c.head_dim)) != hipSuccess) (void)hipGetLastError(), d->prefill->attn_part = nullptr;
+}
+// A prompt's attention split along the keys where that pays (before: keys cached in front of the first row)
 static void split_attn(pie_decoder *d, PrefillAttnArgs &a, int before) {
-    PrefillScratch *s = d->prefill;
-    const int splits = prefill_attn_splits(a.M, before, a.Hkv);
-    const size_t need = prefill_attn_part_bytes(a.M, a.Hq, d->cfg.head_dim, splits);
-    if (need > s->attn_part_bytes) {
-        if (s->attn_part) (void)hipFree(s->attn_part);
-        s->attn_part = nullptr, s->attn_part_bytes = 0, ++s->alloc_gen;
-        if (hipMalloc((void **)&s->attn_part, need) != hipSuccess) {
-            (void)hipGetLastError();
-            return;
-        }
-        s->attn_part_bytes = need;
-    }
-    if (splits > 1) a.splits = splits, a.part = s->attn_part;
+    const int splits = d->prefill->attn_part ? prefill_attn_splits(a.M, before, a.Hkv) : 1;
+    if (splits > 1) a.splits = splits, a.part = d->prefill->attn_part;
 }
 
 // ---------------------------------------------------------------- the batched forward
@@ -754,6 +748,7 @@ static int prefill_t(pie_decoder *d, const int32_t *ids, const void *embeds, int
     if (rc) return rc;
     PrefillScratch *s = d->prefill;
     const bool mfma_attn = pie_knob(PIE_KNOB_PREFILL_ATTN_VALU) != 1;  // 1 forces the row-per-launch-slice VALU kernel (tests compare the two)
+    if (mfma_attn) reserve_attn_part(d);
     for (int c0 = 0; c0 < L; c0 += chunk) {
         const int M = L - c0 < chunk ? L - c0 : chunk;
         // h = embed_tokens(inputs)  (language.py:176)
@@ -1033,6 +1028,7 @@ static int prefill_varlen_t(pie_decoder *d, const int32_t *ids, const int32_t *r
     if (rc) return rc;
     PrefillScratch *s = d->prefill;
     if ((rc = tail_stats_reserve(s, (size_t)TAIL_STAT_TILES * (size_t)S))) return rc;
+    if (n_chunks > 0) reserve_attn_part(d);
     rc = d->mat_fmt(d->glob.embed_codes) == PIE_W_DENSE
              ? pie_embedding_dense(ids, N, d->glob.embed_codes, c.vocab, H, c.dtype, s->x, st)
              : embedding_launch(ids, N, d->glob.embed_codes, d->glob.embed_scales, d->glob.embed_biases, c.vocab, H, c.dtype, s->x, nullptr, nullptr,

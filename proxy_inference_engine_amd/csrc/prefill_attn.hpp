@@ -337,7 +337,8 @@ static inline int prefill_attn_splits(int M, int before, int Hkv) {
     const int s = shares < room ? shares : room;
     return s < 2 ? 1 : s > 16 ? 16 : s;
 }
-static inline size_t prefill_attn_part_bytes(int M, int Hq, int D, int splits) { return splits > 1 ? (size_t)M * Hq * splits * (D + 2) * sizeof(float) : 0; }
+// room for the sums of any split prompt: ceil(M / 32) Hkv splits <= 512
+static inline size_t prefill_attn_part_bytes(int Hq, int Hkv, int D) { return (size_t)(512 / Hkv) * 32 * Hq * (D + 2) * sizeof(float); }
 
 template <class T, int D>
 static int prefill_attn_launch_d(const PrefillAttnArgs &a, hipStream_t st) {

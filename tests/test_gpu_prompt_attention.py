@@ -61,3 +61,27 @@ def test_rows_behind_a_prefix_split_along_the_keys(geometry, paged):
                 layer.trim(n)
         for i in range(n):
             assert_vec_close(got[1][i], got[0][i], "bfloat16", what=f"{n} rows, row {i}")
+
+
+def test_longer_splits_neither_allocate_nor_drop_the_step_s_graph():
+    """Prompts behind longer and longer prefixes take more and more shares of more rows; the room for their sums is there from the first prompt on."""
+    from proxy_inference_engine_amd.models.llama import Model, ModelArgs
+    from proxy_inference_engine_amd.models.utils import synthetic_checkpoint
+    cfg = {"model_type": "llama", "hidden_size": 256, "num_hidden_layers": 2, "intermediate_size": 512, "num_attention_heads": 32, "num_key_value_heads": 8, "head_dim": 128, "vocab_size": 320,
+           "rms_norm_eps": 1e-5, "tie_word_embeddings": False, "quantization": None}
+    m = Model(ModelArgs(**cfg), synthetic_checkpoint(cfg, seed=5))
+    m.enable_paged_kv(num_pages=80, max_blocks=40)
+    ids = torch.from_numpy(np.random.default_rng(1).integers(0, 320, 2048).astype(np.int32)).cuda()
+    cache, other = m.make_cache(), m.make_cache()
+    for n in (300, 200, 64, 40):   # every row count once without a prefix: the other buffers have their sizes
+        m.step(ids[:n], other)
+        other[0].page_manager.release()
+    m.step(ids[:300], cache), m.step(ids[300:600], cache), m.step(ids[600:900], cache)
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    for n in (40, 64, 200, 300):
+        m.step(ids[900:900 + n], cache)
+        for layer in cache:
+            layer.trim(n)
+    torch.cuda.synchronize()
+    assert torch.cuda.mem_get_info()[0] == free
