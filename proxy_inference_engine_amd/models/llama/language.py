@@ -546,6 +546,8 @@ class Model:
         valid until the next step_batch of that size; every cache advances by one position.  graph: replay a captured hipGraph
         of the step while the batch size and table width stay the same (captured on the second such step).
         The weights stream once for the whole batch: int4 models run the few-row MFMA GEMM up to 32 sequences."""
+        if torch.cuda.is_current_stream_capturing():  # the lengths on the device would not move now, those of the caches would
+            raise RuntimeError("step_batch cannot be captured: it moves the caches on the host (graph=True replays a graph of its own)")
         seqs = []
         for c in caches:
             if len(c) != len(self.layers) or not isinstance(c[0], PagedKVCache):
@@ -587,10 +589,10 @@ class Model:
             buf["key"] = key
         buf["tokens"].copy_(tokens)
         # the lengths stay on the device from step to step: a copy from the host would wait until the previous step is done and leave the GPU idle while this one is prepared
-        at = [s.offset + 1 for s in seqs]
-        if buf["at"] == [n - 1 for n in at]:
+        at, held, buf["at"] = [s.offset + 1 for s in seqs], buf["at"], None
+        if held == [n - 1 for n in at]:
             buf["ctx"].add_(1)
-        elif buf["at"] != at:
+        elif held != at:
             buf["ctx"].copy_(torch.tensor(at, dtype=torch.int32))
         buf["at"] = at
         n = len(self.layers)

@@ -89,3 +89,26 @@ def test_a_step_that_opens_a_page_reads_no_row_that_nobody_wrote(hidden, Hq, Hkv
             c[0].page_manager.release()
     assert not torch.isnan(got[0]).any()
     assert torch.equal(got[0], got[1]) and torch.equal(got[0], got[2])
+
+
+@pytest.mark.filterwarnings("ignore:The CUDA Graph is empty")
+def test_a_step_of_a_batch_refuses_a_caller_s_capture():
+    """A step moves the lengths on the device and the sequences on the host together; in a captured stream only the host's half would happen now."""
+    model = _model(512, 8, 2, 64, False, False, False)
+    model.enable_paged_kv(num_pages=16, max_blocks=4)
+    caches = [model.make_cache() for _ in range(2)]
+    for i, c in enumerate(caches):
+        model.step(torch.arange(9 + i, dtype=torch.int32, device="cuda"), c)
+    feed = torch.tensor([5, 6], dtype=torch.int32, device="cuda")
+    want = []
+    for _ in range(3):
+        want.append(model.step_batch(feed, caches, graph=False)[2].clone())
+    for c in caches:
+        for layer in c:
+            layer.trim(2)
+    assert torch.equal(model.step_batch(feed, caches, graph=False)[2], want[1])
+    with pytest.raises(RuntimeError, match="captur"):
+        with torch.cuda.graph(torch.cuda.CUDAGraph()):
+            model.step_batch(feed, caches, graph=False)
+    torch.cuda.synchronize()
+    assert torch.equal(model.step_batch(feed, caches, graph=False)[2], want[2])
