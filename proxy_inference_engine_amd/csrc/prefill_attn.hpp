@@ -229,7 +229,8 @@ __global__ void __launch_bounds__(REP * QT * 64, 2) k_prefill_attn(const Prefill
         for (int n = 0; n < NB; ++n)
 #pragma unroll
             for (int i = 0; i < 16; ++i) mloc = fmaxf(mloc, sc[n][i]);
-        mloc = xor32_max(mloc) * sl2;  // the other half of the block's keys lives in the partner lane
+        const float top = xor32_max(mloc);  // the other half of the block's keys lives in the partner lane
+        mloc = top * sl2;
         const float m_new = fmaxf(m_run, mloc);
         if (m_new > m_run) {  // rare after the first blocks
             const float alpha = attn_exp2(m_run - m_new);
@@ -240,12 +241,22 @@ __global__ void __launch_bounds__(REP * QT * 64, 2) k_prefill_attn(const Prefill
                 for (int i = 0; i < 16; ++i) oacc[dt][i] *= alpha;
             m_run = m_new;
         }
+        // one fma per score is exact against a maximum that is itself rounded: beyond 2^24 by more than one, which the exponential turns into 0 or infinity.  There
+        // the scores are rounded like their maximum first (rare: a uniform branch; a row that sees no key of the block does not ask for it)
+        float slope = sl2;
+        if (__any(fabsf(m_run) > 16777216.0f && top > ATTN_NEG)) {
+            slope = 1.0f;
+#pragma unroll
+            for (int n = 0; n < NB; ++n)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) sc[n][i] *= sl2;
+        }
         u32 phi[NB][8], plo[NB][8];
 #pragma unroll
         for (int n = 0; n < NB; ++n)
 #pragma unroll
             for (int i = 0; i < 16; i += 2) {
-                float pa = attn_exp2(fmaf(sc[n][i], sl2, -m_run)), pb = attn_exp2(fmaf(sc[n][i + 1], sl2, -m_run));
+                float pa = attn_exp2(fmaf(sc[n][i], slope, -m_run)), pb = attn_exp2(fmaf(sc[n][i + 1], slope, -m_run));
                 if (masked) pa = sees(n, i) ? pa : 0.0f, pb = sees(n, i + 1) ? pb : 0.0f;
                 l_run += pa + pb;
                 const u32 hi = pa_pack2<T>(pa, pb);

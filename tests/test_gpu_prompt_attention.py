@@ -85,3 +85,26 @@ def test_longer_splits_neither_allocate_nor_drop_the_step_s_graph():
             layer.trim(n)
     torch.cuda.synchronize()
     assert torch.cuda.mem_get_info()[0] == free
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("heads", [(2, 2), (8, 2)], ids=str)
+def test_scores_whose_rounding_is_more_than_one(heads, dtype):
+    """Scores of 2^24 to 2^36: the largest key takes all the weight, and a score's rounding (up to 2^11) must not reach the exponential.  Sums of 64 products in fp32 are good to 2^-18 of the
+    largest score, far below the distance of the two best keys for these draws, so the row is that key's value."""
+    Hq, Hkv = heads
+    g = torch.Generator().manual_seed(Hq)
+    for power in (9, 12, 15):
+        gain = 2.0 ** power if dtype == torch.float16 else 2.0 ** (power + 2)   # (float16: up to 4 x 2^15 would overflow, see the clamp)
+        q, k, v = (torch.randn(1, n, m, 64, generator=g) for n, m in ((Hq, 70), (Hkv, 130), (Hkv, 130)))
+        q, k, v = (q * gain).clamp(-6e4, 6e4).to(dtype), (k * gain).clamp(-6e4, 6e4).to(dtype), v.to(dtype)
+        got = ops.scaled_dot_product_attention(q.cuda(), k.cuda(), v.cuda(), 0.5, mask="causal").double().cpu()
+        r = Hq // Hkv
+        s = q.double() @ k.double().repeat_interleave(r, 1).transpose(-1, -2).contiguous() * 0.5
+        s = s.masked_fill(torch.arange(130)[None] > torch.arange(70)[:, None] + 60, -torch.inf)
+        want = torch.softmax(s, -1) @ v.double().repeat_interleave(r, 1)
+        top = s.topk(2, -1).values
+        clear = (top[..., 0] - top[..., 1] > 2.0 ** -16 * s.masked_fill(s == -torch.inf, 0).abs().amax(-1))
+        assert clear.float().mean() > 0.95
+        assert torch.isfinite(got).all()
+        assert ((got - want).abs().amax(-1)[clear] <= EPS[dtype] * want.abs().max()).all(), power
