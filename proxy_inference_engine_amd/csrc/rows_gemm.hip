@@ -266,7 +266,7 @@ __global__ void __launch_bounds__(512) k_rows_w16m(const RowsArgs a) {
 // matrix cores idle).  Here a workgroup of WV (eight) waves takes 16 NN features and all of K in chunks of 32 WV U columns: the chunk's rows come in as whole lines, once per workgroup
 // (registers, then one of two LDS buffers; rows padded by 16 B, conflict-free both ways), each wave multiplies every WV-th 32-column step by weights that it streams two chunks ahead.
 // Loads go by descriptors whose bounds drop what lies behind a row, a matrix or K (zeros), so no load has a branch around it.  Two workgroups of eight waves share a CU (launch bounds: 128 registers),
-// one loads while the other finishes.  Sixteen features per wave and step re-read x most (NN = 1), four blocks least: NN follows from how many workgroups are left (rows_gemm_launch).
+// one loads while the other finishes.  Sixteen features per wave and step re-read x most (NN = 1), four blocks least: NN follows from how many workgroups are left (rows_lds_pick).
 // [28672, 4096] with 8 / 16 / 32 / 64 rows: 39 / 40 / 42 / 64 us = 6.0 / 5.8 / 5.6 / 3.7 TB/s.  Experts have fewer bytes per workgroup, and workgroups of four waves (WV) fill the gaps that
 // others leave better: 60 active ones of [2816, 2048] with 3 rows each 131 (k_rows_w16m) -> 110 (eight waves) -> 103 us (6.7 TB/s), of [2048, 1408] 90 -> 58 -> 53 us.
 template <class E, int NT, int NN, int U, int WV = 8>
@@ -437,17 +437,17 @@ int rows_lds_go(RowsArgs a, int n_max, int batches, hipStream_t st) {
     return PIE_OK;
 }
 
-// Which of the two, and how many features a workgroup of k_rows_lds takes; blocks: 16-feature blocks of the whole launch.  Measured, us (k_rows_w16m / NN = 1 / 2 / 4; x in LDS wins from
-// about 5 rows on, where the rows are long enough for eight waves to share them):
-//   [28672, 4096]: 8 rows 41 / 43 / 39 / 39, 32 rows 58 / 59 / 48 / 42    [11264, 2048]: 8 rows 11.1 / 14.1 / 13.1 / 11.4, 32 rows 17.5 / 17.2 / 15.9 / 13.9    [32768, 4096]: 8 rows 47 / 49 / 42 / 45
-//   [6144, 4096]: 8 rows 13.6 / 14.6 / 12.3 / 17.5, 32 rows 17.0 / 19.1 / 15.2 / 20.3    [4096, 14336]: 8 rows 23.6 / 22.3 / 27.9 / 46.9, 32 rows 41 / 30 / 37 / 54
-// Fewer blocks than that leave CUs without a workgroup; more than 32 rows of x per CU take the room of the fourth block.
+// How many features a workgroup of k_rows_lds takes; blocks: 16-feature blocks of the whole launch.  As few as leave at most one workgroup per CU (a few more workgroups than that and most
+// CUs wait for those with two), and beyond 1024 blocks two, four where 17 to 32 rows make x the larger part.  us with NN = 1 / 2 / 4:
+//   8 rows   [4608, 2048] 10.1 / 8.2 / 10.2   [9216, 3072] 16.5 / 16.5 / 14.2   [11264, 2048] 14.0 / 13.1 / 11.4   [12320, 4096] 24.3 / 21.1 / 18.9   [18944, 4096] 31.3 / 29.9 / 34.7   [28672, 4096] 42.7 / 39.6 / 39.6
+//   20 rows  [4608, 2048] 11.0 / 9.1 / 11.7   [9216, 3072] 19.3 / 18.6 / 16.1   [11264, 2048] 15.9 / 15.0 / 12.9   [18944, 4096] 37.0 / 33.5 / 37.1   [24576, 4096] 44.5 / 35.5 / 39.3   [28672, 4096] 51.0 / 43.9 / 40.7
+// More than 32 rows of x per CU take the room of the fourth block.
 template <class E>
 int rows_lds_pick(const RowsArgs &a, int n_max, long blocks, int batches, hipStream_t st) {
     if (a.active) return rows_lds_go<E, 1, 2, 2, 4>(a, n_max, batches, st);
-    if (a.M <= 16) return blocks < 320 ? rows_lds_go<E, 1, 1, 4>(a, n_max, batches, st) : rows_lds_go<E, 1, 2, 2>(a, n_max, batches, st);
-    if (a.M <= 32)
-        return blocks < 320 ? rows_lds_go<E, 2, 1, 2>(a, n_max, batches, st) : blocks < 640 ? rows_lds_go<E, 2, 2, 2>(a, n_max, batches, st) : rows_lds_go<E, 2, 4, 1>(a, n_max, batches, st);
+    const int nn = blocks <= 256 ? 1 : blocks <= 512 ? 2 : blocks <= 1024 ? 4 : a.M <= 16 || blocks <= 1600 ? 2 : 4;
+    if (a.M <= 16) return nn == 1 ? rows_lds_go<E, 1, 1, 4>(a, n_max, batches, st) : nn == 2 ? rows_lds_go<E, 1, 2, 2>(a, n_max, batches, st) : rows_lds_go<E, 1, 4, 1>(a, n_max, batches, st);
+    if (a.M <= 32) return nn == 1 ? rows_lds_go<E, 2, 1, 2>(a, n_max, batches, st) : nn == 2 ? rows_lds_go<E, 2, 2, 2>(a, n_max, batches, st) : rows_lds_go<E, 2, 4, 1>(a, n_max, batches, st);
     return blocks < 320 ? rows_lds_go<E, 4, 1, 1>(a, n_max, batches, st) : rows_lds_go<E, 4, 2, 1>(a, n_max, batches, st);
 }
 
@@ -484,8 +484,37 @@ static bool rows_lds_reaches(const RowsArgs &a) {
     const size_t rows = a.rows ? (size_t)a.x_rows : a.gather ? (size_t)a.M : 64;
     return rows * (size_t)a.m.ldx * 2 < (1u << 31);
 }
+static long rows_blocks(const RowsArgs &a, int batches) {  // of 16 features, over the whole launch
+    long blocks = a.n_mats ? 0 : (long)batches * ((a.m.N + 15) / 16);
+    for (int i = 0; i < a.n_mats; ++i) blocks += (a.mats[i].N + 15) / 16;
+    return blocks;
+}
+// x through LDS costs a start and an end per workgroup, the operands straight into the lanes cost x again per 16 features: the latter is the faster up to so many rows, fewer the longer the
+// rows (its eight waves walk K in rounds of 2048, a part of one costs a whole one) and the better the chip is filled by k_rows_lds.  us, k_rows_w16m / k_rows_lds:
+//   up to 256 blocks   [2048, 2048] 5 rows 5.2 / 6.7, 16 rows 6.4 / 7.3, 32 rows 8.3 / 8.2   [3072, 3072] 8 rows 8.0 / 8.0, 12 rows 8.6 / 8.3   [4096, 4096] 8 rows 8.8 / 9.9, 16 rows 10.4 / 10.4
+//                      [2048, 1024] 8 rows 5.1 / 5.8, 16 rows 5.9 / 5.9   [2048, 6144] 5 rows 10.0 / 10.5, 10 rows 11.4 / 11.1
+//   up to 512          [8192, 2048] 5 rows 8.3 / 9.7, 12 rows 9.1 / 9.6, 16 rows 10.1 / 9.8   [6144, 1536] 6 rows 7.5 / 7.7, 8 rows 7.9 / 7.8   [4608, 4096] 5 rows 12.1 / 11.2
+//   up to 1024         [9216, 3072] 5 rows 16.1 / 14.1   [11264, 2048] 8 rows 11.7 / 11.4   [12320, 4096] 5 rows 21.2 / 19.0   [16384, 2048] 5 rows 13.8 / 14.5, 12 rows 15.4 / 14.6
+//   beyond             [16896, 2048] 8 rows 16.0 / 17.9, 12 rows 17.5 / 18.3, 16 rows 19.4 / 18.4   [18944, 4096] 5 rows 27.8 / 29.7, 10 rows 31.3 / 30.3   [24576, 2048] 5 rows 19.5 / 21.2, 10 rows 20.5 / 20.1
+//                      [28672, 4096] 5 rows 38.9 / 39.4, 8 rows 41.3 / 39.6   [32768, 2048] 5 rows 24.6 / 25.0, 8 rows 25.6 / 24.9
+static bool rows_direct_faster(int M, int K, long blocks) {
+    const long rounds = (K + 2047) / 2048, rows = blocks <= 256 ? 26 : blocks <= 512 ? 10 : blocks <= 1024 ? 0 : blocks <= 1280 ? 13 : blocks <= 1600 ? 10 : 0;  // (at K = 2048)
+    return M * rounds * rounds * 2048 < rows * K;
+}
 static bool rows_lds_serves(const RowsArgs &a, int n_max, int k_max, int batches) {
-    return a.M > 4 && k_max >= 1024 && !rows_narrow(a, n_max, batches) && !a.x_norm && a.merge.splits <= 0 && rows_lds_reaches(a);
+    if (a.M <= 4 || k_max < 1024 || rows_narrow(a, n_max, batches) || a.x_norm || a.merge.splits > 0 || !rows_lds_reaches(a)) return false;
+    return a.active || !rows_direct_faster(a.M, k_max, rows_blocks(a, batches));
+}
+template <class E>
+static int rows_launch(const RowsArgs &a, int n_max, int k_max, int batches, hipStream_t st) {
+    if (rows_lds_serves(a, n_max, k_max, batches)) return rows_lds_pick<E>(a, n_max, rows_blocks(a, batches), batches, st);
+    if (a.M <= 16 || a.active || rows_narrow(a, n_max, batches)) return rows_go<E, 1, 1>(a, n_max, k_max, batches, st);
+    int n_all = batches == 1 ? n_max : 0;
+    for (int i = 0; i < a.n_mats; ++i) n_all += a.mats[i].N;
+    const bool wide = n_all >= 32 * 140;  // two feature blocks per wave where half as many workgroups still fill most of the chip
+    if (a.M <= 32) return wide ? rows_go<E, 2, 2>(a, n_max, k_max, batches, st) : rows_go<E, 2, 1>(a, n_max, k_max, batches, st);
+    if constexpr (__is_same(E, ElemBF16)) return wide ? rows_go<E, 4, 2>(a, n_max, k_max, batches, st) : rows_go<E, 4, 1>(a, n_max, k_max, batches, st);
+    else return pie::fail(PIE_E_SHAPE, "few-row 16-bit Linear: at most 32 rows");
 }
 
 size_t rows_weight_bytes(int dtype, int N, int K) {
@@ -514,21 +543,7 @@ int rows_gemm_launch(int dtype, const RowsArgs &a, int batches, hipStream_t st) 
     PIE_REQUIRE(a.merge.splits <= 64 && (a.merge.splits <= 0 || (a.merge.M == a.M && a.M <= MERGE_ROWS && a.merge.ldr <= MERGE_LDR && a.merge.ldr % 8 == 0 && !a.active && !a.rows)), PIE_E_SHAPE,
                 "row-wise Linear: too many rows or columns to merge key splits on the way in");
     PIE_REQUIRE(a.m.ldx % 8 == 0 && a.x_batch % 8 == 0 && pie_aligned(a.m.x, 16) && pie_aligned(a.m.w, 16), PIE_E_ALIGN, "row-wise Linear: 16-byte alignment required");
-    int n_all = batches == 1 ? n_max : 0;
-    for (int i = 0; i < a.n_mats; ++i) n_all += a.mats[i].N;
-    long blocks = 0;  // of 16 features, over the whole launch
-    for (int i = 0; i < a.n_mats; ++i) blocks += (a.mats[i].N + 15) / 16;
-    if (!a.n_mats) blocks = (long)batches * ((a.m.N + 15) / 16);
-    if (rows_lds_serves(a, n_max, k_max, batches)) return rows_lds_pick<ElemBF16>(a, n_max, blocks, batches, st);
-    if (a.M <= 16 || a.active || rows_narrow(a, n_max, batches)) return rows_go<ElemBF16, 1, 1>(a, n_max, k_max, batches, st);
-    const bool wide = n_all >= 32 * 140;  // two feature blocks per wave where half as many workgroups still fill most of the chip
-    if (a.M <= 32) return wide ? rows_go<ElemBF16, 2, 2>(a, n_max, k_max, batches, st) : rows_go<ElemBF16, 2, 1>(a, n_max, k_max, batches, st);
-    return wide ? rows_go<ElemBF16, 4, 2>(a, n_max, k_max, batches, st) : rows_go<ElemBF16, 4, 1>(a, n_max, k_max, batches, st);
-}
-
-template <class E>
-static int rows_w16_go(const RowsArgs &a, hipStream_t st) {
-    return a.M > 4 && a.m.K >= 1024 ? rows_lds_pick<E>(a, a.m.N, (a.m.N + 15) / 16, 1, st) : rows_go<E, 1, 1>(a, a.m.N, a.m.K, 1, st);
+    return rows_launch<ElemBF16>(a, n_max, k_max, batches, st);
 }
 
 int rows_w16_launch(int dtype, const void *w16m, const void *x, int M, int N, int K, void *y, const void *bias, bool swiglu, hipStream_t st) {
@@ -539,7 +554,7 @@ int rows_w16_launch(int dtype, const void *w16m, const void *x, int M, int N, in
     RowsArgs a = {};
     a.m = {(const char *)w16m, N, K, x, K, y, swiglu ? N / 2 : N};
     a.M = M, a.epi = swiglu ? ROWS_SWIGLU : ROWS_LINEAR, a.bias = (const u16 *)bias;
-    return dtype == PIE_F16 ? rows_w16_go<ElemF16>(a, st) : rows_w16_go<ElemBF16>(a, st);
+    return dtype == PIE_F16 ? rows_launch<ElemF16>(a, N, K, 1, st) : rows_launch<ElemBF16>(a, N, K, 1, st);
 }
 
 extern "C" {

@@ -62,6 +62,33 @@ def test_dense_llama_step_of_several_rows(dtype, vocab):
             c[0].page_manager.release()
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("inter,vocab", [(1472, 330), (5632, 16900)])
+def test_dense_llama_step_on_both_sides_of_the_choice_of_kernel(dtype, inter, vocab):
+    """Rows of 2048 columns, where the number of rows decides between the two kernels: 26 from 256 blocks of features down, 10 or 13 for wider products, and every choice of features per
+    workgroup up to 32 rows.  Each sequence's first step alone (the GEMV) is the reference; bounds as above."""
+    from _util import assert_vec_close
+    from proxy_inference_engine_amd.models.llama import Model, ModelArgs
+    from proxy_inference_engine_amd.models.utils import synthetic_checkpoint
+    cfg = {"model_type": "llama", "hidden_size": 2048, "num_hidden_layers": 1, "intermediate_size": inter, "num_attention_heads": 16, "num_key_value_heads": 4, "head_dim": 128,
+           "vocab_size": vocab, "rms_norm_eps": 1e-5, "tie_word_embeddings": False, "attention_bias": True, "mlp_bias": True, "quantization": None}
+    m = Model(ModelArgs(**cfg), synthetic_checkpoint(cfg, seed=2, dtype=dtype))
+    m.enable_paged_kv(num_pages=40, max_blocks=1)
+    feed = torch.from_numpy(np.random.default_rng(3).integers(0, vocab, 32).astype(np.int32)).cuda()
+    want = []
+    for i in range(32):
+        c = m.make_cache()
+        want.append(m.step(feed[i:i + 1], c)[2].float().cpu().numpy().reshape(-1))
+        c[0].page_manager.release()
+    for B in (5, 9, 10, 12, 13, 16, 17, 25, 26, 32):
+        caches = [m.make_cache() for _ in range(B)]
+        got = m.step_batch(feed[:B], caches, graph=False)[2].float().cpu().numpy()
+        for i in range(B):
+            assert_vec_close(got[i], want[i], "bfloat16" if dtype == torch.bfloat16 else "float16", what=f"B {B} row {i}")
+        for c in caches:
+            c[0].page_manager.release()
+
+
 @pytest.mark.parametrize("bits", [None, 8, 4], ids=["dense", "int8", "int4"])
 def test_a_head_changed_in_place_is_seen_after_set_globals(bits):
     """The head's tiles stay with the decoder; pie_decoder_set_globals says that the weights behind its pointers are others.  Batch steps, eager and replayed, and prompts with logits

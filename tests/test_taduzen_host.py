@@ -124,3 +124,17 @@ def test_rows_picked_from_more_than_2_gib_take_the_kernel_with_64_bit_addresses(
         assert lds(M, 32768, 32768, 32768) == 0 and lds(M, 32768, 32896, 32650) == 0 and lds(M, 32768, 32768, 65535) == 0
         assert lds(M, 16384, 16384, 65535) == 1 and lds(M, 16384, 16400, 65535) == 0
     assert _ffi.base().pie_stack_linear_kernel(0, 1, 1, 1, 0) < 0
+
+
+def test_few_rows_take_the_kernel_that_is_faster_for_their_size():
+    """Short rows of x and few of them: both operands straight into the lanes; long ones, more of them, or a chip that the other kernel fills: x through LDS."""
+    from proxy_inference_engine_amd import _ffi
+
+    def lds(M, N, K):
+        return _ffi.base().pie_stack_linear_kernel(M, N, K, K, 0)
+    assert [lds(M, 2048, 2048) for M in (4, 5, 8, 16, 25, 26, 64)] == [0, 0, 0, 0, 0, 1, 1]
+    assert [lds(M, 4096, 4096) for M in (5, 12, 13, 32)] == [0, 0, 1, 1]
+    assert [lds(M, 3072, 3072) for M in (8, 9, 10)] == [0, 0, 1] and [lds(M, 4096, 14336) for M in (4, 5)] == [0, 1]
+    assert [lds(M, 8192, 2048) for M in (9, 10)] == [0, 1] and [lds(M, 6144, 4096) for M in (4, 5)] == [0, 1]
+    assert [lds(M, 11264, 2048) for M in (4, 5, 64)] == [0, 1, 1] and [lds(M, 16896, 2048) for M in (12, 13)] == [0, 1]
+    assert [lds(M, 28672, 4096) for M in (4, 5)] == [0, 1] and lds(64, 1024, 4096) == 0 and lds(64, 4096, 1000) == 0
