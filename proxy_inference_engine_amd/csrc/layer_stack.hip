@@ -1084,12 +1084,12 @@ void feed_forward(Pass &p, int li, const pie_stack_layer &L, const Into &into, b
         const int groups = (int)std::min((long)L.experts, (long)M * L.top) + (S ? 1 : 0);
         RowsArgs u = {};
         u.m = {(const char *)L.w_gate_up, 2 * F, W, s->h.p, WA, s->act_e.p, FA};
-        u.M = M, u.epi = clipped ? ROWS_CLIP_MUL : ROWS_SILU_MUL, u.act_alpha = L.act_alpha, u.act_limit = L.act_limit, u.w_batch = gu_stride, u.active = r.active, u.offset = r.offset, u.list = r.list, u.gather = true;
+        u.M = M, u.epi = clipped ? ROWS_CLIP_MUL : ROWS_SILU_MUL, u.act_alpha = L.act_alpha, u.act_limit = L.act_limit, u.w_batch = gu_stride, u.active = r.active, u.offset = r.offset, u.list = r.list, u.mean_rows = M * L.top / L.experts, u.gather = true;
         if (S) u.shared = {(const char *)L.s_gate_up, 2 * S, W, s->h.p, WA, s->act_s.p, SA};
         p.linear(u, groups);
         RowsArgs d = {};
         d.m = {(const char *)L.w_expert_down, W, F, s->act_e.p, FA, s->part.p, W64};
-        d.M = M, d.epi = ROWS_SCALE_F32, d.scale = 1.0f, d.w_batch = dn_stride, d.active = r.active, d.offset = r.offset, d.list = r.list;
+        d.M = M, d.epi = ROWS_SCALE_F32, d.scale = 1.0f, d.w_batch = dn_stride, d.active = r.active, d.offset = r.offset, d.list = r.list, d.mean_rows = u.mean_rows;
         if (S) d.shared = {(const char *)L.s_down, W, S, s->act_s.p, SA, s->part_s.p, W64};
         p.linear(d, groups);
         if (p.rc) return;

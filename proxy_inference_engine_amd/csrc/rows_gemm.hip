@@ -327,7 +327,7 @@ __global__ void __launch_bounds__(64 * WV, 4) k_rows_lds(const RowsArgs a) {
             for (int u = 0; u < U; ++u) {
                 const int s = (it * U + u) * WV + wave;
 #pragma unroll
-                for (int n = 0; n < NN; ++n)  // non-temporal: a pass reads a weight once
+                for (int n = 0; n < NN; ++n)  // non-temporal: a weight is read once, except an expert's with more than 16 NT rows
                     wv[u][n] = __builtin_amdgcn_raw_buffer_load_b128(wr, s < steps ? wlane + (unsigned)((n >> 1) * groups * 4096 + s * 2048 + (n & 1) * 256) : NOWHERE, 0, 2);
             }
         };
@@ -437,6 +437,13 @@ int rows_lds_go(RowsArgs a, int n_max, int batches, hipStream_t st) {
     return PIE_OK;
 }
 
+// Experts: blocks of 16 rows, or of 32 where many rows would make a workgroup go through its weights twice -- the shared expert's, which has all rows of the pass (beside so many other experts
+// that it does not matter, 16 stay), or the experts' own.  From two rounds of workgroups on (four a CU) chunks of half the length.  us, 16 / 32 rows in long / 32 in short chunks:
+//   64 experts, 6 a row, shared beside   [2816, 2048] 17 rows 92.4 / 91.3 / 91.0, 32 rows 110.8 / 109.0 / 109.3, 64 rows 126.6 / 121.0 / 121.8   [2048, 1408] 32 rows 57.2 / 60.0 / 56.2, 64 rows 68.3 / 66.6 / 63.4
+//   8 experts, 2 a row   shared [7168, 2048] 17 rows 48.4 / 44.7 / 45.1, 64 rows 83.3 / 53.7 / 52.6   none 32 rows 38.2 / 41.9 / 41.6, 48 rows 50.0 / 42.8 / 42.4   shared [2048, 3584] 17 rows 34.6 / 28.6 / 25.5
+//   16 experts, 2 a row, shared [2048, 2816] beside [2048, 1408]   17 rows 26.7 / 21.8 / 22.7, 64 rows 42.5 / 30.4 / 36.6      128 experts, 8 a row, shared [1536, 2048]   20 rows 86.1 / 88.3 / 87.9
+static bool rows_lds_two(const RowsArgs &a, int batches) { return a.M > 16 && ((a.shared.w && batches <= 65) || a.mean_rows >= 12); }
+
 // How many features a workgroup of k_rows_lds takes; blocks: 16-feature blocks of the whole launch.  As few as leave at most one workgroup per CU (a few more workgroups than that and most
 // CUs wait for those with two), and beyond 1024 blocks two, four where 17 to 32 rows make x the larger part.  us with NN = 1 / 2 / 4:
 //   8 rows   [4608, 2048] 10.1 / 8.2 / 10.2   [9216, 3072] 16.5 / 16.5 / 14.2   [11264, 2048] 14.0 / 13.1 / 11.4   [12320, 4096] 24.3 / 21.1 / 18.9   [18944, 4096] 31.3 / 29.9 / 34.7   [28672, 4096] 42.7 / 39.6 / 39.6
@@ -444,7 +451,11 @@ int rows_lds_go(RowsArgs a, int n_max, int batches, hipStream_t st) {
 // More than 32 rows of x per CU take the room of the fourth block.
 template <class E>
 int rows_lds_pick(const RowsArgs &a, int n_max, long blocks, int batches, hipStream_t st) {
-    if (a.active) return rows_lds_go<E, 1, 2, 2, 4>(a, n_max, batches, st);
+    if (a.active) {
+        if (!rows_lds_two(a, batches)) return rows_lds_go<E, 1, 2, 2, 4>(a, n_max, batches, st);
+        const long wgs = (long)(batches - (a.shared.w != nullptr)) * ((a.m.N + 31) / 32) + (a.shared.w ? (a.shared.N + 31) / 32 : 0);
+        return wgs < 2048 ? rows_lds_go<E, 2, 2, 2, 4>(a, n_max, batches, st) : rows_lds_go<E, 2, 2, 1, 4>(a, n_max, batches, st);
+    }
     const int nn = blocks <= 256 ? 1 : blocks <= 512 ? 2 : blocks <= 1024 ? 4 : a.M <= 16 || blocks <= 1600 ? 2 : 4;
     if (a.M <= 16) return nn == 1 ? rows_lds_go<E, 1, 1, 4>(a, n_max, batches, st) : nn == 2 ? rows_lds_go<E, 1, 2, 2>(a, n_max, batches, st) : rows_lds_go<E, 1, 4, 1>(a, n_max, batches, st);
     if (a.M <= 32) return nn == 1 ? rows_lds_go<E, 2, 1, 2>(a, n_max, batches, st) : nn == 2 ? rows_lds_go<E, 2, 2, 2>(a, n_max, batches, st) : rows_lds_go<E, 2, 4, 1>(a, n_max, batches, st);

@@ -331,6 +331,7 @@ struct RowsArgs {
     int x_batch, y_batch;  // elements
     // grouped over blockIdx.y (experts): active[y] = expert or -1; its rows are list[offset[e] .. offset[e + 1])
     const int *active, *offset, *list;
+    int mean_rows;         // grouped: rows of an expert in the mean
     bool gather;           // grouped: x row = list[position] (else x row = position); y row = position always
     RowsMat shared;        // blockIdx.y == batches - 1 when shared.w: all M rows, this matrix (the expert every token takes)
     const int *rows;       // ungrouped, nullable: x row of result row i

@@ -27,6 +27,22 @@ def test_stack_linears_against_the_oracle(vocab):
         assert tu.err(got, orc.forward(cfg, wn, ids)) < 0.04, n
 
 
+def test_mixtures_whose_shared_expert_has_more_rows_than_a_block():
+    """64 experts and a shared one, 17 to 64 rows: blocks of 32 rows, in long chunks (17 rows: fewer than 2048 workgroups) and short ones.  The same tokens four at a time take the kernel
+    without LDS; bounds as above."""
+    from proxy_inference_engine_amd.models.taduzen import Model, ModelArgs
+    cfg = tu.config([(tu.latent(heads=2, rank=40), tu.moe(ff=512, experts=64, top=3, shared=640))], width=1096, vocab=200)
+    m = Model(ModelArgs(**cfg), {k: v.cuda() for k, v in tu.weights(cfg, seed=9).items()}, dtype=torch.bfloat16)
+    m.enable_paged_kv(num_pages=8)
+    ids, c = tu.tokens(cfg, 64, seed=3), m.make_cache()
+    want = np.concatenate([m.step_portions([(ids[i:i + 4], c)], [list(range(4))]).cpu().numpy() for i in range(0, 64, 4)])
+    c[0].page_manager.release()
+    for n in (17, 32, 33, 49, 64):
+        got = m.step_portions([(ids[:n], c)], [list(range(n))]).cpu().numpy()
+        c[0].page_manager.release()
+        assert tu.err(got, want[:n]) < 0.04, n
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
 @pytest.mark.parametrize("vocab", [330, 5210, 10260])
 def test_dense_llama_step_of_several_rows(dtype, vocab):
