@@ -92,7 +92,7 @@ static bool w16_narrow(int tn, int tm) { return tn < 8 && tm >= 8; }  // column 
 // no_split: one pass over K; two: two strips per wave
 static W16Plan w16_plan(int M, int N, int K, bool no_split = false, bool two = false) {
     const int groups = (K + 63) / 64;
-    if (g_w16_plan_override[0]) return {g_w16_plan_override[0], g_w16_plan_override[1], w16_even_splits(groups, g_w16_plan_override[2])};
+    if (g_w16_plan_override[0]) return {g_w16_plan_override[0], g_w16_plan_override[1], no_split ? 1 : w16_even_splits(groups, g_w16_plan_override[2])};
     const int mb_max = M <= 64 ? 2 : (M <= 128 ? 4 : 8);
     W16Plan best = {mb_max, 2, 1};
     double best_us = 1e30;
