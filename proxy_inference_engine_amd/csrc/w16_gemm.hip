@@ -72,7 +72,8 @@ int w16m_from_w16s_launch(const void *w16s, int N, int K, void *w16m, hipStream_
 // the 256 MB behind the L2s it preferred plans up to 1.4 times slower).  A K step of a (32 mb) x (128 sw) tile costs t(mb, sw) us -- larger tiles are cheaper per MFMA but quantise worse --
 // and no less than its weights take from beyond the caches, which the row tiles of a column share; workgroups run in rounds of 256, counted on the XCD that has most; all weights come
 // once through HBM (5.6 TB/s); a launch costs 5.8 us of ramp, prologue and epilogue; a K split writes and re-reads its fp32 slabs and launches the reduce.  Over those products its choices
-// take 1.4 % longer than the best ones (those of the model before: 6.2 %); [4096, 14336]: 64 / 128 / 509 / 1024 rows 40 / 40 / 91 / 123 -> 34 / 34 / 67 / 113 us.
+// take 1.4 % longer than the best ones (those of the model before: 6.2 %); over 563 products of 40 matrices, most of them others, 1.9 % (6.4 %).  Up to K = 2048 the reduce's launch has little to hide behind:
+// [1024, 1024], 450 rows: 6.5 us, in two splits 8.8; [1280, 1280], 320 rows: 7.7, 9.5.  [4096, 14336]: 64 / 128 / 509 / 1024 rows 40 / 40 / 91 / 123 -> 34 / 34 / 67 / 113 us.
 struct W16Plan {
     int mb, sw, S;
 };
@@ -112,7 +113,7 @@ static W16Plan w16_plan(int M, int N, int K, bool no_split = false, bool two = f
                 const double t = t_light[mi][sw] + (t_full[mi][sw] - t_light[mi][sw]) * load;
                 double us = (most + 31) / 32 * steps * (t > cold ? t : cold);
                 us = (us > stream_us ? us : stream_us) + 5.8;
-                if (S > 1) us += (double)M * N * 4.0 * (2 * S + 0.5) / 5.1e6 + 0.6;
+                if (S > 1) us += (double)M * N * 4.0 * (2 * S + 0.5) / 5.1e6 + (groups <= 32 ? 3.5 : 1.0);
                 if (us < best_us) best_us = us, best = {mb, sw, S};
             }
     best.S = w16_even_splits(groups, best.S);

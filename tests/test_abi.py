@@ -79,3 +79,13 @@ def test_no_library_gemm_behind_the_c_abi():
     assert lib.pie_w16m_bytes(1280, 3420) == 40 * 54 * 4096 and lib.pie_w16m_bytes(0, 64) == 0   # 32-row x 64-column tiles, zero-padded
     assert lib.pie_linear_w16m_workspace(4096, 6144, 4096) == 0                                    # no K split where the tiles fill the chip
     assert lib.pie_linear_w16m_workspace(64, 4096, 14336) % (64 * 4096 * 4) == 0 and lib.pie_linear_w16m_workspace(64, 4096, 14336) > 0
+
+
+def test_short_products_are_not_split_along_k():
+    """Up to K = 2048 the second launch of a split costs more than the split saves; long rows of few features are split (a split asks for a workspace)."""
+    from proxy_inference_engine_amd import _ffi
+    ws = _ffi.base().pie_linear_w16m_workspace
+    for M, N, K in [(450, 1024, 1024), (509, 1000, 1152), (320, 1280, 1280), (33, 8192, 1024), (509, 1280, 2048), (450, 2048, 2048)]:
+        assert ws(M, N, K) == 0, (M, N, K)
+    for M, N, K in [(64, 4096, 14336), (64, 4096, 4096), (509, 64, 4096), (40, 1000, 4096)]:
+        assert ws(M, N, K) > 0, (M, N, K)

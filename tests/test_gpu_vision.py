@@ -106,7 +106,7 @@ def test_fused_gate_up_linear_is_the_gemm_followed_by_bias_silu_mul(ops, dt, M, 
     assert torch.equal(ops.linear_rows(padded, ops.pack_linear(dw)), ops.linear_rows(got, dw))
 
 
-@pytest.mark.parametrize("M,N,K,pad", [(40, 1000, 1152, 64), (300, 1000, 1152, 64), (129, 1176, 1280, 32), (509, 36, 4096, 64), (33, 1000, 1152, 1000)])
+@pytest.mark.parametrize("M,N,K,pad", [(40, 1000, 1152, 64), (300, 1000, 1152, 64), (129, 1176, 1280, 32), (509, 36, 4096, 64), (33, 1000, 1152, 1000), (64, 1000, 4096, 64), (40, 1176, 3456, 32)])
 def test_padded_rows_of_shapes_that_would_split_k(ops, M, N, K, pad):
     """linear_rows(..., pad_to=...): rows wider than the matrix take one pass over K, whatever the plan for packed rows is.  One rounding of a sum of K products that is good to
     K 2^-24 of its terms: half an ulp of the largest result, under 2^-8 of it."""
