@@ -479,9 +479,10 @@ static void reserve_attn_part(pie_decoder *d) {
     if (d->prefill->attn_part || 512 / c.n_kv_heads < 2) return;
     if (hipMalloc((void **)&d->prefill->attn_part, prefill_attn_part_bytes(c.n_heads, c.n_kv_heads, c.head_dim)) != hipSuccess) (void)hipGetLastError(), d->prefill->attn_part = nullptr;
 }
-// A prompt's attention split along the keys where that pays (before: keys cached in front of the first row)
+// How a prompt's attention is launched: split along the keys where that pays (before: keys cached in front of the first row)
 static void split_attn(pie_decoder *d, PrefillAttnArgs &a, int before) {
     const int splits = d->prefill->attn_part ? prefill_attn_splits(a.M, before, a.Hkv) : 1;
+    a.before = before;
     if (splits > 1) a.splits = splits, a.part = d->prefill->attn_part;
 }
 
@@ -845,7 +846,7 @@ extern "C" int pie_sdpa_prefill(const void *q, const void *k, const void *v, int
     PIE_REQUIRE(Hkv > 0 && Hq % Hkv == 0 && Hq / Hkv <= 8, PIE_E_SHAPE, "pie_sdpa_prefill: n_heads / n_kv_heads must be between 1 and 8");
     PIE_REQUIRE(pie_aligned(q, 16) && pie_aligned(k, 16) && pie_aligned(v, 16) && pie_aligned(out, 8), PIE_E_ALIGN, "pie_sdpa_prefill: misaligned pointer");
     PrefillAttnArgs a = {};
-    a.q = (const u16 *)q, a.k = (const u16 *)k, a.v = (const u16 *)v, a.offset = offset, a.cap = cap;
+    a.q = (const u16 *)q, a.k = (const u16 *)k, a.v = (const u16 *)v, a.offset = a.before = offset, a.cap = cap;
     a.M = L, a.Hq = Hq, a.Hkv = Hkv, a.scale = scale, a.out = (u16 *)out;
     if (dtype == PIE_BF16) return prefill_attn_launch_t<BF16>(a, D, (hipStream_t)stream);
     if (dtype == PIE_F16) return prefill_attn_launch_t<F16>(a, D, (hipStream_t)stream);

@@ -46,6 +46,7 @@ struct PrefillAttnArgs {
     const int *seg_lo, *seg_hi;
     const int *block_table;              // paged KV (nullable, decoder only): kv_table holds the layers' slab K / V bases; key t
     int n_pages;                         //   lives in page block_table[t / 64] (each [Hkv, 64, D]) at row t % 64
+    int before;                          // keys in front of the first row, as far as the host knows (plans the launch; the device's position decides)
     int splits;                          // SPLIT instantiation: workgroups along the keys (gridDim.y); their partial sums meet in k_prefill_combine
     float *part;                         //   [M, Hq, splits] x {[D] weighted sums}, then [M, Hq, splits] x {running max, sum}
 };
@@ -91,9 +92,10 @@ __device__ __forceinline__ int pa_off(int row, int ch) {
 // tile, [REP, 2 REP) the second -- and one staged K/V block serves 64 query rows: half the L2 -> LDS traffic and barriers per
 // unit of work, at the same number of waves per CU (one 8-wave workgroup instead of two 4-wave ones for REP = 4).
 // SPLIT: blockIdx.y takes its share of the tile's key blocks and leaves its sums to k_prefill_combine (prefill_attn_splits says when).
-template <class T, int D, int REP, int QT, bool SEG = false, bool SPLIT = false>
+// SHORT: blocks of 32 keys, for prompts that fill few of 64 (prefill_attn_short).
+template <class T, int D, int REP, int QT, bool SEG = false, bool SPLIT = false, bool SHORT = false>
 __global__ void __launch_bounds__(REP * QT * 64, 2) k_prefill_attn(const PrefillAttnArgs a) {
-    constexpr int NT = REP * QT * 64, NB = NT >= 256 ? 2 : 1, BK = 32 * NB;  // keys per block: 64 where enough threads share their loads
+    constexpr int NT = REP * QT * 64, NB = NT >= 256 && !SHORT ? 2 : 1, BK = 32 * NB;  // keys per block: 64 where enough threads share their loads
     constexpr int CH = D / 8, KS = D / 16, DT = D / 32;                      // chunks per row, k-steps of Q.K^T, 32-dim output tiles
     constexpr int BM = 32 * QT;
     constexpr int CPT = (BK * CH + NT - 1) / NT;                                   // 16-byte chunks per thread and tile
@@ -351,6 +353,10 @@ static inline int prefill_attn_splits(int M, int before, int Hkv) {
 // room for the sums of any split prompt: ceil(M / 32) Hkv splits <= 512
 static inline size_t prefill_attn_part_bytes(int Hq, int Hkv, int D) { return (size_t)(512 / Hkv) * 32 * Hq * (D + 2) * sizeof(float); }
 
+// A block of 64 keys costs its whole chain however few of them there are.  us in blocks of 32 / 64 keys, 32 / 8 heads of 128: 8 rows 5.7 / 6.7, 20 rows 6.5 / 7.6, 33 rows 7.4 / 8.4,
+// 48 rows 7.6 / 8.4, 64 rows 8.8 / 8.4; 32 / 4 heads: 8 rows 6.4 / 7.6, 33 rows 9.6 / 10.6, 64 rows 10.7 / 10.5.
+static inline bool prefill_attn_short(const PrefillAttnArgs &a) { return a.M + a.before <= 56; }
+
 template <class T, int D>
 static int prefill_attn_launch_d(const PrefillAttnArgs &a, hipStream_t st) {
     const int rep = a.Hq / a.Hkv;
@@ -378,10 +384,11 @@ static int prefill_attn_launch_d(const PrefillAttnArgs &a, hipStream_t st) {
     const int qt = pie_knob(PIE_KNOB_PREFILL_QT);  // test knob: 1 forces one 32-row query tile per workgroup, 2 forces two wherever they fit
     // 2 tiles need 2*rep <= 8 waves of up to 256 registers, and only pay while the halved grid still fills the 256 CUs
     // (8B model: 4096 tokens 54.9 -> 53.9 ms, 8000 tokens 126.3 -> 125.0 ms; at 1024 tokens it would idle half the chip)
-    const bool two = rep <= 4 && a.M > 32 && (qt > 0 ? qt == 2 : ((a.M + 63) / 64) * a.Hkv >= 256);
+    const bool two = rep <= 4 && a.M > 32 && (qt > 0 ? qt == 2 : ((a.M + 63) / 64) * a.Hkv >= 256), few = prefill_attn_short(a);
     const dim3 grid(((a.M + (two ? 63 : 31)) / (two ? 64 : 32)) * a.Hkv);
 #define PA_LAUNCH(R)                                                                                         \
     if (two && R <= 4) hipLaunchKernelGGL((k_prefill_attn<T, D, R, (R <= 4 ? 2 : 1)>), grid, dim3(R * 128), 0, st, a); \
+    else if (few && R >= 4) hipLaunchKernelGGL((k_prefill_attn<T, D, R, 1, false, false, (R >= 4)>), grid, dim3(R * 64), 0, st, a); \
     else hipLaunchKernelGGL((k_prefill_attn<T, D, R, 1>), grid, dim3(R * 64), 0, st, a);                     \
     break
     switch (rep) {

@@ -28,6 +28,22 @@ def test_causal_rows_against_float64(heads, D, dtype):
         assert (got - want).abs().max() <= EPS[dtype] * want.abs().max(), (L, off, scale)
 
 
+@pytest.mark.parametrize("heads", [(4, 1), (8, 2), (5, 1), (8, 1)], ids=str)
+@pytest.mark.parametrize("D", [64, 128])
+def test_short_prompts_against_float64(heads, D):
+    """Up to 56 keys in blocks of 32, 57 in blocks of 64, a second tile of rows, a few cached keys; bound as above."""
+    Hq, Hkv = heads
+    g = torch.Generator().manual_seed(D + Hq)
+    for L, off in ((3, 0), (33, 0), (48, 0), (56, 0), (57, 0), (20, 36), (20, 37), (40, 9)):
+        q, k, v = (torch.randn(1, n, m, D, generator=g).to(torch.bfloat16) for n, m in ((Hq, L), (Hkv, off + L), (Hkv, off + L)))
+        got = ops.scaled_dot_product_attention(q.cuda(), k.cuda(), v.cuda(), 0.3, mask="causal").double().cpu()
+        r = Hq // Hkv
+        s = q.double() @ k.double().repeat_interleave(r, 1).transpose(-1, -2).contiguous() * 0.3
+        s = s.masked_fill(torch.arange(off + L)[None] > torch.arange(L)[:, None] + off, -torch.inf)
+        want = torch.softmax(s, -1) @ v.double().repeat_interleave(r, 1)
+        assert (got - want).abs().max() <= EPS[torch.bfloat16] * want.abs().max(), (L, off)
+
+
 @pytest.mark.parametrize("paged", [False, True], ids=["contiguous", "paged"])
 @pytest.mark.parametrize("geometry", [(8, 2, 64), (8, 1, 128), (2, 2, 128)], ids=str)
 def test_rows_behind_a_prefix_split_along_the_keys(geometry, paged):
