@@ -299,7 +299,7 @@ int pie_decoder_set_paged_kv(pie_decoder *d, const void *const *slabs, size_t n_
                              void *stream);
 /* One decode step for B sequences at once over the paged KV pool (continuous batching): the weights stream once for all rows;
  * row s is its own sequence -- input token tokens[s], attending context_lens[s] positions INCLUDING the new one (its position is
- * context_lens[s] - 1; 0 = idle slot), K / V appended to page block_tables[s][pos / 64] of every layer's slab (slabs: HOST array
+ * context_lens[s] - 1; 0 = idle slot; no two rows of one sequence: a row need not see what another appends in the same step), K / V appended to page block_tables[s][pos / 64] of every layer's slab (slabs: HOST array
  * [n_layers] of device pointers), attention over its own table row.  Outputs per row: logits T [B, vocab], logprobs fp32
  * [B, vocab], next_tokens int32 [B] (greedy).  What the reference's decode-state batch is meant to be (BatchDetails,
  * include/engine/batch_details.hpp:10-88; Scheduler and the paged attention kernel are skeletons there).  Independent of
@@ -358,6 +358,8 @@ int pie_decoder_prefill(pie_decoder *d, const int32_t *ids, int L, void *logits_
  * features (models/intern/ensemble.py:33-91, :106-108).  Always the batched path, whatever L -- except on int8 pages (PIE_OPT_KV_I8 with a
  * paged cache), where the rows run as decode steps like a prompt of tokens does there. */
 int pie_decoder_prefill_embeds(pie_decoder *d, const void *embeds, int L, void *logits_all, void *stream);
+/* Into how many shares of the keys the attention of the last prompt (or chunk behind a cached prefix) was split; 1: not split, 0: none ran yet. */
+int pie_decoder_prompt_shares(const pie_decoder *d);
 /* Output buffers of the step, allocated by the caller (device): logits T [vocab], logprobs fp32 [vocab],
  * token int32 [1] (the greedy choice), hidden T [hidden] (the residual stream; after a step it holds the
  * output of the last block, the input of the final norm).  history (optional, int32 [history_len]): the tail

@@ -359,6 +359,7 @@ struct PrefillScratch {
     void *w4l_ws = nullptr;   // fp32 partial tiles of the K-split prompt GEMM (w4m_gemm.hip)
     size_t w4l_ws_bytes = 0;
     float *attn_part = nullptr;  // sums of prompt attention split along the keys (reserve_attn_part)
+    int last_shares = 0;         // pie_decoder_prompt_shares
     int resident_mode = -1;   // -1: budget not fixed yet
     size_t resident_left = 0; // bytes still available for resident copies
 };
@@ -482,7 +483,7 @@ static void reserve_attn_part(pie_decoder *d) {
 // How a prompt's attention is launched: split along the keys where that pays (before: keys cached in front of the first row)
 static void split_attn(pie_decoder *d, PrefillAttnArgs &a, int before) {
     const int splits = d->prefill->attn_part ? prefill_attn_splits(a.M, before, a.Hkv) : 1;
-    a.before = before;
+    a.before = before, d->prefill->last_shares = splits;
     if (splits > 1) a.splits = splits, a.part = d->prefill->attn_part;
 }
 
@@ -836,6 +837,8 @@ static int prefill_t(pie_decoder *d, const int32_t *ids, const void *embeds, int
     if ((rc = enqueue_kernel(d, PIE_K_LMHEAD, 0, nullptr, d->logits, st))) return rc;
     return enqueue_kernel(d, PIE_K_TAIL, 0, nullptr, d->logits, st);
 }
+
+extern "C" int pie_decoder_prompt_shares(const pie_decoder *d) { return d && d->prefill ? d->prefill->last_shares : 0; }
 
 // mx.fast.scaled_dot_product_attention(q, k, v, scale, mask=causal) for L > 1 (models/base.py:37-53,111-113), op level.
 extern "C" int pie_sdpa_prefill(const void *q, const void *k, const void *v, int Hq, int Hkv, int L, int offset, int cap, int D, float scale,

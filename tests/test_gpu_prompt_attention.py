@@ -75,6 +75,7 @@ def test_rows_behind_a_prefix_split_along_the_keys(geometry, paged):
                 _ffi.set_knob("prefill_attn_valu", None)
             for layer in cache:
                 layer.trim(n)
+        assert _ffi.load().pie_decoder_prompt_shares(m._dec) == (5 if n <= 64 else 3)   # of 700 keys: two blocks of 64 each, three from 65 rows on
         for i in range(n):
             assert_vec_close(got[1][i], got[0][i], "bfloat16", what=f"{n} rows, row {i}")
 
