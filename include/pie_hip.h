@@ -564,7 +564,8 @@ typedef struct pie_stack pie_stack;
 size_t pie_stack_weight_bytes(int dtype, int N, int K);
 int pie_stack_pack_weight(const void *w, int N, int K, int dtype, void *packed, void *stream);
 /* Which kernel a plain bf16 Linear [N, K] of M rows takes (host only): 0 the one that fetches both operands itself, 1 the one that brings x through LDS.
- * ldx: elements from one row of x to the next; x_rows: how many rows x holds where a list picks the M from them (0: they follow one another). */
+ * ldx: elements from one row of x to the next; x_rows: how many rows x holds where a list picks the M from them (0: they follow one another;
+ * -1: so they do, and the matrix is the one of a list). */
 int pie_stack_linear_kernel(int M, int N, int K, int ldx, int x_rows);
 
 /* A norm.  NONE: the identity.  DYN_TANH: w * tanh(param x) + b, element by element.  RMS: x / sqrt(mean(x^2) + param) * w.

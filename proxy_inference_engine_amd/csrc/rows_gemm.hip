@@ -490,10 +490,12 @@ __global__ void __launch_bounds__(256) k_pack_f32(const u16 *w, int N, int K, in
 }  // namespace
 
 static bool rows_narrow(const RowsArgs &a, int n_max, int batches) { return (long)batches * n_max <= 16 * 64 && !a.merge.splits; }  // so few workgroups that they should not all read all rows
-// k_rows_lds counts the bytes behind its first row of x in 31 bits: all of x where a list picks rows from it, 64 rows otherwise
+// k_rows_lds counts the bytes behind its first row of x in 31 bits: all of x where a list picks rows from it, 64 rows otherwise; of the widest operand that the launch has
 static bool rows_lds_reaches(const RowsArgs &a) {
     const size_t rows = a.rows ? (size_t)a.x_rows : a.gather ? (size_t)a.M : 64;
-    return rows * (size_t)a.m.ldx * 2 < (1u << 31);
+    int ldx = a.n_mats ? 0 : a.shared.w ? std::max(a.m.ldx, a.shared.ldx) : a.m.ldx;
+    for (int i = 0; i < a.n_mats; ++i) ldx = std::max(ldx, a.mats[i].ldx);
+    return rows * (size_t)ldx * 2 < (1u << 31);
 }
 static long rows_blocks(const RowsArgs &a, int batches) {  // of 16 features, over the whole launch
     long blocks = a.n_mats ? 0 : (long)batches * ((a.m.N + 15) / 16);
@@ -575,10 +577,11 @@ size_t pie_stack_weight_bytes(int dtype, int N, int K) {
 }
 
 int pie_stack_linear_kernel(int M, int N, int K, int ldx, int x_rows) {
-    PIE_REQUIRE(M > 0 && N > 0 && K > 0 && ldx >= K && x_rows >= 0, -1, "pie_stack_linear_kernel: bad sizes");
+    PIE_REQUIRE(M > 0 && N > 0 && K > 0 && ldx >= K && x_rows >= -1, -1, "pie_stack_linear_kernel: bad sizes");
     RowsArgs a = {};
     const int any = 0;
-    a.m.N = N, a.m.K = K, a.m.ldx = ldx, a.M = M, a.rows = x_rows ? &any : nullptr, a.x_rows = x_rows;
+    a.m.N = N, a.m.K = K, a.m.ldx = ldx, a.M = M, a.rows = x_rows > 0 ? &any : nullptr, a.x_rows = x_rows;
+    if (x_rows < 0) a.mats[0] = a.m, a.n_mats = 1, a.m = {};
     return rows_lds_serves(a, N, K, 1);
 }
 

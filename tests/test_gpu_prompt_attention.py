@@ -80,7 +80,7 @@ def test_rows_behind_a_prefix_split_along_the_keys(geometry, paged):
             assert_vec_close(got[1][i], got[0][i], "bfloat16", what=f"{n} rows, row {i}")
 
 
-def test_longer_splits_neither_allocate_nor_drop_the_step_s_graph():
+def test_longer_splits_do_not_allocate():
     """Prompts behind longer and longer prefixes take more and more shares of more rows; the room for their sums is there from the first prompt on."""
     from proxy_inference_engine_amd.models.llama import Model, ModelArgs
     from proxy_inference_engine_amd.models.utils import synthetic_checkpoint

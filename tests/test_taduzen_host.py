@@ -123,6 +123,8 @@ def test_rows_picked_from_more_than_2_gib_take_the_kernel_with_64_bit_addresses(
         assert lds(M, 32768, 32768, 0) == 1 and lds(M, 32768, 32768, M) == 1 and lds(M, 32768, 32768, 32767) == 1
         assert lds(M, 32768, 32768, 32768) == 0 and lds(M, 32768, 32896, 32650) == 0 and lds(M, 32768, 32768, 65535) == 0
         assert lds(M, 16384, 16384, 65535) == 1 and lds(M, 16384, 16400, 65535) == 0
+        for where in (0, -1):   # 64 rows, one behind the other, of a matrix alone and of one in a list
+            assert lds(M, 32768, (1 << 24) - 8, where) == 1 and lds(M, 32768, 1 << 24, where) == 0
     assert _ffi.base().pie_stack_linear_kernel(0, 1, 1, 1, 0) < 0
 
 
