@@ -131,9 +131,9 @@ __global__ void __launch_bounds__(STEP_WAVES * 64, REP <= 4 ? 3 : 2) k_attn_step
 
     const int first = t_begin + wave * 16;  // the wave's block b begins at first + 16 WAVES b
     const int n_blk = first < t_end ? (t_end - first + 16 * WAVES - 1) / (16 * WAVES) : 0;
-    int pages = 0;  // lane i: page of block i, of the 64 that b is in
+    int pages = 0;  // lane i: page of block i, of the 64 that b is in; past the wave's last block that one's, whose row issue() reads again (t_end may lie a page further on)
     auto page_ids = [&](int b0) {
-        const int t = min(first + (b0 + lane) * 16 * WAVES, t_end - 1);
+        const int t = first + min(b0 + lane, n_blk - 1) * 16 * WAVES;
         pages = (int)min((unsigned)bt[t >> 6], last_page);
     };
     uint4 kq[STEP_DEPTH][KS], vq[STEP_DEPTH][VI];

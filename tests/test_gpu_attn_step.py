@@ -99,3 +99,45 @@ def test_a_step_is_the_prompt_with_its_token(rep, D, dtype):
     for i, n in enumerate(lens):
         assert_vec_close(alone[i].float().cpu().numpy(), want[i], dtype, c_max=8.0, c_rms=8.0, what=f"alone, {n} positions")
         assert_vec_close(batch[i].float().cpu().numpy(), want[i], dtype, c_max=8.0, c_rms=8.0, what=f"batch, {n} positions")
+
+
+def bits_over_pools(model, lens, max_blocks, run):
+    """What `run(caches, feed)` gives behind prompts of these lengths, with a pool full of zeros, of NaN and of infinities."""
+    prompts = [torch.from_numpy(np.random.default_rng(i).integers(0, 512, n).astype(np.int32)).cuda() for i, n in enumerate(lens)]
+    pool = model.enable_paged_kv(num_pages=sum(n // 64 + 1 for n in lens) + 1, max_blocks=max_blocks)
+    feed, got = torch.arange(3, 3 + len(lens), dtype=torch.int32, device="cuda"), []
+    for fill in (0.0, float("nan"), float("inf")):
+        for slab in pool.slab:
+            slab.view(torch.bfloat16).fill_(fill)
+        caches = [model.make_cache() for _ in lens]
+        for p, c in zip(prompts, caches):
+            model.step(p, c)
+        got.append(run(caches, feed))
+        for c in caches:
+            c[0].page_manager.release()
+    return got
+
+
+@pytest.mark.parametrize("Hq,Hkv,D", [(24, 8, 128), (4, 4, 128), (8, 1, 128), (32, 4, 64), (8, 2, 64), (5, 5, 64)])
+def test_a_paged_sequence_reads_no_row_that_nobody_wrote(Hq, Hkv, D):
+    """Splits of a multiple of 16 positions that end on another page than some wave's last block: what lies behind the sequence in the pool counts nothing, not even with weight 0.  The new
+    position included, 129 .. 145 and some up to the 1024 where the consumer merges the splits."""
+    model = _model(512, Hq, Hkv, D, False, False, False)
+    lens = [*range(128, 145), 149, 159, 192, 199, 256, 299, 399, 449, 640, 830, 1000]
+    got = bits_over_pools(model, lens, 16, lambda caches, feed: torch.stack([model.step(feed[i:i + 1], c)[2].clone().reshape(-1) for i, c in enumerate(caches)]))
+    assert torch.isfinite(got[0]).all()
+    for g in got[1:]:
+        assert [lens[i] for i in range(len(lens)) if not torch.equal(g[i], got[0][i])] == []
+
+
+@pytest.mark.parametrize("Hq,Hkv,D", [(8, 8, 128), (24, 8, 128), (16, 8, 64)])
+@pytest.mark.parametrize("short", [4, 7])
+def test_a_batch_reads_no_row_that_nobody_wrote(short, Hq, Hkv, D):
+    """One row in pieces beside rows in one: pieces that end on another page than some wave's last block, in front of a last piece that is short."""
+    model = _model(512, Hq, Hkv, D, False, False, False)
+    for n in (*range(400, 417, 3), 415, *range(672, 689, 4)):
+        lens = [40] * short
+        lens.insert(2, n)
+        got = bits_over_pools(model, lens, 12, lambda caches, feed: model.step_batch(feed, caches, graph=False)[2].clone())
+        assert torch.isfinite(got[0]).all()
+        assert torch.equal(got[0], got[1]) and torch.equal(got[0], got[2]), n
