@@ -422,10 +422,11 @@ struct PrefillScratch {
     int rows = 0;           // chunk capacity (rows)
     size_t w_elems = 0;     // capacity of the dequantised-weight buffer (elements)
     u16 *wT = nullptr, *wM = nullptr, *x = nullptr, *xn = nullptr, *qkv = nullptr, *q = nullptr, *attn = nullptr, *gu = nullptr, *act = nullptr, *r = nullptr;
-    float *part_acc = nullptr, *part_ml = nullptr, *rope_cs = nullptr;
+    float *rope_cs = nullptr;
     int *arrived = nullptr;   // k_attn_step's counters, [rows, n_kv_heads]
     u16 *kc = nullptr, *vc = nullptr;  // [n_kv_heads, rows, head_dim]: this pass's K / V rows, contiguous (several prompts in one pass)
-    int part_splits = 0;
+    float *part_acc = nullptr, *part_ml = nullptr;  // sums of rows whose decode attention is split: sized by what takes them, not by the rows of a prompt
+    size_t parts = 0;                               // their capacity in (row, split)s
     // Resident T copies of the layer matrices, keyed by the packed-weight pointer: the per-chunk dequantisation moves
     // 4.6 B per parameter (7 ms of a 10.8 ms 128-token prefill on the 8B model) for 2 B per parameter of HBM; kept when
     // that is a small share of the free memory (PIE_KNOB_PREFILL_RESIDENT overrides), built on first use.
@@ -458,7 +459,7 @@ static int tail_stats_reserve(PrefillScratch *s, size_t entries) {
 }
 
 static void scratch_release(PrefillScratch *s) {  // the chunk buffers; resident weight copies survive a re-size
-    void *ptrs[] = {s->wT, s->wM, s->x, s->xn, s->qkv, s->q, s->attn, s->gu, s->act, s->r, s->part_acc, s->part_ml, s->arrived, s->rope_cs, s->kc, s->vc};
+    void *ptrs[] = {s->wT, s->wM, s->x, s->xn, s->qkv, s->q, s->attn, s->gu, s->act, s->r, s->arrived, s->rope_cs, s->kc, s->vc};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     auto keep = std::move(s->resident);
@@ -471,9 +472,10 @@ static void scratch_release(PrefillScratch *s) {  // the chunk buffers; resident
     const size_t left = s->resident_left;
     void *keep_ws = s->w4l_ws;
     const size_t keep_wsb = s->w4l_ws_bytes;
-    float *keep_part = s->attn_part;
+    float *keep_part = s->attn_part, *keep_acc = s->part_acc, *keep_ml = s->part_ml;
+    const size_t keep_parts = s->parts;
     *s = PrefillScratch();
-    s->w4l_ws = keep_ws, s->w4l_ws_bytes = keep_wsb, s->attn_part = keep_part;
+    s->w4l_ws = keep_ws, s->w4l_ws_bytes = keep_wsb, s->attn_part = keep_part, s->part_acc = keep_acc, s->part_ml = keep_ml, s->parts = keep_parts;
     s->resident = std::move(keep), s->resident_w4m = std::move(keep_m), s->resident_mode = mode, s->resident_left = left;
     s->tail_stats = keep_ts, s->tail_entries = keep_tr, s->alloc_gen = gen;
 }
@@ -486,6 +488,8 @@ void prefill_free(pie_decoder *d) {
     if (d->prefill->tail_stats) (void)hipFree(d->prefill->tail_stats);
     if (d->prefill->w4l_ws) (void)hipFree(d->prefill->w4l_ws);
     if (d->prefill->attn_part) (void)hipFree(d->prefill->attn_part);
+    if (d->prefill->part_acc) (void)hipFree(d->prefill->part_acc);
+    if (d->prefill->part_ml) (void)hipFree(d->prefill->part_ml);
     if (d->prefill->batch_graph) (void)hipGraphExecDestroy(d->prefill->batch_graph);
     delete d->prefill;
     d->prefill = nullptr;
@@ -516,12 +520,14 @@ static int prefill_chunk_rows() {
     return n < 16 ? 16 : (n > 8192 ? 8192 : n);
 }
 
-static int scratch_reserve(pie_decoder *d, int rows, size_t w_elems, int splits) {
+// parts: rows whose decode attention is split, times the splits.  Every buffer only grows: prompts have many rows and no such parts, a batch's step few rows and many, and a serving loop
+// takes them in turn (sized by the call at hand each took the buffers from the other, all of them anew twice a prompt, and the captured step with them).
+static int scratch_reserve(pie_decoder *d, int rows, size_t w_elems, size_t parts) {
     if (!d->prefill) d->prefill = new PrefillScratch();
     PrefillScratch *s = d->prefill;
     const pie_decoder_config &c = d->cfg;
     const size_t QD = (size_t)c.n_heads * c.head_dim, NQKV = QD + 2 * (size_t)c.n_kv_heads * c.head_dim;
-    if (rows > s->rows || splits > s->part_splits) {
+    if (rows > s->rows) {
         const size_t we = s->w_elems > w_elems ? s->w_elems : w_elems;
         scratch_release(s);
         const size_t R = (size_t)rows;
@@ -534,8 +540,6 @@ static int scratch_reserve(pie_decoder *d, int rows, size_t w_elems, int splits)
         PF_ALLOC(s->attn, 2 * R * QD);
         PF_ALLOC(s->gu, 2 * R * 2 * c.inter);
         PF_ALLOC(s->act, 2 * R * c.inter);
-        PF_ALLOC(s->part_acc, 4 * R * c.n_heads * splits * c.head_dim);
-        PF_ALLOC(s->part_ml, 4 * R * c.n_heads * splits * 2);
         PF_ALLOC(s->arrived, 4 * R * c.n_kv_heads);
         PIE_HIP_TRY(hipMemset(s->arrived, 0, 4 * R * c.n_kv_heads));
         PIE_HIP_TRY(hipStreamSynchronize(nullptr));  // (a pass on a stream that does not wait for the null stream)
@@ -544,7 +548,7 @@ static int scratch_reserve(pie_decoder *d, int rows, size_t w_elems, int splits)
         PF_ALLOC(s->vc, 2 * R * c.n_kv_heads * c.head_dim);
         PF_ALLOC(s->wT, 2 * we);
         PF_ALLOC(s->wM, 2 * we);
-        s->rows = rows, s->part_splits = splits, s->w_elems = we;
+        s->rows = rows, s->w_elems = we;
     }
     if (w_elems > s->w_elems) {
         if (s->wT) (void)hipFree(s->wT);
@@ -553,6 +557,14 @@ static int scratch_reserve(pie_decoder *d, int rows, size_t w_elems, int splits)
         PF_ALLOC(s->wT, 2 * w_elems);
         PF_ALLOC(s->wM, 2 * w_elems);
         s->w_elems = w_elems, ++s->alloc_gen;
+    }
+    if (parts > s->parts) {
+        if (s->part_acc) (void)hipFree(s->part_acc);
+        if (s->part_ml) (void)hipFree(s->part_ml);
+        s->part_acc = s->part_ml = nullptr, s->parts = 0, ++s->alloc_gen;
+        PF_ALLOC(s->part_acc, 4 * parts * c.n_heads * c.head_dim);
+        PF_ALLOC(s->part_ml, 4 * parts * c.n_heads * 2);
+        s->parts = parts;
     }
 #undef PF_ALLOC
     return PIE_OK;
@@ -875,10 +887,10 @@ static int prefill_t(pie_decoder *d, const int32_t *ids, const void *embeds, int
     if (w16m_size(NQKV, H) / 2 > w_elems) w_elems = w16m_size(NQKV, H) / 2;
     if (w16m_size(H, I) / 2 > w_elems) w_elems = w16m_size(H, I) / 2;
     if (logits_all && w16m_size(c.vocab, H) / 2 > w_elems) w_elems = w16m_size(c.vocab, H) / 2;
-    int rc = scratch_reserve(d, chunk, w_elems, d->splits);
+    const bool mfma_attn = pie_knob(PIE_KNOB_PREFILL_ATTN_VALU) != 1;  // 1 forces the row-per-launch-slice VALU kernel (tests compare the two)
+    int rc = scratch_reserve(d, chunk, w_elems, mfma_attn ? 0 : (size_t)chunk * d->splits);
     if (rc) return rc;
     PrefillScratch *s = d->prefill;
-    const bool mfma_attn = pie_knob(PIE_KNOB_PREFILL_ATTN_VALU) != 1;  // 1 forces the row-per-launch-slice VALU kernel (tests compare the two)
     if (mfma_attn) reserve_attn_part(d);
     for (int c0 = 0; c0 < L; c0 += chunk) {
         const int M = L - c0 < chunk ? L - c0 : chunk;
@@ -1033,7 +1045,7 @@ static int decode_batch_t(pie_decoder *d, const int32_t *tokens, const int32_t *
     if (w16m_size(H, I) / 2 > w_elems) w_elems = w16m_size(H, I) / 2;
     if (w16m_size(c.vocab, H) / 2 > w_elems) w_elems = w16m_size(c.vocab, H) / 2;
     const int splits = batch_attn_splits(d, B, max_blocks, !batch_fused(d, B));
-    int rc = scratch_reserve(d, B, w_elems, splits > d->splits ? splits : d->splits);
+    int rc = scratch_reserve(d, B, w_elems, (size_t)B * splits);
     if (rc) return rc;
     PrefillScratch *s = d->prefill;
     int32_t *lens = advance ? const_cast<int32_t *>(ctx_len) : nullptr;
@@ -1154,7 +1166,7 @@ static int prefill_varlen_t(pie_decoder *d, const int32_t *ids, const int32_t *r
     if (w16m_size(H, I) / 2 > w_elems) w_elems = w16m_size(H, I) / 2;
     if (w16m_size(c.vocab, H) / 2 > w_elems) w_elems = w16m_size(c.vocab, H) / 2;
     const int dsplits = n_decode > 0 ? batch_attn_splits(d, n_decode, max_blocks, false) : 1;
-    int rc = scratch_reserve(d, N > S ? N : S, w_elems, dsplits > d->splits ? dsplits : d->splits);
+    int rc = scratch_reserve(d, N > S ? N : S, w_elems, (size_t)n_decode * dsplits);
     if (rc) return rc;
     PrefillScratch *s = d->prefill;
     if (n_chunks > 0) reserve_attn_part(d);
