@@ -995,9 +995,9 @@ extern "C" int pie_sdpa_prefill(const void *q, const void *k, const void *v, int
 
 
 // attention splits of a batch of B decode rows over block tables of max_blocks pages
-static int batch_attn_splits(const pie_decoder *d, int B, int max_blocks, bool step) {  // step: for k_attn_step
+static int batch_attn_splits(const pie_decoder *d, int B, int max_blocks, bool step) {  // step: for k_attn_step (T pages)
     const pie_decoder_config &c = d->cfg;
-    if (step && !d->kv_i8) {
+    if (step) {
         // Room for pieces, as many as the kernel may want of a row: how many it cuts depends on the lengths (step_split).  More than rows of like lengths need, for a row that is longer.
         const int n = B * c.n_kv_heads, most = max_blocks < ATTN_MAX_SPLITS ? max_blocks : ATTN_MAX_SPLITS, pieces = 512 / n > 4 ? 512 / n : 4;
         return pieces < most ? pieces : most;
@@ -1044,13 +1044,14 @@ static int decode_batch_t(pie_decoder *d, const int32_t *tokens, const int32_t *
     if (w16m_size(NQKV, H) / 2 > w_elems) w_elems = w16m_size(NQKV, H) / 2;
     if (w16m_size(H, I) / 2 > w_elems) w_elems = w16m_size(H, I) / 2;
     if (w16m_size(c.vocab, H) / 2 > w_elems) w_elems = w16m_size(c.vocab, H) / 2;
-    const int splits = batch_attn_splits(d, B, max_blocks, !batch_fused(d, B));
-    int rc = scratch_reserve(d, B, w_elems, (size_t)B * splits);
+    // (the layers' products say whether they rotated and appended themselves, and with it which kernel attends)
+    const bool fused_rows = batch_fused(d, B);
+    const int splits = batch_attn_splits(d, B, max_blocks, false), step_splits = fused_rows ? splits : batch_attn_splits(d, B, max_blocks, true);
+    int rc = scratch_reserve(d, B, w_elems, (size_t)B * (step_splits > splits ? step_splits : splits));
     if (rc) return rc;
     PrefillScratch *s = d->prefill;
     int32_t *lens = advance ? const_cast<int32_t *>(ctx_len) : nullptr;
     if (tokens && (rc = batch_rows(d, tokens, ctx_len, B, st))) return rc;  // (nullptr: they are there already)
-    const bool fused_rows = batch_fused(d, B);
     const int lm_waves = w4s_gemv_waves(c.vocab, H);
     if (fused_rows && (rc = tail_stats_reserve(s, (size_t)lm_waves * (size_t)B))) return rc;
     if (fused_rows) {
@@ -1106,7 +1107,7 @@ static int decode_batch_t(pie_decoder *d, const int32_t *tokens, const int32_t *
         }
         AttnRopeArgs a = {};
         a.q = s->q, a.slab = (const u16 *)slabs[li], a.block_table = block_tables, a.ctx_len = ctx_len, a.bt_stride = max_blocks, a.n_pages = n_pages;
-        a.rows = B, a.Hq = c.n_heads, a.Hkv = c.n_kv_heads, a.splits = splits, a.scale = 1.0f / sqrtf((float)D);
+        a.rows = B, a.Hq = c.n_heads, a.Hkv = c.n_kv_heads, a.splits = rope_in_attn ? step_splits : splits, a.scale = 1.0f / sqrtf((float)D);
         a.nt_kv = (size_t)B * max_blocks * 64 >= 2048;
         a.part_acc = s->part_acc, a.part_ml = s->part_ml, a.out = s->attn;
         a.qkv = s->qkv, a.part = sq.part, a.S = sq.S, a.MN = sq.MN, a.n_cols = NQKV, a.rope_cs = s->rope_cs, a.traditional = c.rope_traditional, a.pages = (u16 *)slabs[li], a.arrived = s->arrived;

@@ -112,3 +112,32 @@ def test_a_step_of_a_batch_refuses_a_caller_s_capture():
             model.step_batch(feed, caches, graph=False)
     torch.cuda.synchronize()
     assert torch.equal(model.step_batch(feed, caches, graph=False)[2], want[2])
+
+
+def test_rows_rotated_by_their_product_take_that_kernel_s_splits():
+    """int4 of so few columns that q|k|v is not split: its epilogue rotates and appends, and the attention behind it takes short rows in one piece, whatever the tables have room for.  Tables
+    of one page, where there is nothing else, give the same bits -- of sums that cancel, so that their order shows: keys of 0, values of up to 2^30 and their negatives."""
+    from proxy_inference_engine_amd import _ffi
+    import ctypes as C
+    model, B = _model(256, 8, 8, 64, False, True, False), 8
+    pool = model.enable_paged_kv(num_pages=2 * B, max_blocks=4)
+    caches = [model.make_cache() for _ in range(B)]
+    lens = [40 + 3 * i for i in range(B)]
+    for n, c in zip(lens, caches):
+        model.step(torch.arange(n, dtype=torch.int32, device="cuda"), c)
+    gen = torch.Generator().manual_seed(1)
+    for n, c in zip(lens, caches):
+        half = torch.randn(8, n // 2, 64, generator=gen) * 2.0 ** torch.randint(10, 30, (8, n // 2, 64), generator=gen)
+        rows = torch.cat([half, -half[:, torch.randperm(n // 2, generator=gen)], torch.zeros(8, n % 2, 64)], 1).to(torch.bfloat16).cuda()
+        page = pool.slab[0].view(torch.bfloat16).view(-1, 2, 8, 64, 64)[c[0].page_manager.pages[0]]
+        page[0, :, :n], page[1, :, :n] = 0, rows
+    feed, ctx = torch.arange(B, dtype=torch.int32, device="cuda"), torch.tensor(lens, dtype=torch.int32, device="cuda") + 1
+    slabs, got = (C.c_void_p * 2)(*[s.data_ptr() for s in pool.slab]), []
+    for width in (1, 4):
+        table = torch.zeros((B, width), dtype=torch.int32)
+        table[:, 0] = torch.tensor([c[0].page_manager.pages[0] for c in caches])
+        table, logits, logprobs, token = table.cuda(), torch.empty((B, 512), dtype=torch.bfloat16, device="cuda"), torch.empty((B, 512), device="cuda"), torch.empty(B, dtype=torch.int32, device="cuda")
+        _ffi.check(_ffi.load().pie_decoder_step_batch(model._dec, _ffi.p(feed), _ffi.p(ctx), slabs, pool.size(), pool.slab[0].numel() * pool.slab[0].element_size(), _ffi.p(table), width, B,
+                                                      _ffi.p(logits), _ffi.p(logprobs), _ffi.p(token), 0, _ffi.stream()))
+        got.append(logits.clone())
+    assert torch.isfinite(got[0]).all() and torch.equal(*got)
