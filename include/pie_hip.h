@@ -305,10 +305,14 @@ int pie_decoder_set_paged_kv(pie_decoder *d, const void *const *slabs, size_t n_
  * include/engine/batch_details.hpp:10-88; Scheduler and the paged attention kernel are skeletons there).  Independent of
  * pie_decoder_set_kv / set_state / bind_outputs; all device arrays are caller-owned.  flags: PIE_STEP_GRAPH replays a captured
  * hipGraph of the step while the caller passes the same buffers (their contents may change; tokens may be another buffer every time) --
- * captured on the second such call; PIE_STEP_ADVANCE adds 1 to every context_lens[s] > 0 behind the step: the next step's lengths. */
+ * captured on the second such call.
+ * pie_decoder_step_batch_advance: the same step, and context_lens[s] + 1 for every context_lens[s] > 0 behind it: the next step's lengths. */
 int pie_decoder_step_batch(pie_decoder *d, const int32_t *tokens, const int32_t *context_lens, const void *const *slabs, size_t n_pages, size_t slab_bytes,
                            const int32_t *block_tables, int max_blocks, int B, void *logits, float *logprobs, int32_t *next_tokens,
                            int flags, void *stream);
+int pie_decoder_step_batch_advance(pie_decoder *d, const int32_t *tokens, int32_t *context_lens, const void *const *slabs, size_t n_pages, size_t slab_bytes,
+                                   const int32_t *block_tables, int max_blocks, int B, void *logits, float *logprobs, int32_t *next_tokens,
+                                   int flags, void *stream);
 /* Several FRESH prompts in one pass (the prefill-state half of BatchDetails, batch_details.hpp:10-88): their N rows are
  * concatenated -- ids [N]; per row: row_context_lens (position + 1), row_seq (which prompt, = its block-table row), seg_lo
  * (index of its prompt's first row), seg_hi (row index + 1: causal); per prompt: last_rows [S] (index of its last row).  K / V
@@ -340,7 +344,7 @@ int pie_decoder_set_state(pie_decoder *d, int offset, int token, void *stream);
  * the KV caches: prompt tokens before the last); PIE_STEP_GRAPH replays a captured hipGraph of the step
  * (captured on first use per flag set).  After the step the device-side offset is incremented and, with
  * PIE_STEP_LOGITS, the device-side token is the greedy choice. */
-enum { PIE_STEP_LOGITS = 1, PIE_STEP_GRAPH = 2, PIE_STEP_ADVANCE = 4 /* pie_decoder_step_batch */ };
+enum { PIE_STEP_LOGITS = 1, PIE_STEP_GRAPH = 2 };
 int pie_decoder_step(pie_decoder *d, int flags, void *stream);
 /* Kernel nodes of the captured step graph (read back with hipGraphGetNodes when it was instantiated); -1 while no step with these flags has
  * been captured.  bench.py reports it as config.launches_per_step. */

@@ -1037,7 +1037,7 @@ static int batch_rows(pie_decoder *d, const int32_t *tokens, const int32_t *ctx_
 // skeleton (src/pie_core/include/engine/batch_details.hpp:10-88, scheduler.hpp) describes for decode-state sequences.
 template <class T>
 static int decode_batch_t(pie_decoder *d, const int32_t *tokens, const int32_t *ctx_len, const void *const *slabs, int n_pages,
-                          const int32_t *block_tables, int max_blocks, int B, u16 *logits, float *logprobs, int32_t *next_tokens, bool advance, hipStream_t st) {
+                          const int32_t *block_tables, int max_blocks, int B, u16 *logits, float *logprobs, int32_t *next_tokens, int32_t *lens, hipStream_t st) {
     const pie_decoder_config &c = d->cfg;
     const int H = c.hidden, D = c.head_dim, QD = c.n_heads * D, KVD = c.n_kv_heads * D, NQKV = QD + 2 * KVD, I = c.inter;
     size_t w_elems = w16m_size(2 * I, H) / 2;  // the 16-bit copies are W16M tiles (rows padded to 32, columns to 64)
@@ -1050,7 +1050,6 @@ static int decode_batch_t(pie_decoder *d, const int32_t *tokens, const int32_t *
     int rc = scratch_reserve(d, B, w_elems, (size_t)B * (step_splits > splits ? step_splits : splits));
     if (rc) return rc;
     PrefillScratch *s = d->prefill;
-    int32_t *lens = advance ? const_cast<int32_t *>(ctx_len) : nullptr;
     if (tokens && (rc = batch_rows(d, tokens, ctx_len, B, st))) return rc;  // (nullptr: they are there already)
     const int lm_waves = w4s_gemv_waves(c.vocab, H);
     if (fused_rows && (rc = tail_stats_reserve(s, (size_t)lm_waves * (size_t)B))) return rc;
@@ -1285,10 +1284,10 @@ extern "C" int pie_decoder_step_mixed(pie_decoder *d, const int32_t *ids, const 
 }
 
 static int decode_batch(pie_decoder *d, const int32_t *tokens, const int32_t *ctx_len, const void *const *slabs, int n_pages, const int32_t *block_tables,
-                        int max_blocks, int B, void *logits, float *logprobs, int32_t *next_tokens, bool advance, hipStream_t st) {
+                        int max_blocks, int B, void *logits, float *logprobs, int32_t *next_tokens, int32_t *lens, hipStream_t st) {
     return d->cfg.dtype == PIE_BF16
-               ? decode_batch_t<BF16>(d, tokens, ctx_len, slabs, n_pages, block_tables, max_blocks, B, (u16 *)logits, logprobs, next_tokens, advance, st)
-               : decode_batch_t<F16>(d, tokens, ctx_len, slabs, n_pages, block_tables, max_blocks, B, (u16 *)logits, logprobs, next_tokens, advance, st);
+               ? decode_batch_t<BF16>(d, tokens, ctx_len, slabs, n_pages, block_tables, max_blocks, B, (u16 *)logits, logprobs, next_tokens, lens, st)
+               : decode_batch_t<F16>(d, tokens, ctx_len, slabs, n_pages, block_tables, max_blocks, B, (u16 *)logits, logprobs, next_tokens, lens, st);
 }
 
 // bytes one page of the active format takes in a layer's slab: K block + V block of T rows, or the int8 page with its scales
@@ -1297,9 +1296,9 @@ static size_t active_page_bytes(const pie_decoder *d) {
     return d->kv_i8 ? pie_page_i8_bytes(c.n_kv_heads, c.head_dim) : (size_t)2 * PIE_PAGE_TOKENS * c.n_kv_heads * c.head_dim * 2;
 }
 
-extern "C" int pie_decoder_step_batch(pie_decoder *d, const int32_t *tokens, const int32_t *context_lens, const void *const *slabs, size_t n_pages, size_t slab_bytes,
-                                      const int32_t *block_tables, int max_blocks, int B, void *logits, float *logprobs, int32_t *next_tokens,
-                                      int flags, void *stream) {
+// lens: context_lens where the step moves them on, else nullptr
+static int step_batch(pie_decoder *d, const int32_t *tokens, const int32_t *context_lens, int32_t *lens, const void *const *slabs, size_t n_pages, size_t slab_bytes,
+                      const int32_t *block_tables, int max_blocks, int B, void *logits, float *logprobs, int32_t *next_tokens, int flags, void *stream) {
     PIE_REQUIRE(d && tokens && context_lens && slabs && block_tables && logits && logprobs && next_tokens, PIE_E_ARG, "pie_decoder_step_batch: null pointer");
     PIE_REQUIRE(d->glob_set, PIE_E_STATE, "pie_decoder_step_batch: set_globals must be called first");
     PIE_REQUIRE(!d->tp(), PIE_E_STATE, "pie_decoder_step_batch: not available on a tensor-parallel shard");
@@ -1311,13 +1310,12 @@ extern "C" int pie_decoder_step_batch(pie_decoder *d, const int32_t *tokens, con
     PIE_REQUIRE(rep >= 1 && rep <= 8, PIE_E_SHAPE, "pie_decoder_step_batch: n_heads / n_kv_heads must be between 1 and 8");
     for (int i = 0; i < d->cfg.n_layers; ++i) PIE_REQUIRE(slabs[i] && pie_aligned(slabs[i], 16), PIE_E_ALIGN, "pie_decoder_step_batch: null or misaligned slab");
     hipStream_t st = (hipStream_t)stream;
-    const bool advance = (flags & PIE_STEP_ADVANCE) != 0;
-    if (!(flags & PIE_STEP_GRAPH)) return decode_batch(d, tokens, context_lens, slabs, (int)n_pages, block_tables, max_blocks, B, logits, logprobs, next_tokens, advance, st);
+    if (!(flags & PIE_STEP_GRAPH)) return decode_batch(d, tokens, context_lens, slabs, (int)n_pages, block_tables, max_blocks, B, logits, logprobs, next_tokens, lens, st);
     // Graph replay, behind the launch that reads the tokens: those may be another buffer every time (copied to a fixed place first, and the lengths moved on by a launch of their own,
     // a step of 8 sequences took 2 % more).  The launches bake in the caller's buffers and this library's scratch / resident weight copies, so a graph is
     // captured only for a call that repeats the previous call's buffers after that call allocated nothing, and is dropped when
     // either changes.  (First call with new buffers: eager, it may allocate; second: capture; from the third: replay.)
-    std::vector<uintptr_t> key = {(uintptr_t)advance, (uintptr_t)context_lens, (uintptr_t)block_tables, (uintptr_t)logits, (uintptr_t)logprobs,
+    std::vector<uintptr_t> key = {(uintptr_t)lens, (uintptr_t)context_lens, (uintptr_t)block_tables, (uintptr_t)logits, (uintptr_t)logprobs,
                                   (uintptr_t)next_tokens, (uintptr_t)n_pages, (uintptr_t)max_blocks, (uintptr_t)B, (uintptr_t)d->kv_i8 /* the page format is baked into the launches too */};
     for (int i = 0; i < d->cfg.n_layers; ++i) key.push_back((uintptr_t)slabs[i]);
     if (!d->prefill) d->prefill = new PrefillScratch();
@@ -1338,14 +1336,14 @@ extern "C" int pie_decoder_step_batch(pie_decoder *d, const int32_t *tokens, con
             return pie::fail(PIE_E_HIP, std::string("hipStreamBeginCapture: ") + hipGetErrorString(e));
         }
         const unsigned gen = s->alloc_gen;
-        const int rc = decode_batch(d, nullptr, context_lens, slabs, (int)n_pages, block_tables, max_blocks, B, logits, logprobs, next_tokens, advance, cs);
+        const int rc = decode_batch(d, nullptr, context_lens, slabs, (int)n_pages, block_tables, max_blocks, B, logits, logprobs, next_tokens, lens, cs);
         e = hipStreamEndCapture(cs, &g);
         (void)hipStreamDestroy(cs);
         if (rc || e != hipSuccess || d->prefill->alloc_gen != gen) {  // something allocated or failed under capture: run this call eagerly instead
             if (g) (void)hipGraphDestroy(g);
             (void)hipGetLastError();
             d->prefill->warm_key.clear();
-            return decode_batch(d, tokens, context_lens, slabs, (int)n_pages, block_tables, max_blocks, B, logits, logprobs, next_tokens, advance, st);
+            return decode_batch(d, tokens, context_lens, slabs, (int)n_pages, block_tables, max_blocks, B, logits, logprobs, next_tokens, lens, st);
         }
         s = d->prefill;
         e = hipGraphInstantiate(&s->batch_graph, g, nullptr, nullptr, 0);
@@ -1356,9 +1354,19 @@ extern "C" int pie_decoder_step_batch(pie_decoder *d, const int32_t *tokens, con
         PIE_HIP_TRY(hipGraphLaunch(s->batch_graph, st));
         return PIE_OK;
     }
-    const int rc = decode_batch(d, tokens, context_lens, slabs, (int)n_pages, block_tables, max_blocks, B, logits, logprobs, next_tokens, advance, st);
+    const int rc = decode_batch(d, tokens, context_lens, slabs, (int)n_pages, block_tables, max_blocks, B, logits, logprobs, next_tokens, lens, st);
     d->prefill->warm_key = key, d->prefill->warm_gen = d->prefill->alloc_gen;
     return rc;
+}
+extern "C" int pie_decoder_step_batch(pie_decoder *d, const int32_t *tokens, const int32_t *context_lens, const void *const *slabs, size_t n_pages, size_t slab_bytes,
+                                      const int32_t *block_tables, int max_blocks, int B, void *logits, float *logprobs, int32_t *next_tokens,
+                                      int flags, void *stream) {
+    return step_batch(d, tokens, context_lens, nullptr, slabs, n_pages, slab_bytes, block_tables, max_blocks, B, logits, logprobs, next_tokens, flags, stream);
+}
+extern "C" int pie_decoder_step_batch_advance(pie_decoder *d, const int32_t *tokens, int32_t *context_lens, const void *const *slabs, size_t n_pages, size_t slab_bytes,
+                                              const int32_t *block_tables, int max_blocks, int B, void *logits, float *logprobs, int32_t *next_tokens,
+                                              int flags, void *stream) {
+    return step_batch(d, tokens, context_lens, context_lens, slabs, n_pages, slab_bytes, block_tables, max_blocks, B, logits, logprobs, next_tokens, flags, stream);
 }
 
 int prefill_batched(pie_decoder *d, const int32_t *ids, const void *embeds, int L, void *logits_all, hipStream_t st) {

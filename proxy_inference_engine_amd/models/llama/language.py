@@ -595,9 +595,9 @@ class Model:
         n = len(self.layers)
         slabs = (C.c_void_p * n)(*[a.slab[i].data_ptr() for i in range(n)])
         self._match_page_format(a)
-        _ffi.check(_ffi.load().pie_decoder_step_batch(self._dec, _ffi.p(tokens), _ffi.p(buf["ctx"]), slabs, a.size(), a.slab[0].numel() * a.slab.element_size(), _ffi.p(buf["table"]),
+        _ffi.check(_ffi.load().pie_decoder_step_batch_advance(self._dec, _ffi.p(tokens), _ffi.p(buf["ctx"]), slabs, a.size(), a.slab[0].numel() * a.slab.element_size(), _ffi.p(buf["table"]),
                                                       buf["table"].shape[1], B, _ffi.p(buf["logits"]), _ffi.p(buf["logprobs"]), _ffi.p(buf["next"]),
-                                                      _ffi.PIE_STEP_ADVANCE | (_ffi.PIE_STEP_GRAPH if graph else 0), _ffi.stream()))
+                                                      _ffi.PIE_STEP_GRAPH if graph else 0, _ffi.stream()))
         buf["at"] = [n + 1 for n in at]
         nxt, logprobs, logits = buf["next"], buf["logprobs"], buf["logits"]
         for s in seqs:

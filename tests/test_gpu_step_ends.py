@@ -102,3 +102,23 @@ def test_batch_steps_take_tokens_where_they_lie_and_move_the_lengths_on(B):
             c[0].page_manager.release()
     for a, b in zip(*runs):
         assert all(torch.equal(x, y) for x, y in zip(a, b))
+
+
+@pytest.mark.parametrize("B", [3, 7])
+def test_lengths_move_where_they_were_given_to_be_written(B):
+    """pie_decoder_step_batch leaves them, whatever bits its flags have; pie_decoder_step_batch_advance adds one to those of slots in use."""
+    import ctypes as C
+    m = llama(320, 2, (4, 64))
+    pool = m.enable_paged_kv(num_pages=2 * B, max_blocks=4)
+    caches = [m.make_cache() for _ in range(B)]
+    m.prefill_batch([np.arange(9 + i, dtype=np.int32) for i in range(B)], caches)
+    lens = torch.tensor([0] + [10 + i for i in range(1, B)], dtype=torch.int32)
+    table = torch.tensor([[c[0].page_manager.pages[0], 0] for c in caches], dtype=torch.int32, device="cuda")
+    feed, token = torch.arange(B, dtype=torch.int32, device="cuda"), torch.empty(B, dtype=torch.int32, device="cuda")
+    logits, logprobs = torch.empty((B, 328), dtype=torch.bfloat16, device="cuda"), torch.empty((B, 328), device="cuda")
+    slabs, lib = (C.c_void_p * 2)(*[s.data_ptr() for s in pool.slab]), _ffi.load()
+    for step, flags, moved in ((lib.pie_decoder_step_batch, 0, 0), (lib.pie_decoder_step_batch, 4, 0), (lib.pie_decoder_step_batch_advance, 0, 1)):
+        ctx = lens.cuda()
+        _ffi.check(step(m._dec, _ffi.p(feed), _ffi.p(ctx), slabs, pool.size(), pool.slab[0].numel() * pool.slab[0].element_size(), _ffi.p(table), 2, B, _ffi.p(logits), _ffi.p(logprobs),
+                        _ffi.p(token), flags, _ffi.stream()))
+        assert torch.equal(ctx.cpu(), torch.where(lens > 0, lens + moved, lens)), (flags, moved)
