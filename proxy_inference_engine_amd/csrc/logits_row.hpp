@@ -27,13 +27,19 @@ template <> struct LogitOctet<float> {
     template <class T>
     __device__ __forceinline__ void get(float (&v)[8]) const { v[0] = a.x, v[1] = a.y, v[2] = a.z, v[3] = a.w, v[4] = b.x, v[5] = b.y, v[6] = b.z, v[7] = b.w; }
 };
-// exp(x) for x <= 0 in three instructions: v_exp_f32 is good to one ulp like expf, and the argument's rounding moves a term of the sum by at most x e^x 2^-24 <= 0.4 2^-24 of the largest one
-__device__ __forceinline__ float logits_exp(float x) { return __builtin_amdgcn_exp2f(x * 1.4426950408889634f); }
+// exp(x) for x <= 0: 2^t (1 + r), t = x log2 e as rounded, r = x - t ln 2 what the roundings left out.  (2^t alone is off by up to |x| 2^-24, alike for like logits: a sum of terms far below
+// the maximum takes it whole.)  From -104 down e^x is below the smallest number there is, and -inf would make r a NaN.  A NaN counts nothing.
+__device__ __forceinline__ float logits_exp(float x) {
+    constexpr float LN2 = 0.69314718055994531f, REST = (float)(0.69314718055994531 - (double)LN2);
+    x = fmaxf(x, -104.0f);
+    const float t = x * 1.4426950408889634f, e = __builtin_amdgcn_exp2f(t);
+    return fmaf(e, fmaf(-t, REST, fmaf(-t, LN2, x)), e);
+}
 template <class T> __device__ __forceinline__ float logit_f32(u16 x) { return T::to_f32(x); }
 template <class T> __device__ __forceinline__ float logit_f32(float x) { return x; }
 
-// -> log(sum exp(row)) and the first index of the row's maximum, in every thread of the workgroup.  A thread's sum that is not a number (a NaN among its logits, an infinite maximum) does not
-// count, as a tile's did not when tiles were merged; a row of nothing above -inf has token INT_MAX.
+// -> log(sum exp(row)) and the first index of the row's maximum, in every thread of the workgroup.  A NaN counts nothing, in an infinite maximum's row neither does
+// what is finite; a row of nothing above -inf has token INT_MAX.
 template <class T, class L>
 __device__ __forceinline__ void logits_row_stats(const L *row, int V, float &lse, int &token) {
     constexpr int NT = LOGITS_ROW_THREADS, WAVES = NT / 64, U = 4;  // U octets of a thread in flight
@@ -41,7 +47,7 @@ __device__ __forceinline__ void logits_row_stats(const L *row, int V, float &lse
     __shared__ int s_arg[WAVES];
     float m = -INFINITY, s = 0.0f;
     int arg = 0x7fffffff;
-    auto take = [&](const float (&v)[8], int at, int n) {  // the first n of v: logits at, at + 1, ...
+    auto take = [&](const float (&v)[8], int at, int step, int n) {  // the first n of v: logits at, at + step, ...
         float top = v[0];
 #pragma unroll
         for (int j = 1; j < 8; ++j)
@@ -50,12 +56,14 @@ __device__ __forceinline__ void logits_row_stats(const L *row, int V, float &lse
             s *= logits_exp(m - top), m = top;
 #pragma unroll
             for (int j = 7; j >= 0; --j)
-                if (j < n && v[j] == top) arg = at + j;
+                if (j < n && v[j] == top) arg = at + j * step;
         }
-        if (m > -INFINITY)
+        if (m > -INFINITY) {
+            float e[8];
 #pragma unroll
-            for (int j = 0; j < 8; ++j)
-                if (j < n) s += logits_exp(v[j] - m);
+            for (int j = 0; j < 8; ++j) e[j] = j < n ? logits_exp(v[j] - m) : 0.0f;
+            s += ((e[0] + e[1]) + (e[2] + e[3])) + ((e[4] + e[5]) + (e[6] + e[7]));
+        }
     };
     if ((V & 7) == 0 && ((size_t)row & 15) == 0) {
         for (int base = threadIdx.x * 8; base < V; base += U * NT * 8) {
@@ -71,13 +79,15 @@ __device__ __forceinline__ void logits_row_stats(const L *row, int V, float &lse
                 if (base + u * NT * 8 < V) {
                     float v[8];
                     q[u].template get<T>(v);
-                    take(v, base + u * NT * 8, 8);
+                    take(v, base + u * NT * 8, 1, 8);
                 }
         }
     } else {
-        for (int i = threadIdx.x; i < V; i += NT) {
-            const float v[8] = {logit_f32<T>(row[i])};
-            take(v, i, 1);
+        for (int i = threadIdx.x; i < V; i += NT * 8) {
+            float v[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) v[j] = logit_f32<T>(row[min(i + j * NT, V - 1)]);
+            take(v, i, NT, min(8, (V - 1 - i) / NT + 1));
         }
     }
     const int wave = threadIdx.x >> 6;
@@ -88,14 +98,13 @@ __device__ __forceinline__ void logits_row_stats(const L *row, int V, float &lse
     const float ws = wave_sum(s > 0.0f ? s * logits_exp(m - wm) : 0.0f);
     if ((threadIdx.x & 63) == 0) s_max[wave] = wm, s_sum[wave] = ws, s_arg[wave] = cand;
     __syncthreads();
-    float M = -INFINITY, S = 0.0f;
-    token = 0x7fffffff;
+    // every wave merges the waves', one a lane (and adds them as a tree)
+    const int lane = threadIdx.x & 63, w = lane & (WAVES - 1);
+    const float wmax = s_max[w], M = wave_max(wmax);
+    token = wmax == M ? s_arg[w] : 0x7fffffff;
 #pragma unroll
-    for (int w = 0; w < WAVES; ++w)
-        if (s_max[w] > M || (s_max[w] == M && s_arg[w] < token)) M = s_max[w], token = s_arg[w];
-#pragma unroll
-    for (int w = 0; w < WAVES; ++w) S += s_sum[w] > 0.0f ? s_sum[w] * logits_exp(s_max[w] - M) : 0.0f;
-    lse = M + logf(S);
+    for (int o = WAVES / 2; o > 0; o >>= 1) token = min(token, __shfl_xor(token, o, 64));
+    lse = M + logf(wave_sum(lane < WAVES && s_sum[w] > 0.0f ? s_sum[w] * logits_exp(wmax - M) : 0.0f));
 }
 
 // logprobs = row - lse over share `part` of `parts`

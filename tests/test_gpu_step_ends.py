@@ -122,3 +122,21 @@ def test_lengths_move_where_they_were_given_to_be_written(B):
         _ffi.check(step(m._dec, _ffi.p(feed), _ffi.p(ctx), slabs, pool.size(), pool.slab[0].numel() * pool.slab[0].element_size(), _ffi.p(table), 2, B, _ffi.p(logits), _ffi.p(logprobs),
                         _ffi.p(token), flags, _ffi.stream()))
         assert torch.equal(ctx.cpu(), torch.where(lens > 0, lens + moved, lens)), (flags, moved)
+
+
+@pytest.mark.parametrize("V", [8, 1023, 1024, 8192, 32768, 33001, 131072, 131075])
+def test_the_sum_of_a_row_takes_exponentials_to_their_last_bit(V):
+    """Rows of one logit of 0 and V - 1 equal ones below it, so that an exponential's error is the sum's, and rows of log-probabilities with a spike of 0: log sum exp is read off the spike, near
+    1 where a float has steps of 2^-24 .. 2^-23.  An exponential and a logarithm of an ulp each (2^-24 rms), the result's rounding and the roundings of sums that are added pairwise: an rms of
+    2^-23 together.  (An exponential of a rounded product, 2^-24 |x| log2 e off, gives 1.5 to 2.5 2^-23.)"""
+    square = 0.0
+    for i in range(150):
+        if i % 2:
+            x = torch.full((V,), 1.0 + i / 100 - np.log(V))
+        else:
+            x = torch.randn(V, generator=torch.Generator().manual_seed(i)) * 2
+            x -= torch.logsumexp(x.double(), 0).float() + i / 150
+        x[V // 2] = 0.0
+        lp = ops.logprobs_argmax(x.cuda())[1]
+        square += float(lp[V // 2].double().cpu() + torch.logsumexp(x.double(), 0)) ** 2
+    assert (square / 150) ** 0.5 <= 2.0 ** -23
