@@ -556,7 +556,7 @@ int pie_repack_w4s_to_w4m(const void *w4s, int N, int K, void *w4m, void *stream
 int pie_qgemm_w4m(const void *x, const void *w4m, int M, int N, int K, int dtype, void *y, void *stream);
 
 
-/* The tail over fp32 logits [rows][V] (logprobs nullable); workspace: pie_logprobs_argmax_f32_workspace(rows) bytes of device scratch. */
+/* The tail over fp32 logits [rows][V] (logprobs nullable; it may be logits); workspace: pie_logprobs_argmax_f32_workspace(rows) bytes of device scratch. */
 size_t pie_logprobs_argmax_f32_workspace(int rows);
 int pie_logprobs_argmax_f32(const float *logits, int rows, int V, float *logprobs, int32_t *tokens, void *workspace, void *stream);
 

@@ -235,6 +235,8 @@ __global__ void __launch_bounds__(256) k_point_residual(const u16 *y, int ldy, P
     }
 }
 
+// In place (logprobs == logits) one workgroup has a row to itself: it has read all of it before it writes any
+static int f32_row_parts(int rows, const float *logits, const float *logprobs) { return logprobs && logprobs != logits ? logits_row_parts(rows) : 1; }
 // log-softmax and greedy token over fp32 logits (logits_row.hpp), grid (rows, parts); a decode step feeds itself
 __global__ void __launch_bounds__(LOGITS_ROW_THREADS) k_f32_rows(const float *logits, int V, float *logprobs, int *next, int advance, int *ids, int *pos, int *history, int history_len) {
     const size_t r = blockIdx.x;
@@ -1130,7 +1132,7 @@ int stack_enqueue(pie_stack *s, const pie_stack_batch &b, const Plan &plan, hipS
         a.M = b.n_want, a.epi = s->cfg.logit_cap > 0.0f ? ROWS_SOFTCAP : ROWS_SCALE_F32, a.scale = s->cfg.logit_scale, a.act_limit = s->cfg.logit_cap, a.rows = b.want, a.x_rows = M;
         p.linear(a);
         if (!p.rc && b.next) {
-            hipLaunchKernelGGL(k_f32_rows, dim3((unsigned)b.n_want, b.logprobs ? logits_row_parts(b.n_want) : 1), dim3(LOGITS_ROW_THREADS), 0, st, b.logits, V, b.logprobs, b.next, b.advance, b.ids, b.pos,
+            hipLaunchKernelGGL(k_f32_rows, dim3((unsigned)b.n_want, f32_row_parts(b.n_want, b.logits, b.logprobs)), dim3(LOGITS_ROW_THREADS), 0, st, b.logits, V, b.logprobs, b.next, b.advance, b.ids, b.pos,
                                b.history, b.history_len);
             PIE_LAUNCH_CHECK();
             ++p.launches;
@@ -1255,7 +1257,7 @@ size_t pie_logprobs_argmax_f32_workspace(int rows) { return rows > 0 ? (size_t)r
 int pie_logprobs_argmax_f32(const float *logits, int rows, int V, float *logprobs, int32_t *tokens, void *workspace, void *stream) {
     PIE_REQUIRE(logits && tokens && workspace, PIE_E_ARG, "pie_logprobs_argmax_f32: null pointer");
     PIE_REQUIRE(rows > 0 && rows <= 65535 && V > 0, PIE_E_SHAPE, "pie_logprobs_argmax_f32: bad shape");
-    hipLaunchKernelGGL(k_f32_rows, dim3((unsigned)rows, logprobs ? logits_row_parts(rows) : 1), dim3(LOGITS_ROW_THREADS), 0, (hipStream_t)stream, logits, V, logprobs, tokens, 0, nullptr, nullptr, nullptr, 0);
+    hipLaunchKernelGGL(k_f32_rows, dim3((unsigned)rows, f32_row_parts(rows, logits, logprobs)), dim3(LOGITS_ROW_THREADS), 0, (hipStream_t)stream, logits, V, logprobs, tokens, 0, nullptr, nullptr, nullptr, 0);
     PIE_LAUNCH_CHECK();
     return PIE_OK;
 }

@@ -140,3 +140,16 @@ def test_the_sum_of_a_row_takes_exponentials_to_their_last_bit(V):
         lp = ops.logprobs_argmax(x.cuda())[1]
         square += float(lp[V // 2].double().cpu() + torch.logsumexp(x.double(), 0)) ** 2
     assert (square / 150) ** 0.5 <= 2.0 ** -23
+
+
+@pytest.mark.parametrize("V", [33, 32768, 131072])
+@pytest.mark.parametrize("rows", [1, 5, 40])
+def test_log_probabilities_in_the_logits_place(rows, V):
+    x = torch.randn(rows, V, generator=torch.Generator().manual_seed(rows)).cuda()
+    lib, got = _ffi.load(), []
+    ws = torch.empty(lib.pie_logprobs_argmax_f32_workspace(rows), dtype=torch.uint8, device="cuda")
+    for lp, logits in ((torch.empty_like(x), x), (x, x)):
+        token = torch.empty(rows, dtype=torch.int32, device="cuda")
+        _ffi.check(lib.pie_logprobs_argmax_f32(_ffi.p(logits), rows, V, _ffi.p(lp), _ffi.p(token), _ffi.p(ws), _ffi.stream()))
+        got.append((lp.clone(), token))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
