@@ -235,14 +235,12 @@ __global__ void __launch_bounds__(256) k_point_residual(const u16 *y, int ldy, P
     }
 }
 
-// In place (logprobs == logits) one workgroup has a row to itself: it has read all of it before it writes any
-static int f32_row_parts(int rows, const float *logits, const float *logprobs) { return logprobs && logprobs != logits ? logits_row_parts(rows) : 1; }
 // log-softmax and greedy token over fp32 logits (logits_row.hpp), grid (rows, parts); a decode step feeds itself
-__global__ void __launch_bounds__(LOGITS_ROW_THREADS) k_f32_rows(const float *logits, int V, float *logprobs, int *next, int advance, int *ids, int *pos, int *history, int history_len) {
+__global__ void __launch_bounds__(LOGITS_ROW_THREADS) k_f32_rows(const float *logits, int V, const RowStat *tiles, float *logprobs, int *next, int advance, int *ids, int *pos, int *history, int history_len) {
     const size_t r = blockIdx.x;
     float lse;
     int token;
-    logits_row_stats<BF16>(logits + r * V, V, lse, token);
+    logits_row_stats<BF16>(logits + r * V, V, tiles ? tiles + r * LOGITS_TILES : nullptr, lse, token);
     if (logprobs) logits_row_write<BF16>(logits + r * V, V, lse, blockIdx.y, gridDim.y, logprobs + r * V);
     if (blockIdx.y == 0 && threadIdx.x == 0) {
         next[r] = token;
@@ -252,6 +250,21 @@ __global__ void __launch_bounds__(LOGITS_ROW_THREADS) k_f32_rows(const float *lo
             if (history && r == 0 && p < history_len) history[p] = token;
         }
     }
+}
+// tiles: LOGITS_TILES a row of scratch.  In place (logprobs == logits) and not in tiles one workgroup has a row to itself: it has read all of it before it writes any
+static int f32_rows_launch(const float *logits, int rows, int V, float *logprobs, int *next, RowStat *tiles, hipStream_t st, int &launches, int advance = 0, int *ids = nullptr, int *pos = nullptr,
+                           int *history = nullptr, int history_len = 0) {
+    const bool in_tiles = logits_in_tiles(rows, V);
+    if (in_tiles) {
+        hipLaunchKernelGGL((k_logits_tiles<BF16, float>), dim3(LOGITS_TILES, (unsigned)rows), dim3(LOGITS_TILE_THREADS), 0, st, logits, V, tiles);
+        PIE_LAUNCH_CHECK();
+        ++launches;
+    }
+    const int parts = logprobs && (logprobs != logits || in_tiles) ? logits_row_parts(rows) : 1;
+    hipLaunchKernelGGL(k_f32_rows, dim3((unsigned)rows, parts), dim3(LOGITS_ROW_THREADS), 0, st, logits, V, in_tiles ? tiles : nullptr, logprobs, next, advance, ids, pos, history, history_len);
+    PIE_LAUNCH_CHECK();
+    ++launches;
+    return PIE_OK;
 }
 
 template <class T>
@@ -298,6 +311,7 @@ struct pie_stack {
     // workspace, by rows of a pass
     Buf<float> x, c_raw, part, part_s, attn_ws, gemm_ws, y32, logits_e, rec_ws, rec_o, rec_den;
     Buf<char> h, hc, q, qu, cq, ql, oc, o, act, act_e, act_s, y, ctx, kv, mixes, mixed, side;
+    Buf<RowStat> stats;             // tiles of the wanted rows' logits
     Buf<int> route_ints;
     Buf<RouteLayer> route_dev;
     Buf<int> arrived;               // rows that have chosen their experts (zero between launches)
@@ -478,7 +492,7 @@ int stack_reserve(pie_stack *s, const pie_stack_batch &b, const Plan &plan, hipS
     if ((rc = s->x.need(M * streams * W64, &moved)) || (rc = s->c_raw.need(M * c, &moved)) || (rc = s->part.need(M * part, &moved)) || (rc = s->part_s.need(M * part_s, &moved)) ||
         (rc = s->h.need(M * WA * E, &moved)) || (rc = s->q.need(M * q * E, &moved)) || (rc = s->ql.need(M * ql * E, &moved)) || (rc = s->oc.need(M * ql * E, &moved)) ||
         (rc = s->o.need(M * o * E, &moved)) || (rc = s->act.need(M * act * E, &moved)) || (rc = s->act_e.need(M * act_e * E, &moved)) ||
-        (rc = s->act_s.need(M * act_s * E, &moved)) || (rc = s->y.need(plan.big ? M * W64 * E : 0, &moved)) ||
+        (rc = s->act_s.need(M * act_s * E, &moved)) || (rc = s->stats.need((size_t)b.n_want * LOGITS_TILES, &moved)) || (rc = s->y.need(plan.big ? M * W64 * E : 0, &moved)) ||
         (rc = s->y32.need(plan.big ? 0 : M * W64, &moved)) || (rc = s->logits_e.need(M * le, &moved)) || (rc = s->rec_ws.need(rw, &moved)) || (rc = s->rec_o.need(M * ro, &moved)) ||
         (rc = s->rec_den.need(M * rd, &moved)) || (rc = s->hc.need(M * hc * E, &moved)) || (rc = s->mixes.need(M * mx * E, &moved)) || (rc = s->mixed.need(M * md * E, &moved)) || (rc = s->side.need(M * sd * E, &moved)) || (rc = s->qu.need(M * qu * E, &moved)) || (rc = s->cq.need(M * cq * E, &moved)) || (rc = s->ctx.need(ctx * E, &moved)) ||
         (rc = s->kv.need(kv * E, &moved)) || (rc = s->gemm_ws.need(ws, &moved)))
@@ -1132,10 +1146,7 @@ int stack_enqueue(pie_stack *s, const pie_stack_batch &b, const Plan &plan, hipS
         a.M = b.n_want, a.epi = s->cfg.logit_cap > 0.0f ? ROWS_SOFTCAP : ROWS_SCALE_F32, a.scale = s->cfg.logit_scale, a.act_limit = s->cfg.logit_cap, a.rows = b.want, a.x_rows = M;
         p.linear(a);
         if (!p.rc && b.next) {
-            hipLaunchKernelGGL(k_f32_rows, dim3((unsigned)b.n_want, f32_row_parts(b.n_want, b.logits, b.logprobs)), dim3(LOGITS_ROW_THREADS), 0, st, b.logits, V, b.logprobs, b.next, b.advance, b.ids, b.pos,
-                               b.history, b.history_len);
-            PIE_LAUNCH_CHECK();
-            ++p.launches;
+            p.rc = f32_rows_launch(b.logits, b.n_want, V, b.logprobs, b.next, s->stats.p, st, p.launches, b.advance, b.ids, b.pos, b.history, b.history_len);
         }
     }
     s->launches = p.launches;
@@ -1252,14 +1263,12 @@ int pie_stack_set_layer(pie_stack *s, int i, const pie_stack_layer *L) {
     return PIE_OK;
 }
 
-// (the rows need no scratch any more; callers size and pass it as before)
-size_t pie_logprobs_argmax_f32_workspace(int rows) { return rows > 0 ? (size_t)rows * 1024 : 0; }
+size_t pie_logprobs_argmax_f32_workspace(int rows) { return rows > 0 ? (size_t)rows * LOGITS_TILES * sizeof(RowStat) : 0; }
 int pie_logprobs_argmax_f32(const float *logits, int rows, int V, float *logprobs, int32_t *tokens, void *workspace, void *stream) {
     PIE_REQUIRE(logits && tokens && workspace, PIE_E_ARG, "pie_logprobs_argmax_f32: null pointer");
     PIE_REQUIRE(rows > 0 && rows <= 65535 && V > 0, PIE_E_SHAPE, "pie_logprobs_argmax_f32: bad shape");
-    hipLaunchKernelGGL(k_f32_rows, dim3((unsigned)rows, f32_row_parts(rows, logits, logprobs)), dim3(LOGITS_ROW_THREADS), 0, (hipStream_t)stream, logits, V, logprobs, tokens, 0, nullptr, nullptr, nullptr, 0);
-    PIE_LAUNCH_CHECK();
-    return PIE_OK;
+    int launches = 0;
+    return f32_rows_launch(logits, rows, V, logprobs, tokens, (RowStat *)workspace, (hipStream_t)stream, launches);
 }
 
 int pie_stack_page_row(const pie_stack *s, int i) {

@@ -1,9 +1,9 @@
-// logits_row.hpp -- log-softmax normaliser and greedy token of whole logit rows in one launch (engine/inference_engine.py:254,268-271, samplers/__init__.py:37-38).
+// logits_row.hpp -- log-softmax normaliser and greedy token of whole logit rows, in one launch or in two (engine/inference_engine.py:254,268-271, samplers/__init__.py:37-38).
 //
 // Every workgroup of a row reads the whole row (from L2: a row's workgroups share an XCD where the rows come in eights), keeps one running (max, sum, first index of the max) per thread and
-// merges them once; then it writes its share of the log-probabilities.  What bounds it is the launch and one workgroup's 32 exponentials a thread.  Rows of 32768 logits, traced, us:
-// 8 rows 6.8, 32 rows 7.2 (fp32: 8.0).  Partials in one launch and their merge in another took 4.7 + 5.2 and 10.6 + 12.6 (the merging workgroups fetched 16 partials a thread of the one that
-// there was; fp32: 4.8 + 4.4).  With expf, a dozen instructions, 9.9 and 11.
+// merges them once; then it writes its share of the log-probabilities.  What bounds it is the launch and one workgroup's exponentials, 32 a thread of 32768 logits.  16-bit rows of 32768, traced,
+// us: 8 rows 6.9, 32 rows 8.0; with expf, a dozen instructions, 9.9 and 11.  Few rows of many more logits come in tiles, a launch in front of this one (logits_in_tiles): 128256 logits, traced,
+// us, 8 rows 17.3 -> 8.6, 32 rows 21.2 -> 13.0; tiles of 32768 7.6 and 9.0.
 #pragma once
 #include "common.hpp"
 
@@ -38,11 +38,11 @@ __device__ __forceinline__ float logits_exp(float x) {
 template <class T> __device__ __forceinline__ float logit_f32(u16 x) { return T::to_f32(x); }
 template <class T> __device__ __forceinline__ float logit_f32(float x) { return x; }
 
-// -> log(sum exp(row)) and the first index of the row's maximum, in every thread of the workgroup.  A NaN counts nothing, in an infinite maximum's row neither does
+// -> maximum M of the n logits from row on, sum of exp(logit - M) and the first index of the maximum (the first logit's is at), in every thread of the workgroup.  A NaN counts nothing, in an infinite maximum's row neither does
 // what is finite; a row of nothing above -inf has token INT_MAX.
-template <class T, class L>
-__device__ __forceinline__ void logits_row_stats(const L *row, int V, float &lse, int &token) {
-    constexpr int NT = LOGITS_ROW_THREADS, WAVES = NT / 64, U = 4;  // U octets of a thread in flight
+template <class T, int NT, class L>
+__device__ __forceinline__ void logits_stats(const L *row, int V, int first, float &M, float &S, int &token) {
+    constexpr int WAVES = NT / 64, U = 4;  // U octets of a thread in flight
     __shared__ float s_max[WAVES], s_sum[WAVES];
     __shared__ int s_arg[WAVES];
     float m = -INFINITY, s = 0.0f;
@@ -100,11 +100,42 @@ __device__ __forceinline__ void logits_row_stats(const L *row, int V, float &lse
     __syncthreads();
     // every wave merges the waves', one a lane (and adds them as a tree)
     const int lane = threadIdx.x & 63, w = lane & (WAVES - 1);
-    const float wmax = s_max[w], M = wave_max(wmax);
+    const float wmax = s_max[w];
+    M = wave_max(wmax);
     token = wmax == M ? s_arg[w] : 0x7fffffff;
 #pragma unroll
     for (int o = WAVES / 2; o > 0; o >>= 1) token = min(token, __shfl_xor(token, o, 64));
-    lse = M + logf(wave_sum(lane < WAVES && s_sum[w] > 0.0f ? s_sum[w] * logits_exp(wmax - M) : 0.0f));
+    S = wave_sum(lane < WAVES && s_sum[w] > 0.0f ? s_sum[w] * logits_exp(wmax - M) : 0.0f);
+    if (token != 0x7fffffff) token += first;
+}
+
+// Rows in 64 tiles, for a launch of their own
+constexpr int LOGITS_TILES = 64, LOGITS_TILE_THREADS = 256;
+struct RowStat {  // of a tile (of an empty one: -inf, 0, INT_MAX)
+    float max, sum;
+    int arg, pad;
+};
+template <class T, class L>
+__global__ void __launch_bounds__(LOGITS_TILE_THREADS) k_logits_tiles(const L *logits, int V, RowStat *stats) {  // grid (tiles, rows)
+    const int len = ((V + LOGITS_TILES - 1) / LOGITS_TILES + 7) & ~7, begin = blockIdx.x * len;
+    RowStat s;
+    s.pad = 0;
+    logits_stats<T, LOGITS_TILE_THREADS>(logits + (size_t)blockIdx.y * V + begin, min(V - begin, len), begin, s.max, s.sum, s.arg);
+    if (threadIdx.x == 0) stats[blockIdx.y * LOGITS_TILES + blockIdx.x] = s;
+}
+
+// -> log(sum exp(row)) and the row's first maximum, in every thread: of the row's tiles where a launch in front of this one left them, else of the row
+template <class T, class L>
+__device__ __forceinline__ void logits_row_stats(const L *row, int V, const RowStat *tiles, float &lse, int &token) {
+    float M, S;
+    if (tiles) {  // (every wave merges them, one a lane)
+        const RowStat s = tiles[threadIdx.x & 63];
+        M = wave_max(s.max), token = s.max == M ? s.arg : 0x7fffffff;
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) token = min(token, __shfl_xor(token, o, 64));
+        S = wave_sum(s.sum > 0.0f ? s.sum * logits_exp(s.max - M) : 0.0f);
+    } else logits_stats<T, LOGITS_ROW_THREADS>(row, V, 0, M, S, token);
+    lse = M + logf(S);
 }
 
 // logprobs = row - lse over share `part` of `parts`
@@ -126,3 +157,10 @@ __device__ __forceinline__ void logits_row_write(const L *row, int V, float lse,
 
 // workgroups per row: a workgroup on every CU while the rows are few, so that a CU's writes are a fraction of a row (all read all of it)
 static inline int logits_row_parts(int rows) { return rows >= 256 ? 1 : rows <= 16 ? 16 : 256 / rows; }
+// A row's exponentials are taken by each of its workgroups, by tiles only once but in two launches (fp32: 9.5 us whatever the row is, until the tiles fill the chip): worth it for rows of a large
+// vocabulary that are not many.  One launch / two, us, fp32: 49152 logits, 8 rows 8.7 / 9.4; 65536, 8 rows 10.2 / 9.5, 48 rows 12.8 / 12.8; 128256, 1 row 15.7 / 9.7, 64 rows 23.3 / 20.7,
+// 128 rows 34.3 / 36.7; 262144, 8 rows 29.8 / 9.7.  Rows that are no multiple of eight logits are loaded one by one and cost two fifths more: 50257, 8 rows 11.9 / 9.6, 64 rows 14.2 / 16.1.
+static inline bool logits_in_tiles(int rows, int V) {
+    const int work = V & 7 ? V + V / 5 * 2 : V;
+    return work >= 60000 && rows <= work / 1500;
+}

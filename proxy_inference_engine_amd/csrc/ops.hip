@@ -306,7 +306,7 @@ int pie_stream_read(const void *p, size_t bytes, void *stream) {
 int pie_logprobs_argmax(const void *logits, int V, int dtype, float *logprobs, int32_t *token, void *stream) {
     PIE_REQUIRE(logits && logprobs && token, PIE_E_ARG, "pie_logprobs_argmax: null pointer");
     PIE_REQUIRE(V > 0, PIE_E_SHAPE, "pie_logprobs_argmax: empty vocabulary");
-    return logits_tail_rows_launch(dtype, (const u16 *)logits, V, 1, logprobs, token, (hipStream_t)stream);
+    return logits_tail_rows_launch(dtype, (const u16 *)logits, V, 1, nullptr, logprobs, token, (hipStream_t)stream);
 }
 
 }  // extern "C"

@@ -433,8 +433,8 @@ struct PrefillScratch {
     std::map<const void *, u16 *> resident;
     // W4M tile copies (w4m_gemm.hip) of int4 layer matrices for prompts of at most small_rows() rows: 0.5625 B per weight each
     std::map<const void *, void *> resident_w4m;
-    LogitStat *tail_stats = nullptr;  // fused few-sequence step: the lm_head GEMV's tail partials, one per wave and row
-    size_t tail_entries = 0;           // its capacity in entries (rows x waves)
+    LogitStat *tail_stats = nullptr;  // fused few-sequence step: the lm_head GEMV's tail partials, one per wave and row; other rows' tiles (RowStat) where the tail takes two launches
+    size_t tail_entries = 0;           // its capacity in entries
     // Captured multi-sequence step (pie_decoder_step_batch with PIE_STEP_GRAPH): valid while the caller's buffers (key) and every
     // device allocation baked into the launches (alloc_gen) stay what they were at capture time.
     unsigned alloc_gen = 0;
@@ -449,6 +449,7 @@ struct PrefillScratch {
     size_t resident_left = 0; // bytes still available for resident copies
 };
 
+static_assert(sizeof(RowStat) == sizeof(LogitStat), "one buffer for both");
 static int tail_stats_reserve(PrefillScratch *s, size_t entries) {
     if (s->tail_entries >= entries) return PIE_OK;
     if (s->tail_stats) (void)hipFree(s->tail_stats);
@@ -1052,7 +1053,8 @@ static int decode_batch_t(pie_decoder *d, const int32_t *tokens, const int32_t *
     PrefillScratch *s = d->prefill;
     if (tokens && (rc = batch_rows(d, tokens, ctx_len, B, st))) return rc;  // (nullptr: they are there already)
     const int lm_waves = w4s_gemv_waves(c.vocab, H);
-    if (fused_rows && (rc = tail_stats_reserve(s, (size_t)lm_waves * (size_t)B))) return rc;
+    const bool tiles = !fused_rows && logits_in_tiles(B, c.vocab);
+    if ((fused_rows || tiles) && (rc = tail_stats_reserve(s, (size_t)(tiles ? LOGITS_TILES : lm_waves) * (size_t)B))) return rc;
     if (fused_rows) {
         for (int li = 0; li < c.n_layers; ++li) {
             const pie_layer_weights &w = d->layers[li];
@@ -1135,7 +1137,7 @@ static int decode_batch_t(pie_decoder *d, const int32_t *tokens, const int32_t *
     // the head's 16-bit tiles stay, like the layers' (int4: its W4M tiles do): laid out anew for every step they cost more than the product (268 MB: 115 us beside 42)
     const bool keep_head = d->mat_fmt(d->glob.lm_head) != PIE_W_INT4_G64;
     if ((rc = linear_rows<T>(d, d->glob.lm_head, c.vocab, H, s->xn, B, logits, st, keep_head, nullptr, true))) return rc;
-    return logits_tail_rows_launch(c.dtype, logits, c.vocab, B, logprobs, next_tokens, st, lens);
+    return logits_tail_rows_launch(c.dtype, logits, c.vocab, B, tiles ? (RowStat *)s->tail_stats : nullptr, logprobs, next_tokens, st, lens);
 }
 
 
@@ -1169,6 +1171,8 @@ static int prefill_varlen_t(pie_decoder *d, const int32_t *ids, const int32_t *r
     int rc = scratch_reserve(d, N > S ? N : S, w_elems, (size_t)n_decode * dsplits);
     if (rc) return rc;
     PrefillScratch *s = d->prefill;
+    const bool tiles = logits_in_tiles(S, c.vocab);
+    if (tiles && (rc = tail_stats_reserve(s, (size_t)LOGITS_TILES * S))) return rc;
     if (n_chunks > 0) reserve_attn_part(d);
     if ((rc = pass_rows(d, ids, nullptr, N, row_ctx, d->layers[0].attn_norm, st))) return rc;
     for (int li = 0; li < c.n_layers; ++li) {
@@ -1232,7 +1236,7 @@ static int prefill_varlen_t(pie_decoder *d, const int32_t *ids, const int32_t *r
     // the normalised last row of every prompt -> lm_head -> tail
     const bool keep_head = d->mat_fmt(d->glob.lm_head) != PIE_W_INT4_G64;  // (as in a step)
     if ((rc = linear_rows<T>(d, d->glob.lm_head, c.vocab, H, s->x, S, logits, st, keep_head, nullptr, true))) return rc;
-    return logits_tail_rows_launch(c.dtype, logits, c.vocab, S, logprobs, next_tokens, st);
+    return logits_tail_rows_launch(c.dtype, logits, c.vocab, S, tiles ? (RowStat *)s->tail_stats : nullptr, logprobs, next_tokens, st);
 }
 
 static size_t active_page_bytes(const pie_decoder *d);

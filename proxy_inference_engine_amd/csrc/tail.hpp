@@ -2,7 +2,7 @@
 // (samplers/__init__.py:37-38): logprobs = f32(logits) - logsumexp(f32(logits)); token = first argmax.
 //
 // Behind the lm_head GEMV, whose epilogue (EPI_LOGITS) leaves per-wave (max, sum exp(x - max), first argmax) partials: k_logits_finish, in which every workgroup merges
-// the partials (a few thousand, L2-resident) and writes its slice of the fp32 logprobs.  Behind any other product: k_logits_rows, one launch (logits_row.hpp).
+// the partials (a few thousand, L2-resident) and writes its slice of the fp32 logprobs.  Behind any other product: k_logits_rows, one launch or, behind k_logits_tiles, two (logits_row.hpp).
 #pragma once
 #include "common.hpp"
 #include "logits_row.hpp"
@@ -10,13 +10,13 @@
 
 constexpr int TAIL_FINISH_BLOCKS = 64;
 
-// whole rows at once, grid (rows, parts): no partials.  lens (nullable): the rows' context lengths, moved on by the token that this step appended
+// whole rows at once, grid (rows, parts); tiles (nullable): what k_logits_tiles left of them.  lens (nullable): the rows' context lengths, moved on by the token that this step appended
 template <class T>
-__global__ void __launch_bounds__(LOGITS_ROW_THREADS) k_logits_rows(const u16 *logits, int V, float *logprobs, int *tokens, int *lens) {
+__global__ void __launch_bounds__(LOGITS_ROW_THREADS) k_logits_rows(const u16 *logits, int V, const RowStat *tiles, float *logprobs, int *tokens, int *lens) {
     const size_t at = (size_t)blockIdx.x * V;
     float lse;
     int token;
-    logits_row_stats<T>(logits + at, V, lse, token);
+    logits_row_stats<T>(logits + at, V, tiles ? tiles + (size_t)blockIdx.x * LOGITS_TILES : nullptr, lse, token);
     logits_row_write<T>(logits + at, V, lse, blockIdx.y, gridDim.y, logprobs + at);
     if (blockIdx.y == 0 && threadIdx.x == 0) {
         tokens[blockIdx.x] = token;
@@ -92,12 +92,18 @@ __global__ void __launch_bounds__(256) k_logits_finish(const u16 *logits, int V,
     }
 }
 
-// `rows` logit vectors [rows, V] at once (the multi-sequence decode step, the op-level API)
-static inline int logits_tail_rows_launch(int dtype, const u16 *logits, int V, int rows, float *logprobs, int *tokens, hipStream_t st, int *lens = nullptr) {
+// `rows` logit vectors [rows, V] at once (the multi-sequence decode step, the op-level API).  tiles: LOGITS_TILES a row of scratch, needed where logits_in_tiles says so (nullptr: not in tiles)
+static inline int logits_tail_rows_launch(int dtype, const u16 *logits, int V, int rows, RowStat *tiles, float *logprobs, int *tokens, hipStream_t st, int *lens = nullptr) {
     if (dtype != PIE_BF16 && dtype != PIE_F16) return pie::fail(PIE_E_ARG, "logits tail: dtype must be PIE_BF16 or PIE_F16");
+    if (tiles) {
+        const dim3 gt(LOGITS_TILES, rows);
+        if (dtype == PIE_BF16) hipLaunchKernelGGL((k_logits_tiles<BF16, u16>), gt, dim3(LOGITS_TILE_THREADS), 0, st, logits, V, tiles);
+        else hipLaunchKernelGGL((k_logits_tiles<F16, u16>), gt, dim3(LOGITS_TILE_THREADS), 0, st, logits, V, tiles);
+        PIE_LAUNCH_CHECK();
+    }
     const dim3 g(rows, logits_row_parts(rows));
-    if (dtype == PIE_BF16) hipLaunchKernelGGL(k_logits_rows<BF16>, g, dim3(LOGITS_ROW_THREADS), 0, st, logits, V, logprobs, tokens, lens);
-    else hipLaunchKernelGGL(k_logits_rows<F16>, g, dim3(LOGITS_ROW_THREADS), 0, st, logits, V, logprobs, tokens, lens);
+    if (dtype == PIE_BF16) hipLaunchKernelGGL(k_logits_rows<BF16>, g, dim3(LOGITS_ROW_THREADS), 0, st, logits, V, tiles, logprobs, tokens, lens);
+    else hipLaunchKernelGGL(k_logits_rows<F16>, g, dim3(LOGITS_ROW_THREADS), 0, st, logits, V, tiles, logprobs, tokens, lens);
     PIE_LAUNCH_CHECK();
     return PIE_OK;
 }
