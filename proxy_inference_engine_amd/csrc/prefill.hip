@@ -880,7 +880,7 @@ static int pass_rows(pie_decoder *d, const int32_t *ids, const void *embeds, int
 }
 
 template <class T>
-static int prefill_t(pie_decoder *d, const int32_t *ids, const void *embeds, int L, void *logits_all, hipStream_t st) {
+static int prefill_t(pie_decoder *d, const int32_t *ids, const void *embeds, int L, void *logits_all, int &moved, hipStream_t st) {  // moved: by how much the device's position has
     const pie_decoder_config &c = d->cfg;
     const int H = c.hidden, D = c.head_dim, QD = c.n_heads * D, KVD = c.n_kv_heads * D, NQKV = QD + 2 * KVD, I = c.inter;
     const int chunk = prefill_chunk_rows() < L ? prefill_chunk_rows() : L;
@@ -920,7 +920,7 @@ static int prefill_t(pie_decoder *d, const int32_t *ids, const void *embeds, int
                 if (!last) break;
                 hipLaunchKernelGGL(k_add_pos, dim3(1), dim3(1), 0, st, d->state, M - 1);
                 PIE_LAUNCH_CHECK();
-                R = 1;
+                moved += M - 1, R = 1;
             }
             u16 *x = s->x + (size_t)(M - R) * H, *q = s->q + (size_t)(M - R) * QD, *attn = s->attn + (size_t)(M - R) * QD;
             if (mfma_attn) {  // causal flash attention on the MFMA units (prefill_attn.hpp)
@@ -970,6 +970,7 @@ static int prefill_t(pie_decoder *d, const int32_t *ids, const void *embeds, int
         if (last && !logits_all) break;  // (the position has moved)
         hipLaunchKernelGGL(k_add_pos, dim3(1), dim3(1), 0, st, d->state, last ? M - 1 : M);
         PIE_LAUNCH_CHECK();
+        moved += last ? M - 1 : M;
     }
     // logits[:, -1, :] -> logprobs -> greedy token; the tail advances the device-side offset past the last prompt token
     if ((rc = enqueue_kernel(d, PIE_K_LMHEAD, 0, nullptr, d->logits, st))) return rc;
@@ -1376,7 +1377,9 @@ extern "C" int pie_decoder_step_batch_advance(pie_decoder *d, const int32_t *tok
 int prefill_batched(pie_decoder *d, const int32_t *ids, const void *embeds, int L, void *logits_all, hipStream_t st) {
     const int rep = d->cfg.n_heads / d->cfg.n_kv_heads;
     PIE_REQUIRE(rep >= 1 && rep <= 8, PIE_E_SHAPE, "prefill: n_heads / n_kv_heads must be between 1 and 8");
-    const int rc = d->cfg.dtype == PIE_BF16 ? prefill_t<BF16>(d, ids, embeds, L, logits_all, st) : prefill_t<F16>(d, ids, embeds, L, logits_all, st);
-    d->pos_hint += L;
+    int moved = 0;
+    const int rc = d->cfg.dtype == PIE_BF16 ? prefill_t<BF16>(d, ids, embeds, L, logits_all, moved, st) : prefill_t<F16>(d, ids, embeds, L, logits_all, moved, st);
+    if (rc == PIE_OK) d->pos_hint += L;
+    else if (moved) hipLaunchKernelGGL(k_add_pos, dim3(1), dim3(1), 0, st, d->state, -moved);  // a prompt that fails leaves the sequence where it was
     return rc;
 }

@@ -161,3 +161,41 @@ def test_the_last_layer_of_a_prompt_takes_its_last_row_alone(bits, layers):
     logits = m.prefill_batch([ids[:n].cpu().numpy() for n in (6, 1, 80)], [m.make_cache() for _ in range(3)])[2].float().cpu().numpy()
     for i in (0, 2):   # (a prompt of one token by itself is a decode step, whose weights are not rounded)
         assert_vec_close(logits[i], alone[i], "bfloat16", what=f"prompt {i} of a batch")
+
+
+@pytest.mark.parametrize("n", [40, 150])
+@pytest.mark.parametrize("paged", [False, True])
+def test_a_prompt_that_fails_leaves_the_sequence_where_it_was(n, paged):
+    """The host refuses the last layer's product (a bias at an odd address) behind the launches of everything before it, in one chunk and in three: the prompt again, with its weights, is the prompt."""
+    import ctypes as C
+    from proxy_inference_engine_amd.models.llama import Model, ModelArgs
+    from proxy_inference_engine_amd.models.utils import synthetic_checkpoint
+    cfg = {"model_type": "llama", "hidden_size": 256, "num_hidden_layers": 2, "intermediate_size": 512, "num_attention_heads": 8, "num_key_value_heads": 2, "head_dim": 64, "vocab_size": 320,
+           "rms_norm_eps": 1e-5, "tie_word_embeddings": False, "quantization": {"group_size": 64, "bits": 4}}
+    m = Model(ModelArgs(**cfg), synthetic_checkpoint(cfg, seed=7))
+    ids = torch.from_numpy(np.random.default_rng(3).integers(0, 320, 200).astype(np.int32)).cuda()
+    if paged:
+        m.enable_paged_kv(num_pages=20, max_blocks=8)
+    blk, bias, lib = m.layers[1], torch.zeros(264, dtype=torch.bfloat16, device="cuda"), _ffi.load()
+
+    def layer(o_bias):
+        w = _ffi.pie_layer_weights(blk.input_layernorm.data_ptr(), blk.post_attention_layernorm.data_ptr(), blk.wqkv.packed.data_ptr(), blk.wo.packed.data_ptr(), blk.wgateup.packed.data_ptr(),
+                                   blk.wdown.packed.data_ptr(), None, o_bias, None, None, *blk.formats)
+        _ffi.check(lib.pie_decoder_set_layer(m._dec, 1, C.byref(w)))
+
+    _ffi.set_knob("prefill_chunk", 64)
+    try:
+        got = []
+        for fail in (False, True):
+            cache = m.make_cache()
+            m.step(ids[:30], cache)
+            if fail:
+                layer(bias.data_ptr() + 2)
+                with pytest.raises(ValueError, match="alignment"):
+                    m.step(ids[30:30 + n], cache)
+                layer(None)
+            got.append([m.step(ids[30:30 + n], cache)[2].clone(), m.step(ids[30 + n:31 + n], cache)[2].clone()])
+            assert cache[0].offset == 31 + n
+    finally:
+        _ffi.set_knob("prefill_chunk", None)
+    assert all(torch.equal(a, b) for a, b in zip(*got))
