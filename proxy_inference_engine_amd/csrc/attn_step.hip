@@ -7,8 +7,8 @@
 // Here a wave takes 16 tokens at a time:
 //   * scores S[token][head] = K q^T by v_mfma_f32_16x16x32, K rows straight from memory in operand order (lane: token lane % 16, dims 32 s + 8 (lane / 16) ..), the query heads as
 //     the 16 columns (four or eight, repeated): no cross-lane additions, and a lane is left with four tokens' scores of ONE head, lane % 4 or lane % 8;
-//   * the softmax of 16 tokens x 4 heads is then four exponentials a lane, not sixteen; a stream is rescaled only where a score exceeds its reference by 2^RISE (weights up to 2^RISE
-//     in fp32 lose nothing, and the merge divides them out);
+//   * the softmax of 16 tokens x 4 heads is then four exponentials a lane, not sixteen; a stream is rescaled only where a score exceeds its reference, which is set RISE above it (weights
+//     of 2^-RISE and less lose nothing in fp32, none is above 1, so that a V near the type's largest has room in the sums, and the merge divides the factor out);
 //   * P V stays fp32 products of the vector units, weights unrounded: lane (tokens 4 (lane / 16) .., dims 8 (lane % 16) ..; heads of 64: half of the tokens) finds its tokens' weights
 //     in its own quad or the one beside (DPP).
 // Blocks of 16 tokens begin at multiples of 16 (a page holds 64): a block lies in one page, its page number and its addresses are the wave's.
@@ -218,9 +218,9 @@ __global__ void __launch_bounds__(STEP_WAVES * 64, REP <= 4 ? 3 : 2) k_attn_step
             sc[i] = in[i] ? s4[i] * sl2 : ATTN_NEG;
             most = fmaxf(most, sc[i]);
         }
-        const bool rise = most > m + RISE;
+        const bool rise = most > m;
         if (__any(rise)) {  // (the whole wave: a quad's lanes hold its heads' factors)
-            const float to = rise ? most : m, f = attn_exp2(m - to);
+            const float to = rise ? most + RISE : m, f = attn_exp2(m - to);
             float fh[REP];
             heads_of<REP>(f, beside<REP>(f), fh);
             l *= f, m = to;

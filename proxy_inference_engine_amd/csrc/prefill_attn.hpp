@@ -235,10 +235,12 @@ __global__ void __launch_bounds__(REP * QT * 64, 2) k_prefill_attn(const Prefill
             for (int i = 0; i < 16; ++i) mloc = fmaxf(mloc, sc[n][i]);
         const float top = xor32_max(mloc);  // the other half of the block's keys lives in the partner lane
         mloc = top * sl2;
-        // A row's reference follows its maximum only from 2^PA_RISE above: with 32 rows to a wave some row's maximum grows in most blocks (two of three at 4096 keys), and the rescale is 64
-        // products a lane.  Weights up to 2^PA_RISE lose nothing in fp32 or in their two halves, and the final division takes the factor out.  (4096 tokens, four layers: 5623 -> 5570 us.)
-        if (mloc > m_run + PA_RISE) {
-            const float m_new = mloc, alpha = attn_exp2(m_run - m_new);
+        // A row's reference follows its maximum only every PA_RISE: with 32 rows to a wave some row's maximum grows in most blocks (two of three at 4096 keys), and the rescale is 64
+        // products a lane.  (4096 tokens, four layers: 5623 -> 5570 us.)  bf16: the reference is set PA_RISE above the maximum -- no weight is above 1 then, and a V near the type's largest
+        // keeps its sum in fp32; f16, whose V are no danger to fp32 but whose small weights have no low half, at the maximum, weights up to 2^PA_RISE.  The final division takes the factor out.
+        constexpr float ABOVE = std::is_same<T, BF16>::value ? PA_RISE : 0.0f;
+        if (mloc > m_run + (PA_RISE - ABOVE)) {
+            const float m_new = mloc + ABOVE, alpha = attn_exp2(m_run - m_new);
             l_run *= alpha;
 #pragma unroll
             for (int dt = 0; dt < DT; ++dt)

@@ -141,3 +141,90 @@ def test_a_batch_reads_no_row_that_nobody_wrote(short, Hq, Hkv, D):
         got = bits_over_pools(model, lens, 12, lambda caches, feed: model.step_batch(feed, caches, graph=False)[2].clone())
         assert torch.isfinite(got[0]).all()
         assert torch.equal(got[0], got[1]) and torch.equal(got[0], got[2]), n
+
+
+def attention_shown(Hq, Hkv, D, dtype, gain=1.0):
+    """A layer that shows its attention: embeddings, MLP and the projections' weights are 0, q, k and v their biases -- q and k in dims that position does not turn (theta 1e30: from a quarter of the
+    pairs on no angle reaches 1e-3 of a step, and the bias is 0 in the others) --, o_proj and lm_head identities (o_proj times gain, a
+    power of two, by which v's bias is divided): logits = T(norm(T(attention)))."""
+    from proxy_inference_engine_amd.models.llama import Model, ModelArgs
+    from proxy_inference_engine_amd.models.utils import synthetic_checkpoint
+    H = Hq * D
+    cfg = {"model_type": "llama", "hidden_size": H, "num_hidden_layers": 1, "intermediate_size": 64, "num_attention_heads": Hq, "num_key_value_heads": Hkv, "head_dim": D, "rms_norm_eps": 1e-5,
+           "vocab_size": H, "rope_theta": 1e30, "max_position_embeddings": 2048, "tie_word_embeddings": False, "attention_bias": True}
+    w = {n: torch.zeros_like(t) for n, t in synthetic_checkpoint(cfg, seed=1, dtype=dtype).items()}
+    g = torch.Generator().manual_seed(Hq * D)
+    still = (torch.arange(D) % (D // 2)) >= D // 4
+    for n, heads in (("q", Hq), ("k", Hkv), ("v", Hkv)):
+        b = torch.randn(heads, D, generator=g) / (gain if n == "v" else 1.0)
+        w[f"model.layers.0.self_attn.{n}_proj.bias"] = (b if n == "v" else b * still).reshape(-1).to(dtype).cuda()
+    w["model.layers.0.self_attn.o_proj.weight"] = (torch.eye(H) * gain).to(dtype).cuda()
+    w["lm_head.weight"] = torch.eye(H, dtype=dtype, device="cuda")
+    for n in w:
+        if "norm" in n:
+            w[n] = torch.ones_like(w[n])
+    return Model(ModelArgs(**cfg), w), [w[f"model.layers.0.self_attn.{n}_proj.bias"].double().cpu().view(-1, D) for n in "qkv"]
+
+
+def check_shown(Hq, Hkv, D, dtype, lens, keys, values, gain=1.0, batch=True, paged=True):
+    """The step against float64, from the rows that lie in the cache: attention good to the sums' fp32 (K 2^-24 of the weighted magnitudes, weights to 2^-20 of themselves: their scores are sums of
+    D products of up to 8 log2 units and more), and three roundings of eps each: of attention, in the norm and behind it."""
+    model, (q, k_new, v_new) = attention_shown(Hq, Hkv, D, dtype, gain)
+    pool = model.enable_paged_kv(num_pages=sum(n // 64 + 1 for n in lens) + 1, max_blocks=16) if paged else None
+    if paged:
+        for slab in pool.slab:
+            slab.view(dtype).fill_(torch.nan)
+    caches, rows = [model.make_cache() for _ in lens], []
+    for i, (n, c) in enumerate(zip(lens, caches)):
+        model.step(torch.zeros(n, dtype=torch.int32, device="cuda"), c)
+        K, V = keys(i, n, q).to(dtype), values(i, n).to(dtype)   # [Hkv, n, D]
+        if paged:
+            for p in range(0, n, 64):
+                page = pool.slab[0].view(dtype).view(-1, 2, Hkv, 64, D)[c[0].page_manager.pages[p // 64]]
+                page[0, :, :min(64, n - p)], page[1, :, :min(64, n - p)] = K[:, p:p + 64].cuda(), V[:, p:p + 64].cuda()
+        else:
+            c[0].keys[0, :, :n], c[0].values[0, :, :n] = K.cuda(), V.cuda()
+        rows.append((torch.cat([K.double(), k_new[:, None]], 1), torch.cat([V.double(), v_new[:, None]], 1)))
+    feed = torch.zeros(len(lens), dtype=torch.int32, device="cuda")
+    if batch:
+        got = model.step_batch(feed, caches, graph=False)[2].double().cpu()
+    else:
+        got = torch.stack([model.step(feed[i:i + 1], c)[2].double().cpu().reshape(-1) for i, c in enumerate(caches)])
+    eps = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    for i, (K, V) in enumerate(rows):
+        K, V = K.repeat_interleave(Hq // Hkv, 0), V.repeat_interleave(Hq // Hkv, 0)
+        p = torch.softmax((K @ q[:, :, None]).squeeze(-1) * D ** -0.5, -1)
+        x = (p[:, None] @ V).reshape(-1) * gain
+        noise = ((p[:, None] @ V.abs()).reshape(-1) * abs(gain)) * (2.0 ** -20 + V.shape[1] * 2.0 ** -24)
+        norm = (x.square().mean() + 1e-5).rsqrt()
+        bound = (x.abs() * 3.1 * eps + noise + noise.square().mean().sqrt() * x.abs() * norm) * norm
+        assert torch.isfinite(got[i]).all(), lens[i]
+        assert ((got[i] - x * norm).abs() <= bound).all(), (lens[i], float(((got[i] - x * norm).abs() / bound).max()))
+
+
+SHOWN = [1, 15, 31, 47, 63, 64, 100, 129, 191, 300, 415, 513]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("Hq,Hkv,D", [(8, 8, 64), (6, 2, 64), (8, 1, 64), (4, 4, 128), (4, 2, 128), (6, 2, 128), (5, 1, 128), (8, 1, 128), (8, 2, 128)])
+@pytest.mark.parametrize("how", ["batch", "paged", "alone"])
+def test_the_attention_of_a_step_against_float64(how, Hq, Hkv, D, dtype):
+    """Random keys (scores of a few units, maxima that rise again and again) and values: batches with one long row, one sequence on pages and in its own buffers."""
+    g = torch.Generator().manual_seed(D)
+    draw = lambda i, n, *_: torch.randn(Hkv, n, D, generator=g) * 2
+    lens = SHOWN + [900] if how != "batch" else SHOWN + [1000]
+    check_shown(Hq, Hkv, D, dtype, lens, draw, draw, batch=how == "batch", paged=how != "alone")
+
+
+@pytest.mark.parametrize("power", [118, -124])
+@pytest.mark.parametrize("Hq,Hkv,D", [(6, 2, 64), (4, 4, 128), (8, 2, 128)])
+@pytest.mark.parametrize("how", ["batch", "paged", "alone"])
+def test_values_near_the_limits_of_bf16(how, Hq, Hkv, D, power):
+    """Weights that rise by seven powers of two over the row and values of 2^118 or 2^-124: a value times the row's length at most is what the sums have to hold, and nothing more."""
+    def keys(i, n, q):   # (the scores of a group's first query; the others lean on its direction more or less)
+        u = q.view(Hkv, Hq // Hkv, D)[:, 0]
+        return (u / u.square().sum(-1, keepdim=True))[:, None] * (torch.arange(n)[None, :, None] / n * 5) * D ** 0.5
+
+    g = torch.Generator().manual_seed(D)
+    values = lambda i, n: (1 + torch.rand(Hkv, n, D, generator=g)) * 2.0 ** power
+    check_shown(Hq, Hkv, D, torch.bfloat16, SHOWN[5:], keys, values, gain=2.0 ** -power, batch=how == "batch", paged=how != "alone")

@@ -199,3 +199,25 @@ def test_a_prompt_that_fails_leaves_the_sequence_where_it_was(n, paged):
     finally:
         _ffi.set_knob("prefill_chunk", None)
     assert all(torch.equal(a, b) for a, b in zip(*got))
+
+
+@pytest.mark.parametrize("power", [120, -124])
+@pytest.mark.parametrize("heads", [(2, 2), (8, 2)], ids=str)
+@pytest.mark.parametrize("D", [64, 128])
+def test_values_near_the_limits_of_bf16(D, heads, power):
+    """Scores that rise by seven powers of two over a row's keys and values of 2^120 or 2^-124: up to 60 times a value is what the sums have to hold.  Weights in two halves of bf16 (2^-17), scores
+    good to 2^-20 of 8, one rounding to bf16."""
+    Hq, Hkv = heads
+    g = torch.Generator().manual_seed(D)
+    n, rows = 300, 90
+    u = torch.randn(D, generator=g)
+    q = u.expand(1, Hq, rows, D).to(torch.bfloat16)
+    k = (u / u.square().sum() * (torch.arange(n)[:, None] / n * 5) * D ** 0.5).expand(1, Hkv, n, D).to(torch.bfloat16)
+    v = ((1 + torch.rand(1, Hkv, n, D, generator=g)) * 2.0 ** power).to(torch.bfloat16)
+    got = ops.scaled_dot_product_attention(q.cuda(), k.cuda(), v.cuda(), D ** -0.5, mask="causal").double().cpu()
+    r = Hq // Hkv
+    s = q.double() @ k.double().repeat_interleave(r, 1).transpose(-1, -2).contiguous() * D ** -0.5
+    s = s.masked_fill(torch.arange(n)[None] > torch.arange(rows)[:, None] + n - rows, -torch.inf)
+    want = torch.softmax(s, -1) @ v.double().repeat_interleave(r, 1)
+    assert torch.isfinite(got).all()
+    assert ((got - want).abs() <= want * (2.0 ** -8 + 2.0 ** -15)).all(), float(((got - want).abs() / want).max())
