@@ -440,7 +440,7 @@ struct AttnRopeArgs : AttnArgs {
     size_t MN;
     const float *rope_cs;   // [rows][D / 2] (cos, sin)
     u16 *pages;             // = slab
-    int *arrived;           // [rows, Hkv], 0 between launches: splits that left their sums (k_attn_step: the last one merges them); nullptr: a combine launch does
+    int *arrived;           // [rows, Hkv], 0 between launches: splits that left their sums (k_attn_step: the last one merges them); rows in one piece need none
 };
 // Merge of the active splits for 8 consecutive dims [d0, d0+8) of q-head h (fp32):
 // out[d] = sum_j w_j acc_j[d] / sum_j w_j l_j,  w_j = exp(m_j - max m).  Split in a load half and a math half so a

@@ -717,8 +717,8 @@ static int linear_rows(pie_decoder *d, const void *packed, int N, int K, const u
     if (pie_knob(PIE_KNOB_W4L_SLABS) == 0) slabs = nullptr;  // always reduce in the GEMM's own launch (the bit-equality test)
     // 8B prompt of 64 / 128 / 256 / 512 / 700 tokens, slabs summed by the consumers vs reduce launches: 3.70 / 4.56 / 6.13 / 9.56 / 14.26 ms
     // vs 3.96 / 4.82 / 6.20 / 9.75 / 14.38.  (With ONE workgroup per row the RoPE consumer could not keep enough slab loads in flight
-    // below ~200 rows -- 4.21 ms at 64 tokens -- so few rows get four workgroups each there; that split applies to the RoPE consumer, not to the
-    // add + RMSNorm consumers, whose row-wide reduction keeps them at one workgroup per row.)
+    // below ~200 rows -- 4.21 ms at 64 tokens -- so few rows get several there, one per 2048 columns (rope_append_rows); the add + RMSNorm
+    // consumers, whose reduction is the row's, have one and ask for more slabs at a time.)
     const bool is_int4 = d->mat_fmt(packed) == PIE_W_INT4_G64, qmv = (pass_rows ? pass_rows : M) <= GEMV_ROWS_MAX;
     if ((d->mat_fmt(packed) == PIE_W_INT4_G32 || d->mat_fmt(packed) == PIE_W_INT8_G32 || d->mat_fmt(packed) == PIE_W_INT2_G64 || d->mat_fmt(packed) == PIE_W_INT6_G64) && qmv && K <= 32768 && N % 2 == 0) {  // group-32 / two-bit codes, qmv regime: the streaming GEMV, one pass per row
         GemvArgs a = {};

@@ -803,7 +803,7 @@ struct GemvRowsArgs {
     LogitStat *stats;    // EPI_LOGITS [M, n_waves]
     // EPI_ROPE_KV: every row is its own sequence (pie_decoder_step_batch): position ctx_len[m] - 1 (< 0: idle slot), K / V rows to page
     // block_table[m * bt_stride + pos / 64] of this layer's slab (K block then V block, each [n_kv_heads, 64, head_dim])
-    const float *rope_cs;  // [M, head_dim / 2, 2] (cos, sin) of every row's position (k_rope_cs_rows)
+    const float *rope_cs;  // [M, head_dim / 2, 2] (cos, sin) of every row's position (k_pass_rows)
     const int *ctx_len, *block_table;
     u16 *slab, *q_out;     // q_out [M, n_heads, head_dim]
     int bt_stride, n_pages, n_heads, n_kv_heads, head_dim, rope_traditional;

@@ -93,7 +93,7 @@ __device__ __forceinline__ uint4 w4m_dequant_pk(u32 word, w4m_f32x2 s2, w4m_f32x
 // Sum of the 8 waves' partial tiles (fixed order), rounded once, stored for the live rows.
 // Arguments of the q|k|v epilogue (rope = 2): RoPE on the q and k pairs and the cache append, exactly k_rope_append_rows (prefill.hip).
 struct W4mRope {
-    const float *rope_cs;               // [M, HD / 2, 2] (cos, sin) of every row's position (k_rope_cs_rows)
+    const float *rope_cs;               // [M, HD / 2, 2] (cos, sin) of every row's position (k_pass_rows)
     const DecState *state;              // single sequence: row m sits at state->pos + m, cache capacity state->cap ...
     const int *ctx_len;                 // ... or a batch of sequences: row m at ctx_len[m] - 1 (< 0: idle slot)
     const unsigned long long *kv_table; // per-layer K / V buffer (or slab) bases ...

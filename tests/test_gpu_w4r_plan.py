@@ -21,3 +21,10 @@ def test_against_the_dequantised_weights(M, N, K, dtype):
     got = ops.quantized_matmul_rows(x, ops.repack_w4s(codes, scales, biases))
     bound = want.abs() * 2.0 ** (-8 if dtype == torch.bfloat16 else -11) + K * 2.0 ** -24 * (x.double().abs() @ w.abs().t())
     assert bool(((got.double() - want).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("N,K", [(96, 1024), (320, 5120), (224, 2880), (1024, 7168), (4096, 14336), (6176, 4096)])
+@pytest.mark.parametrize("M", [65, 100, 128, 160, 192, 256])
+def test_many_rows_against_the_dequantised_weights(M, N, K):
+    """Row blocks of three to eight, rings of four, three and two steps: one split (23 steps are a prime number) and up to sixteen, whole rounds of the ring and not."""
+    test_against_the_dequantised_weights(M, N, K, torch.bfloat16)
