@@ -440,6 +440,7 @@ struct AttnRopeArgs : AttnArgs {
     size_t MN;
     const float *rope_cs;   // [rows][D / 2] (cos, sin)
     u16 *pages;             // = slab
+    const int *total;       // sum of the rows' ctx_len (those above 0): k_pass_rows leaves it
     int *arrived;           // [rows, Hkv], 0 between launches: splits that left their sums (k_attn_step: the last one merges them); rows in one piece need none
 };
 // Merge of the active splits for 8 consecutive dims [d0, d0+8) of q-head h (fp32):

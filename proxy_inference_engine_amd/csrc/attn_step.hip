@@ -73,13 +73,9 @@ __device__ __forceinline__ float2 agent_load(const float *p) {
 }
 
 // How a row's positions are cut: into pieces of about what a CU gets of the batch's, one at least and most at most, that begin at multiples of 16.  The lengths are on the device, and
-// so is the choice: rows of like lengths are one piece each where there are CUs for no more, a long row among short ones is spread.
-__device__ __forceinline__ AttnSplit step_split(int T, const int *ctx_len, int rows, int Hkv, int most) {
-    int sum = 0;
-    for (int r = threadIdx.x & 63; r < rows; r += 64) sum += max(ctx_len[r], 0);
-#pragma unroll
-    for (int i = 1; i < 64; i <<= 1) sum += __shfl_xor(sum, i);
-    const int per_cu = (int)(((long long)sum * Hkv) >> 8), share = max(__builtin_amdgcn_readfirstlane(per_cu), STEP_WAVES * 16);  // (256 CUs)
+// so is the choice: rows of like lengths are one piece each where there are CUs for no more, a long row among short ones is spread.  (The lengths are summed once a step.)
+__device__ __forceinline__ AttnSplit step_split(int T, int total, int Hkv, int most) {
+    const int per_cu = (int)(((long long)total * Hkv) >> 8), share = max(per_cu, STEP_WAVES * 16);  // (256 CUs)
     const int n = max(1, min(most, (T + (share >> 1)) / share));
     AttnSplit s;
     s.chunk = max(((T + n - 1) / n + 15) & ~15, 16);
@@ -101,7 +97,7 @@ __global__ void __launch_bounds__(STEP_WAVES * 64, REP <= 4 ? 3 : 2) k_attn_step
     const int g = blockIdx.x, split = blockIdx.z, row = (blockIdx.y + split) % gridDim.y, q0 = g * REP;
     const int Ttot = STEP ? a.ctx_len[row] : a.state ? a.state->pos + 1 : a.T;
     AttnSplit sp;
-    if constexpr (STEP) sp = step_split(Ttot, a.ctx_len, a.rows, a.Hkv, a.splits);
+    if constexpr (STEP) sp = step_split(Ttot, *a.total, a.Hkv, a.splits);
     else {
         sp = attn_split(Ttot, a.splits);
         sp.chunk = (sp.chunk + 15) & ~15, sp.active = (Ttot + sp.chunk - 1) / sp.chunk;
@@ -356,7 +352,7 @@ int step_go(int rep, const AttnRopeArgs &a, hipStream_t st) {
 int attn_rope_decode_launch(int dtype, int D, const AttnRopeArgs &a, hipStream_t st) {
     PIE_REQUIRE(a.Hkv > 0 && a.Hq % a.Hkv == 0, PIE_E_SHAPE, "sdpa_decode: Hq must be a multiple of Hkv");
     PIE_REQUIRE(a.splits >= 1 && a.splits <= ATTN_MAX_SPLITS, PIE_E_ARG, "sdpa_decode: bad split count");
-    PIE_REQUIRE(a.splits == 1 || a.arrived, PIE_E_ARG, "sdpa_decode: a split step needs its counters");
+    PIE_REQUIRE(a.total && (a.splits == 1 || a.arrived), PIE_E_ARG, "sdpa_decode: a step needs the sum of its lengths, a split one its counters");
     const int rep = a.Hq / a.Hkv;
 #define STEP_D(T_, D_) return a.nt_kv ? step_go<T_, D_, true, true, true>(rep, a, st) : step_go<T_, D_, false, true, true>(rep, a, st)
     if (dtype == PIE_BF16 && D == 128) STEP_D(BF16, 128);

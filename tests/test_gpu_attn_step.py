@@ -228,3 +228,10 @@ def test_values_near_the_limits_of_bf16(how, Hq, Hkv, D, power):
     g = torch.Generator().manual_seed(D)
     values = lambda i, n: (1 + torch.rand(Hkv, n, D, generator=g)) * 2.0 ** power
     check_shown(Hq, Hkv, D, torch.bfloat16, SHOWN[5:], keys, values, gain=2.0 ** -power, batch=how == "batch", paged=how != "alone")
+
+
+def test_a_batch_of_many_rows_against_float64():
+    """More rows than one workgroup's threads sum at a time, idle of pieces beside one row that is in several."""
+    g = torch.Generator().manual_seed(7)
+    draw = lambda i, n, *_: torch.randn(1, n, 64, generator=g)
+    check_shown(2, 1, 64, torch.bfloat16, [5 + i % 40 for i in range(700)] + [1000], draw, draw)
