@@ -620,7 +620,7 @@ static int rope_append_rows(const pie_decoder *d, const W4lSlabs &sl, int M, int
 // Byte budget for resident T copies of layer matrices, fixed at the first batched prefill: half of the free device memory
 // (PIE_KNOB_PREFILL_RESIDENT: 0 disables, <GiB> sets it).  Matrices are admitted in first-use order while the budget lasts
 // (8B model: all 15 GB; 70B: ~7/8 of its 140 GB); the rest keep going through the scratch every chunk.
-static size_t resident_budget(pie_decoder *d) {
+static size_t resident_budget(const pie_decoder *d) {
     PrefillScratch *s = d->prefill;
     if (s->resident_mode < 0) {
         size_t free_b = 0, total_b = 0;
@@ -696,6 +696,11 @@ bool w4r_serves(int M, int N, int K);
 int w4r_splits(int M, int N, int K);
 size_t w4r_workspace_bytes(int M, int N, int K);
 bool w4m_wide_scales(const void *w4m);
+bool w4a_serves(int M, int N, int K);
+int w4a_splits(int M, int N, int K);
+size_t w4a_workspace_bytes(int M, int N, int K);
+int w4a_gemm_launch(int dtype, const void *w4m, const void *x, int M, int N, int K, void *y, void *workspace, hipStream_t st, int epi, const void *bias,
+                    const W4mRope *rope, int *slabs, bool *bias_done);
 int w4r_gemm_launch(int dtype, const void *w4m, const void *x, int M, int N, int K, void *y, void *workspace, hipStream_t st, int epi, const void *bias,
                     const W4mRope *rope, int *slabs, bool *bias_done, bool wide_scales);
 
@@ -739,10 +744,6 @@ static int linear_rows(pie_decoder *d, const void *packed, int N, int K, const u
         a.fmt = d->mat_fmt(packed) == PIE_W_INT2_G64 ? FMT_W2S : d->mat_fmt(packed) == PIE_W_INT6_G64 ? FMT_W6S : d->mat_fmt(packed) == PIE_W_INT8_G32 ? FMT_W8S32 : FMT_W4S32, a.w = (const char *)packed, a.K = K, a.N = N, a.x = x, a.y = y, a.lin_bias = (const u16 *)bias;
         return w4s_gemv_launch(d->cfg.dtype, PRO_NONE, EPI_STORE, a, M, st);
     }
-    // Below 6 rows MLX multiplies row by row (qmv: exact fp32 per row, mx.quantized_matmul as reached from nn.QuantizedLinear): the
-    // streaming GEMV with the rows' images side by side -- one pass over the weights, each row with the batch-1 arithmetic.
-    if (is_int4 && qmv && K % 64 == 0 && N % 2 == 0 && gemv_rows_lds_bytes(K, 1) <= 160u * 1024u)
-        return w4s_gemv_rows_launch(d->cfg.dtype, packed, N, K, x, M, y, (const u16 *)bias, st);
     // resident W4M tile copy of an int4 matrix (0.5625 B per weight, built on first use within the residency budget); nullptr: no room
     auto w4m_tiles = [&](void **out) -> int {
         *out = nullptr;
@@ -769,35 +770,52 @@ static int linear_rows(pie_decoder *d, const void *packed, int N, int K, const u
         }
         return PIE_OK;
     };
-    // 6 .. 256 rows (a chat turn behind a cached prefix, a prompt chunk, a multi-sequence step): the weight-streaming MFMA GEMM, every CU
-    // streaming its slab of W4M tiles once (w4r_gemm.hpp).  q|k|v, o_proj and down split K over workgroups and hand fp32 slabs to their
-    // consumers (RoPE + append, add + RMSNorm); gate|up carries the SwiGLU in its epilogue.
+    // A product of W4M tiles: affine: k_w4a_gemm, else k_w4r_gemm.  q|k|v, o_proj and down split K over workgroups and hand fp32 slabs to their consumers (RoPE + append, add + RMSNorm); gate|up
+    // carries the SwiGLU in its epilogue.
+    auto tiles_gemm = [&](void *wm, bool affine) -> int {
+        const bool wide = !affine && w4m_wide_scales(wm);
+        auto go = [&](void *to, void *ws, int epi, const void *b, const W4mRope *r, int *n_slabs, bool *done) {
+            return affine ? w4a_gemm_launch(d->cfg.dtype, wm, x, M, N, K, to, ws, st, epi, b, r, n_slabs, done) : w4r_gemm_launch(d->cfg.dtype, wm, x, M, N, K, to, ws, st, epi, b, r, n_slabs, done, wide);
+        };
+        if (act && used_act) {  // gate|up: SwiGLU (and the Linear's bias) in the epilogue
+            *used_act = true;
+            return go(act, nullptr, 1, bias, nullptr, nullptr, nullptr);
+        }
+        if (rope && used_act && (affine ? w4a_splits(M, N, K) : w4r_splits(M, N, K)) == 1) {  // q|k|v wide enough to fill the chip without a K split: RoPE + append in the epilogue
+            *used_act = true;
+            rope->bias = (const u16 *)bias;
+            return go(nullptr, nullptr, 2, nullptr, rope, nullptr, nullptr);
+        }
+        int rc = w4l_reserve(affine ? slabs ? w4a_workspace_bytes(M, N, K) : 0 : w4r_workspace_bytes(M, N, K));
+        if (rc) return rc;
+        int n_slabs = 0;
+        bool bias_done = false;
+        rc = go(y, s->w4l_ws, 0, bias, nullptr, slabs ? &n_slabs : nullptr, &bias_done);
+        if (!rc && n_slabs > 1) {  // y was NOT written: the consumer sums the slabs, rounds and adds the bias
+            slabs->part = (const float *)s->w4l_ws, slabs->S = n_slabs, slabs->MN = (size_t)M * N;
+            return PIE_OK;
+        }
+        if (rc || !bias || bias_done) return rc;
+        return bias_rows<T>(y, bias, M, N, st);
+    };
+    // Up to 16 rows (8 of a narrow matrix): the scales on the sums.  Passes of one and two rows stay with the GEMV below (batch_fused).
+    if (is_int4 && w4a_serves(M, N, K) && (pass_rows ? pass_rows : M) > GEMV_FUSED_ROWS) {
+        void *wm = nullptr;
+        const int rc = w4m_tiles(&wm);
+        if (rc) return rc;
+        if (wm && !w4m_wide_scales(wm)) return tiles_gemm(wm, true);
+    }
+    // Below 6 rows MLX multiplies row by row (qmv: exact fp32 per row, mx.quantized_matmul as reached from nn.QuantizedLinear): the
+    // streaming GEMV with the rows' images side by side -- one pass over the weights, each row with the batch-1 arithmetic.
+    if (is_int4 && qmv && K % 64 == 0 && N % 2 == 0 && gemv_rows_lds_bytes(K, 1) <= 160u * 1024u)
+        return w4s_gemv_rows_launch(d->cfg.dtype, packed, N, K, x, M, y, (const u16 *)bias, st);
+    // Up to 256 rows (a chat turn behind a cached prefix, a prompt chunk, a multi-sequence step): the weight-streaming MFMA GEMM, every CU
+    // streaming its slab of W4M tiles once (w4r_gemm.hpp).
     if (is_int4 && w4r_serves(M, N, K)) {
         void *wm = nullptr;
-        int rc = w4m_tiles(&wm);
+        const int rc = w4m_tiles(&wm);
         if (rc) return rc;
-        if (wm) {
-            const bool wide = w4m_wide_scales(wm);
-            if (act && used_act) {  // gate|up: SwiGLU (and the Linear's bias) in the epilogue
-                *used_act = true;
-                return w4r_gemm_launch(d->cfg.dtype, wm, x, M, N, K, act, nullptr, st, 1, bias, nullptr, nullptr, nullptr, wide);
-            }
-            if (rope && used_act && w4r_splits(M, N, K) == 1) {  // q|k|v wide enough to fill the chip without a K split: RoPE + append in the epilogue
-                *used_act = true;
-                rope->bias = (const u16 *)bias;
-                return w4r_gemm_launch(d->cfg.dtype, wm, x, M, N, K, nullptr, nullptr, st, 2, nullptr, rope, nullptr, nullptr, wide);
-            }
-            if ((rc = w4l_reserve(w4r_workspace_bytes(M, N, K)))) return rc;
-            int n_slabs = 0;
-            bool bias_done = false;
-            rc = w4r_gemm_launch(d->cfg.dtype, wm, x, M, N, K, y, s->w4l_ws, st, 0, bias, nullptr, slabs ? &n_slabs : nullptr, &bias_done, wide);
-            if (!rc && n_slabs > 1) {  // y was NOT written: the consumer sums the slabs, rounds and adds the bias
-                slabs->part = (const float *)s->w4l_ws, slabs->S = n_slabs, slabs->MN = (size_t)M * N;
-                return PIE_OK;
-            }
-            if (rc || !bias || bias_done) return rc;
-            return bias_rows<T>(y, bias, M, N, st);
-        }
+        if (wm) return tiles_gemm(wm, false);
     }
     // Up to 32 rows of a shape k_w4r_gemm does not take (K < 256) -- or all of them with knob PIE_KNOB_W4R = 0, the tests' comparator: round 2's
     // first few-row kernel, one workgroup per 32-column strip
@@ -1034,15 +1052,33 @@ static int batch_attn_splits(const pie_decoder *d, int B, int max_blocks, bool s
     return splits;
 }
 
-// Up to 5 sequences on an int4 checkpoint: the batch-1 launch sequence, once, with every GEMV multiplying all rows per weight
+// Whether every matrix of an int4 step has its W4M tiles, or room for them, and k_w4a_gemm takes it.
+static bool step_tiles(const pie_decoder *d, int B) {
+    const pie_decoder_config &c = d->cfg;
+    const int QD = c.n_heads * c.head_dim, NQKV = QD + 2 * c.n_kv_heads * c.head_dim;
+    size_t more = 0;
+    auto has = [&](const void *packed, int N, int K) {
+        if (!w4a_serves(B, N, K)) return false;
+        const auto it = d->prefill->resident_w4m.find(packed);
+        if (it != d->prefill->resident_w4m.end()) return !w4m_wide_scales(it->second);
+        more += w4m_bytes(N, K);
+        return true;
+    };
+    for (const pie_layer_weights &w : d->layers)
+        if (!has(w.wqkv, NQKV, c.hidden) || !has(w.wo, c.hidden, QD) || !has(w.wgateup, 2 * c.inter, c.hidden) || !has(w.wdown, c.hidden, c.inter)) return false;
+    return has(d->glob.lm_head, c.vocab, c.hidden) && more <= resident_budget(d);
+}
+
+// Up to 2 sequences on an int4 checkpoint (5 without W4M tiles): the batch-1 launch sequence, once, with every GEMV multiplying all rows per weight
 // unit (k_w4s_gemv_rows: RMSNorm prologues; RoPE + page append, residual, SwiGLU and logits epilogues, per row) -- 6 launches per
-// layer instead of 9-10, each row in MLX's row-by-row fp32 regime.  Biases, int8 pages and hidden sizes beyond 8192 take the
-// general path.
+// layer instead of 7, each row in MLX's row-by-row fp32 regime.  Biases, int8 pages and hidden sizes beyond 8192 take the
+// general path, and from 3 rows on every step whose matrices k_w4a_gemm takes: the GEMV's work grows with its rows (Llama-3-8B, four layers, 16 steps at 200 positions, 2 / 3 / 4 / 5 rows
+// 3823 / 4515 / 5283 / 6332 us; the general path, 3 / 4 / 5 / 6 / 8 rows 4156 / 4363 / 4415 / 4465 / 4570).
 static bool batch_fused(const pie_decoder *d, int B) {
     if (B > GEMV_ROWS_MAX || !d->uniform_int4() || d->kv_i8 || d->cfg.hidden > 8192 || w4s_gemv_waves(d->cfg.vocab, d->cfg.hidden) > TAIL_MAX_STATS) return false;
     for (const pie_layer_weights &w : d->layers)
         if (w.bqkv || w.bo || w.bgateup || w.bdown) return false;
-    return true;
+    return B <= GEMV_FUSED_ROWS || !step_tiles(d, B);
 }
 static int batch_rows(pie_decoder *d, const int32_t *tokens, const int32_t *ctx_len, int B, hipStream_t st) {
     const bool fused = batch_fused(d, B);
@@ -1063,6 +1099,7 @@ static int decode_batch_t(pie_decoder *d, const int32_t *tokens, const int32_t *
     if (w16m_size(NQKV, H) / 2 > w_elems) w_elems = w16m_size(NQKV, H) / 2;
     if (w16m_size(H, I) / 2 > w_elems) w_elems = w16m_size(H, I) / 2;
     if (w16m_size(c.vocab, H) / 2 > w_elems) w_elems = w16m_size(c.vocab, H) / 2;
+    if (!d->prefill) d->prefill = new PrefillScratch();
     // (the layers' products say whether they rotated and appended themselves, and with it which kernel attends)
     const bool fused_rows = batch_fused(d, B);
     const int splits = batch_attn_splits(d, B, max_blocks, false), step_splits = fused_rows ? splits : batch_attn_splits(d, B, max_blocks, true);

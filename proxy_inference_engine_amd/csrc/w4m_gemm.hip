@@ -708,6 +708,7 @@ int w4l_gemm_launch(int dtype, const void *w4m, const void *x, int M, int N, int
 
 // ---------------------------------------------------------------- 6 .. 256 rows: the weight-streaming form (w4r_gemm.hpp)
 #include "w4r_gemm.hpp"
+#include "w4a_gemm.hpp"
 
 // Decomposition: 4 strips (128 columns) per workgroup, 2 where that leaves at most 128 column workgroups of up to 64 rows or the splits are the better for it, all rows; K split over blockIdx.y into runs of whole steps where the column
 // workgroups alone cannot fill the chip (q|k|v: 48, o_proj / down: 32 on the 8B model) -- the splits' fp32 slabs are summed by the consumer.
@@ -783,6 +784,64 @@ static void w4r_go(const W4rPlan &pl, int N, hipStream_t st, const W4rArgs &a, c
     case 6: hipLaunchKernelGGL((k_w4r_gemm<T, 8, 6, 1, 2, 3, PLAIN>), grid, block, 0, st, a, r); break;
     default: hipLaunchKernelGGL((k_w4r_gemm<T, 8, 8, 1, 2, 2, PLAIN>), grid, block, 0, st, a, r); break;
     }
+}
+
+size_t w4m_bytes(int N, int K);
+// Up to 16 rows with the scales on the sums (k_w4a_gemm).  Workgroups: of as many half strips as give every CU one (at most eight); what stays below 1024 half strips takes four and splits of
+// K, in one round of workgroups and of at least two steps: q|k|v two splits, o_proj and down four (8 rows, four half strips in two / four / seven splits, two in two: q|k|v 6.8 / 7.6 / - / 7.3 us,
+// o_proj - / 5.2 / - / 5.2, down - / 11.4 / 11.2 / 12.2, [3072, 8192] - / 6.6 / - / 7.6).  Beyond eight rows only what needs no splits: there k_w4r_gemm is as good or better at the others.
+struct W4aPlan {
+    int halves, S, groups;  // half strips per workgroup; K splits, groups of each; halves == 0: shape not served
+};
+static W4aPlan w4a_plan(int M, int N, int K, bool may_split) {
+    if (M < 1 || M > W4A_ROWS || N < 32 || N % 32 || K < 64 || K % 64 || w4m_bytes(N, K) >= (1ull << 31)) return {0, 0, 0};
+    const int units = N / 16, groups = K / 64, steps = (groups + 7) / 8;
+    if (M > 8 && units < 1024) return {0, 0, 0};
+    const int halves = units >= 2048 ? 8 : (units + 255) / 256;
+    if (units >= 1024 || !may_split) return {halves, 1, 8 * steps};
+    const int wgs = (units + 3) / 4;
+    int S = 1;
+    for (int n = 2; n <= 8 && n * wgs <= 256; ++n)
+        if (steps % n == 0 && steps / n >= 2) S = n;
+    if (S == 1) return {halves, 1, 8 * steps};
+    return {4, S, 8 * (steps / S)};
+}
+bool w4a_serves(int M, int N, int K) { return pie_knob(PIE_KNOB_W4R) != 0 && w4a_plan(M, N, K, false).halves != 0; }
+int w4a_splits(int M, int N, int K) { return w4a_plan(M, N, K, true).S; }
+size_t w4a_workspace_bytes(int M, int N, int K) {
+    const int s = w4a_splits(M, N, K);
+    return s > 1 ? (size_t)s * M * N * sizeof(float) : 0;
+}
+template <class T, int MT>
+static void w4a_go(const W4aArgs &a, int S, hipStream_t st, const W4mRope &r) {
+    const dim3 grid((unsigned)((a.N / 16 + a.halves - 1) / a.halves), (unsigned)S), block(512);
+    switch ((a.halves + 1) / 2) {  // (rings of two steps and more: 8 KB and more of weights per wave)
+    case 1: hipLaunchKernelGGL((k_w4a_gemm<T, MT, 1, 5>), grid, block, 0, st, a, r); break;
+    case 2: hipLaunchKernelGGL((k_w4a_gemm<T, MT, 2, 4>), grid, block, 0, st, a, r); break;
+    case 3: hipLaunchKernelGGL((k_w4a_gemm<T, MT, 3, 3>), grid, block, 0, st, a, r); break;
+    default: hipLaunchKernelGGL((k_w4a_gemm<T, MT, 4, 2>), grid, block, 0, st, a, r); break;
+    }
+}
+// epi, rope, slabs, bias_done: as for w4r_gemm_launch; a matrix with wide scales stays there (bias - 128 scale has to be finite)
+int w4a_gemm_launch(int dtype, const void *w4m, const void *x, int M, int N, int K, void *y, void *workspace, hipStream_t st, int epi, const void *bias,
+                    const W4mRope *rope, int *slabs, bool *bias_done) {
+    if (slabs) *slabs = 0;
+    if (bias_done) *bias_done = false;
+    PIE_REQUIRE(dtype == PIE_BF16 || dtype == PIE_F16, PIE_E_ARG, "W4A GEMM: dtype must be PIE_BF16 or PIE_F16");
+    PIE_REQUIRE((epi == W4R_ROPE) == (rope != nullptr), PIE_E_ARG, "W4A GEMM: the q|k|v epilogue needs its arguments");
+    const bool may_split = epi == W4R_STORE && workspace != nullptr && slabs != nullptr;  // (the caller's consumer sums them)
+    const W4aPlan pl = w4a_plan(M, N, K, may_split);
+    PIE_REQUIRE(pl.halves != 0, PIE_E_SHAPE, "W4A GEMM: 1..16 rows, N a multiple of 32, K of 64");
+    PIE_REQUIRE(pie_aligned(w4m, 16) && pie_aligned(x, 16) && pie_aligned(y, 16) && pie_aligned(bias, 16), PIE_E_ALIGN, "W4A GEMM: 16-byte alignment required");
+    const W4aArgs a = {(const char *)w4m, (const u16 *)x, M, N, K, pl.halves, pl.groups, (u16 *)y, pl.S > 1 ? (float *)workspace : nullptr, pl.S > 1 ? nullptr : (const u16 *)bias,
+                       pl.S > 1 ? W4R_SLAB : epi};
+    const W4mRope r = rope ? *rope : W4mRope{};
+    if (dtype == PIE_BF16) M <= 8 ? w4a_go<BF16, 8>(a, pl.S, st, r) : w4a_go<BF16, 16>(a, pl.S, st, r);
+    else M <= 8 ? w4a_go<F16, 8>(a, pl.S, st, r) : w4a_go<F16, 16>(a, pl.S, st, r);
+    PIE_LAUNCH_CHECK();
+    if (pl.S > 1) *slabs = pl.S;
+    else if (bias_done) *bias_done = true;
+    return PIE_OK;
 }
 
 // epi: W4R_STORE (y [M, N], + bias), W4R_SWIGLU (y = activation [M, N / 2], + bias), W4R_ROPE (rope != nullptr; q -> rope->q_out, k / v -> cache).
