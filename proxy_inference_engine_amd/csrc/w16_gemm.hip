@@ -73,9 +73,12 @@ int w16m_from_w16s_launch(const void *w16s, int N, int K, void *w16m, hipStream_
 // and no less than its weights take from beyond the caches, which the row tiles of a column share; workgroups run in rounds of 256, counted on the XCD that has most; all weights come
 // once through HBM (5.6 TB/s); a launch costs 5.8 us of ramp, prologue and epilogue; a K split writes and re-reads its fp32 slabs and launches the reduce.  Over those products its choices
 // take 1.4 % longer than the best ones (those of the model before: 6.2 %); over 563 products of 40 matrices, most of them others, 1.9 % (6.4 %).  Up to K = 2048 the reduce's launch has little to hide behind:
+// The fused activation takes the same tiles (while it was built for two strips per wave alone, us: 64 / 128 / 256 / 320 rows of [28672, 4096] 68 / 67 / 76 / 102, now 48 / 55 / 70 / 99; of
+// [11264, 2048] 29 / 29 / 28 / 29, now 20 / 20 / 24 / 28; of the tower's [6840, 1280] 21 / 20 / 20 / 20, now 11 / 13 / 13 / 16).
 // [1024, 1024], 450 rows: 6.5 us, in two splits 8.8; [1280, 1280], 320 rows: 7.7, 9.5.  [4096, 14336]: 64 / 128 / 509 / 1024 rows 40 / 40 / 91 / 123 -> 34 / 34 / 67 / 113 us.
 struct W16Plan {
     int mb, sw, S;
+    double us = 0.0;  // what the model says
 };
 static int g_w16_plan_override[3] = {0, 0, 0};  // developer override (tools/w16_bench)
 static int g_w16_block[2] = {4, 8};              // XCD-local traversal block (row tiles x column tiles)
@@ -90,8 +93,8 @@ static int w16_even_splits(int groups, int S) {  // the largest split count <= S
     }
 }
 static bool w16_narrow(int tn, int tm) { return tn < 8 && tm >= 8; }  // column tiles that would leave XCDs without work: row tiles go over the XCDs instead
-// no_split: one pass over K; two: two strips per wave
-static W16Plan w16_plan(int M, int N, int K, bool no_split = false, bool two = false) {
+// no_split: one pass over K
+static W16Plan w16_plan(int M, int N, int K, bool no_split = false) {
     const int groups = (K + 63) / 64;
     if (g_w16_plan_override[0]) return {g_w16_plan_override[0], g_w16_plan_override[1], no_split ? 1 : w16_even_splits(groups, g_w16_plan_override[2])};
     const int mb_max = M <= 64 ? 2 : (M <= 128 ? 4 : 8);
@@ -103,7 +106,7 @@ static W16Plan w16_plan(int M, int N, int K, bool no_split = false, bool two = f
     const double stream_us = 2.0 * N * (64.0 * groups) / 5.6e6;
     for (int S = 1; S <= (no_split ? 1 : 16) && (S == 1 || 8 * S <= groups); ++S)
         for (int mb = mb_max; mb >= 2; mb >>= 1)
-            for (int sw = 2; sw >= (two ? 2 : 1); --sw) {
+            for (int sw = 2; sw >= 1; --sw) {
                 const int tn = (N + 128 * sw - 1) / (128 * sw), tm = (M + 32 * mb - 1) / (32 * mb), wgs = tn * tm * S;
                 const int most = (w16_narrow(tn, tm) ? (tm + 7) / 8 * tn : (tn + 7) / 8 * tm) * S;  // workgroups of the XCD that has most: 32 run at once
                 const int steps = ((groups + S - 1) / S + 3) & ~3;
@@ -114,10 +117,14 @@ static W16Plan w16_plan(int M, int N, int K, bool no_split = false, bool two = f
                 double us = (most + 31) / 32 * steps * (t > cold ? t : cold);
                 us = (us > stream_us ? us : stream_us) + 5.8;
                 if (S > 1) us += (double)M * N * 4.0 * (2 * S + 0.5) / 5.1e6 + (groups <= 32 ? 3.5 : 1.0);
-                if (us < best_us) best_us = us, best = {mb, sw, S};
+                if (us < best_us) best_us = us, best = {mb, sw, S, us};
             }
     best.S = w16_even_splits(groups, best.S);
     return best;
+}
+void w16l_tile(int M, int N, int K, int *mb, int *sw) {  // of one pass over K (the forms with an activation: w16_grouped.hip)
+    const W16Plan pl = w16_plan(M, N, K, true);
+    *mb = pl.mb, *sw = pl.sw;
 }
 int w16l_splits(int M, int N, int K) { return w16_plan(M, N, K).S; }
 size_t w16l_workspace_bytes(int M, int N, int K) {
@@ -144,12 +151,14 @@ static int w16l_gemm_launch_z(int dtype, const void *w16m, const void *x, int ld
     PIE_REQUIRE(pie_aligned(w16m, 16) && pie_aligned(x, 16) && pie_aligned(y, 8) && (!bias || pie_aligned(bias, (N & 3) ? 2 : 8)), PIE_E_ALIGN, "16-bit GEMM: 16-byte alignment required");
     PIE_REQUIRE(dtype == PIE_BF16 || dtype == PIE_F16, PIE_E_ARG, "16-bit GEMM: dtype must be PIE_BF16 or PIE_F16");
     // One pass over K where the slabs do not fit the output: rows that are not a multiple of 16 bytes, a row stride of the caller's; and where swiglu_act comes without `fused`: the caller
-    // has no fallback (the C ABI's fused MLP).  The fused activation is built for two strips per wave: the best tile among those.
+    // has no fallback (the C ABI's fused MLP).  A split product's activation is a launch of its own behind the reduce's: about 6 us.
     const bool one_pass = (swiglu_act && !fused) || (N & 3) || (!swiglu_act && ldy && ldy != N);
     W16Plan plan = w16_plan(M, N, K, one_pass);
-    if (swiglu_act && plan.S == 1) plan = w16_plan(M, N, K, true, true);
+    if (swiglu_act && plan.S > 1) {
+        const W16Plan whole = w16_plan(M, N, K, true);
+        if (whole.us < plan.us + 6.0) plan = whole;
+    }
     const bool sg = swiglu_act && plan.S == 1;
-    if (sg) plan.sw = 2;  // (a developer's override)
     PIE_REQUIRE(plan.S == 1 || workspace, PIE_E_ARG, "16-bit GEMM: this shape splits K and needs its workspace");
     W16Args a = {};
     int rc = w16_zero_block(&a.zero);
@@ -172,7 +181,8 @@ static int w16l_gemm_launch_z(int dtype, const void *w16m, const void *x, int ld
     const dim3 grid((unsigned)(a.narrow ? 8 * ((a.tm + 7) / 8) * a.tn : 8 * ((a.tn + 7) / 8) * a.tm), (unsigned)plan.S);
 #define W16_GO(TT, MB_, SW_, SG_) hipLaunchKernelGGL((k_w16l_gemm<TT, MB_, SW_, SG_>), grid, dim3(256), 0, st, a)
 #define W16_SW(TT, MB_) \
-    if (sg) W16_GO(TT, MB_, 2, true); \
+    if (sg && plan.sw == 1) W16_GO(TT, MB_, 1, true); \
+    else if (sg) W16_GO(TT, MB_, 2, true); \
     else if (plan.sw == 2) W16_GO(TT, MB_, 2, false); \
     else W16_GO(TT, MB_, 1, false)
 #define W16_MB(TT) \

@@ -7,6 +7,7 @@ typedef __attribute__((address_space(3))) void w4l_lds_void;
 #include "w16_gemm.hpp"
 
 int w16_zero_block(const char **out);  // w16_gemm.hip
+void w16l_tile(int M, int N, int K, int *mb, int *sw);
 
 static int w16_fill(W16Args &a, const void *w16m, const void *x, int ldx, int N, int K, void *y, int ldy) {
     const int Kx = 64 * ((K + 63) / 64);
@@ -26,19 +27,24 @@ int w16l_act_launch(const void *w16m, const void *x, int ldx, int M, int N, int 
     PIE_REQUIRE(act == MFMA_ACT_NONE || act == MFMA_ACT_RELU2 || act == MFMA_ACT_XIELU || (act == MFMA_ACT_GELU && N % 8 == 0), PIE_E_ARG, "16-bit GEMM: unknown activation");
     PIE_REQUIRE(!bias || (act == MFMA_ACT_GELU && pie_aligned(bias, 8)), PIE_E_ARG, "16-bit GEMM: a bias goes with the paired gelu");
     a.bias = (const u16 *)bias;
-    int mb = 8;  // the largest row tile that still gives the chip a round of workgroups
-    while (mb > 2 && (M <= 16 * mb || a.tn * ((M + 32 * mb - 1) / (32 * mb)) < 200)) mb >>= 1;
+    int mb, sw;
+    w16l_tile(M, N, K, &mb, &sw);
+    a.tn = (N + 128 * sw - 1) / (128 * sw);
     a.M = M, a.tm = (M + 32 * mb - 1) / (32 * mb), a.bm = a.bm < a.tm ? a.bm : a.tm, a.act_alpha = alpha, a.act_limit = beta;
     a.narrow = a.tn < 8 && a.tm >= 8;
     const dim3 grid((unsigned)(a.narrow ? 8 * ((a.tm + 7) / 8) * a.tn : 8 * ((a.tn + 7) / 8) * a.tm));
-#define ACT_GO(MB_) \
-    if (act == MFMA_ACT_RELU2) hipLaunchKernelGGL((k_w16l_gemm<BF16, MB_, 2, MFMA_ACT_RELU2>), grid, dim3(256), 0, st, a); \
-    else if (act == MFMA_ACT_GELU) hipLaunchKernelGGL((k_w16l_gemm<BF16, MB_, 2, MFMA_ACT_GELU>), grid, dim3(256), 0, st, a); \
-    else if (act == MFMA_ACT_NONE) hipLaunchKernelGGL((k_w16l_gemm<BF16, MB_, 2, MFMA_ACT_NONE>), grid, dim3(256), 0, st, a); \
-    else hipLaunchKernelGGL((k_w16l_gemm<BF16, MB_, 2, MFMA_ACT_XIELU>), grid, dim3(256), 0, st, a)
-    if (mb == 2) { ACT_GO(2); }
-    else if (mb == 4) { ACT_GO(4); }
-    else { ACT_GO(8); }
+#define ACT_GO(MB_, SW_) \
+    if (act == MFMA_ACT_RELU2) hipLaunchKernelGGL((k_w16l_gemm<BF16, MB_, SW_, MFMA_ACT_RELU2>), grid, dim3(256), 0, st, a); \
+    else if (act == MFMA_ACT_GELU) hipLaunchKernelGGL((k_w16l_gemm<BF16, MB_, SW_, MFMA_ACT_GELU>), grid, dim3(256), 0, st, a); \
+    else if (act == MFMA_ACT_NONE) hipLaunchKernelGGL((k_w16l_gemm<BF16, MB_, SW_, MFMA_ACT_NONE>), grid, dim3(256), 0, st, a); \
+    else hipLaunchKernelGGL((k_w16l_gemm<BF16, MB_, SW_, MFMA_ACT_XIELU>), grid, dim3(256), 0, st, a)
+#define ACT_SW(MB_) \
+    if (sw == 1) { ACT_GO(MB_, 1); } \
+    else { ACT_GO(MB_, 2); }
+    if (mb == 2) { ACT_SW(2) }
+    else if (mb == 4) { ACT_SW(4) }
+    else { ACT_SW(8) }
+#undef ACT_SW
 #undef ACT_GO
     PIE_LAUNCH_CHECK();
     return PIE_OK;
