@@ -92,7 +92,7 @@ class BaseCache(ABC):
     def to_quantized(self, group_size: int = 64, bits: int = 4) -> "BaseCache": ...
 
 
-from .reusable import ReusableKVCache  # noqa: E402
+from .reusable import ReusableKVCache, reserve_layers  # noqa: E402
 from .paged import PageAllocator, PagedKVCache, PagedSequence  # noqa: E402
 from .latent import LatentPageAllocator, PagedLatentCache, SavedLatentCache  # noqa: E402
 from .stack import PagedStackCache, SavedStackCache, StackPageAllocator, StackSequence  # noqa: E402

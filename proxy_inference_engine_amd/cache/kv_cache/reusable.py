@@ -102,3 +102,15 @@ class ReusableKVCache(BaseCache):
 
     def to_quantized(self, group_size: int = 64, bits: int = 4) -> BaseCache:
         return self  # the reference returns self too (reusable.py:250-254): KV stays 16-bit on this path
+
+
+def reserve_layers(caches: list[ReusableKVCache], needed: int, n_kv_heads: int, head_dim: int, dtype: torch.dtype, device) -> None:
+    """`reserve` of a model's layers.  The first buffers of all of them are slices of one: a fill each was a launch each, two a layer."""
+    first = caches[0]
+    if all(type(c) is ReusableKVCache and c.keys is None and c.values is None and (c.step, c.max_capacity) == (first.step, first.max_capacity) for c in caches):
+        cap = first._aligned(needed)
+        rows = torch.zeros((2 * len(caches), 1, n_kv_heads, cap, head_dim), dtype=dtype, device=device)
+        for i, c in enumerate(caches):
+            c.keys, c.values, c.offset = rows[2 * i], rows[2 * i + 1], 0
+    for c in caches:
+        c.reserve(needed, n_kv_heads, head_dim, dtype, device)

@@ -19,7 +19,7 @@ import torch
 
 from .. import base
 from ... import _ffi, hip_ops
-from ...cache.kv_cache import BaseCache, PageAllocator, PagedKVCache, PagedSequence, ReusableKVCache
+from ...cache.kv_cache import BaseCache, PageAllocator, PagedKVCache, PagedSequence, ReusableKVCache, reserve_layers
 from .utils import Llama3RoPE
 
 
@@ -392,7 +392,7 @@ class Model:
                 raise TypeError("the decode path runs on ReusableKVCache (prompt_cache.py:73)")
             if c.offset != off:
                 raise ValueError("layer caches disagree on offset")
-            c.reserve(n_new, self.n_kv_heads, self.head_dim, self.dtype, self.device)
+        reserve_layers(cache, n_new, self.n_kv_heads, self.head_dim, self.dtype, self.device)
         cap = min(c.capacity for c in cache)
         key = (tuple(c.keys.data_ptr() for c in cache), tuple(c.values.data_ptr() for c in cache), cap)
         lib = _ffi.load()

@@ -238,3 +238,23 @@ def test_generate_step_mask_arrays_that_the_reference_loop_can_carry():
                      (torch.full((1, 1), float("-inf")), "hides every key")):
         with pytest.raises(ValueError, match=why):
             check_generate_mask(bad, 4)
+
+
+@pytest.mark.parametrize("tokens", [1, 256, 257])
+def test_first_buffers_of_all_layers_are_slices_of_one(tokens):
+    """reserve_layers gives every layer what reserve gives it: zeros of the same capacity, each its own rows; layers that already hold something, and growth, go one by one."""
+    from proxy_inference_engine_amd.cache.kv_cache import reserve_layers
+    caches, want = [ReusableKVCache() for _ in range(3)], ReusableKVCache()
+    reserve_layers(caches, tokens, 2, 8, torch.float32, "cpu")
+    want.reserve(tokens, 2, 8, torch.float32, "cpu")
+    for i, c in enumerate(caches):
+        assert c.keys.shape == c.values.shape == want.keys.shape and c.offset == 0 and c.keys.is_contiguous() and c.values.is_contiguous() and not c.keys.any() and not c.values.any()
+        c.update_and_fetch(torch.full((1, 2, tokens, 8), 2.0 * i + 1), torch.full((1, 2, tokens, 8), 2.0 * i + 2))
+    for i, c in enumerate(caches):
+        assert (c.keys[:, :, :tokens] == 2 * i + 1).all() and (c.values[:, :, :tokens] == 2 * i + 2).all() and not c.keys[:, :, tokens:].any()
+    held = caches[0].keys
+    mixed = [caches[0], ReusableKVCache(max_capacity=300)]
+    reserve_layers(mixed, 1, 2, 8, torch.float32, "cpu")
+    assert mixed[0].keys.shape[2] >= tokens + 1 and (mixed[0].keys is held) == (tokens % 256 != 0) and mixed[1].keys.shape[2] == 256
+    with pytest.raises(RuntimeError):
+        reserve_layers([ReusableKVCache(max_capacity=300) for _ in range(2)], 301, 2, 8, torch.float32, "cpu")
