@@ -95,14 +95,18 @@ __device__ __forceinline__ int pa_off(int row, int ch) {
 // unit of work, at the same number of waves per CU (one 8-wave workgroup instead of two 4-wave ones for REP = 4).
 // SPLIT: blockIdx.y takes its share of the tile's key blocks and leaves its sums to k_prefill_combine (prefill_attn_splits says when).
 // SHORT: blocks of 32 keys, for prompts that fill few of 64 (prefill_attn_short).
-template <class T, int D, int REP, int QT, bool SEG = false, bool SPLIT = false, bool SHORT = false>
-__global__ void __launch_bounds__(REP * QT * 64, 2) k_prefill_attn(const PrefillAttnArgs a) {
-    constexpr int NT = REP * QT * 64, NB = NT >= 256 && !SHORT ? 2 : 1, BK = 32 * NB;  // keys per block: 64 where enough threads share their loads
+// KG = 2: two waves per head and tile, which take a staged block's first and second 64 keys and meet in LDS at the end: half the serial blocks, and a wave's softmax beside the other's
+// products (prefill_attn_pairs says when).
+template <class T, int D, int REP, int QT, bool SEG = false, bool SPLIT = false, bool SHORT = false, int KG = 1>
+__global__ void __launch_bounds__(REP * QT * KG * 64, 2) k_prefill_attn(const PrefillAttnArgs a) {
+    static_assert(KG == 1 || (KG == 2 && QT == 1 && !SEG && !SHORT), "two waves per tile: causal, one tile");
+    constexpr int NT = REP * QT * KG * 64, NB = (NT >= 256 && !SHORT) || KG == 2 ? 2 : 1, BK = 32 * NB * KG;  // keys per block: 64 (a wave's) where enough threads share their loads
     constexpr int CH = D / 8, KS = D / 16, DT = D / 32;                      // chunks per row, k-steps of Q.K^T, 32-dim output tiles
     constexpr int BM = 32 * QT;
     constexpr int CPT = (BK * CH + NT - 1) / NT;                                   // 16-byte chunks per thread and tile
     __shared__ __attribute__((aligned(16))) char kv_lds[2][2][BK * 2 * D];         // [block parity][K, V]
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63, wave_id = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wave = KG == 2 ? wave_id % REP : wave_id, kg = KG == 2 ? wave_id / REP : 0;  // (kg: which half of a block's keys)
     const int c = lane & 31, h = lane >> 5;
     // XCD-aware tile mapping: workgroups go round-robin over the 8 XCDs by linear id, so the kv-head group is the FASTEST
     // index (id % Hkv): with 8 kv-heads every XCD's L2 only ever holds one group's K/V (4 MB at 4096 tokens) instead of all
@@ -110,7 +114,7 @@ __global__ void __launch_bounds__(REP * QT * 64, 2) k_prefill_attn(const Prefill
     const int g = (int)blockIdx.x % a.Hkv, tile = (int)blockIdx.x / a.Hkv;
     const int wg_r0 = ((a.M + BM - 1) / BM - 1 - tile) * BM;                  // first query row of the workgroup
     const int r0 = wg_r0 + 32 * (wave / REP), hq = g * REP + wave % REP;     // this wave's 32-row tile and q-head
-    // paged KV: a key block (BK = 32 or 64 rows) never straddles a 64-row page, so its page is one scalar table lookup per fetch;
+    // paged KV: a key block (BK = 32 or 64 rows) never straddles a 64-row page, so its page is one scalar table lookup per fetch (KG = 2: two);
     // the contiguous case is the same code with one "page" of `cap` rows (mask keeps every row bit, page offset 0)
     const bool paged = a.block_table != nullptr;
     const int pos0 = a.state ? a.state->pos : a.offset, cap = paged ? 64 : a.state ? a.state->cap : a.cap;
@@ -125,7 +129,7 @@ __global__ void __launch_bounds__(REP * QT * 64, 2) k_prefill_attn(const Prefill
     const int n_blocks = SPLIT ? min(b_first + share, n_all) : n_all;
     if constexpr (SPLIT)
         if (b_first >= n_blocks) {  // fewer blocks than workgroups: an empty share weighs nothing
-            if (h == 0 && r0 + c < a.M) {
+            if (h == 0 && kg == 0 && r0 + c < a.M) {
                 float *ml = a.part + (size_t)a.M * a.Hq * a.splits * D + (((size_t)(r0 + c) * a.Hq + hq) * a.splits + blockIdx.y) * 2;
                 ml[0] = ATTN_NEG, ml[1] = 0.0f;
             }
@@ -144,8 +148,9 @@ __global__ void __launch_bounds__(REP * QT * 64, 2) k_prefill_attn(const Prefill
         x = x < BK * CH ? x : BK * CH - 1;                                                       \
         int t = b * BK + x / CH;                                                                 \
         t = t < t_last ? t : t_last;                                                             \
-        kr = *reinterpret_cast<const uint4 *>(kbase + pg_off + (size_t)(t & row_mask) * D + (x % CH) * 8); \
-        vr = *reinterpret_cast<const uint4 *>(vbase + pg_off + (size_t)(t & row_mask) * D + (x % CH) * 8); \
+        const size_t po = KG == 2 && x >= 64 * CH ? pg_off1 : pg_off;                            \
+        kr = *reinterpret_cast<const uint4 *>(kbase + po + (size_t)(t & row_mask) * D + (x % CH) * 8); \
+        vr = *reinterpret_cast<const uint4 *>(vbase + po + (size_t)(t & row_mask) * D + (x % CH) * 8); \
     }
 #define PA_PUBLISH1(i, kr, vr)                                                                 \
     if constexpr (i < CPT) {                                                                     \
@@ -155,8 +160,9 @@ __global__ void __launch_bounds__(REP * QT * 64, 2) k_prefill_attn(const Prefill
             *reinterpret_cast<uint4 *>(kv_lds[buf][1] + pa_off<D>(x / CH, x % CH)) = vr;                  \
         }                                                                                        \
     }
+    auto page_at = [&](int t) { return paged ? (size_t)min((unsigned)a.block_table[t >> 6], (unsigned)a.n_pages - 1u) * page_elems : (size_t)0; };
     auto fetch = [&](int b) {
-        const size_t pg_off = paged ? (size_t)min((unsigned)a.block_table[(b * BK) >> 6], (unsigned)a.n_pages - 1u) * page_elems : 0;
+        const size_t pg_off = page_at(b * BK), pg_off1 = KG == 2 ? page_at(min(b * BK + 64, t_last)) : 0;
         PA_FETCH1(0, k0, v0) PA_FETCH1(1, k1, v1) PA_FETCH1(2, k2, v2) PA_FETCH1(3, k3, v3)
         PA_FETCH1(4, k4, v4) PA_FETCH1(5, k5, v5) PA_FETCH1(6, k6, v6) PA_FETCH1(7, k7, v7)
     };
@@ -200,8 +206,10 @@ __global__ void __launch_bounds__(REP * QT * 64, 2) k_prefill_attn(const Prefill
     __syncthreads();
     for (int b = b_first; b < n_blocks; ++b) {
         const int buf = (b - b_first) & 1;
-        const char *k_lds = kv_lds[buf][0], *v_lds = kv_lds[buf][1];
+        const char *k_lds = kv_lds[buf][0] + kg * (64 * 2 * D), *v_lds = kv_lds[buf][1] + kg * (64 * 2 * D);
         if (b + 1 < n_blocks) fetch(b + 1);
+        const int t0 = b * BK + (KG == 2 ? 64 * kg : 0);
+        if (KG == 1 || t0 <= t_last) {
 
         // S^T = K . Q^T : rows = keys (registers), cols = query rows (lanes); the blocks of 32 keys are independent chains
         f32x16_t sc[NB];
@@ -217,8 +225,7 @@ __global__ void __launch_bounds__(REP * QT * 64, 2) k_prefill_attn(const Prefill
                 sc[n] = MfmaT<T>::run(kf, qf[s], sc[n]);
             }
         // online softmax over keys: register i of block n <-> key t0 + 32 n + (i & 3) + 8 (i >> 2) + 4 h
-        const int t0 = b * BK;
-        const bool masked = t0 + BK - 1 > all_hi || (SEG && t0 < all_lo);  // uniform for the wave
+        const bool masked = t0 + 32 * NB - 1 > all_hi || (SEG && t0 < all_lo);  // uniform for the wave
         auto sees = [&](int n, int i) {
             const int t = t0 + 32 * n + (i & 3) + 8 * (i >> 2) + 4 * h;
             return t <= t_row && (!SEG || t >= t_lo);
@@ -292,10 +299,32 @@ __global__ void __launch_bounds__(REP * QT * 64, 2) k_prefill_attn(const Prefill
 #pragma unroll
             for (int dt = 0; dt < DT; ++dt) oacc[dt] = MfmaT<T>::run(vf[dt], bl, oacc[dt]);
         }
+        }
         if (b + 1 < n_blocks) {  // (the other image: its last readers passed the barrier in front of this block)
             publish(buf ^ 1);
             __syncthreads();
         }
+    }
+    if constexpr (KG == 2) {  // the second wave's sums join the first's: 16 floats of a lane at a time, lanes side by side
+        static_assert(REP * 64 * (DT * 16 + 2) * 4 <= (int)sizeof(kv_lds), "the sums fit the images");
+        float *meet = reinterpret_cast<float *>(kv_lds) + wave * (64 * (DT * 16 + 2)) + lane;
+        __syncthreads();
+        if (kg == 1) {
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) meet[(16 * dt + i) * 64] = oacc[dt][i];
+            meet[DT * 16 * 64] = m_run, meet[(DT * 16 + 1) * 64] = l_run;
+        }
+        __syncthreads();
+        if (kg == 1) return;
+        const float m1 = meet[DT * 16 * 64], m_new = fmaxf(m_run, m1), w0 = attn_exp2(m_run - m_new), w1 = attn_exp2(m1 - m_new);
+        l_run = l_run * w0 + meet[(DT * 16 + 1) * 64] * w1;
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) oacc[dt][i] = oacc[dt][i] * w0 + meet[(16 * dt + i) * 64] * w1;
+        m_run = m_new;
     }
     if constexpr (SPLIT) {
         const float l = xor32_sum(l_run);
@@ -349,9 +378,11 @@ __global__ void __launch_bounds__(256) k_prefill_combine(const float *part, int 
 // Workgroups along the keys: rows behind a long cached prefix are few tiles with many blocks each (37 rows: 16 workgroups of 30 blocks).  `before`: keys in front of the first row.  Every
 // share costs its sums (4 D bytes per row and head, twice): at least two blocks of 64 keys per share up to 64 rows, three beyond, up to two workgroups per CU.  us, 1 / 2 / 4 / 8 shares:
 // 8 rows behind 500: 20 / 14 / 12 / 12; 37 behind 900: 35 / 24 / 18 / 17; 100: 38 / 26 / 21 / 23; 200: 41 / 30 / 26 / 30; 509: 53 / 42 / 40 / 46; 32 behind 4000: 131 / 73 / 42 / 29 (16: 28).
-// Rows of a fresh prompt see half of the blocks on average and gain nothing (509 rows: 22 / 26).
-static inline int prefill_attn_splits(int M, int before, int Hkv) {
-    const int shares = before / 64 / (M <= 64 ? 2 : 3), room = 512 / ((M + 31) / 32 * Hkv);
+// Rows of a fresh prompt see half of the blocks on average and gain nothing (509 rows: 22 / 26).  With two waves per tile (prefill_attn_pairs, whose images fill a CU) one workgroup per CU:
+// 509 behind 900 in four shares of one wave / two of two 39 / 36, 1000 behind 900 in two of one / one of two 65 / 53.
+static inline bool prefill_attn_duo(int rep) { return rep >= 2 && rep <= 4; }  // (four waves of 64 keys, 240 registers each, leave room for four more)
+static inline int prefill_attn_splits(int M, int before, int Hq, int Hkv) {
+    const int shares = before / 64 / (M <= 64 ? 2 : 3), room = (M > 256 && prefill_attn_duo(Hq / Hkv) ? 256 : 512) / ((M + 31) / 32 * Hkv);
     const int s = shares < room ? shares : room;
     return s < 2 ? 1 : s > 16 ? 16 : s;
 }
@@ -362,12 +393,21 @@ static inline size_t prefill_attn_part_bytes(int Hq, int Hkv, int D) { return (s
 // 48 rows 7.6 / 8.4, 64 rows 8.8 / 8.4; 32 / 4 heads: 8 rows 6.4 / 7.6, 33 rows 9.6 / 10.6, 64 rows 10.7 / 10.5.
 static inline bool prefill_attn_short(const PrefillAttnArgs &a) { return a.M + a.before <= 56; }
 
+// Two waves per tile (KG) pay from about five blocks of 64 keys on, where they save blocks that wait for each other; below, and in shares of a few blocks, their meeting costs more.  us, one wave /
+// two, 32 / 8 heads: 128 rows 9.1 / 9.8, 300 15.4 / 15.1, 509 21.9 / 19.0, 1000 39.5 / 32.3, 1900 76.9 / 66.7; 24 / 8: 509 24.9 / 19.3, 1000 49.5 / 33.4, 1900 92.9 / 62.6; 32 / 16: 300 15.3 / 13.0;
+// 37 behind 900 in seven shares 17.2 / 17.9.  Against two tiles per workgroup (two waves per SIMD either way, K and V staged once for both): 2000 rows 89.5 / 71.3, 2300 103 / 94, 3000 139 / 148.
+static inline bool prefill_attn_pairs(const PrefillAttnArgs &a) { return prefill_attn_duo(a.Hq / a.Hkv) && a.M + a.before >= 256 && (a.splits <= 1 || a.M > 256); }
+
 template <class T, int D>
 static int prefill_attn_launch_d(const PrefillAttnArgs &a, hipStream_t st) {
     const int rep = a.Hq / a.Hkv;
+    const bool pairs = prefill_attn_pairs(a);
     if (a.splits > 1) {
         const dim3 grid((a.M + 31) / 32 * a.Hkv, a.splits);
-#define PA_SPLIT(R) hipLaunchKernelGGL((k_prefill_attn<T, D, R, 1, false, true>), grid, dim3(R * 64), 0, st, a); break
+#define PA_SPLIT(R)                                                                                                                                      \
+    if (pairs && R >= 2 && R <= 4) hipLaunchKernelGGL((k_prefill_attn<T, D, R, 1, false, true, false, (R >= 2 && R <= 4 ? 2 : 1)>), grid, dim3(R * 128), 0, st, a); \
+    else hipLaunchKernelGGL((k_prefill_attn<T, D, R, 1, false, true>), grid, dim3(R * 64), 0, st, a);                                                    \
+    break
         switch (rep) {
             case 1: PA_SPLIT(1);
             case 2: PA_SPLIT(2);
@@ -381,18 +421,19 @@ static int prefill_attn_launch_d(const PrefillAttnArgs &a, hipStream_t st) {
         }
 #undef PA_SPLIT
         PIE_LAUNCH_CHECK();
-        const int pairs = a.M * a.Hq;
-        hipLaunchKernelGGL((k_prefill_combine<T, D>), dim3((unsigned)(((size_t)pairs * (D / 4) + 255) / 256)), dim3(256), 0, st, a.part, a.splits, pairs, a.out);
+        const int rows = a.M * a.Hq;
+        hipLaunchKernelGGL((k_prefill_combine<T, D>), dim3((unsigned)(((size_t)rows * (D / 4) + 255) / 256)), dim3(256), 0, st, a.part, a.splits, rows, a.out);
         PIE_LAUNCH_CHECK();
         return PIE_OK;
     }
     const int qt = pie_knob(PIE_KNOB_PREFILL_QT);  // test knob: 1 forces one 32-row query tile per workgroup, 2 forces two wherever they fit
     // 2 tiles need 2*rep <= 8 waves of up to 256 registers, and only pay while the halved grid still fills the 256 CUs
     // (8B model: 4096 tokens 54.9 -> 53.9 ms, 8000 tokens 126.3 -> 125.0 ms; at 1024 tokens it would idle half the chip)
-    const bool two = rep <= 4 && a.M > 32 && (qt > 0 ? qt == 2 : ((a.M + 63) / 64) * a.Hkv >= 256), few = prefill_attn_short(a);
+    const bool two = rep <= 4 && a.M > 32 && (qt > 0 ? qt == 2 : ((a.M + 63) / 64) * a.Hkv >= (prefill_attn_duo(rep) ? 320 : 256)), few = prefill_attn_short(a);
     const dim3 grid(((a.M + (two ? 63 : 31)) / (two ? 64 : 32)) * a.Hkv);
 #define PA_LAUNCH(R)                                                                                         \
     if (two && R <= 4) hipLaunchKernelGGL((k_prefill_attn<T, D, R, (R <= 4 ? 2 : 1)>), grid, dim3(R * 128), 0, st, a); \
+    else if (pairs && !few && R >= 2 && R <= 4) hipLaunchKernelGGL((k_prefill_attn<T, D, R, 1, false, false, false, (R >= 2 && R <= 4 ? 2 : 1)>), grid, dim3(R * 128), 0, st, a); \
     else if (few && R >= 4) hipLaunchKernelGGL((k_prefill_attn<T, D, R, 1, false, false, (R >= 4)>), grid, dim3(R * 64), 0, st, a); \
     else hipLaunchKernelGGL((k_prefill_attn<T, D, R, 1>), grid, dim3(R * 64), 0, st, a);                     \
     break

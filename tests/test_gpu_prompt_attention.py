@@ -44,8 +44,28 @@ def test_short_prompts_against_float64(heads, D):
         assert (got - want).abs().max() <= EPS[torch.bfloat16] * want.abs().max(), (L, off)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("heads", [(2, 1), (3, 1), (8, 2)], ids=str)
+@pytest.mark.parametrize("D", [64, 128])
+def test_two_waves_per_tile_against_float64(heads, D, dtype):
+    """From 256 keys on, two to four heads a group: block pairs whose second half is empty, masked in part or whole, rows of one and of several tiles; bound as above.  The second half's
+    values are much larger in one key each, so that a half that is lost or counted twice shows."""
+    Hq, Hkv = heads
+    g = torch.Generator().manual_seed(D + Hq)
+    for L, off, scale in ((256, 0, 0.3), (257, 0, 0.3), (320, 0, -0.3), (321, 63, 0.3), (7, 249, 0.3), (40, 280, 0.2), (33, 400, 0.0), (450, 1, 0.2)):
+        T = off + L
+        q, k, v = (torch.randn(1, n, m, D, generator=g).to(dtype) for n, m in ((Hq, L), (Hkv, T), (Hkv, T)))
+        v[:, :, 64::128] *= 8
+        got = ops.scaled_dot_product_attention(q.cuda(), k.cuda(), v.cuda(), scale, mask="causal").double().cpu()
+        r = Hq // Hkv
+        s = q.double() @ k.double().repeat_interleave(r, 1).transpose(-1, -2).contiguous() * scale
+        s = s.masked_fill(torch.arange(T)[None] > torch.arange(L)[:, None] + off, -torch.inf)
+        want = torch.softmax(s, -1) @ v.double().repeat_interleave(r, 1)
+        assert (got - want).abs().max() <= EPS[dtype] * want.abs().max(), (L, off, scale)
+
+
 @pytest.mark.parametrize("paged", [False, True], ids=["contiguous", "paged"])
-@pytest.mark.parametrize("geometry", [(8, 2, 64), (8, 1, 128), (2, 2, 128)], ids=str)
+@pytest.mark.parametrize("geometry", [(8, 2, 64), (8, 1, 128), (2, 2, 128), (6, 2, 128)], ids=str)
 def test_rows_behind_a_prefix_split_along_the_keys(geometry, paged):
     """700 cached tokens: 2 to 5 shares, the last ones empty or partly masked.  Two layers against the kernel that takes one query row at a time: both keep fp32 until one rounding, so four ulps of the
     largest logit as everywhere in this suite."""
