@@ -44,6 +44,7 @@ EXPORTS = BASE_EXPORTS + [
     "pie_paged_attn_workspace_bytes", "pie_paged_attn_decode", "pie_paged_kv_append",
     "pie_page_i8_set_scales", "pie_paged_kv_append_i8", "pie_paged_attn_decode_i8",
     "pie_gelu", "pie_vision_qkv_rope", "pie_sdpa_segments", "pie_bias_silu_mul", "pie_add_bias", "pie_add_bias_rms_norm",
+    "pie_vision_blocks", "pie_vision_blocks_workspace",
     "pie_w4m_bytes", "pie_repack_w4s_to_w4m", "pie_qgemm_w4m",
     "pie_comm_create", "pie_comm_rccl_unique_id", "pie_comm_create_rccl", "pie_comm_export", "pie_comm_connect", "pie_allreduce_f32", "pie_comm_status", "pie_comm_destroy", "pie_decoder_set_comm", "pie_sample", "pie_sample_workspace_bytes",
 ]
@@ -67,6 +68,10 @@ class pie_global_weights(C.Structure):
     _fields_ = [("embed_codes", C.c_void_p), ("embed_scales", C.c_void_p), ("embed_biases", C.c_void_p),
                 ("final_norm", C.c_void_p), ("lm_head", C.c_void_p), ("rope_freqs", C.c_void_p),
                 ("fmt_embed", C.c_int), ("fmt_lm_head", C.c_int)]
+
+
+class pie_vision_block(C.Structure):
+    _fields_ = [(n, C.c_void_p) for n in ("qkv_w", "qkv_b", "proj_w", "proj_b", "norm2", "gateup_w", "gateup_b", "down_w", "down_b", "next_norm")] + [("full", C.c_int)]
 
 
 class pie_stack_norm(C.Structure):
@@ -239,6 +244,9 @@ def load() -> C.CDLL:
     lib.pie_bias_silu_mul.argtypes = [C.c_void_p] * 4 + [C.c_int] * 4 + [C.c_void_p] * 2
     lib.pie_add_bias_rms_norm.argtypes = [C.c_void_p] * 4 + [C.c_float] + [C.c_int] * 3 + [C.c_void_p] * 3
     lib.pie_add_bias.argtypes = [C.c_void_p] * 3 + [C.c_int] * 3 + [C.c_void_p] * 2
+    lib.pie_vision_blocks_workspace.restype = C.c_size_t
+    lib.pie_vision_blocks_workspace.argtypes = [C.c_int] * 5
+    lib.pie_vision_blocks.argtypes = [C.POINTER(pie_vision_block)] + [C.c_int] * 6 + [C.c_float] + [C.c_void_p] * 6 + [C.c_int] + [C.c_void_p] * 3 + [C.c_size_t, C.c_void_p]
     lib.pie_sdpa_segments.argtypes = [C.c_void_p] * 5 + [C.c_int] * 3 + [C.c_float, C.c_int, C.c_void_p, C.c_void_p]
     lib.pie_w4m_bytes.restype = C.c_size_t
     lib.pie_repack_w4s_to_w4m.argtypes = [C.c_void_p, C.c_int, C.c_int, C.c_void_p, C.c_void_p]

@@ -44,6 +44,7 @@ struct PrefillAttnArgs {
     // SEG instantiation (vision tower: block-diagonal, non-causal attention -- the mask of models/intern/vision.py:160-167):
     // query row r attends keys [seg_lo[r], seg_hi[r]); both int32 [M], non-decreasing in r.  Op level only (k, v, cap = M).
     const int *seg_lo, *seg_hi;
+    int out_d;                           // SEG: columns of a head's output that are stored (a multiple of 4; 0: D): heads of 80, padded to 128 for the products, side by side again
     const int *block_table;              // paged KV (nullable, decoder only): kv_table holds the layers' slab K / V bases; key t
     int n_pages;                         //   lives in page block_table[t / 64] (each [Hkv, 64, D]) at row t % 64
     int before;                          // keys in front of the first row, as far as the host knows (plans the launch; the device's position decides)
@@ -343,14 +344,15 @@ __global__ void __launch_bounds__(REP * QT * KG * 64, 2) k_prefill_attn(const Pr
     // normalise: the pair (lane, lane ^ 32) shares the query row and holds the two halves of the row sum
     const float inv = 1.0f / xor32_sum(l_run);
     if (r0 + c < a.M) {
-        u16 *orow = a.out + ((size_t)(r0 + c) * a.Hq + hq) * D;
+        const int od = SEG && a.out_d ? a.out_d : D;
+        u16 *orow = a.out + ((size_t)(r0 + c) * a.Hq + hq) * od;
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
             for (int k = 0; k < 4; ++k) {  // registers 4k .. 4k+3 <-> dims 32 dt + 8 k + 4 h + {0..3}
                 const uint2 o = make_uint2(pack2<T>(oacc[dt][4 * k] * inv, oacc[dt][4 * k + 1] * inv),
                                            pack2<T>(oacc[dt][4 * k + 2] * inv, oacc[dt][4 * k + 3] * inv));
-                *reinterpret_cast<uint2 *>(orow + 32 * dt + 8 * k + 4 * h) = o;
+                if (!SEG || 32 * dt + 8 * k + 4 * h < od) *reinterpret_cast<uint2 *>(orow + 32 * dt + 8 * k + 4 * h) = o;
             }
     }
 }

@@ -654,6 +654,42 @@ def sdpa_segments(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, seg_lo: tor
     return out
 
 
+def vision_blocks_served(hidden: int, inter: int, heads: int, head_dim: int) -> bool:
+    """Whether pie_vision_blocks takes a tower of these widths."""
+    return _ffi.load().pie_vision_blocks_workspace(64, hidden, inter, heads, head_dim) > 0
+
+
+def vision_block_table(blocks: list[dict], after: list[torch.Tensor], full: list[int]):
+    """The blocks' weights (qkv_w, qkv_b, ..; packed Linears and tensors, which the caller keeps) for vision_blocks; after[i]: the norm behind block i, full: the blocks over whole images."""
+    def ptr(v):
+        return (v.tiles if isinstance(v, PackedLinear) else v).data_ptr()
+    table = (_ffi.pie_vision_block * len(blocks))()
+    for i, (b, n) in enumerate(zip(blocks, after)):
+        for name in ("qkv_w", "qkv_b", "proj_w", "proj_b", "norm2", "gateup_w", "gateup_b", "down_w", "down_b"):
+            setattr(table[i], name, ptr(b[name]))
+        table[i].next_norm, table[i].full = ptr(n), int(i in full)
+    return table
+
+
+def vision_blocks(table, first: int, count: int, x: torch.Tensor, xn: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, seg_full, seg_win, inter: int, heads: int, head_dim: int,
+                  eps: float) -> None:
+    """Blocks first .. first + count of a vision tower on x [N, hidden] and xn = norm1(x), both updated in place (pie_vision_blocks); seg_full, seg_win: segment_bounds of whole images and windows."""
+    for t in (x, xn, cos, sin, *seg_full, *seg_win):
+        _dev(t)
+    N, hidden = x.shape
+    if first < 0 or count < 1 or first + count > len(table) or xn.shape != x.shape or xn.dtype != x.dtype or not (x.is_contiguous() and xn.is_contiguous()):
+        raise ValueError("vision_blocks: blocks of the table; x, xn [N, hidden], contiguous, of one dtype")
+    if any(t.shape != (N, head_dim // 2) or t.dtype != torch.float32 or not t.is_contiguous() for t in (cos, sin)):
+        raise ValueError("vision_blocks: cos / sin must be float32 [N, head_dim / 2], contiguous")
+    if any(t.shape != (N,) or t.dtype != torch.int32 or not t.is_contiguous() for t in (*seg_full, *seg_win)):
+        raise ValueError("vision_blocks: segment bounds must be int32 [N]")
+    lib = _ffi.load()
+    ws = torch.empty(int(lib.pie_vision_blocks_workspace(N, hidden, inter, heads, head_dim)), dtype=torch.uint8, device=x.device)
+    at = C.cast(C.byref(table, first * C.sizeof(_ffi.pie_vision_block)), C.POINTER(_ffi.pie_vision_block))
+    _ffi.check(lib.pie_vision_blocks(at, count, N, hidden, inter, heads, head_dim, float(eps), _ffi.p(cos), _ffi.p(sin), _ffi.p(seg_full[0]), _ffi.p(seg_full[1]), _ffi.p(seg_win[0]),
+                                     _ffi.p(seg_win[1]), _ffi.dtype_code(x.dtype), _ffi.p(x), _ffi.p(xn), _ffi.p(ws), ws.numel(), _ffi.stream()))
+
+
 def bias_silu_mul(gate: torch.Tensor, up: torch.Tensor, bias_gate: torch.Tensor, bias_up: torch.Tensor) -> torch.Tensor:
     """silu(gate + bias_gate) * (up + bias_up) on [M, N] GEMM outputs (MLP of vision.py:196-197, biases folded in).  gate and up
     may be the two column halves of one [M, 2N] GEMM output (equal row strides, unit column stride)."""

@@ -7,8 +7,8 @@ MFMA units (full-image layers and 64-patch-window layers are the same kernel wit
 pie_silu_mul, pie_add, pie_gelu.  Index bookkeeping (positions, window order, cu_seqlens) is host numpy, as it is host
 Python in the reference; the row permutations are device gathers.
 
-Layout notes: head_dim (80 for the 7B tower) is zero-padded to the attention kernel's 128 inside q / k / v; `proj`'s weight
-is widened to match once at load (zero columns), so no un-padding pass exists.  PatchEmbed's Conv3d (stride = kernel) is a
+Layout notes: head_dim (80 for the 7B tower) is zero-padded to the attention kernel's 128 inside q / k / v; the attention stores
+the heads' own columns side by side.  PatchEmbed's Conv3d (stride = kernel) is a
 GEMM over the flattened patches; its weight is flattened once at load in the pixel rows' (C, T, P, P) order."""
 from __future__ import annotations
 
@@ -71,18 +71,12 @@ class VisionModel:
         # tiled in MFMA operand order once, here (ops.pack_linear); rounds 1-4 called hipBLASLt
         self.patch_w = ops.pack_linear(w.reshape(w.shape[0], -1).to(device=self.device, dtype=dtype).contiguous())   # [hidden, C*T*P*P]
         self.blocks = []
-        H, D, DP = c.num_heads, self.head_dim, self.padded_head_dim
         for i in range(c.depth):
             p = f"blocks.{i}."
-            proj = get(p + "attn.proj.weight")                                  # [hidden, H*D] -> [hidden, H*DP], zero columns
-            if DP != D:
-                wide = torch.zeros((proj.shape[0], H, DP), dtype=dtype, device=self.device)
-                wide[:, :, :D] = proj.view(proj.shape[0], H, D)
-                proj = wide.view(proj.shape[0], H * DP).contiguous()
             self.blocks.append({
                 "norm1": get(p + "norm1.weight"), "norm2": get(p + "norm2.weight"),
                 "qkv_w": ops.pack_linear(get(p + "attn.qkv.weight")), "qkv_b": get(p + "attn.qkv.bias"),
-                "proj_w": ops.pack_linear(proj), "proj_b": get(p + "attn.proj.bias"),
+                "proj_w": ops.pack_linear(get(p + "attn.proj.weight")), "proj_b": get(p + "attn.proj.bias"),
                 # gate_proj and up_proj as ONE GEMM [2 * intermediate, hidden] with rows (gate_i, up_i) interleaved: the biases and
                 # silu(gate) * up ride in its epilogue (vision.py:196-197), the [N, 2 * intermediate] block is never written
                 "gateup_w": ops.pack_linear(ops.interleave_gate_up(get(p + "mlp.gate_proj.weight"), get(p + "mlp.up_proj.weight"))),
@@ -93,6 +87,11 @@ class VisionModel:
         self._graphs: dict = {}
         self.merger = {"ln_q": get("merger.ln_q.weight"), "w0": ops.pack_linear(get("merger.mlp.0.weight")), "b0": get("merger.mlp.0.bias"),
                        "w2": ops.pack_linear(get("merger.mlp.2.weight")), "b2": get("merger.mlp.2.bias")}
+        # widths that pie_vision_blocks takes: the blocks in one native call
+        self._native = None
+        if c.depth and c.hidden_size == c.num_heads * self.head_dim and ops.vision_blocks_served(c.hidden_size, c.intermediate_size, c.num_heads, self.head_dim):
+            after = [b["norm1"] for b in self.blocks[1:]] + [self.merger["ln_q"]]   # the next consumer's norm
+            self._native = ops.vision_block_table(self.blocks, after, c.fullatt_block_indexes)
 
     # ------------------------------------------------------------------ vision.py:245-279
     def rot_pos_emb(self, grid_thw) -> np.ndarray:
@@ -170,13 +169,21 @@ class VisionModel:
         scale = self.head_dim ** -0.5
         fuse_norm = c.hidden_size % 8 == 0 and c.hidden_size <= 8192
         xn = ops.rms_norm(x, self.blocks[0]["norm1"], 1e-6) if self.blocks else None
-        for i, b in enumerate(self.blocks):
+        if self._native is not None:
+            at = range(0, c.depth, 1 if output_hidden_states else c.depth)   # (one call, or one for each state that is handed out)
+            for i in at:
+                if states:
+                    x = x.clone()
+                ops.vision_blocks(self._native, i, at.step, x, xn, cos, sin, t["seg_full"], t["seg_win"], c.intermediate_size, c.num_heads, self.head_dim, 1e-6)
+                if output_hidden_states:
+                    states = (*states, x)
+        for i, b in enumerate(self.blocks if self._native is None else ()):
             lo, hi = t["seg_full"] if i in c.fullatt_block_indexes else t["seg_win"]
             # hidden_states + attn(norm1(hidden_states))  (vision.py:212-217); xn = norm1(x) comes from the previous fused pass
             qkv = ops.linear_rows(xn, b["qkv_w"])                                           # bias folded into the rotary kernel
             q, k, v = ops.vision_qkv_rope(qkv, cos, sin, c.num_heads, self.padded_head_dim, bias=b["qkv_b"])
             att = ops.sdpa_segments(q, k, v, lo, hi, scale)
-            r = ops.linear_rows(att.view(seq_len, -1), b["proj_w"])
+            r = ops.linear_rows(att[..., :self.head_dim].reshape(seq_len, -1), b["proj_w"])
             if fuse_norm:
                 x, xn = ops.add_bias_rms_norm(x, r, b["proj_b"], b["norm2"], 1e-6)
             else:
