@@ -445,7 +445,8 @@ struct PrefillScratch {
     // that is a small share of the free memory (PIE_KNOB_PREFILL_RESIDENT overrides), built on first use.
     std::map<const void *, u16 *> resident;
     // W4M tile copies (w4m_gemm.hip) of int4 layer matrices for prompts of at most small_rows() rows: 0.5625 B per weight each
-    std::map<const void *, void *> resident_w4m;
+    struct Tiles { void *p; size_t bytes; };
+    std::map<const void *, Tiles> resident_w4m;
     LogitStat *tail_stats = nullptr;  // fused few-sequence step: the lm_head GEMV's tail partials, one per wave and row; other rows' tiles (RowStat) where the tail takes two launches
     size_t tail_entries = 0;           // its capacity in entries
     // Captured multi-sequence step (pie_decoder_step_batch with PIE_STEP_GRAPH): valid while the caller's buffers (key) and every
@@ -498,7 +499,7 @@ void prefill_free(pie_decoder *d) {
     if (!d->prefill) return;
     scratch_release(d->prefill);
     for (auto &kv : d->prefill->resident) (void)hipFree(kv.second);
-    for (auto &kv : d->prefill->resident_w4m) (void)hipFree(kv.second);
+    for (auto &kv : d->prefill->resident_w4m) (void)hipFree(kv.second.p);
     if (d->prefill->tail_stats) (void)hipFree(d->prefill->tail_stats);
     if (d->prefill->w4l_ws) (void)hipFree(d->prefill->w4l_ws);
     if (d->prefill->attn_part) (void)hipFree(d->prefill->attn_part);
@@ -518,7 +519,7 @@ void prefill_globals_changed(pie_decoder *d, const void *new_head) {
     for (const void *head : {(const void *)d->glob.lm_head, new_head}) {
         const int N = d->cfg.vocab, K = d->cfg.hidden;
         if (auto it = s->resident.find(head); it != s->resident.end()) (void)hipFree(it->second), s->resident.erase(it), s->resident_left += w16m_size(N, K);
-        if (auto it = s->resident_w4m.find(head); it != s->resident_w4m.end()) (void)hipFree(it->second), s->resident_w4m.erase(it), s->resident_left += w4m_bytes(N, K);
+        if (auto it = s->resident_w4m.find(head); it != s->resident_w4m.end()) (void)hipFree(it->second.p), s->resident_left += it->second.bytes, s->resident_w4m.erase(it);
     }
 }
 
@@ -696,11 +697,13 @@ bool w4r_serves(int M, int N, int K);
 int w4r_splits(int M, int N, int K);
 size_t w4r_workspace_bytes(int M, int N, int K);
 bool w4m_wide_scales(const void *w4m);
-bool w4a_serves(int M, int N, int K);
-int w4a_splits(int M, int N, int K);
-size_t w4a_workspace_bytes(int M, int N, int K);
+bool w4a_serves(int M, int N, int K, int bits = 4);
+int w4a_splits(int M, int N, int K, int bits);
+size_t w4a_workspace_bytes(int M, int N, int K, int bits);
+size_t w8m_bytes(int N, int K);
+int w8m_repack_launch(const void *w8s, int N, int K, void *w8m, hipStream_t st);
 int w4a_gemm_launch(int dtype, const void *w4m, const void *x, int M, int N, int K, void *y, void *workspace, hipStream_t st, int epi, const void *bias,
-                    const W4mRope *rope, int *slabs, bool *bias_done);
+                    const W4mRope *rope, int *slabs, bool *bias_done, int bits);
 int w4r_gemm_launch(int dtype, const void *w4m, const void *x, int M, int N, int K, void *y, void *workspace, hipStream_t st, int epi, const void *bias,
                     const W4mRope *rope, int *slabs, bool *bias_done, bool wide_scales);
 
@@ -744,19 +747,21 @@ static int linear_rows(pie_decoder *d, const void *packed, int N, int K, const u
         a.fmt = d->mat_fmt(packed) == PIE_W_INT2_G64 ? FMT_W2S : d->mat_fmt(packed) == PIE_W_INT6_G64 ? FMT_W6S : d->mat_fmt(packed) == PIE_W_INT8_G32 ? FMT_W8S32 : FMT_W4S32, a.w = (const char *)packed, a.K = K, a.N = N, a.x = x, a.y = y, a.lin_bias = (const u16 *)bias;
         return w4s_gemv_launch(d->cfg.dtype, PRO_NONE, EPI_STORE, a, M, st);
     }
-    // resident W4M tile copy of an int4 matrix (0.5625 B per weight, built on first use within the residency budget); nullptr: no room
+    // resident W4M (W8M) tile copy of an int4 (int8) matrix (0.5625 B, 1.0625 B per weight, built on first use within the residency budget); nullptr: no room
+    const bool is_int8 = d->mat_fmt(packed) == PIE_W_INT8_G64;
+    const size_t tile_bytes = is_int8 ? w8m_bytes(N, K) : w4m_bytes(N, K);
     auto w4m_tiles = [&](void **out) -> int {
         *out = nullptr;
         auto it = s->resident_w4m.find(packed);
         if (it != s->resident_w4m.end()) {
-            *out = it->second;
+            *out = it->second.p;
             return PIE_OK;
         }
         void *wm = nullptr;
-        if (resident_budget(d) >= w4m_bytes(N, K) && hipMalloc(&wm, w4m_bytes(N, K)) == hipSuccess) {
-            s->resident_w4m[packed] = wm, s->resident_left -= w4m_bytes(N, K), ++s->alloc_gen;
+        if (resident_budget(d) >= tile_bytes && hipMalloc(&wm, tile_bytes) == hipSuccess) {
+            s->resident_w4m[packed] = {wm, tile_bytes}, s->resident_left -= tile_bytes, ++s->alloc_gen;
             *out = wm;
-            return w4m_repack_launch(packed, N, K, wm, st);
+            return is_int8 ? w8m_repack_launch(packed, N, K, wm, st) : w4m_repack_launch(packed, N, K, wm, st);
         }
         (void)hipGetLastError();
         return PIE_OK;
@@ -773,20 +778,21 @@ static int linear_rows(pie_decoder *d, const void *packed, int N, int K, const u
     // A product of W4M tiles: affine: k_w4a_gemm, else k_w4r_gemm.  q|k|v, o_proj and down split K over workgroups and hand fp32 slabs to their consumers (RoPE + append, add + RMSNorm); gate|up
     // carries the SwiGLU in its epilogue.
     auto tiles_gemm = [&](void *wm, bool affine) -> int {
+        const int bits = is_int8 ? 8 : 4;
         const bool wide = !affine && w4m_wide_scales(wm);
         auto go = [&](void *to, void *ws, int epi, const void *b, const W4mRope *r, int *n_slabs, bool *done) {
-            return affine ? w4a_gemm_launch(d->cfg.dtype, wm, x, M, N, K, to, ws, st, epi, b, r, n_slabs, done) : w4r_gemm_launch(d->cfg.dtype, wm, x, M, N, K, to, ws, st, epi, b, r, n_slabs, done, wide);
+            return affine ? w4a_gemm_launch(d->cfg.dtype, wm, x, M, N, K, to, ws, st, epi, b, r, n_slabs, done, bits) : w4r_gemm_launch(d->cfg.dtype, wm, x, M, N, K, to, ws, st, epi, b, r, n_slabs, done, wide);
         };
         if (act && used_act) {  // gate|up: SwiGLU (and the Linear's bias) in the epilogue
             *used_act = true;
             return go(act, nullptr, 1, bias, nullptr, nullptr, nullptr);
         }
-        if (rope && used_act && (affine ? w4a_splits(M, N, K) : w4r_splits(M, N, K)) == 1) {  // q|k|v wide enough to fill the chip without a K split: RoPE + append in the epilogue
+        if (rope && used_act && (affine ? w4a_splits(M, N, K, bits) : w4r_splits(M, N, K)) == 1) {  // q|k|v wide enough to fill the chip without a K split: RoPE + append in the epilogue
             *used_act = true;
             rope->bias = (const u16 *)bias;
             return go(nullptr, nullptr, 2, nullptr, rope, nullptr, nullptr);
         }
-        int rc = w4l_reserve(affine ? slabs ? w4a_workspace_bytes(M, N, K) : 0 : w4r_workspace_bytes(M, N, K));
+        int rc = w4l_reserve(affine ? slabs ? w4a_workspace_bytes(M, N, K, bits) : 0 : w4r_workspace_bytes(M, N, K));
         if (rc) return rc;
         int n_slabs = 0;
         bool bias_done = false;
@@ -804,6 +810,13 @@ static int linear_rows(pie_decoder *d, const void *packed, int N, int K, const u
         const int rc = w4m_tiles(&wm);
         if (rc) return rc;
         if (wm && !w4m_wide_scales(wm)) return tiles_gemm(wm, true);
+    }
+    // Int8 codes, up to 32 rows: the same form (no scale is too large for it: a code has no offset)
+    if (is_int8 && (keep || keep_w4m) && w4a_serves(M, N, K, 8)) {
+        void *wm = nullptr;
+        const int rc = w4m_tiles(&wm);
+        if (rc) return rc;
+        if (wm) return tiles_gemm(wm, true);
     }
     // Below 6 rows MLX multiplies row by row (qmv: exact fp32 per row, mx.quantized_matmul as reached from nn.QuantizedLinear): the
     // streaming GEMV with the rows' images side by side -- one pass over the weights, each row with the batch-1 arithmetic.
@@ -1060,7 +1073,7 @@ static bool step_tiles(const pie_decoder *d, int B) {
     auto has = [&](const void *packed, int N, int K) {
         if (!w4a_serves(B, N, K)) return false;
         const auto it = d->prefill->resident_w4m.find(packed);
-        if (it != d->prefill->resident_w4m.end()) return !w4m_wide_scales(it->second);
+        if (it != d->prefill->resident_w4m.end()) return !w4m_wide_scales(it->second.p);
         more += w4m_bytes(N, K);
         return true;
     };

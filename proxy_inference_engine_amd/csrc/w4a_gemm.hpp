@@ -13,9 +13,10 @@
 // Error (2-norm, before the rounding to T) against 64 bits: 9e-7; of weights rounded to bf16 1.7e-3.
 #pragma once
 
-constexpr int W4A_ROWS = 16;
+constexpr int W4A_ROWS = 16, W8A_ROWS = 32;
+constexpr int W8M_TILE_BYTES = 2176;  // W8M (below)
 struct W4aArgs {
-    const char *w4m;   // W4M tiles of the [N, K] matrix
+    const char *w4m;   // W4M (W8M) tiles of the [N, K] matrix
     const u16 *x;      // [M, K]
     int M, N, K;
     int halves;        // half strips (16 columns) per workgroup
@@ -35,9 +36,24 @@ __device__ __forceinline__ uint4 w4a_codes(u32 w) {
 template <class T>
 constexpr float w4a_offset() { return std::is_same<T, F16>::value ? 0.0f : 128.0f; }
 
-template <class T, int MT, int SPW, int D>
+// Int8 codes, W8M tiles: as W4M, 32 rows x 64 columns, two pieces of 1 KiB and the 32 {scale, bias} words: lane l = 32 kh + n holds in piece h the codes of row n of k-steps 2 h and 2 h + 1, two words
+// each, in the W8S word format (codes 0, 2, 1, 3).  Up to 255 a code is a bf16 and an f16 as it stands.
+// Bound by the stream; before, two and more rows multiplied a 16-bit copy, twice the bytes.  us of 16 steps of four layers at 200 positions, 16-bit copy / this: Llama-3-8B 2 rows 6924 / 5080, 4 7209 / 5288,
+// 8 7440 / 5474, 16 8042 / 6015, 32 9319 / 6719; Llama-3.2-3B 4 rows 5357 / 3881, 8 5142 / 4033.  Error of a step against 64 bits 0.0095-0.0100 / 0.0089-0.0095.
+template <class T>
+__device__ __forceinline__ u32 w8a_pair(u32 a, u32 b) {  // two codes as T, b in the high half
+    if constexpr (std::is_same<T, F16>::value) return __builtin_bit_cast(u32, __builtin_amdgcn_cvt_pkrtz((float)a, (float)b));
+    return __builtin_amdgcn_perm(__builtin_bit_cast(u32, (float)b), __builtin_bit_cast(u32, (float)a), 0x07060302u);
+}
+template <class T>
+__device__ __forceinline__ uint4 w8a_codes(u32 lo, u32 hi) {
+    return make_uint4(w8a_pair<T>(lo & 0xFFu, (lo >> 16) & 0xFFu), w8a_pair<T>((lo >> 8) & 0xFFu, lo >> 24), w8a_pair<T>(hi & 0xFFu, (hi >> 16) & 0xFFu), w8a_pair<T>((hi >> 8) & 0xFFu, hi >> 24));
+}
+
+template <class T, int MT, int SPW, int D, int BITS = 4>
 __global__ void __launch_bounds__(512) k_w4a_gemm(const W4aArgs a, const W4mRope rp) {
-    constexpr int KW = 8, XJ = MT / 8, WL = 2 * SPW, CHUNK = MT * 128;  // K-phases = waves; DMA instructions (eight rows of a group each), weight loads per step; bytes of x of a step
+    constexpr int PC = BITS / 4, TILE = BITS == 8 ? W8M_TILE_BYTES : W4M_TILE_BYTES;  // code pieces (16 bytes a lane) of a tile; bytes of one
+    constexpr int KW = 8, XJ = MT / 8, WL = (PC + 1) * SPW, CHUNK = MT * 128;  // K-phases = waves; DMA instructions (eight rows of a group each), weight loads per step; bytes of x of a step
     constexpr int RL = MT / 2;                                  // accumulators that hold rows < MT
     constexpr int RSTR = 36, BLK = MT * RSTR * 4;               // reduction: one (phase, strip) block, rows of 32 + 4 floats
     constexpr int RED = KW * SPW * BLK, LDS = KW * D * CHUNK > RED ? KW * D * CHUNK : RED;
@@ -50,14 +66,14 @@ __global__ void __launch_bounds__(512) k_w4a_gemm(const W4aArgs a, const W4mRope
     const int g_lo = blockIdx.y * a.groups + p, g_hi = min(all_groups, ((int)blockIdx.y + 1) * a.groups);  // this wave's groups: g_lo, g_lo + 8, ..
     const int steps = g_hi > g_lo ? (g_hi - g_lo + KW - 1) / KW : 0;
     const int h0 = blockIdx.x * a.halves, h1 = min(h0 + a.halves, n_halves), strip0 = h0 >> 1;
-    const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>(a.w4m), 0, (a.N >> 5) * all_groups * W4M_TILE_BYTES, 0x00020000);
+    const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>(a.w4m), 0, (a.N >> 5) * all_groups * TILE, 0x00020000);
     unsigned code_at[SPW], scale_at[SPW], strip_at[SPW];
 #pragma unroll
     for (int s = 0; s < SPW; ++s) {
         const int h = 2 * (strip0 + s) + (n >> 4);
         const bool mine = h >= h0 && h < h1;  // (the strips at both ends may be another workgroup's by half)
-        code_at[s] = mine ? 16u * lane : NOWHERE, scale_at[s] = mine ? 1024u + 4u * n : NOWHERE;
-        strip_at[s] = (unsigned)((strip0 + s) * all_groups + g_lo) * W4M_TILE_BYTES;
+        code_at[s] = mine ? 16u * lane : NOWHERE, scale_at[s] = mine ? 1024u * PC + 4u * n : NOWHERE;
+        strip_at[s] = (unsigned)((strip0 + s) * all_groups + g_lo) * TILE;
     }
     u32 xoffs[XJ];
 #pragma unroll
@@ -67,7 +83,7 @@ __global__ void __launch_bounds__(512) k_w4a_gemm(const W4aArgs a, const W4mRope
     }
     const unsigned lds0 = (unsigned)(size_t)(__attribute__((address_space(3))) void *)smem + (unsigned)(p * D * CHUNK);
     typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
-    uint4 cw[D][SPW];
+    uint4 cw[D][SPW][PC];
     u32 sb[D][SPW];
     auto issue = [&](int d, int j) {
         const char *src = reinterpret_cast<const char *>(a.x) + (size_t)(g_lo + (j < steps ? j : steps - 1) * KW) * 128;
@@ -79,11 +95,14 @@ __global__ void __launch_bounds__(512) k_w4a_gemm(const W4aArgs a, const W4mRope
                          : "v"(xoffs[i]), "s"(src), "s"(lds0 + (unsigned)(d * CHUNK + i * 1024))
                          : "memory");
         }
-        const unsigned o = (unsigned)j * (KW * W4M_TILE_BYTES), dead = j < steps ? 0u : NOWHERE;
+        const unsigned o = (unsigned)j * (KW * TILE), dead = j < steps ? 0u : NOWHERE;
 #pragma unroll
         for (int s = 0; s < SPW; ++s) {
-            const u32x4 c = __builtin_amdgcn_raw_buffer_load_b128(wr, code_at[s] | dead, strip_at[s] + o, 2);
-            cw[d][s] = make_uint4(c.x, c.y, c.z, c.w);
+#pragma unroll
+            for (int q = 0; q < PC; ++q) {
+                const u32x4 c = __builtin_amdgcn_raw_buffer_load_b128(wr, (code_at[s] | dead) + 1024u * q, strip_at[s] + o, 2);
+                cw[d][s][q] = make_uint4(c.x, c.y, c.z, c.w);
+            }
             sb[d][s] = __builtin_amdgcn_raw_buffer_load_b32(wr, scale_at[s] | dead, strip_at[s] + o, 2);
         }
     };
@@ -120,12 +139,19 @@ __global__ void __launch_bounds__(512) k_w4a_gemm(const W4aArgs a, const W4mRope
                     for (int kk = 0; kk < 4; ++kk)
 #pragma unroll
                         for (int s = s0; s < s0 + 2 && s < SPW; ++s) {
-                            const u32 wk = kk == 0 ? cw[d][s].x : (kk == 1 ? cw[d][s].y : (kk == 2 ? cw[d][s].z : cw[d][s].w));
-                            dot[s - s0] = MfmaT<T>::run(xq[kk], w4a_codes<T>(wk), kk ? dot[s - s0] : zero);
+                            uint4 wf;
+                            if constexpr (BITS == 8) {
+                                const uint4 &c = cw[d][s][kk >> 1];
+                                wf = kk & 1 ? w8a_codes<T>(c.z, c.w) : w8a_codes<T>(c.x, c.y);
+                            } else {
+                                const uint4 &c = cw[d][s][0];
+                                wf = w4a_codes<T>(kk == 0 ? c.x : (kk == 1 ? c.y : (kk == 2 ? c.z : c.w)));
+                            }
+                            dot[s - s0] = MfmaT<T>::run(xq[kk], wf, kk ? dot[s - s0] : zero);
                         }
 #pragma unroll
                     for (int s = s0; s < s0 + 2 && s < SPW; ++s) {
-                        const float sc = lo_f32<T>(sb[d][s]), bi = fmaf(-w4a_offset<T>(), sc, hi_f32<T>(sb[d][s]));
+                        const float sc = lo_f32<T>(sb[d][s]), bi = BITS == 8 ? hi_f32<T>(sb[d][s]) : fmaf(-w4a_offset<T>(), sc, hi_f32<T>(sb[d][s]));
 #pragma unroll
                         for (int i = 0; i < RL; ++i) acc[s][i] = fmaf(bi, xs[i], fmaf(sc, dot[s - s0][i], acc[s][i]));
                     }

@@ -787,16 +787,40 @@ static void w4r_go(const W4rPlan &pl, int N, hipStream_t st, const W4rArgs &a, c
 }
 
 size_t w4m_bytes(int N, int K);
+size_t w8m_bytes(int N, int K) { return (size_t)(N >> 5) * (K >> 6) * W8M_TILE_BYTES; }
+
+// W8S unit stream -> W8M tiles (w4a_gemm.hpp).  One thread per (tile, lane, piece).
+__global__ void __launch_bounds__(256) k_w8s_to_w8m(const u32 *w8s, int N, int K, int ns, u32 *w8m) {
+    const int groups = K >> 6;
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= (size_t)(N >> 5) * groups * 128) return;
+    const int lane = (int)(i & 63), q = (int)((i >> 6) & 1), g = (int)((i >> 7) % groups), nt = (int)((i >> 7) / groups);
+    const int n = lane & 31, kh = lane >> 5, r = 32 * nt + n;
+    const u32 *unit = w8s + ((size_t)(r >> 1) * ns + (g >> 5)) * (W8S_UNIT_BYTES / 4);
+    const int src_lane = (r & 1) * 32 + (g & 31);
+    u32 *tile = w8m + ((size_t)nt * groups + g) * (W8M_TILE_BYTES / 4);
+    const uint2 a = *reinterpret_cast<const uint2 *>(unit + 512 * q + 4 * src_lane + 2 * kh), b = *reinterpret_cast<const uint2 *>(unit + 512 * q + 256 + 4 * src_lane + 2 * kh);  // k-steps 2 q, 2 q + 1
+    *reinterpret_cast<uint4 *>(tile + 256 * q + 4 * lane) = make_uint4(a.x, a.y, b.x, b.y);
+    if (q == 0 && kh == 0) tile[512 + n] = unit[1024 + src_lane];
+}
+int w8m_repack_launch(const void *w8s, int N, int K, void *w8m, hipStream_t st) {
+    PIE_REQUIRE(N > 0 && K > 0 && N % 32 == 0 && K % 64 == 0, PIE_E_SHAPE, "W8M repack: N must be a multiple of 32 and K of 64");
+    const size_t n = (size_t)(N >> 5) * (K >> 6) * 128;
+    hipLaunchKernelGGL(k_w8s_to_w8m, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, (const u32 *)w8s, N, K, w4s_slices(K), (u32 *)w8m);
+    PIE_LAUNCH_CHECK();
+    return PIE_OK;
+}
 // Up to 16 rows with the scales on the sums (k_w4a_gemm).  Workgroups: of as many half strips as give every CU one (at most eight); what stays below 1024 half strips takes four and splits of
 // K, in one round of workgroups and of at least two steps: q|k|v two splits, o_proj and down four (8 rows, four half strips in two / four / seven splits, two in two: q|k|v 6.8 / 7.6 / - / 7.3 us,
 // o_proj - / 5.2 / - / 5.2, down - / 11.4 / 11.2 / 12.2, [3072, 8192] - / 6.6 / - / 7.6).  Beyond eight rows only what needs no splits: there k_w4r_gemm is as good or better at the others.
 struct W4aPlan {
     int halves, S, groups;  // half strips per workgroup; K splits, groups of each; halves == 0: shape not served
 };
-static W4aPlan w4a_plan(int M, int N, int K, bool may_split) {
-    if (M < 1 || M > W4A_ROWS || N < 32 || N % 32 || K < 64 || K % 64 || w4m_bytes(N, K) >= (1ull << 31)) return {0, 0, 0};
+// Int8 codes (bits == 8): up to 32 rows, narrow matrices in the same splits: the other form reads 16 bits a weight (32 rows 9319 / 6719 us, w4a_gemm.hpp).
+static W4aPlan w4a_plan(int M, int N, int K, bool may_split, int bits) {
+    if (M < 1 || M > (bits == 8 ? W8A_ROWS : W4A_ROWS) || N < 32 || N % 32 || K < 64 || K % 64 || (bits == 8 ? w8m_bytes(N, K) : w4m_bytes(N, K)) >= (1ull << 31)) return {0, 0, 0};
     const int units = N / 16, groups = K / 64, steps = (groups + 7) / 8;
-    if (M > 8 && units < 1024) return {0, 0, 0};
+    if (bits == 4 && M > 8 && units < 1024) return {0, 0, 0};
     const int halves = units >= 2048 ? 8 : (units + 255) / 256;
     if (units >= 1024 || !may_split) return {halves, 1, 8 * steps};
     const int wgs = (units + 3) / 4;
@@ -806,10 +830,10 @@ static W4aPlan w4a_plan(int M, int N, int K, bool may_split) {
     if (S == 1) return {halves, 1, 8 * steps};
     return {4, S, 8 * (steps / S)};
 }
-bool w4a_serves(int M, int N, int K) { return pie_knob(PIE_KNOB_W4R) != 0 && w4a_plan(M, N, K, false).halves != 0; }
-int w4a_splits(int M, int N, int K) { return w4a_plan(M, N, K, true).S; }
-size_t w4a_workspace_bytes(int M, int N, int K) {
-    const int s = w4a_splits(M, N, K);
+bool w4a_serves(int M, int N, int K, int bits) { return pie_knob(PIE_KNOB_W4R) != 0 && w4a_plan(M, N, K, false, bits).halves != 0; }
+int w4a_splits(int M, int N, int K, int bits) { return w4a_plan(M, N, K, true, bits).S; }
+size_t w4a_workspace_bytes(int M, int N, int K, int bits) {
+    const int s = w4a_splits(M, N, K, bits);
     return s > 1 ? (size_t)s * M * N * sizeof(float) : 0;
 }
 template <class T, int MT>
@@ -822,21 +846,33 @@ static void w4a_go(const W4aArgs &a, int S, hipStream_t st, const W4mRope &r) {
     default: hipLaunchKernelGGL((k_w4a_gemm<T, MT, 4, 2>), grid, block, 0, st, a, r); break;
     }
 }
+template <class T, int MT>
+static void w8a_go(const W4aArgs &a, int S, hipStream_t st, const W4mRope &r) {
+    const dim3 grid((unsigned)((a.N / 16 + a.halves - 1) / a.halves), (unsigned)S), block(512);
+    switch ((a.halves + 1) / 2) {  // (half as many steps in flight as int4's: as many bytes)
+    case 1: hipLaunchKernelGGL((k_w4a_gemm<T, MT, 1, 4, 8>), grid, block, 0, st, a, r); break;
+    case 2: hipLaunchKernelGGL((k_w4a_gemm<T, MT, 2, 3, 8>), grid, block, 0, st, a, r); break;
+    case 3: hipLaunchKernelGGL((k_w4a_gemm<T, MT, 3, 2, 8>), grid, block, 0, st, a, r); break;
+    default: hipLaunchKernelGGL((k_w4a_gemm<T, MT, 4, 2, 8>), grid, block, 0, st, a, r); break;
+    }
+}
 // epi, rope, slabs, bias_done: as for w4r_gemm_launch; a matrix with wide scales stays there (bias - 128 scale has to be finite)
 int w4a_gemm_launch(int dtype, const void *w4m, const void *x, int M, int N, int K, void *y, void *workspace, hipStream_t st, int epi, const void *bias,
-                    const W4mRope *rope, int *slabs, bool *bias_done) {
+                    const W4mRope *rope, int *slabs, bool *bias_done, int bits) {
     if (slabs) *slabs = 0;
     if (bias_done) *bias_done = false;
     PIE_REQUIRE(dtype == PIE_BF16 || dtype == PIE_F16, PIE_E_ARG, "W4A GEMM: dtype must be PIE_BF16 or PIE_F16");
     PIE_REQUIRE((epi == W4R_ROPE) == (rope != nullptr), PIE_E_ARG, "W4A GEMM: the q|k|v epilogue needs its arguments");
     const bool may_split = epi == W4R_STORE && workspace != nullptr && slabs != nullptr;  // (the caller's consumer sums them)
-    const W4aPlan pl = w4a_plan(M, N, K, may_split);
-    PIE_REQUIRE(pl.halves != 0, PIE_E_SHAPE, "W4A GEMM: 1..16 rows, N a multiple of 32, K of 64");
+    const W4aPlan pl = w4a_plan(M, N, K, may_split, bits);
+    PIE_REQUIRE(pl.halves != 0, PIE_E_SHAPE, "W4A GEMM: 1..16 rows (32 of int8 codes), N a multiple of 32, K of 64");
     PIE_REQUIRE(pie_aligned(w4m, 16) && pie_aligned(x, 16) && pie_aligned(y, 16) && pie_aligned(bias, 16), PIE_E_ALIGN, "W4A GEMM: 16-byte alignment required");
     const W4aArgs a = {(const char *)w4m, (const u16 *)x, M, N, K, pl.halves, pl.groups, (u16 *)y, pl.S > 1 ? (float *)workspace : nullptr, pl.S > 1 ? nullptr : (const u16 *)bias,
                        pl.S > 1 ? W4R_SLAB : epi};
     const W4mRope r = rope ? *rope : W4mRope{};
-    if (dtype == PIE_BF16) M <= 8 ? w4a_go<BF16, 8>(a, pl.S, st, r) : w4a_go<BF16, 16>(a, pl.S, st, r);
+    if (bits == 8 && dtype == PIE_BF16) M <= 8 ? w8a_go<BF16, 8>(a, pl.S, st, r) : M <= 16 ? w8a_go<BF16, 16>(a, pl.S, st, r) : w8a_go<BF16, 32>(a, pl.S, st, r);
+    else if (bits == 8) M <= 8 ? w8a_go<F16, 8>(a, pl.S, st, r) : M <= 16 ? w8a_go<F16, 16>(a, pl.S, st, r) : w8a_go<F16, 32>(a, pl.S, st, r);
+    else if (dtype == PIE_BF16) M <= 8 ? w4a_go<BF16, 8>(a, pl.S, st, r) : w4a_go<BF16, 16>(a, pl.S, st, r);
     else M <= 8 ? w4a_go<F16, 8>(a, pl.S, st, r) : w4a_go<F16, 16>(a, pl.S, st, r);
     PIE_LAUNCH_CHECK();
     if (pl.S > 1) *slabs = pl.S;
