@@ -444,7 +444,7 @@ struct PrefillScratch {
     // 4.6 B per parameter (7 ms of a 10.8 ms 128-token prefill on the 8B model) for 2 B per parameter of HBM; kept when
     // that is a small share of the free memory (PIE_KNOB_PREFILL_RESIDENT overrides), built on first use.
     std::map<const void *, u16 *> resident;
-    // W4M tile copies (w4m_gemm.hip) of int4 layer matrices for prompts of at most small_rows() rows: 0.5625 B per weight each
+    // W4M (W8M) tile copies (w4m_gemm.hip) of int4 (int8) matrices: 0.5625 (1.0625) B per weight each
     struct Tiles { void *p; size_t bytes; };
     std::map<const void *, Tiles> resident_w4m;
     LogitStat *tail_stats = nullptr;  // fused few-sequence step: the lm_head GEMV's tail partials, one per wave and row; other rows' tiles (RowStat) where the tail takes two launches
@@ -869,7 +869,7 @@ static int linear_rows(pie_decoder *d, const void *packed, int N, int K, const u
             return bias_rows<T>(y, bias, M, N, st);
         }
     }
-    // Everything else -- dense modules, int8 and group-32 modules beyond the GEMV's rows -- multiplies a 16-bit copy of the matrix in W16M
+    // Everything else -- dense modules, int8 beyond 32 rows, group-32 modules beyond the GEMV's rows -- multiplies a 16-bit copy of the matrix in W16M
     // tiles with the hand-written MFMA GEMM (w16_gemm.hpp); resident copies are built on first use within the budget.
     PIE_REQUIRE(K % 64 == 0, PIE_E_SHAPE, "prefill: a many-row Linear needs in_features % 64 == 0 (pie_set_knob(PIE_KNOB_PREFILL_MIN, 1000000) processes prompts as iterated decode steps)");
     u16 *wM = s->wM;

@@ -660,7 +660,7 @@ def vision_blocks_served(hidden: int, inter: int, heads: int, head_dim: int) -> 
 
 
 def vision_block_table(blocks: list[dict], after: list[torch.Tensor], full: list[int]):
-    """The blocks' weights (qkv_w, qkv_b, ..; packed Linears and tensors, which the caller keeps) for vision_blocks; after[i]: the norm behind block i, full: the blocks over whole images."""
+    """The blocks' weights (qkv_w, qkv_b, ..; packed Linears and tensors, which the table keeps) for vision_blocks; after[i]: the norm behind block i, full: the blocks over whole images."""
     def ptr(v):
         return (v.tiles if isinstance(v, PackedLinear) else v).data_ptr()
     table = (_ffi.pie_vision_block * len(blocks))()
@@ -668,6 +668,7 @@ def vision_block_table(blocks: list[dict], after: list[torch.Tensor], full: list
         for name in ("qkv_w", "qkv_b", "proj_w", "proj_b", "norm2", "gateup_w", "gateup_b", "down_w", "down_b"):
             setattr(table[i], name, ptr(b[name]))
         table[i].next_norm, table[i].full = ptr(n), int(i in full)
+    table.weights = [dict(b) for b in blocks], list(after)   # alive as long as the pointers
     return table
 
 
