@@ -445,7 +445,7 @@ struct PrefillScratch {
     // that is a small share of the free memory (PIE_KNOB_PREFILL_RESIDENT overrides), built on first use.
     std::map<const void *, u16 *> resident;
     // W4M (W8M) tile copies (w4m_gemm.hip) of int4 (int8) matrices: 0.5625 (1.0625) B per weight each
-    struct Tiles { void *p; size_t bytes; };
+    struct Tiles { void *p; size_t bytes; bool wide; };  // wide: some scale is too large for k_w4a_gemm (w4m_wide_scales)
     std::map<const void *, Tiles> resident_w4m;
     LogitStat *tail_stats = nullptr;  // fused few-sequence step: the lm_head GEMV's tail partials, one per wave and row; other rows' tiles (RowStat) where the tail takes two launches
     size_t tail_entries = 0;           // its capacity in entries
@@ -455,6 +455,7 @@ struct PrefillScratch {
     hipGraphExec_t batch_graph = nullptr;
     std::vector<uintptr_t> batch_key, warm_key;
     unsigned batch_gen = 0, warm_gen = 0;
+    bool batch_form = false;  // batch_fused() of the captured step
     void *w4l_ws = nullptr;   // fp32 partial tiles of the K-split prompt GEMM (w4m_gemm.hip)
     size_t w4l_ws_bytes = 0;
     float *attn_part = nullptr;  // sums of prompt attention split along the keys (reserve_attn_part)
@@ -750,18 +751,21 @@ static int linear_rows(pie_decoder *d, const void *packed, int N, int K, const u
     // resident W4M (W8M) tile copy of an int4 (int8) matrix (0.5625 B, 1.0625 B per weight, built on first use within the residency budget); nullptr: no room
     const bool is_int8 = d->mat_fmt(packed) == PIE_W_INT8_G64;
     const size_t tile_bytes = is_int8 ? w8m_bytes(N, K) : w4m_bytes(N, K);
+    bool wide = false;  // of the tiles that w4m_tiles found
     auto w4m_tiles = [&](void **out) -> int {
         *out = nullptr;
         auto it = s->resident_w4m.find(packed);
         if (it != s->resident_w4m.end()) {
-            *out = it->second.p;
+            *out = it->second.p, wide = it->second.wide;
             return PIE_OK;
         }
         void *wm = nullptr;
         if (resident_budget(d) >= tile_bytes && hipMalloc(&wm, tile_bytes) == hipSuccess) {
-            s->resident_w4m[packed] = {wm, tile_bytes}, s->resident_left -= tile_bytes, ++s->alloc_gen;
+            const int rc = is_int8 ? w8m_repack_launch(packed, N, K, wm, st) : w4m_repack_launch(packed, N, K, wm, st);
+            wide = !is_int8 && w4m_wide_scales(wm);
+            s->resident_w4m[packed] = {wm, tile_bytes, wide}, s->resident_left -= tile_bytes, ++s->alloc_gen;
             *out = wm;
-            return is_int8 ? w8m_repack_launch(packed, N, K, wm, st) : w4m_repack_launch(packed, N, K, wm, st);
+            return rc;
         }
         (void)hipGetLastError();
         return PIE_OK;
@@ -779,7 +783,6 @@ static int linear_rows(pie_decoder *d, const void *packed, int N, int K, const u
     // carries the SwiGLU in its epilogue.
     auto tiles_gemm = [&](void *wm, bool affine) -> int {
         const int bits = is_int8 ? 8 : 4;
-        const bool wide = !affine && w4m_wide_scales(wm);
         auto go = [&](void *to, void *ws, int epi, const void *b, const W4mRope *r, int *n_slabs, bool *done) {
             return affine ? w4a_gemm_launch(d->cfg.dtype, wm, x, M, N, K, to, ws, st, epi, b, r, n_slabs, done, bits) : w4r_gemm_launch(d->cfg.dtype, wm, x, M, N, K, to, ws, st, epi, b, r, n_slabs, done, wide);
         };
@@ -809,7 +812,7 @@ static int linear_rows(pie_decoder *d, const void *packed, int N, int K, const u
         void *wm = nullptr;
         const int rc = w4m_tiles(&wm);
         if (rc) return rc;
-        if (wm && !w4m_wide_scales(wm)) return tiles_gemm(wm, true);
+        if (wm && !wide) return tiles_gemm(wm, true);
     }
     // Int8 codes, up to 32 rows: the same form (no scale is too large for it: a code has no offset)
     if (is_int8 && (keep || keep_w4m) && w4a_serves(M, N, K, 8)) {
@@ -1073,7 +1076,7 @@ static bool step_tiles(const pie_decoder *d, int B) {
     auto has = [&](const void *packed, int N, int K) {
         if (!w4a_serves(B, N, K)) return false;
         const auto it = d->prefill->resident_w4m.find(packed);
-        if (it != d->prefill->resident_w4m.end()) return !w4m_wide_scales(it->second.p);
+        if (it != d->prefill->resident_w4m.end()) return !it->second.wide;
         more += w4m_bytes(N, K);
         return true;
     };
@@ -1093,8 +1096,8 @@ static bool batch_fused(const pie_decoder *d, int B) {
         if (w.bqkv || w.bo || w.bgateup || w.bdown) return false;
     return B <= GEMV_FUSED_ROWS || !step_tiles(d, B);
 }
-static int batch_rows(pie_decoder *d, const int32_t *tokens, const int32_t *ctx_len, int B, hipStream_t st) {
-    const bool fused = batch_fused(d, B);
+// fused: the form of the layers that follow, replayed ones too (step_batch keeps it with the graph): with norm and lengths' sum they take another pass's rows
+static int batch_rows(pie_decoder *d, const int32_t *tokens, const int32_t *ctx_len, int B, bool fused, hipStream_t st) {
     return pass_rows(d, tokens, nullptr, B, ctx_len, fused ? nullptr : d->layers[0].attn_norm, st, !fused);
 }
 
@@ -1105,21 +1108,19 @@ static int batch_rows(pie_decoder *d, const int32_t *tokens, const int32_t *ctx_
 // skeleton (src/pie_core/include/engine/batch_details.hpp:10-88, scheduler.hpp) describes for decode-state sequences.
 template <class T>
 static int decode_batch_t(pie_decoder *d, const int32_t *tokens, const int32_t *ctx_len, const void *const *slabs, int n_pages,
-                          const int32_t *block_tables, int max_blocks, int B, u16 *logits, float *logprobs, int32_t *next_tokens, int32_t *lens, hipStream_t st) {
+                          const int32_t *block_tables, int max_blocks, int B, u16 *logits, float *logprobs, int32_t *next_tokens, int32_t *lens, bool fused_rows, hipStream_t st) {
     const pie_decoder_config &c = d->cfg;
     const int H = c.hidden, D = c.head_dim, QD = c.n_heads * D, KVD = c.n_kv_heads * D, NQKV = QD + 2 * KVD, I = c.inter;
     size_t w_elems = w16m_size(2 * I, H) / 2;  // the 16-bit copies are W16M tiles (rows padded to 32, columns to 64)
     if (w16m_size(NQKV, H) / 2 > w_elems) w_elems = w16m_size(NQKV, H) / 2;
     if (w16m_size(H, I) / 2 > w_elems) w_elems = w16m_size(H, I) / 2;
     if (w16m_size(c.vocab, H) / 2 > w_elems) w_elems = w16m_size(c.vocab, H) / 2;
-    if (!d->prefill) d->prefill = new PrefillScratch();
     // (the layers' products say whether they rotated and appended themselves, and with it which kernel attends)
-    const bool fused_rows = batch_fused(d, B);
     const int splits = batch_attn_splits(d, B, max_blocks, false), step_splits = fused_rows ? splits : batch_attn_splits(d, B, max_blocks, true);
     int rc = scratch_reserve(d, B, w_elems, (size_t)B * (step_splits > splits ? step_splits : splits));
     if (rc) return rc;
     PrefillScratch *s = d->prefill;
-    if (tokens && (rc = batch_rows(d, tokens, ctx_len, B, st))) return rc;  // (nullptr: they are there already)
+    if (tokens && (rc = batch_rows(d, tokens, ctx_len, B, fused_rows, st))) return rc;  // (nullptr: they are there already)
     const int lm_waves = w4s_gemv_waves(c.vocab, H);
     const bool tiles = !fused_rows && logits_in_tiles(B, c.vocab);
     if ((fused_rows || tiles) && (rc = tail_stats_reserve(s, (size_t)(tiles ? LOGITS_TILES : lm_waves) * (size_t)B))) return rc;
@@ -1356,10 +1357,10 @@ extern "C" int pie_decoder_step_mixed(pie_decoder *d, const int32_t *ids, const 
 }
 
 static int decode_batch(pie_decoder *d, const int32_t *tokens, const int32_t *ctx_len, const void *const *slabs, int n_pages, const int32_t *block_tables,
-                        int max_blocks, int B, void *logits, float *logprobs, int32_t *next_tokens, int32_t *lens, hipStream_t st) {
+                        int max_blocks, int B, void *logits, float *logprobs, int32_t *next_tokens, int32_t *lens, bool fused, hipStream_t st) {
     return d->cfg.dtype == PIE_BF16
-               ? decode_batch_t<BF16>(d, tokens, ctx_len, slabs, n_pages, block_tables, max_blocks, B, (u16 *)logits, logprobs, next_tokens, lens, st)
-               : decode_batch_t<F16>(d, tokens, ctx_len, slabs, n_pages, block_tables, max_blocks, B, (u16 *)logits, logprobs, next_tokens, lens, st);
+               ? decode_batch_t<BF16>(d, tokens, ctx_len, slabs, n_pages, block_tables, max_blocks, B, (u16 *)logits, logprobs, next_tokens, lens, fused, st)
+               : decode_batch_t<F16>(d, tokens, ctx_len, slabs, n_pages, block_tables, max_blocks, B, (u16 *)logits, logprobs, next_tokens, lens, fused, st);
 }
 
 // bytes one page of the active format takes in a layer's slab: K block + V block of T rows, or the int8 page with its scales
@@ -1382,7 +1383,8 @@ static int step_batch(pie_decoder *d, const int32_t *tokens, const int32_t *cont
     PIE_REQUIRE(rep >= 1 && rep <= 8, PIE_E_SHAPE, "pie_decoder_step_batch: n_heads / n_kv_heads must be between 1 and 8");
     for (int i = 0; i < d->cfg.n_layers; ++i) PIE_REQUIRE(slabs[i] && pie_aligned(slabs[i], 16), PIE_E_ALIGN, "pie_decoder_step_batch: null or misaligned slab");
     hipStream_t st = (hipStream_t)stream;
-    if (!(flags & PIE_STEP_GRAPH)) return decode_batch(d, tokens, context_lens, slabs, (int)n_pages, block_tables, max_blocks, B, logits, logprobs, next_tokens, lens, st);
+    if (!d->prefill) d->prefill = new PrefillScratch();
+    if (!(flags & PIE_STEP_GRAPH)) return decode_batch(d, tokens, context_lens, slabs, (int)n_pages, block_tables, max_blocks, B, logits, logprobs, next_tokens, lens, batch_fused(d, B), st);
     // Graph replay, behind the launch that reads the tokens: those may be another buffer every time (copied to a fixed place first, and the lengths moved on by a launch of their own,
     // a step of 8 sequences took 2 % more).  The launches bake in the caller's buffers and this library's scratch / resident weight copies, so a graph is
     // captured only for a call that repeats the previous call's buffers after that call allocated nothing, and is dropped when
@@ -1390,13 +1392,13 @@ static int step_batch(pie_decoder *d, const int32_t *tokens, const int32_t *cont
     std::vector<uintptr_t> key = {(uintptr_t)lens, (uintptr_t)context_lens, (uintptr_t)block_tables, (uintptr_t)logits, (uintptr_t)logprobs,
                                   (uintptr_t)next_tokens, (uintptr_t)n_pages, (uintptr_t)max_blocks, (uintptr_t)B, (uintptr_t)d->kv_i8 /* the page format is baked into the launches too */};
     for (int i = 0; i < d->cfg.n_layers; ++i) key.push_back((uintptr_t)slabs[i]);
-    if (!d->prefill) d->prefill = new PrefillScratch();
     PrefillScratch *s = d->prefill;
     if (s->batch_graph && s->batch_key == key && s->batch_gen == s->alloc_gen) {
-        if (const int rc = batch_rows(d, tokens, context_lens, B, st)) return rc;
+        if (const int rc = batch_rows(d, tokens, context_lens, B, s->batch_form, st)) return rc;
         PIE_HIP_TRY(hipGraphLaunch(s->batch_graph, st));
         return PIE_OK;
     }
+    const bool fused = batch_fused(d, B);
     if (s->warm_key == key && s->warm_gen == s->alloc_gen) {
         if (s->batch_graph) (void)hipGraphExecDestroy(s->batch_graph), s->batch_graph = nullptr;
         hipGraph_t g = nullptr;
@@ -1408,25 +1410,25 @@ static int step_batch(pie_decoder *d, const int32_t *tokens, const int32_t *cont
             return pie::fail(PIE_E_HIP, std::string("hipStreamBeginCapture: ") + hipGetErrorString(e));
         }
         const unsigned gen = s->alloc_gen;
-        const int rc = decode_batch(d, nullptr, context_lens, slabs, (int)n_pages, block_tables, max_blocks, B, logits, logprobs, next_tokens, lens, cs);
+        const int rc = decode_batch(d, nullptr, context_lens, slabs, (int)n_pages, block_tables, max_blocks, B, logits, logprobs, next_tokens, lens, fused, cs);
         e = hipStreamEndCapture(cs, &g);
         (void)hipStreamDestroy(cs);
         if (rc || e != hipSuccess || d->prefill->alloc_gen != gen) {  // something allocated or failed under capture: run this call eagerly instead
             if (g) (void)hipGraphDestroy(g);
             (void)hipGetLastError();
             d->prefill->warm_key.clear();
-            return decode_batch(d, tokens, context_lens, slabs, (int)n_pages, block_tables, max_blocks, B, logits, logprobs, next_tokens, lens, st);
+            return decode_batch(d, tokens, context_lens, slabs, (int)n_pages, block_tables, max_blocks, B, logits, logprobs, next_tokens, lens, fused, st);
         }
         s = d->prefill;
         e = hipGraphInstantiate(&s->batch_graph, g, nullptr, nullptr, 0);
         (void)hipGraphDestroy(g);
         if (e != hipSuccess) return pie::fail(PIE_E_HIP, std::string("hipGraphInstantiate: ") + hipGetErrorString(e));
-        s->batch_key = key, s->batch_gen = s->alloc_gen;
-        if (const int rows = batch_rows(d, tokens, context_lens, B, st)) return rows;
+        s->batch_key = key, s->batch_gen = s->alloc_gen, s->batch_form = fused;
+        if (const int rows = batch_rows(d, tokens, context_lens, B, fused, st)) return rows;
         PIE_HIP_TRY(hipGraphLaunch(s->batch_graph, st));
         return PIE_OK;
     }
-    const int rc = decode_batch(d, tokens, context_lens, slabs, (int)n_pages, block_tables, max_blocks, B, logits, logprobs, next_tokens, lens, st);
+    const int rc = decode_batch(d, tokens, context_lens, slabs, (int)n_pages, block_tables, max_blocks, B, logits, logprobs, next_tokens, lens, fused, st);
     d->prefill->warm_key = key, d->prefill->warm_gen = d->prefill->alloc_gen;
     return rc;
 }
