@@ -307,8 +307,9 @@ def test_batched_decode_step_matches_each_sequence_alone(golden_dir, B):
     """B sequences of different lengths decode together (pie_decoder_step_batch): the weights stream once per step, every row
     has its own position, pages and attention span.  Each row's logits must be what the oracle gives for that sequence alone
     (teacher-forced along the oracle's greedy tokens, margins permitting), with the oracle in ITS OWN default regime for that
-    many rows: below 6 rows row-by-row exact fp32 (MLX's qmv; here the multi-row streaming GEMV k_w4s_gemv_rows), from 6 rows the
-    many-row regime (weights dequantised to T, MFMA: the few-row kernel up to 32 rows, the many-row GEMM beyond)."""
+    many rows: below 6 rows row-by-row exact fp32 (MLX's qmv; here the multi-row streaming GEMV k_w4s_gemv_rows for two, k_w4a_gemm
+    with the scales on its fp32 sums from 3 to 16), from 6 rows the many-row regime (weights dequantised to T, MFMA: the few-row
+    kernel up to 32 rows, the many-row GEMM beyond)."""
     from tests._util import assert_vec_close
     from tests.test_gpu_decode import margin_bound
     g, cfg, model = _tiny(golden_dir)
@@ -695,6 +696,19 @@ def test_prompt_pass_then_few_sequence_step_with_a_large_vocabulary():
         assert_vec_close(got[i], alone[i][0], "bfloat16", what=f"row {i} of the step after the prompt pass")
         assert abs(float(np.exp(got_lp[i].astype(np.float64)).sum()) - 1.0) < 1e-4
         assert np.abs(got_lp[i] - alone[i][1]).max() < 0.05
+
+
+@pytest.mark.parametrize("B", [3, 5])
+def test_batched_decode_step_without_tiles(golden_dir, B, knobs):
+    """No room for W4M tiles (the budget is a new decoder's first pass's): 3 to 5 int4 rows take the multi-row streaming GEMV with everything else of the layer in its launches."""
+    knobs("prefill_resident", 0)
+    test_batched_decode_step_matches_each_sequence_alone(golden_dir, B)
+
+
+def test_prompt_pass_then_few_sequence_step_without_tiles(knobs):
+    """The step that writes one partial per GEMV wave and row behind the prompt pass that takes fewer, three rows wide."""
+    knobs("prefill_resident", 0)
+    test_prompt_pass_then_few_sequence_step_with_a_large_vocabulary()
 
 
 # ---------------------------------------------------------------- int8 pages with per-head scales (page.hpp:25-32)
