@@ -104,13 +104,20 @@ class ReusableKVCache(BaseCache):
         return self  # the reference returns self too (reusable.py:250-254): KV stays 16-bit on this path
 
 
+SHARED_BYTES = 64 << 20   # of one buffer that several layers share: it lives until the last of them has grown out of it
+
+
 def reserve_layers(caches: list[ReusableKVCache], needed: int, n_kv_heads: int, head_dim: int, dtype: torch.dtype, device) -> None:
-    """`reserve` of a model's layers.  The first buffers of all of them are slices of one: a fill each was a launch each, two a layer."""
+    """`reserve` of a model's layers.  Their first buffers are slices of a few, up to SHARED_BYTES each: a fill each was a launch each, two a layer.  Larger ones are a layer's own, as is what they grow
+    into: a layer that has grown gives its old rows back, but a shared buffer only goes with the last of its layers."""
     first = caches[0]
     if all(type(c) is ReusableKVCache and c.keys is None and c.values is None and (c.step, c.max_capacity) == (first.step, first.max_capacity) for c in caches):
         cap = first._aligned(needed)
-        rows = torch.zeros((2 * len(caches), 1, n_kv_heads, cap, head_dim), dtype=dtype, device=device)
-        for i, c in enumerate(caches):
-            c.keys, c.values, c.offset = rows[2 * i], rows[2 * i + 1], 0
+        together = SHARED_BYTES // max(1, 2 * n_kv_heads * cap * head_dim * dtype.itemsize)   # layers of one buffer
+        for at in range(0, len(caches), together) if together > 1 else ():
+            group = caches[at:at + together]
+            rows = torch.zeros((2 * len(group), 1, n_kv_heads, cap, head_dim), dtype=dtype, device=device)
+            for i, c in enumerate(group):
+                c.keys, c.values, c.offset = rows[2 * i], rows[2 * i + 1], 0
     for c in caches:
         c.reserve(needed, n_kv_heads, head_dim, dtype, device)

@@ -258,3 +258,16 @@ def test_first_buffers_of_all_layers_are_slices_of_one(tokens):
     assert mixed[0].keys.shape[2] >= tokens + 1 and (mixed[0].keys is held) == (tokens % 256 != 0) and mixed[1].keys.shape[2] == 256
     with pytest.raises(RuntimeError):
         reserve_layers([ReusableKVCache(max_capacity=300) for _ in range(2)], 301, 2, 8, torch.float32, "cpu")
+
+
+@pytest.mark.parametrize("dim,storages", [(8, 1), (256, 2), (512, 3), (1024, 10)])
+def test_shared_buffers_of_layers_are_small(dim, storages):
+    """What outlives a layer that has grown, until its neighbours have: at most 64 MiB, whatever the model's cache takes (layers of 16 MiB by
+    four, of 32 MiB by two, of 64 MiB and more by themselves, keys and values apart)."""
+    from proxy_inference_engine_amd.cache.kv_cache import reserve_layers
+    caches = [ReusableKVCache() for _ in range(5)]
+    reserve_layers(caches, 4000, 2, dim, torch.float32, "cpu")   # 4096 positions
+    held = {t.untyped_storage().data_ptr(): t.untyped_storage().nbytes() for c in caches for t in (c.keys, c.values)}
+    own = caches[0].keys.nbytes
+    assert len(held) == storages and all(n <= max(64 << 20, own) for n in held.values())
+    assert sum(held.values()) == 10 * own and all(c.keys.shape == c.values.shape == (1, 2, 4096, dim) for c in caches)
