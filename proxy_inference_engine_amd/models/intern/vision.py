@@ -7,8 +7,8 @@ MFMA units (full-image layers and 64-patch-window layers are the same kernel wit
 pie_silu_mul, pie_add, pie_gelu.  Index bookkeeping (positions, window order, cu_seqlens) is host numpy, as it is host
 Python in the reference; the row permutations are device gathers.
 
-Layout notes: head_dim (80 for the 7B tower) is zero-padded to the attention kernel's 128 inside q / k / v; the attention stores
-the heads' own columns side by side.  PatchEmbed's Conv3d (stride = kernel) is a
+Layout notes: head_dim (80 for the 7B tower) is zero-padded to the attention kernel's 128 inside q / k / v; the attention of
+pie_vision_blocks stores the heads' own columns side by side.  PatchEmbed's Conv3d (stride = kernel) is a
 GEMM over the flattened patches; its weight is flattened once at load in the pixel rows' (C, T, P, P) order."""
 from __future__ import annotations
 
@@ -70,13 +70,22 @@ class VisionModel:
         # every Linear of the tower is a dense GEMM on the hand-written 16-bit MFMA kernel (ops.linear_rows -> pie_linear_w16m): the weights are
         # tiled in MFMA operand order once, here (ops.pack_linear); rounds 1-4 called hipBLASLt
         self.patch_w = ops.pack_linear(w.reshape(w.shape[0], -1).to(device=self.device, dtype=dtype).contiguous())   # [hidden, C*T*P*P]
+        # widths that pie_vision_blocks takes: the blocks in one native call.  The others go op by op, and where their heads are padded `proj` is widened to match (zero columns): the attention's rows
+        # are its operand as they stand
+        native = c.depth and c.hidden_size == c.num_heads * self.head_dim and ops.vision_blocks_served(c.hidden_size, c.intermediate_size, c.num_heads, self.head_dim)
+        self.proj_dim = self.head_dim if native else self.padded_head_dim   # columns of a head that `proj` takes
+
+        def proj(name):
+            t, more = get(name), self.proj_dim - self.head_dim
+            return torch.nn.functional.pad(t.view(t.shape[0], c.num_heads, self.head_dim), (0, more)).view(t.shape[0], -1) if more else t
+
         self.blocks = []
         for i in range(c.depth):
             p = f"blocks.{i}."
             self.blocks.append({
                 "norm1": get(p + "norm1.weight"), "norm2": get(p + "norm2.weight"),
                 "qkv_w": ops.pack_linear(get(p + "attn.qkv.weight")), "qkv_b": get(p + "attn.qkv.bias"),
-                "proj_w": ops.pack_linear(get(p + "attn.proj.weight")), "proj_b": get(p + "attn.proj.bias"),
+                "proj_w": ops.pack_linear(proj(p + "attn.proj.weight")), "proj_b": get(p + "attn.proj.bias"),
                 # gate_proj and up_proj as ONE GEMM [2 * intermediate, hidden] with rows (gate_i, up_i) interleaved: the biases and
                 # silu(gate) * up ride in its epilogue (vision.py:196-197), the [N, 2 * intermediate] block is never written
                 "gateup_w": ops.pack_linear(ops.interleave_gate_up(get(p + "mlp.gate_proj.weight"), get(p + "mlp.up_proj.weight"))),
@@ -87,9 +96,8 @@ class VisionModel:
         self._graphs: dict = {}
         self.merger = {"ln_q": get("merger.ln_q.weight"), "w0": ops.pack_linear(get("merger.mlp.0.weight")), "b0": get("merger.mlp.0.bias"),
                        "w2": ops.pack_linear(get("merger.mlp.2.weight")), "b2": get("merger.mlp.2.bias")}
-        # widths that pie_vision_blocks takes: the blocks in one native call
         self._native = None
-        if c.depth and c.hidden_size == c.num_heads * self.head_dim and ops.vision_blocks_served(c.hidden_size, c.intermediate_size, c.num_heads, self.head_dim):
+        if native:
             after = [b["norm1"] for b in self.blocks[1:]] + [self.merger["ln_q"]]   # the next consumer's norm
             self._native = ops.vision_block_table(self.blocks, after, c.fullatt_block_indexes)
 
@@ -183,7 +191,7 @@ class VisionModel:
             qkv = ops.linear_rows(xn, b["qkv_w"])                                           # bias folded into the rotary kernel
             q, k, v = ops.vision_qkv_rope(qkv, cos, sin, c.num_heads, self.padded_head_dim, bias=b["qkv_b"])
             att = ops.sdpa_segments(q, k, v, lo, hi, scale)
-            r = ops.linear_rows(att[..., :self.head_dim].reshape(seq_len, -1), b["proj_w"])
+            r = ops.linear_rows(att[..., :self.proj_dim].reshape(seq_len, -1), b["proj_w"])
             if fuse_norm:
                 x, xn = ops.add_bias_rms_norm(x, r, b["proj_b"], b["norm2"], 1e-6)
             else:

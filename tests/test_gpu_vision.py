@@ -222,6 +222,28 @@ def test_blocks_in_one_call_are_the_blocks_op_by_op(cfg, grid, dt):
     assert all(torch.equal(a, b) for a, b in zip(states, want_states))
 
 
+def test_rows_of_padded_heads_are_the_projection_s_operand(monkeypatch):
+    """A tower whose blocks go op by op (hidden 160): the attention's rows of 128 columns a head go into `proj` as they stand, with no copy and no padding in between."""
+    from proxy_inference_engine_amd.models.intern import vision
+    _, model = _tower(CFG80, seed=4)
+    assert model._native is None
+    attended, multiplied = [], []
+    sdpa, linear = vision.ops.sdpa_segments, vision.ops.linear_rows
+
+    def sdpa_segments(*args):
+        attended.append(sdpa(*args))
+        return attended[-1]
+
+    def linear_rows(x, *args, **kwargs):
+        multiplied.append(x)
+        return linear(x, *args, **kwargs)
+    monkeypatch.setattr(vision.ops, "sdpa_segments", sdpa_segments), monkeypatch.setattr(vision.ops, "linear_rows", linear_rows)
+    model(dev(po.round_T(np.random.default_rng(7).standard_normal((92, 3 * 2 * 14 * 14)), DT)), torch.tensor([(1, 6, 10), (2, 4, 4)]))
+    assert len(attended) == CFG80["depth"]
+    for rows in attended:
+        assert [x.shape for x in multiplied if x.data_ptr() == rows.data_ptr()] == [(92, 2 * 128)]
+
+
 # BASELINE.json configs[3] at ITS geometry (VERDICT r3 item 1a): the Qwen2.5-VL-7B tower's shapes -- hidden 1280, 16 heads of 80 (zero-padded
 # to 128 inside the attention kernel), SwiGLU 3420 (not a multiple of 64: the K = 3420 GEMM rows), patch 14 x 14 x 2 frames, 112-pixel windows,
 # merger 5120 -> 3584 -- with 2 of its 32 blocks: one windowed, one full-attention (vision.py:87-442).
