@@ -596,7 +596,7 @@ static void reserve_attn_part(pie_decoder *d) {
 }
 // How a prompt's attention is launched: split along the keys where that pays (before: keys cached in front of the first row)
 static void split_attn(pie_decoder *d, PrefillAttnArgs &a, int before, bool told = true) {  // told: pie_decoder_prompt_shares hears of it
-    const int splits = d->prefill->attn_part ? prefill_attn_splits(a.M, before, a.Hq, a.Hkv) : 1;
+    const int splits = d->prefill->attn_part ? prefill_attn_splits(a.M, before, a.Hq, a.Hkv, d->cfg.head_dim) : 1;
     a.before = before;
     if (told) d->prefill->last_shares = splits;
     if (splits > 1) a.splits = splits, a.part = d->prefill->attn_part;

@@ -380,14 +380,24 @@ __global__ void __launch_bounds__(256) k_prefill_combine(const float *part, int 
 // Workgroups along the keys: rows behind a long cached prefix are few tiles with many blocks each (37 rows: 16 workgroups of 30 blocks).  `before`: keys in front of the first row.  Every
 // share costs its sums (4 D bytes per row and head, twice): at least two blocks of 64 keys per share up to 64 rows, three beyond, up to two workgroups per CU.  us, 1 / 2 / 4 / 8 shares:
 // 8 rows behind 500: 20 / 14 / 12 / 12; 37 behind 900: 35 / 24 / 18 / 17; 100: 38 / 26 / 21 / 23; 200: 41 / 30 / 26 / 30; 509: 53 / 42 / 40 / 46; 32 behind 4000: 131 / 73 / 42 / 29 (16: 28).
-// Rows of a fresh prompt see half of the blocks on average and gain nothing (509 rows: 22 / 26).  With two waves per tile (prefill_attn_pairs, whose images fill a CU) one workgroup per CU:
-// 509 behind 900 in four shares of one wave / two of two 39 / 36, 1000 behind 900 in two of one / one of two 65 / 53.
+// Rows of a fresh prompt see half of the blocks on average and gain nothing (509 rows: 22 / 26).
+// More than 256 rows of two to four heads a group may take two waves per tile instead (KG), one workgroup a CU (their images fill it for heads of 128), and so half as many shares where the chip and not the
+// prefix sets their number.  Two heads a group and heads of 64 gain from it unless one share is left of three.  The others want as many shares, four, a full round of workgroups or, behind no more keys than rows come, most of one.  Prompts of four layers of
+// attention alone, us, shares of one wave / of two, heads of 128: 32 / 8 heads, 509 rows behind 900 four / two 300 / 291, 400 behind 2000 four / two 328 / 332, 600 three / one 368 / 398; 24 / 8, 600 behind
+// 4000 473 / 581; 12 / 4, 400 behind 2000 nine / four 291 / 276, 1250 behind 4000 three / one 508 / 639; 16 / 8, 1000 behind 2000 two / one 459 / 412; heads of 64, 32 / 8, 600 behind 2000 294 / 310.
 static inline bool prefill_attn_duo(int rep) { return rep >= 2 && rep <= 4; }  // (four waves of 64 keys, 240 registers each, leave room for four more)
-static inline int prefill_attn_splits(int M, int before, int Hq, int Hkv) {
-    const int shares = before / 64 / (M <= 64 ? 2 : 3), room = (M > 256 && prefill_attn_duo(Hq / Hkv) ? 256 : 512) / ((M + 31) / 32 * Hkv);
+static inline bool prefill_attn_slim(int rep, int D) { return rep == 2 || D == 64; }
+static inline int prefill_attn_shares(int M, int before, int Hkv, int chip) {  // chip: workgroups that run at once
+    const int shares = before / 64 / (M <= 64 ? 2 : 3), room = chip / ((M + 31) / 32 * Hkv);
     const int s = shares < room ? shares : room;
     return s < 2 ? 1 : s > 16 ? 16 : s;
 }
+static inline bool prefill_attn_duo_shares(int M, int before, int Hq, int Hkv, int D) {  // whether shares are (or one is) of two waves per tile
+    const int one = prefill_attn_shares(M, before, Hkv, 512), two = prefill_attn_shares(M, before, Hkv, 256), workgroups = (M + 31) / 32 * Hkv * two;
+    if (M <= 256 || one < 2 || !prefill_attn_duo(Hq / Hkv)) return false;
+    return prefill_attn_slim(Hq / Hkv, D) ? 8 * two >= 3 * one : 2 * two > one || two >= 4 || workgroups >= 240 || (two == 1 && workgroups >= 200 && before <= M);
+}
+static inline int prefill_attn_splits(int M, int before, int Hq, int Hkv, int D) { return prefill_attn_shares(M, before, Hkv, prefill_attn_duo_shares(M, before, Hq, Hkv, D) ? 256 : 512); }
 // room for the sums of any split prompt: ceil(M / 32) Hkv splits <= 512
 static inline size_t prefill_attn_part_bytes(int Hq, int Hkv, int D) { return (size_t)(512 / Hkv) * 32 * Hq * (D + 2) * sizeof(float); }
 
@@ -397,13 +407,23 @@ static inline bool prefill_attn_short(const PrefillAttnArgs &a) { return a.M + a
 
 // Two waves per tile (KG) pay from about five blocks of 64 keys on, where they save blocks that wait for each other; below, and in shares of a few blocks, their meeting costs more.  us, one wave /
 // two, 32 / 8 heads: 128 rows 9.1 / 9.8, 300 15.4 / 15.1, 509 21.9 / 19.0, 1000 39.5 / 32.3, 1900 76.9 / 66.7; 24 / 8: 509 24.9 / 19.3, 1000 49.5 / 33.4, 1900 92.9 / 62.6; 32 / 16: 300 15.3 / 13.0;
-// 37 behind 900 in seven shares 17.2 / 17.9.  Against two tiles per workgroup (two waves per SIMD either way, K and V staged once for both): 2000 rows 89.5 / 71.3, 2300 103 / 94, 3000 139 / 148.
-static inline bool prefill_attn_pairs(const PrefillAttnArgs &a) { return prefill_attn_duo(a.Hq / a.Hkv) && a.M + a.before >= 256 && (a.splits <= 1 || a.M > 256); }
+// 37 behind 900 in seven shares 17.2 / 17.9.  Beyond one round of workgroups not behind many more cached keys than rows come, where all tiles are long and a last round costs as much as a full one (four
+// layers of attention alone, heads of 128, one wave / two: 32 / 8 heads, 1500 rows behind 900 532 / 508, behind 4000 884 / 920; 24 / 8, 1500 behind 2000 747 / 695, 2000 behind 4000 1085 / 1107); 16 / 8
+// and heads of 64 gain there too (16 / 8, 1500 behind 4000 971 / 819).  Against two tiles per workgroup, where those fill the chip: two waves per SIMD either way, K and V staged once for both: fresh
+// prompts (2000 rows 89.5 / 71.3, 2300 103 / 94, 3000 139 / 148; layers as above, 24 / 8 heads, 2050 551 / 536, 2400 574 / 591), behind cached keys hardly but heads of 64 (32 / 8
+// heads of 128, 2050 behind 400 609 / 588, behind 900 696 / 718; 24 / 8, 2300 behind 400 627 / 678; 16 / 8 565 / 601; 32 / 8 heads of 64 520 / 491, behind 4000 1067 / 994).
+static inline bool prefill_attn_pairs(const PrefillAttnArgs &a, int D) {
+    const int rep = a.Hq / a.Hkv, tiles = (a.M + 31) / 32 * a.Hkv, doubles = (a.M + 63) / 64 * a.Hkv;
+    if (a.splits > 1) return prefill_attn_duo_shares(a.M, a.before, a.Hq, a.Hkv, D);
+    if (!prefill_attn_duo(rep) || a.M + a.before < 256 || doubles >= 320) return false;
+    if (doubles >= 256) return D == 64 || (rep == 4 ? a.before <= (doubles < 288 ? a.M / 4 : 0) : a.before == 0 && doubles < 288);
+    return prefill_attn_slim(rep, D) || tiles <= 256 || a.before <= (rep == 3 ? a.M + a.M / 2 : a.M);
+}
 
 template <class T, int D>
 static int prefill_attn_launch_d(const PrefillAttnArgs &a, hipStream_t st) {
     const int rep = a.Hq / a.Hkv;
-    const bool pairs = prefill_attn_pairs(a);
+    const bool pairs = prefill_attn_pairs(a, D);
     if (a.splits > 1) {
         const dim3 grid((a.M + 31) / 32 * a.Hkv, a.splits);
 #define PA_SPLIT(R)                                                                                                                                      \
@@ -431,7 +451,7 @@ static int prefill_attn_launch_d(const PrefillAttnArgs &a, hipStream_t st) {
     const int qt = pie_knob(PIE_KNOB_PREFILL_QT);  // test knob: 1 forces one 32-row query tile per workgroup, 2 forces two wherever they fit
     // 2 tiles need 2*rep <= 8 waves of up to 256 registers, and only pay while the halved grid still fills the 256 CUs
     // (8B model: 4096 tokens 54.9 -> 53.9 ms, 8000 tokens 126.3 -> 125.0 ms; at 1024 tokens it would idle half the chip)
-    const bool two = rep <= 4 && a.M > 32 && (qt > 0 ? qt == 2 : ((a.M + 63) / 64) * a.Hkv >= (prefill_attn_duo(rep) ? 320 : 256)), few = prefill_attn_short(a);
+    const bool two = rep <= 4 && a.M > 32 && (qt > 0 ? qt == 2 : ((a.M + 63) / 64) * a.Hkv >= 256 && !pairs), few = prefill_attn_short(a);
     const dim3 grid(((a.M + (two ? 63 : 31)) / (two ? 64 : 32)) * a.Hkv);
 #define PA_LAUNCH(R)                                                                                         \
     if (two && R <= 4) hipLaunchKernelGGL((k_prefill_attn<T, D, R, (R <= 4 ? 2 : 1)>), grid, dim3(R * 128), 0, st, a); \

@@ -100,6 +100,50 @@ def test_rows_behind_a_prefix_split_along_the_keys(geometry, paged):
             assert_vec_close(got[1][i], got[0][i], "bfloat16", what=f"{n} rows, row {i}")
 
 
+@pytest.mark.parametrize("paged", [False, True], ids=["contiguous", "paged"])
+@pytest.mark.parametrize("geometry,calls", [((4, 2, 64), ((257, 700, 3), (300, 390, 2))), ((3, 1, 128), ((300, 700, 3), (257, 770, 4))), ((8, 2, 128), ((257, 700, 3), (300, 400, 2))),
+                                            ((32, 16, 64), ((257, 600, 3), (257, 400, 1))), ((48, 16, 128), ((330, 400, 2),)), ((51, 17, 128), ((500, 500, 1), (490, 736, 1)))], ids=str)
+def test_more_than_256_rows_behind_a_prefix(geometry, calls, paged):
+    """Two to four heads a group.  Shares of two waves a tile (the first three geometries: the last share empty, its last block's second half empty), shares of one where the chip allows few of two (three of
+    144 tiles, two of 176), no shares: two waves a tile, and one where many more keys are cached than rows come and 256 workgroups do not hold the tiles (490
+    behind 736).  Against the kernel that takes one query row at a time; pages out of order.  One layer, so that no second layer's sharp scores multiply what one rounding of the first one's rows leaves
+    between them: an ulp through o_proj, the MLP and the head, four of the largest logit as everywhere."""
+    from _util import assert_vec_close
+    from proxy_inference_engine_amd.models.llama import Model, ModelArgs
+    from proxy_inference_engine_amd.models.utils import synthetic_checkpoint
+    Hq, Hkv, D = geometry
+    cfg = {"model_type": "llama", "hidden_size": 256, "num_hidden_layers": 1, "intermediate_size": 512, "num_attention_heads": Hq, "num_key_value_heads": Hkv, "head_dim": D, "vocab_size": 320,
+           "rms_norm_eps": 1e-5, "tie_word_embeddings": False, "quantization": None}
+    w = synthetic_checkpoint(cfg, seed=5)
+    for n in list(w):
+        if "q_proj" in n or "k_proj" in n:
+            w[n] = w[n] * 6   # sharp attention: single keys decide
+    m = Model(ModelArgs(**cfg), w)
+    if paged:
+        m.enable_paged_kv(num_pages=60, max_blocks=20)
+    ids = torch.from_numpy(np.random.default_rng(1).integers(0, 320, 1300).astype(np.int32)).cuda()
+    for n, before, shares in calls:
+        cache, other = m.make_cache(), m.make_cache()
+        for lo in range(0, before, 100):   # (two sequences take their pages in turn)
+            m.step(ids[lo:min(lo + 100, before)], cache)
+            if paged:
+                m.step(ids[lo + 1:lo + 101], other)
+        got = []
+        for valu in (1, None):
+            _ffi.set_knob("prefill_attn_valu", valu)
+            try:
+                got.append(m(ids[None, before:before + n], cache=cache).float().cpu().numpy()[0])
+            finally:
+                _ffi.set_knob("prefill_attn_valu", None)
+            for layer in cache:
+                layer.trim(n)
+        assert _ffi.load().pie_decoder_prompt_shares(m._dec) == shares, (n, before)
+        for i in range(n):
+            assert_vec_close(got[1][i], got[0][i], "bfloat16", what=f"{n} rows behind {before}, row {i}")
+        if paged:
+            cache[0].page_manager.release(), other[0].page_manager.release()
+
+
 def test_longer_splits_do_not_allocate():
     """Prompts behind longer and longer prefixes take more and more shares of more rows; the room for their sums is there from the first prompt on."""
     from proxy_inference_engine_amd.models.llama import Model, ModelArgs
