@@ -807,8 +807,9 @@ static int linear_rows(pie_decoder *d, const void *packed, int N, int K, const u
         if (rc || !bias || bias_done) return rc;
         return bias_rows<T>(y, bias, M, N, st);
     };
-    // Up to 16 rows (8 of a narrow matrix): the scales on the sums.  Passes of one and two rows stay with the GEMV below (batch_fused).
-    if (is_int4 && w4a_serves(M, N, K) && (pass_rows ? pass_rows : M) > GEMV_FUSED_ROWS) {
+    // Three to 16 rows (8 of a narrow matrix): the scales on the sums.  One and two of a pass of up to five go to the GEMV below (batch_fused), the one that a longer pass leaves to its last layer to
+    // k_w4r_gemm, as the pass's other rows do: gate|up and down of Llama-3-8B 15.5 us each there, 17.1 here, where down has nobody to sum its splits.
+    if (is_int4 && w4a_serves(M, N, K) && M > GEMV_FUSED_ROWS) {
         void *wm = nullptr;
         const int rc = w4m_tiles(&wm);
         if (rc) return rc;

@@ -227,6 +227,23 @@ def test_the_last_layer_of_a_prompt_takes_its_last_row_alone(bits, layers):
         assert_vec_close(logits[i], alone[i], "bfloat16", what=f"prompt {i} of a batch")
 
 
+@pytest.mark.parametrize("layers", [1, 2])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+def test_the_last_row_alone_is_multiplied_as_the_rows_are(dtype, layers):
+    """Int4 prompts of 17 to 56 tokens: the row that the last layer goes on with takes the kernels, splits and sums that all of them take in the pass that returns every position's logits: the same bits."""
+    from proxy_inference_engine_amd.models.llama import Model, ModelArgs
+    from proxy_inference_engine_amd.models.utils import synthetic_checkpoint
+    cfg = {"model_type": "llama", "hidden_size": 512, "num_hidden_layers": layers, "intermediate_size": 2048, "num_attention_heads": 8, "num_key_value_heads": 2, "head_dim": 64, "vocab_size": 320,
+           "rms_norm_eps": 1e-5, "tie_word_embeddings": False, "quantization": {"group_size": 64, "bits": 4}}
+    m = Model(ModelArgs(**cfg), synthetic_checkpoint(cfg, seed=7, dtype=dtype))
+    ids = torch.from_numpy(np.random.default_rng(3).integers(0, 320, 56).astype(np.int32)).cuda()
+    for n in (17, 32, 33, 56):
+        m(ids[None, :n], cache=m.make_cache())
+        want = m.hidden.clone()
+        m.step(ids[:n], m.make_cache())
+        assert torch.equal(m.hidden, want), n
+
+
 @pytest.mark.parametrize("n", [40, 150])
 @pytest.mark.parametrize("paged", [False, True])
 def test_a_prompt_that_fails_leaves_the_sequence_where_it_was(n, paged):
