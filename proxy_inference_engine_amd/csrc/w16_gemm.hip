@@ -123,9 +123,10 @@ static W16Plan w16_plan(int M, int N, int K, bool no_split = false) {
     return best;
 }
 // Of one pass over K (the forms with an activation: w16_grouped.hip).  From two rounds of the largest tile on that one: the model counts whole rounds, which overlap, and its smaller tiles fetch more for the same
-// time ([28672, 4096], 2000 rows: 423.5 us in 1792 workgroups, 422.5 in 896; the prompt around it 5571-5533 us, 5512).
+// time ([28672, 4096], 2000 rows: 423.5 us in 1792 workgroups, 422.5 in 896; the prompt around it 5571-5533 us, 5512).  Rows that fill no more than half of it stay with the plan's
+// (four layers with an MLP [131072, 2048], 65 / 100 / 128 rows: 1539 / 1559 / 1604 us on the largest tile, 1447 / 1434 / 1477).
 void w16l_tile(int M, int N, int K, int *mb, int *sw) {
-    if ((long long)((N + 255) / 256) * ((M + 255) / 256) >= 512) {
+    if (M > 128 && (long long)((N + 255) / 256) * ((M + 255) / 256) >= 512) {
         *mb = 8, *sw = 2;
         return;
     }

@@ -1,0 +1,17 @@
+"""CPU: the tile that a 16-bit product with an activation takes, for rows and columns of every size (no kernel runs)."""
+import ctypes
+
+import pytest
+
+
+@pytest.mark.parametrize("N", [128, 5632, 28672, 57344, 131072, 262144])
+def test_few_rows_take_low_tiles(N):
+    """A tile of 32 mb rows is never twice as high as the rows need: 64 up to 64 rows, 128 up to 128, also where the columns alone are two rounds of workgroups."""
+    from proxy_inference_engine_amd import _ffi
+    tile = ctypes.CDLL(str(_ffi.lib_path().parent / "libpie_base.so"))["_Z9w16l_tileiiiPiS_"]   # w16l_tile(M, N, K, &mb, &sw)
+    mb, sw = ctypes.c_int(), ctypes.c_int()
+    for K in (64, 2048, 8192):
+        for M in (33, 64, 65, 100, 128, 129, 256, 257, 1000, 4096):
+            tile(M, N, K, ctypes.byref(mb), ctypes.byref(sw))
+            assert mb.value in (2, 4, 8) and sw.value in (1, 2), (M, K)
+            assert 32 * mb.value < 2 * max(M, 33), (M, K, mb.value)
