@@ -790,7 +790,10 @@ static int linear_rows(pie_decoder *d, const void *packed, int N, int K, const u
             *used_act = true;
             return go(act, nullptr, 1, bias, nullptr, nullptr, nullptr);
         }
-        if (rope && used_act && (affine ? w4a_splits(M, N, K, bits) : w4r_splits(M, N, K)) == 1) {  // q|k|v wide enough to fill the chip without a K split: RoPE + append in the epilogue
+        // q|k|v wide enough to fill the chip without a K split: RoPE + append in the epilogue.  Not for a step over T pages of an int8 model, whose attention's launch can rotate as well
+        // (24 layers of hidden 1024, 2 / 6 / 32 rows, us a step: 803 / 930 / 1138 rotated here, 755 / 811 / 1050 there).
+        const bool rotates = rope && used_act && !(is_int8 && rope->slab && !rope->i8_page_bytes);
+        if (rotates && (affine ? w4a_splits(M, N, K, bits) : w4r_splits(M, N, K)) == 1) {
             *used_act = true;
             rope->bias = (const u16 *)bias;
             return go(nullptr, nullptr, 2, nullptr, rope, nullptr, nullptr);

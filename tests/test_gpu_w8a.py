@@ -43,3 +43,22 @@ def test_rows_against_single_sequences(hidden, inter, vocab, heads, kv, dim, bia
     assert_vec_close(m.step(feed[:12], p)[2].float().cpu().numpy().reshape(-1), last, name, what="prompt")
     for cache in (c, p):
         cache[0].page_manager.release()
+
+
+def test_a_step_over_pages_rotates_in_its_attention():
+    """Up to 1024 columns (q|k|v in one pass over K): the product could rotate, but the attention's launch does it for less.  The kernels of one step, by name."""
+    from torch.profiler import ProfilerActivity, profile
+    from proxy_inference_engine_amd.models.llama import Model, ModelArgs
+    from proxy_inference_engine_amd.models.utils import synthetic_checkpoint
+    cfg = {"model_type": "llama", "hidden_size": 1024, "num_hidden_layers": 2, "intermediate_size": 512, "num_attention_heads": 8, "num_key_value_heads": 4, "head_dim": 128, "vocab_size": 320,
+           "rms_norm_eps": 1e-5, "tie_word_embeddings": False, "quantization": {"group_size": 64, "bits": 8}}
+    m = Model(ModelArgs(**cfg), synthetic_checkpoint(cfg, seed=2))
+    m.enable_paged_kv(num_pages=8, max_blocks=1)
+    caches, feed = [m.make_cache() for _ in range(2)], torch.arange(2, dtype=torch.int32, device="cuda")
+    m.step_batch(feed, caches, graph=False)
+    torch.cuda.synchronize()
+    with profile(activities=[ProfilerActivity.CUDA]) as p:
+        m.step_batch(feed, caches, graph=False)
+        torch.cuda.synchronize()
+    names = [(e.key, e.count) for e in p.key_averages()]
+    assert sum(n for k, n in names if "k_w4a_gemm" in k) == 9 and sum(n for k, n in names if "k_attn_step" in k) == 2, names
