@@ -634,6 +634,20 @@ static size_t resident_budget(const pie_decoder *d) {
     return s->resident_left;
 }
 
+// Bytes of the 16-bit copies that an int8 model may still make: its prompts beyond 32 rows multiply those, steps and short prompts only prefer the codes' tiles, which take what is left of the budget.
+// (First come first served, a model of more copies than budget that stepped first expanded most of its matrices anew in every chunk of its prompts.)
+static size_t w16_to_come(const pie_decoder *d) {
+    const pie_decoder_config &c = d->cfg;
+    const int QD = c.n_heads * c.head_dim, NQKV = QD + 2 * c.n_kv_heads * c.head_dim;
+    size_t bytes = 0;
+    auto add = [&](const void *packed, int N, int K) {
+        if (d->mat_fmt(packed) == PIE_W_INT8_G64 && !d->prefill->resident.count(packed)) bytes += w16m_size(N, K);
+    };
+    for (const pie_layer_weights &w : d->layers) add(w.wqkv, NQKV, c.hidden), add(w.wo, c.hidden, QD), add(w.wgateup, 2 * c.inter, c.hidden), add(w.wdown, c.hidden, c.inter);
+    add(d->glob.lm_head, c.vocab, c.hidden);
+    return bytes;
+}
+
 // w16_gemm.hpp / w4m_gemm.hip: the 16-bit many-row MFMA GEMM on W16M tiles (weights in MFMA A-fragment order)
 int w16m_from_rows_launch(const void *w, int N, int K, void *w16m, hipStream_t st);
 int w16m_from_w16s_launch(const void *w16s, int N, int K, void *w16m, hipStream_t st);
@@ -760,7 +774,7 @@ static int linear_rows(pie_decoder *d, const void *packed, int N, int K, const u
             return PIE_OK;
         }
         void *wm = nullptr;
-        if (resident_budget(d) >= tile_bytes && hipMalloc(&wm, tile_bytes) == hipSuccess) {
+        if (resident_budget(d) >= tile_bytes + (is_int8 ? w16_to_come(d) : 0) && hipMalloc(&wm, tile_bytes) == hipSuccess) {
             const int rc = is_int8 ? w8m_repack_launch(packed, N, K, wm, st) : w4m_repack_launch(packed, N, K, wm, st);
             wide = !is_int8 && w4m_wide_scales(wm);
             s->resident_w4m[packed] = {wm, tile_bytes, wide}, s->resident_left -= tile_bytes, ++s->alloc_gen;

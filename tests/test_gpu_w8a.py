@@ -62,3 +62,33 @@ def test_a_step_over_pages_rotates_in_its_attention():
         torch.cuda.synchronize()
     names = [(e.key, e.count) for e in p.key_averages()]
     assert sum(n for k, n in names if "k_w4a_gemm" in k) == 9 and sum(n for k, n in names if "k_attn_step" in k) == 2, names
+
+
+@pytest.mark.parametrize("budget,copies", [(1, True), (2, False)], ids=["tight", "ample"])
+def test_prompts_copies_come_before_steps_tiles(budget, copies, knobs):
+    """Steps of two sequences before the first long prompt, 0.9 GiB of 16-bit copies, half of that of the codes' tiles: in a budget of 1 GiB the steps multiply the copies that the prompt finds there, in one
+    of 2 GiB they take tiles, and the prompt's copies have room beside them."""
+    from proxy_inference_engine_amd.models.llama import Model, ModelArgs
+    from proxy_inference_engine_amd.models.utils import synthetic_checkpoint
+    cfg = {"model_type": "llama", "hidden_size": 2048, "num_hidden_layers": 7, "intermediate_size": 8192, "num_attention_heads": 16, "num_key_value_heads": 4, "head_dim": 128, "vocab_size": 16384,
+           "rms_norm_eps": 1e-5, "tie_word_embeddings": False, "quantization": {"group_size": 64, "bits": 8}}
+    layers = 7 * 2048 * (3072 + 2048 + 3 * 8192)   # weights
+    head = 16384 * 2048
+    knobs("prefill_resident", budget)
+    m = Model(ModelArgs(**cfg), synthetic_checkpoint(cfg, seed=2))
+    m.enable_paged_kv(num_pages=40, max_blocks=2)
+    caches = [m.make_cache() for _ in range(2)]
+    feed = torch.arange(2, dtype=torch.int32, device="cuda")
+    torch.cuda.synchronize()
+    free = [torch.cuda.mem_get_info()[0]]
+    m.step_batch(feed, caches, graph=False)
+    torch.cuda.synchronize()
+    free.append(torch.cuda.mem_get_info()[0])
+    m.step(torch.arange(100, dtype=torch.int32, device="cuda"), m.make_cache())
+    torch.cuda.synchronize()
+    free.append(torch.cuda.mem_get_info()[0])
+    steps, prompt = free[0] - free[1], free[1] - free[2]
+    if copies:   # (tiles and scratch would be 0.6 GiB; what the prompt takes beside is its own scratch)
+        assert steps >= 2 * (layers + head)
+    else:   # (the last layer's o_proj, gate|up and down have one row left and take tiles, which are there)
+        assert 1.0625 * (layers + head) <= steps < 1.6 * (layers + head) and prompt >= 2 * layers * 6 // 7
