@@ -824,8 +824,7 @@ static int linear_rows(pie_decoder *d, const void *packed, int N, int K, const u
         if (rc || !bias || bias_done) return rc;
         return bias_rows<T>(y, bias, M, N, st);
     };
-    // Three to 16 rows (8 of a narrow matrix): the scales on the sums.  One and two of a pass of up to five go to the GEMV below (batch_fused), the one that a longer pass leaves to its last layer to
-    // k_w4r_gemm, as the pass's other rows do: gate|up and down of Llama-3-8B 15.5 us each there, 17.1 here, where down has nobody to sum its splits.
+    // Three to 16 rows (8 of a narrow matrix): the scales on the sums.  One and two go to the GEMV below, as a step's do (batch_fused), also the one that a longer pass leaves to its last layer.
     if (is_int4 && w4a_serves(M, N, K) && M > GEMV_FUSED_ROWS) {
         void *wm = nullptr;
         const int rc = w4m_tiles(&wm);
@@ -840,9 +839,14 @@ static int linear_rows(pie_decoder *d, const void *packed, int N, int K, const u
         if (wm) return tiles_gemm(wm, true);
     }
     // Below 6 rows MLX multiplies row by row (qmv: exact fp32 per row, mx.quantized_matmul as reached from nn.QuantizedLinear): the
-    // streaming GEMV with the rows' images side by side -- one pass over the weights, each row with the batch-1 arithmetic.
-    if (is_int4 && qmv && K % 64 == 0 && N % 2 == 0 && gemv_rows_lds_bytes(K, 1) <= 160u * 1024u)
+    // streaming GEMV with the rows' images side by side -- one pass over the weights, each row with the batch-1 arithmetic.  One or two rows of any pass are cheapest there: four
+    // layers, 37 rows behind 900, us, the last layer's row in k_w4r_gemm / k_w4a_gemm / here: Llama-3-8B 386 / 386 / 371, Llama-3.2-3B 298 / 304 / 294 (16 rows 262 / 273 / 265: down has nobody to sum
+    // its splits, which costs the first a launch of its own and the second the splits).
+    const bool last_rows = !qmv && M <= GEMV_FUSED_ROWS && w4r_serves(M, N, K);
+    if (is_int4 && (qmv || last_rows) && K % 64 == 0 && N % 2 == 0 && gemv_rows_lds_bytes(K, 1) <= 160u * 1024u) {
+        PIE_REQUIRE(!last_rows || pie_aligned(bias, 16), PIE_E_ALIGN, "a prompt's last rows: a Linear's bias needs 16-byte alignment");
         return w4s_gemv_rows_launch(d->cfg.dtype, packed, N, K, x, M, y, (const u16 *)bias, st);
+    }
     // Up to 256 rows (a chat turn behind a cached prefix, a prompt chunk, a multi-sequence step): the weight-streaming MFMA GEMM, every CU
     // streaming its slab of W4M tiles once (w4r_gemm.hpp).
     if (is_int4 && w4r_serves(M, N, K)) {

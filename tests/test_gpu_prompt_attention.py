@@ -227,21 +227,23 @@ def test_the_last_layer_of_a_prompt_takes_its_last_row_alone(bits, layers):
         assert_vec_close(logits[i], alone[i], "bfloat16", what=f"prompt {i} of a batch")
 
 
-@pytest.mark.parametrize("layers", [1, 2])
-@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
-def test_the_last_row_alone_is_multiplied_as_the_rows_are(dtype, layers):
-    """Int4 prompts of 17 to 56 tokens: the row that the last layer goes on with takes the kernels, splits and sums that all of them take in the pass that returns every position's logits: the same bits."""
+@pytest.mark.parametrize("n", [6, 17, 40, 300])
+def test_the_last_row_alone_goes_to_the_gemv(n):
+    """Int4 prompts: the products of the row that the last layer goes on with (o_proj, gate|up, down), and the head's, by the kernels' names."""
+    from torch.profiler import ProfilerActivity, profile
     from proxy_inference_engine_amd.models.llama import Model, ModelArgs
     from proxy_inference_engine_amd.models.utils import synthetic_checkpoint
-    cfg = {"model_type": "llama", "hidden_size": 512, "num_hidden_layers": layers, "intermediate_size": 2048, "num_attention_heads": 8, "num_key_value_heads": 2, "head_dim": 64, "vocab_size": 320,
+    cfg = {"model_type": "llama", "hidden_size": 512, "num_hidden_layers": 1, "intermediate_size": 2048, "num_attention_heads": 8, "num_key_value_heads": 2, "head_dim": 64, "vocab_size": 320,
            "rms_norm_eps": 1e-5, "tie_word_embeddings": False, "quantization": {"group_size": 64, "bits": 4}}
-    m = Model(ModelArgs(**cfg), synthetic_checkpoint(cfg, seed=7, dtype=dtype))
-    ids = torch.from_numpy(np.random.default_rng(3).integers(0, 320, 56).astype(np.int32)).cuda()
-    for n in (17, 32, 33, 56):
-        m(ids[None, :n], cache=m.make_cache())
-        want = m.hidden.clone()
-        m.step(ids[:n], m.make_cache())
-        assert torch.equal(m.hidden, want), n
+    m = Model(ModelArgs(**cfg), synthetic_checkpoint(cfg, seed=7))
+    ids = torch.from_numpy(np.random.default_rng(3).integers(0, 320, n).astype(np.int32)).cuda()
+    m.step(ids, m.make_cache())
+    torch.cuda.synchronize()
+    with profile(activities=[ProfilerActivity.CUDA]) as p:
+        m.step(ids, m.make_cache())
+        torch.cuda.synchronize()
+    names = [(e.key, e.count) for e in p.key_averages()]
+    assert sum(c for k, c in names if "k_w4s_gemv" in k) == 4 and sum(c for k, c in names if "k_w4a_gemm" in k or "k_w4r_gemm" in k or "k_w4l2_gemm" in k) == 1, names
 
 
 @pytest.mark.parametrize("n", [40, 150])
