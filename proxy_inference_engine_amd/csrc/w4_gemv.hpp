@@ -1119,7 +1119,7 @@ int w4s_gemv_launch(int dtype, int pro, int epi, GemvArgs &a, int M, hipStream_t
 int w4s_gemv_waves(int N, int K);
 // y[M, N] = T(x[M, K] @ W^T) (+ bias) for 1 <= M <= GEMV_ROWS_MAX rows of one W4S matrix in one pass over the weights (see k_w4s_gemv_rows)
 constexpr int GEMV_ROWS_MAX = 5;
-constexpr int GEMV_FUSED_ROWS = 2;  // rows of an int4 pass that it takes where k_w4a_gemm is there for more
+constexpr int GEMV_FUSED_ROWS = 2;  // int4 rows that it takes where k_w4a_gemm is there for more
 int w4s_gemv_rows_launch(int dtype, const void *packed, int N, int K, const u16 *x, int M, u16 *y, const u16 *lin_bias, hipStream_t stream);
 // the fused forms (pro: PRO_NONE / PRO_RMSNORM; epi: EPI_STORE / EPI_RESIDUAL / EPI_SWIGLU / EPI_ROPE_KV / EPI_LOGITS): w, K, N, M and the operands of the
 // chosen prologue / epilogue set by the caller

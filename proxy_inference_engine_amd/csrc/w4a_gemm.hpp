@@ -1,4 +1,4 @@
-// w4a_gemm.hpp -- int4 g=64 x T GEMM for up to 16 rows with the scales and biases applied to the sums: y = sum over groups of s (q . x) + b sum(x), the weights never rounded to T
+// w4a_gemm.hpp -- int4 (int8) g=64 x T GEMM for 3 to 16 (1 to 32) rows with the scales and biases applied to the sums: y = sum over groups of s (q . x) + b sum(x), the weights never rounded to T
 // (mx.quantized_matmul's row-by-row arithmetic: models/llama/language.py:83,108,127).  (Included by w4m_gemm.hip.)
 //
 // k_w4r_gemm turns every weight into T in front of its product, 17 vector instructions per eight of them, and its waves wait for each other at every step for the x that they share.  For a
@@ -9,7 +9,10 @@
 //   * a workgroup takes `halves` half strips of 16 columns, so that 1792 of them are seven for each CU (896 strips: four for 224 CUs); the lanes of the other half of a strip load nothing.
 // us, k_w4r_gemm / this, weights from HBM, 8 rows: gate|up [28672, 4096] 19.0 / 16.4-17.6, down [4096, 14336] 11.9 / 11.4, q|k|v [6144, 4096] 7.3 / 6.8, o [4096, 4096] 5.65 / 5.2, head [32768, 4096]
 // 20.5 / 19.1; [16384, 3072] 10.9 / 9.8, [3072, 8192] 7.3 / 6.6, [3072, 3072] 5.3 / 4.6.  16 rows: 18.5 / 16.2-17.6, 11.3 / 11.1, 7.0 / 7.4, 5.65 / 6.0, 21.1 / 18.8; 32 rows: 19.1 / 19.8 and
-// worse.  What is left is the stream: 15 us of gate|up's without the products (5.4 TB/s and a launch).  Deeper rings were slower.
+// worse.  Without the products gate|up takes 15 us (5.4 TB/s and a launch): 2 us are not hidden.
+// The ring is less deep than written.  The compiler does not count the DMAs, so in front of a weight's use it lets no more loads be in flight, x among them, than (D - 1) steps have of weights: one strip
+// of 8 rows 9 and 8 instead of 12, of 16 rows 9 and 8 instead of 16 (two steps, not four), int8 of 32 rows 11 to 9 instead of 21.  Strict, never too weak; but that deeper rings were slower and that
+// int4 of 32 rows is better off elsewhere was measured with it.
 // Error (2-norm, before the rounding to T) against 64 bits: 9e-7; of weights rounded to bf16 1.7e-3.
 #pragma once
 
