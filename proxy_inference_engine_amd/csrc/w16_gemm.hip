@@ -122,12 +122,13 @@ static W16Plan w16_plan(int M, int N, int K, bool no_split = false) {
     best.S = w16_even_splits(groups, best.S);
     return best;
 }
-// Of one pass over K (the forms with an activation: w16_grouped.hip).  From two rounds of the largest tile on that one: the model counts whole rounds, which overlap, and its smaller tiles fetch more for the same
-// time ([28672, 4096], 2000 rows: 423.5 us in 1792 workgroups, 422.5 in 896; the prompt around it 5571-5533 us, 5512).  Rows that fill no more than half of it stay with the plan's
-// (four layers with an MLP [131072, 2048], 65 / 100 / 128 rows: 1539 / 1559 / 1604 us on the largest tile, 1447 / 1434 / 1477).
+// Of one pass over K (the forms with an activation: w16_grouped.hip).  From two rounds of the largest tile that the rows fill by more than half on that one: the model counts whole rounds, which overlap, and its smaller tiles fetch more for the same
+// time ([28672, 4096], 2000 rows: 423.5 us in 1792 workgroups, 422.5 in 896; the prompt around it 5571-5533 us, 5512).  Four layers with an MLP [131072, 2048], us, tiles of 256
+// rows / of the plan / of the rows: 65 rows 1549 / 1447 / 1441, 100 rows 1559 / 1434 / 1448, 33 rows 1647 / 1675 / 1636.
 void w16l_tile(int M, int N, int K, int *mb, int *sw) {
-    if (M > 128 && (long long)((N + 255) / 256) * ((M + 255) / 256) >= 512) {
-        *mb = 8, *sw = 2;
+    const int high = M <= 64 ? 2 : M <= 128 ? 4 : 8;
+    if ((long long)((N + 255) / 256) * ((M + 32 * high - 1) / (32 * high)) >= 512) {
+        *mb = high, *sw = 2;
         return;
     }
     const W16Plan pl = w16_plan(M, N, K, true);
