@@ -804,9 +804,10 @@ static int linear_rows(pie_decoder *d, const void *packed, int N, int K, const u
             *used_act = true;
             return go(act, nullptr, 1, bias, nullptr, nullptr, nullptr);
         }
-        // q|k|v wide enough to fill the chip without a K split: RoPE + append in the epilogue.  Not for a step over T pages of an int8 model, whose attention's launch can rotate as well
-        // (24 layers of hidden 1024, 2 / 6 / 32 rows, us a step: 803 / 930 / 1138 rotated here, 755 / 811 / 1050 there).
-        const bool rotates = rope && used_act && !(is_int8 && rope->slab && !rope->i8_page_bytes);
+        // q|k|v wide enough to fill the chip without a K split: RoPE + append in the epilogue.  Not from k_w4a_gemm for a step over T pages: its attention's launch can rotate as
+        // well (int8, 24 layers of hidden 1024, 2 / 6 / 32 rows, us a step: 803 / 930 / 1138 rotated here, 755 / 811 / 1050 there; int4, 16 layers
+        // of Llama-3-70B, 3 / 8 rows, 2222 / 2316 and 2098 / 2182).
+        const bool rotates = rope && used_act && !(affine && rope->slab && !rope->i8_page_bytes);
         if (rotates && (affine ? w4a_splits(M, N, K, bits) : w4r_splits(M, N, K)) == 1) {
             *used_act = true;
             rope->bias = (const u16 *)bias;

@@ -45,16 +45,17 @@ def test_rows_against_single_sequences(hidden, inter, vocab, heads, kv, dim, bia
         cache[0].page_manager.release()
 
 
-def test_a_step_over_pages_rotates_in_its_attention():
+@pytest.mark.parametrize("bits,rows", [(8, 2), (4, 3), (4, 8)])
+def test_a_step_over_pages_rotates_in_its_attention(bits, rows):
     """Up to 1024 columns (q|k|v in one pass over K): the product could rotate, but the attention's launch does it for less.  The kernels of one step, by name."""
     from torch.profiler import ProfilerActivity, profile
     from proxy_inference_engine_amd.models.llama import Model, ModelArgs
     from proxy_inference_engine_amd.models.utils import synthetic_checkpoint
     cfg = {"model_type": "llama", "hidden_size": 1024, "num_hidden_layers": 2, "intermediate_size": 512, "num_attention_heads": 8, "num_key_value_heads": 4, "head_dim": 128, "vocab_size": 320,
-           "rms_norm_eps": 1e-5, "tie_word_embeddings": False, "quantization": {"group_size": 64, "bits": 8}}
+           "rms_norm_eps": 1e-5, "tie_word_embeddings": False, "quantization": {"group_size": 64, "bits": bits}}
     m = Model(ModelArgs(**cfg), synthetic_checkpoint(cfg, seed=2))
-    m.enable_paged_kv(num_pages=8, max_blocks=1)
-    caches, feed = [m.make_cache() for _ in range(2)], torch.arange(2, dtype=torch.int32, device="cuda")
+    m.enable_paged_kv(num_pages=16, max_blocks=1)
+    caches, feed = [m.make_cache() for _ in range(rows)], torch.arange(rows, dtype=torch.int32, device="cuda")
     m.step_batch(feed, caches, graph=False)
     torch.cuda.synchronize()
     with profile(activities=[ProfilerActivity.CUDA]) as p:
