@@ -825,7 +825,7 @@ static int linear_rows(pie_decoder *d, const void *packed, int N, int K, const u
         if (rc || !bias || bias_done) return rc;
         return bias_rows<T>(y, bias, M, N, st);
     };
-    // Three to 16 rows (8 of a narrow matrix): the scales on the sums.  One and two go to the GEMV below, as a step's do (batch_fused), also the one that a longer pass leaves to its last layer.
+    // Three to 16 rows: the scales on the sums.  One and two go to the GEMV below, as a step's do (batch_fused), also the one that a longer pass leaves to its last layer.
     if (is_int4 && w4a_serves(M, N, K) && M > GEMV_FUSED_ROWS) {
         void *wm = nullptr;
         const int rc = w4m_tiles(&wm);

@@ -2,17 +2,19 @@
 // (mx.quantized_matmul's row-by-row arithmetic: models/llama/language.py:83,108,127).  (Included by w4m_gemm.hip.)
 //
 // k_w4r_gemm turns every weight into T in front of its product, 17 vector instructions per eight of them, and its waves wait for each other at every step for the x that they share.  For a
-// few rows that is most of its time: gate|up of Llama-3-8B, 66 MB, 19 us for 8 rows; without its products 14, of which 3 are a launch's.  Here
+// few rows that is most of its time.  Here
 //   * the codes are operands as they stand -- bf16: under the exponent of 128, one v_and_or for two, f16: less 1024 -- and a group's products are multiplied by its scale and joined by bias
-//     times the group's sum of x (another product, by ones) in fp32: 2 fused operations per row (of eight) and 32 columns instead of 68;
-//   * a wave's K-phase is its own: it stages the x of its groups itself, by LDS-DMA into a ring of its own, and waits for nothing but its loads;
-//   * a workgroup takes `halves` half strips of 16 columns, so that 1792 of them are seven for each CU (896 strips: four for 224 CUs); the lanes of the other half of a strip load nothing.
-// us, k_w4r_gemm / this, weights from HBM, 8 rows: gate|up [28672, 4096] 19.0 / 16.4-17.6, down [4096, 14336] 11.9 / 11.4, q|k|v [6144, 4096] 7.3 / 6.8, o [4096, 4096] 5.65 / 5.2, head [32768, 4096]
-// 20.5 / 19.1; [16384, 3072] 10.9 / 9.8, [3072, 8192] 7.3 / 6.6, [3072, 3072] 5.3 / 4.6.  16 rows: 18.5 / 16.2-17.6, 11.3 / 11.1, 7.0 / 7.4, 5.65 / 6.0, 21.1 / 18.8; 32 rows: 19.1 / 19.8 and
-// worse.  Without the products gate|up takes 15 us (5.4 TB/s and a launch): 2 us are not hidden.
-// The ring is less deep than written.  The compiler does not count the DMAs, so in front of a weight's use it lets no more loads be in flight, x among them, than (D - 1) steps have of weights: one strip
-// of 8 rows 9 and 8 instead of 12, of 16 rows 9 and 8 instead of 16 (two steps, not four), int8 of 32 rows 11 to 9 instead of 21.  Strict, never too weak; but that deeper rings were slower and that
-// int4 of 32 rows is better off elsewhere was measured with it.
+//     times the group's sum of x (another product, by ones) in fp32;
+//   * products are 16 x 16 x 32: sixteen rows and sixteen columns, the even or the odd ones of a strip (a v_permlane16_swap of two words makes two such operands of a tile's).  Up to eight
+//     rows, rows 8..15 of a product are the same rows against the odd columns (zeros in the others' place), so that no lane of the sums is idle;
+//   * a wave's K-phase is its own: it loads the x of its groups straight into the operand's lanes (a group of eight rows is one load) and waits for nothing but its loads, all of them ordinary
+//     ones, so that the compiler's waits are exact; the scales of a step's four strips are one load.
+// Bound by the stream, a launch (3 us) and the conversion, of which 1.7 us are not hidden.  us, weights from HBM, k_w4r_gemm / the form before (32 x 32 products, x by LDS-DMA, which the compiler's
+// waits do not count: rings shallower than written) / this, 8 rows: gate|up [28672, 4096] 18.0 / 17.0 / 14.0, down [4096, 14336] 11.1 / 10.6 / 8.9, q|k|v [6144, 4096] 7.2 / 6.7 / 6.1, o [4096, 4096]
+// 5.6 / 5.3 / 4.7, head [32768, 4096] 18.3 / 17.6 / 14.7; [16384, 3072] 9.8 / 9.9 / 8.1, [3072, 8192] 7.2 / 6.7 / 6.1.  16 rows: 17.9 / 18.4 / 15.2, 11.4 / 11.2 / 9.4, 7.3 / 7.6 / 6.4,
+// 5.6 / 6.0 / 4.8, 19.8 / 19.5 / 15.7.  32 rows of int4: 18.5 / 19.8 / 21.4, 11.6 / - / 13.0: k_w4r_gemm's.  Without the conversion gate|up takes 12.8 us, without any arithmetic 11.9 to 12.8.
+// Two steps in flight per wave are enough (eight waves of 4.6 KB each); three and four cost 0.3 to 1 us, since the loads past a wave's last step, which return nothing, take their issue slots too (a
+// loop that leaves them out makes the compiler move registers about or wait for all of them: 17.8).
 // Error (2-norm, before the rounding to T) against 64 bits: 9e-7; of weights rounded to bf16 1.7e-3.
 #pragma once
 
@@ -22,7 +24,7 @@ struct W4aArgs {
     const char *w4m;   // W4M (W8M) tiles of the [N, K] matrix
     const u16 *x;      // [M, K]
     int M, N, K;
-    int halves;        // half strips (16 columns) per workgroup
+    int strips;        // strips (32 columns) per workgroup
     int groups;        // of K (64 columns) per blockIdx.y
     u16 *y;            // STORE: [M, N]; SWIGLU: the activation [M, N / 2]
     float *part;       // SLAB: [gridDim.y][M][N] un-rounded fp32 sums
@@ -41,8 +43,8 @@ constexpr float w4a_offset() { return std::is_same<T, F16>::value ? 0.0f : 128.0
 
 // Int8 codes, W8M tiles: as W4M, 32 rows x 64 columns, two pieces of 1 KiB and the 32 {scale, bias} words: lane l = 32 kh + n holds in piece h the codes of row n of k-steps 2 h and 2 h + 1, two words
 // each, in the W8S word format (codes 0, 2, 1, 3).  Up to 255 a code is a bf16 and an f16 as it stands.
-// Bound by the stream; before, two and more rows multiplied a 16-bit copy, twice the bytes.  us of 16 steps of four layers at 200 positions, 16-bit copy / this: Llama-3-8B 2 rows 6924 / 5080, 4 7209 / 5288,
-// 8 7440 / 5474, 16 8042 / 6015, 32 9319 / 6719; Llama-3.2-3B 4 rows 5357 / 3881, 8 5142 / 4033.  Error of a step against 64 bits 0.0095-0.0100 / 0.0089-0.0095.
+// Bound by the stream, half the bytes of a 16-bit copy's.  us, the form with 32 x 32 products / this, 8 rows: gate|up 23.3 / 22.6, down 13.3 / 12.7, q|k|v 8.8 / 7.8, o 6.5 / 5.8, head 24.9 / 24.5; 32 rows: 27.0 / 27.5,
+// 17.1 / 17.1, 12.1 / 10.5, 8.8 / 7.6, 28.4 / 28.5.
 template <class T>
 __device__ __forceinline__ u32 w8a_pair(u32 a, u32 b) {  // two codes as T, b in the high half
     if constexpr (std::is_same<T, F16>::value) return __builtin_bit_cast(u32, __builtin_amdgcn_cvt_pkrtz((float)a, (float)b));
@@ -53,130 +55,175 @@ __device__ __forceinline__ uint4 w8a_codes(u32 lo, u32 hi) {
     return make_uint4(w8a_pair<T>(lo & 0xFFu, (lo >> 16) & 0xFFu), w8a_pair<T>((lo >> 8) & 0xFFu, lo >> 24), w8a_pair<T>(hi & 0xFFu, (hi >> 16) & 0xFFu), w8a_pair<T>((hi >> 8) & 0xFFu, hi >> 24));
 }
 
+typedef __attribute__((ext_vector_type(4))) float w4a_f32x4;
+template <class T>
+__device__ __forceinline__ w4a_f32x4 w4a_mfma(const uint4 &a, const uint4 &b, const w4a_f32x4 &c) {
+    if constexpr (std::is_same<T, F16>::value) return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b), c, 0, 0, 0);
+    else return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
+}
+// lanes 16..31 and 48..63 of a for lanes 0..15 and 32..47 of b
+__device__ __forceinline__ void w4a_swap16(u32 &a, u32 &b) {
+    const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+    a = r[0], b = r[1];
+}
+__device__ __forceinline__ void w4a_swap32(u32 &a, u32 &b) {  // the upper lanes of a for the lower ones of b
+    const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+    a = r[0], b = r[1];
+}
+// lanes 0..7 of every 16 (LOW: for themselves, else 8..15) to lanes AT .. + 7, the others zero
+template <bool LOW, int AT>
+__device__ __forceinline__ u32 w4a_eight(u32 v) {
+    constexpr int from = LOW ? 0 : 8, ctrl = from == AT ? 0xE4 : 0x128;  // quad_perm 0 1 2 3 / row_ror:8
+    return (u32)__builtin_amdgcn_update_dpp(0, (int)v, ctrl, 0xF, AT ? 0xC : 0x3, false);
+}
+template <bool LOW, int AT>
+__device__ __forceinline__ uint4 w4a_eight(const uint4 &v) { return make_uint4(w4a_eight<LOW, AT>(v.x), w4a_eight<LOW, AT>(v.y), w4a_eight<LOW, AT>(v.z), w4a_eight<LOW, AT>(v.w)); }
+
 template <class T, int MT, int SPW, int D, int BITS = 4>
 __global__ void __launch_bounds__(512) k_w4a_gemm(const W4aArgs a, const W4mRope rp) {
     constexpr int PC = BITS / 4, TILE = BITS == 8 ? W8M_TILE_BYTES : W4M_TILE_BYTES;  // code pieces (16 bytes a lane) of a tile; bytes of one
-    constexpr int KW = 8, XJ = MT / 8, WL = (PC + 1) * SPW, CHUNK = MT * 128;  // K-phases = waves; DMA instructions (eight rows of a group each), weight loads per step; bytes of x of a step
-    constexpr int RL = MT / 2;                                  // accumulators that hold rows < MT
+    constexpr int KW = 8, RB = (MT + 15) / 16;                  // K-phases = waves; blocks of 16 rows
+    constexpr bool PAIR = MT == 8;                              // rows 8..15 of a product: the strip's odd columns
+    constexpr int XL = PAIR ? 1 : 2 * RB;                       // loads of x per step, 1 KiB each
+    constexpr int AC = PAIR ? 1 : 2 * RB;                       // accumulators of a strip: [block][even, odd columns]
     constexpr int RSTR = 36, BLK = MT * RSTR * 4;               // reduction: one (phase, strip) block, rows of 32 + 4 floats
-    constexpr int RED = KW * SPW * BLK, LDS = KW * D * CHUNK > RED ? KW * D * CHUNK : RED;
     constexpr unsigned NOWHERE = 0x80000000u;
-    static_assert((D - 1) * (XJ + WL) <= 63 && LDS <= 160 * 1024, "limits");
-    __shared__ __attribute__((aligned(1024))) char smem[LDS];
+    static_assert(SPW <= 4 && D * (XL + 1 + SPW * PC) <= 63, "a strip to 16 lanes of the scales' load; loads in flight");
+    __shared__ __attribute__((aligned(16))) char smem[KW * SPW * BLK];
     const int lane = threadIdx.x & 63, p = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int n = lane & 31, kh = lane >> 5;
-    const int all_groups = a.K >> 6, n_halves = a.N >> 4;
+    const int c16 = lane & 15, r16 = lane >> 4;
+    const int all_groups = a.K >> 6;
     const int g_lo = blockIdx.y * a.groups + p, g_hi = min(all_groups, ((int)blockIdx.y + 1) * a.groups);  // this wave's groups: g_lo, g_lo + 8, ..
     const int steps = g_hi > g_lo ? (g_hi - g_lo + KW - 1) / KW : 0;
-    const int h0 = blockIdx.x * a.halves, h1 = min(h0 + a.halves, n_halves), strip0 = h0 >> 1;
+    const int strip0 = blockIdx.x * a.strips, n_strips = min(a.strips, (a.N >> 5) - strip0);
     const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>(a.w4m), 0, (a.N >> 5) * all_groups * TILE, 0x00020000);
-    unsigned code_at[SPW], scale_at[SPW], strip_at[SPW];
+    const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<u16 *>(a.x), 0, a.M * a.K * 2, 0x00020000);
+    // lanes by 16: the even and the odd columns' codes of a k-step's first eight numbers, of its other eight; the scales of strips 0 .. 3, an even and an odd column's
+    const unsigned code_at = 16u * (32 * (r16 >> 1) + 2 * c16 + (r16 & 1)), scale_at = r16 < n_strips ? (unsigned)(r16 * all_groups * TILE) + 1024u * PC + 8u * c16 : NOWHERE;
+    unsigned strip_at[SPW], gone[SPW];
 #pragma unroll
-    for (int s = 0; s < SPW; ++s) {
-        const int h = 2 * (strip0 + s) + (n >> 4);
-        const bool mine = h >= h0 && h < h1;  // (the strips at both ends may be another workgroup's by half)
-        code_at[s] = mine ? 16u * lane : NOWHERE, scale_at[s] = mine ? 1024u * PC + 4u * n : NOWHERE;
-        strip_at[s] = (unsigned)((strip0 + s) * all_groups + g_lo) * TILE;
-    }
-    u32 xoffs[XJ];
+    for (int s = 0; s < SPW; ++s) strip_at[s] = (unsigned)((strip0 + s) * all_groups + g_lo) * TILE, gone[s] = s < n_strips ? 0u : NOWHERE;
+    // A product takes 32 columns of x: runs of eight 0, 2, 1, 3 of one half of a group (as the tile's words lie), a run to 16 lanes.  PAIR: the lanes of rows 8..15 load the group's other half
+    unsigned x_at[RB];
 #pragma unroll
-    for (int j = 0; j < XJ; ++j) {
-        const int r = 8 * j + (lane >> 3), rr = r < a.M ? r : a.M - 1;  // rows past the end repeat the last one (never stored)
-        xoffs[j] = (u32)(((size_t)rr * a.K + (size_t)(((lane & 7) ^ ((r >> 1) & 7)) * 8)) * 2);
+    for (int t = 0; t < RB; ++t) {
+        const int r = PAIR ? c16 & 7 : 16 * t + c16;
+        x_at[t] = r < a.M ? (unsigned)(r * a.K + 16 * (r16 & 1) + 8 * (r16 >> 1) + (PAIR ? 32 * (c16 >> 3) : 0)) * 2u : NOWHERE;  // (rows past the end are zeros)
     }
-    const unsigned lds0 = (unsigned)(size_t)(__attribute__((address_space(3))) void *)smem + (unsigned)(p * D * CHUNK);
     typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
-    uint4 cw[D][SPW][PC];
-    u32 sb[D][SPW];
+    typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+    uint4 xv[D][XL], cw[D][SPW][PC];
+    u32x2 sb[D];
     auto issue = [&](int d, int j) {
-        const char *src = reinterpret_cast<const char *>(a.x) + (size_t)(g_lo + (j < steps ? j : steps - 1) * KW) * 128;
+        const unsigned dead = j < steps ? 0u : NOWHERE, o = (unsigned)j * (KW * TILE), xo = (unsigned)(g_lo + j * KW) * 128u;
 #pragma unroll
-        for (int i = 0; i < XJ; ++i) {
-            unsigned keep;
-            asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0"
-                         : "=&s"(keep)
-                         : "v"(xoffs[i]), "s"(src), "s"(lds0 + (unsigned)(d * CHUNK + i * 1024))
-                         : "memory");
+        for (int t = 0; t < XL; ++t) {
+            const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(xr, (x_at[PAIR ? 0 : t >> 1] | dead) + 64u * (t & 1), xo, 0);
+            xv[d][t] = make_uint4(v.x, v.y, v.z, v.w);
         }
-        const unsigned o = (unsigned)j * (KW * TILE), dead = j < steps ? 0u : NOWHERE;
+        sb[d] = __builtin_amdgcn_raw_buffer_load_b64(wr, scale_at | dead, strip_at[0] + o, 2);
 #pragma unroll
-        for (int s = 0; s < SPW; ++s) {
+        for (int s = 0; s < SPW; ++s)
 #pragma unroll
             for (int q = 0; q < PC; ++q) {
-                const u32x4 c = __builtin_amdgcn_raw_buffer_load_b128(wr, (code_at[s] | dead) + 1024u * q, strip_at[s] + o, 2);
+                const u32x4 c = __builtin_amdgcn_raw_buffer_load_b128(wr, (code_at | gone[s] | dead) + 1024u * q, strip_at[s] + o, 2);
                 cw[d][s][q] = make_uint4(c.x, c.y, c.z, c.w);
             }
-            sb[d][s] = __builtin_amdgcn_raw_buffer_load_b32(wr, scale_at[s] | dead, strip_at[s] + o, 2);
-        }
+        __builtin_amdgcn_sched_barrier(0);  // (the loads stay in the order that the compiler's counted waits rely on)
     };
     if (steps > 0)
 #pragma unroll
         for (int d = 0; d < D; ++d) issue(d, d);
-    int xoff[4];
-    const int xrow = n & (MT - 1);
-#pragma unroll
-    for (int kk = 0; kk < 4; ++kk) xoff[kk] = p * D * CHUNK + xrow * 128 + (((2 * kk + kh) ^ ((xrow >> 1) & 7)) << 4);
-    float acc[SPW][RL];
+    const w4a_f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+    w4a_f32x4 acc[SPW][AC];
 #pragma unroll
     for (int s = 0; s < SPW; ++s)
 #pragma unroll
-        for (int i = 0; i < RL; ++i) acc[s][i] = 0.0f;
+        for (int i = 0; i < AC; ++i) acc[s][i] = zero;
     const u32 one = std::is_same<T, F16>::value ? 0x3C003C00u : 0x3F803F80u;
     const uint4 ones = make_uint4(one, one, one, one);
-    const f32x16_t zero = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
     for (int base = 0; base < steps; base += D) {
 #pragma unroll
         for (int d = 0; d < D; ++d) {
             if (base + d < steps) {
-                W4R_WAIT_VM((D - 1) * (XJ + WL));
-                uint4 xq[4];
+                uint4 xa[PAIR ? 4 : XL];  // PAIR: the group's halves as rows 0..7, as rows 8..15
+                if constexpr (PAIR) xa[0] = w4a_eight<true, 0>(xv[d][0]), xa[1] = w4a_eight<false, 0>(xv[d][0]), xa[2] = w4a_eight<true, 8>(xv[d][0]), xa[3] = w4a_eight<false, 8>(xv[d][0]);
+                else
 #pragma unroll
-                for (int kk = 0; kk < 4; ++kk) xq[kk] = *reinterpret_cast<const uint4 *>(smem + d * CHUNK + xoff[kk]);
-                f32x16_t xs = zero;
+                    for (int t = 0; t < XL; ++t) xa[t] = xv[d][t];
+                w4a_f32x4 xs[RB];
 #pragma unroll
-                for (int kk = 0; kk < 4; ++kk) xs = MfmaT<T>::run(xq[kk], ones, kk ? xs : zero);
+                for (int t = 0; t < RB; ++t) xs[t] = w4a_mfma<T>(xa[2 * t + 1], ones, w4a_mfma<T>(xa[2 * t], ones, zero));
+                if constexpr (PAIR) xs[0] = w4a_mfma<T>(xa[3], ones, w4a_mfma<T>(xa[2], ones, xs[0]));
+                u32 sw[4][2];  // every lane's scale word of a strip's even, of its odd column; PAIR: the one of the rows that it sums
+                {
+                    u32 e0 = sb[d].x, e1 = sb[d].x, o0 = sb[d].y, o1 = sb[d].y;
+                    w4a_swap16(e0, e1), w4a_swap16(o0, o1);  // strips 0 0 2 2, 1 1 3 3
+                    if constexpr (PAIR) {
+                        w4a_swap32(e0, o0), w4a_swap32(e1, o1);
+                        sw[0][0] = e0, sw[2][0] = o0, sw[1][0] = e1, sw[3][0] = o1;
+                    } else {
+                        sw[0][0] = sw[2][0] = e0, sw[1][0] = sw[3][0] = e1, sw[0][1] = sw[2][1] = o0, sw[1][1] = sw[3][1] = o1;
 #pragma unroll
-                for (int s0 = 0; s0 < SPW; s0 += 2) {
-                    f32x16_t dot[2];
+                        for (int s = 0; s < 2; ++s) w4a_swap32(sw[s][0], sw[s + 2][0]), w4a_swap32(sw[s][1], sw[s + 2][1]);
+                    }
+                }
 #pragma unroll
-                    for (int kk = 0; kk < 4; ++kk)
+                for (int s = 0; s < SPW; ++s) {
+                    float sc[2], bi[2];
 #pragma unroll
-                        for (int s = s0; s < s0 + 2 && s < SPW; ++s) {
-                            uint4 wf;
-                            if constexpr (BITS == 8) {
-                                const uint4 &c = cw[d][s][kk >> 1];
-                                wf = kk & 1 ? w8a_codes<T>(c.z, c.w) : w8a_codes<T>(c.x, c.y);
-                            } else {
-                                const uint4 &c = cw[d][s][0];
-                                wf = w4a_codes<T>(kk == 0 ? c.x : (kk == 1 ? c.y : (kk == 2 ? c.z : c.w)));
-                            }
-                            dot[s - s0] = MfmaT<T>::run(xq[kk], wf, kk ? dot[s - s0] : zero);
+                    for (int h = 0; h < (PAIR ? 1 : 2); ++h) sc[h] = lo_f32<T>(sw[s][h]), bi[h] = BITS == 8 ? hi_f32<T>(sw[s][h]) : fmaf(-w4a_offset<T>(), sc[h], hi_f32<T>(sw[s][h]));
+                    uint4 wf[2][2];  // [even, odd columns][half of the group]
+                    if constexpr (BITS == 8) {
+#pragma unroll
+                        for (int h = 0; h < 2; ++h) {
+                            uint4 c = cw[d][s][h];
+                            w4a_swap16(c.x, c.z), w4a_swap16(c.y, c.w);
+                            wf[0][h] = w8a_codes<T>(c.x, c.y), wf[1][h] = w8a_codes<T>(c.z, c.w);
                         }
+                    } else {
+                        uint4 c = cw[d][s][0];
+                        w4a_swap16(c.x, c.y), w4a_swap16(c.z, c.w);
+                        wf[0][0] = w4a_codes<T>(c.x), wf[1][0] = w4a_codes<T>(c.y), wf[0][1] = w4a_codes<T>(c.z), wf[1][1] = w4a_codes<T>(c.w);
+                    }
+                    if constexpr (PAIR) {
+                        w4a_f32x4 dot = w4a_mfma<T>(xa[1], wf[0][1], w4a_mfma<T>(xa[0], wf[0][0], zero));
+                        dot = w4a_mfma<T>(xa[3], wf[1][1], w4a_mfma<T>(xa[2], wf[1][0], dot));
 #pragma unroll
-                    for (int s = s0; s < s0 + 2 && s < SPW; ++s) {
-                        const float sc = lo_f32<T>(sb[d][s]), bi = BITS == 8 ? hi_f32<T>(sb[d][s]) : fmaf(-w4a_offset<T>(), sc, hi_f32<T>(sb[d][s]));
+                        for (int i = 0; i < 4; ++i) acc[s][0][i] = fmaf(bi[0], xs[0][i], fmaf(sc[0], dot[i], acc[s][0][i]));
+                    } else {
 #pragma unroll
-                        for (int i = 0; i < RL; ++i) acc[s][i] = fmaf(bi, xs[i], fmaf(sc, dot[s - s0][i], acc[s][i]));
+                        for (int t = 0; t < RB; ++t)
+#pragma unroll
+                            for (int h = 0; h < 2; ++h) {
+                                const w4a_f32x4 dot = w4a_mfma<T>(xa[2 * t + 1], wf[h][1], w4a_mfma<T>(xa[2 * t], wf[h][0], zero));
+#pragma unroll
+                                for (int i = 0; i < 4; ++i) acc[s][2 * t + h][i] = fmaf(bi[h], xs[t][i], fmaf(sc[h], dot[i], acc[s][2 * t + h][i]));
+                            }
                     }
                 }
             }
             __builtin_amdgcn_sched_barrier(0);
             issue(d, base + d + D);
-            __builtin_amdgcn_sched_barrier(0);
         }
     }
-    W4R_WAIT_VM(0);  // (the DMAs past the end)
-    __syncthreads();
-    // accumulator i of lane (n, kh): row (i & 3) + 8 (i >> 2) + 4 kh, column n
+    // a product's lane: columns 2 c16 (+ 1), rows 4 r16 .. + 3
 #pragma unroll
     for (int s = 0; s < SPW; ++s)
 #pragma unroll
-        for (int i = 0; i < RL; ++i) *reinterpret_cast<float *>(smem + (p * SPW + s) * BLK + (((i & 3) + 8 * (i >> 2) + 4 * kh) * RSTR + n) * 4) = acc[s][i];
+        for (int t = 0; t < RB; ++t)
+#pragma unroll
+            for (int h = 0; h < (PAIR ? 1 : 2); ++h)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int row = 4 * r16 + i, m = PAIR ? row & 7 : 16 * t + row, col = 2 * c16 + (PAIR ? row >> 3 : h);
+                    *reinterpret_cast<float *>(smem + (p * SPW + s) * BLK + (m * RSTR + col) * 4) = acc[s][PAIR ? 0 : 2 * t + h][i];
+                }
     __syncthreads();
     const int EPI = a.epi;
     for (int o = threadIdx.x; o < MT * SPW * 4; o += 512) {  // a row's eight columns
-        const int m = o / (4 * SPW), ts = (o >> 2) % SPW, ec = o & 3, col = 32 * (strip0 + ts) + 8 * ec, h = col >> 4;
-        if (m >= a.M || h < h0 || h >= h1) continue;
+        const int m = o / (4 * SPW), ts = (o >> 2) % SPW, ec = o & 3, col = 32 * (strip0 + ts) + 8 * ec;
+        if (m >= a.M || ts >= n_strips) continue;
         float v[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int ph = 0; ph < KW; ++ph) {

@@ -810,50 +810,38 @@ int w8m_repack_launch(const void *w8s, int N, int K, void *w8m, hipStream_t st) 
     PIE_LAUNCH_CHECK();
     return PIE_OK;
 }
-// Up to 16 rows with the scales on the sums (k_w4a_gemm).  Workgroups: of as many half strips as give every CU one (at most eight); what stays below 1024 half strips takes four and splits of
-// K, in one round of workgroups and of at least two steps: q|k|v two splits, o_proj and down four (8 rows, four half strips in two / four / seven splits, two in two: q|k|v 6.8 / 7.6 / - / 7.3 us,
-// o_proj - / 5.2 / - / 5.2, down - / 11.4 / 11.2 / 12.2, [3072, 8192] - / 6.6 / - / 7.6).  Beyond eight rows only what needs no splits: there k_w4r_gemm is as good or better at the others.
+// Up to 16 rows (32 of int8 codes) with the scales on the sums (k_w4a_gemm).  Workgroups of as many strips as give every CU one (at most four: 896 strips in 224 workgroups 14.0 us, two strips each 15.4,
+// three 19.1; 640 in threes 11.5, in twos 14.9, in fours 13.0; 384 in twos 9.2, one by one 10.9; 352 of 2048 columns in twos 6.3, one by one 7.2); what stays below 512 strips takes two and splits of K, in one round of
+// workgroups and of at least two steps: q|k|v two splits, o_proj and down four (8 rows, two strips in splits / one strip in half as many: q|k|v 6.1 / 7.1 us, o_proj 4.7 / 5.1, [3072, 8192] 6.1 / 7.0, [8192, 4096] 6.6 / 7.4).
 struct W4aPlan {
-    int halves, S, groups;  // half strips per workgroup; K splits, groups of each; halves == 0: shape not served
+    int strips, S, groups;  // strips per workgroup; K splits, groups of each; strips == 0: shape not served
 };
-// Int8 codes (bits == 8): up to 32 rows, narrow matrices in the same splits: the other form reads 16 bits a weight (32 rows 9319 / 6719 us, w4a_gemm.hpp).
 static W4aPlan w4a_plan(int M, int N, int K, bool may_split, int bits) {
     if (M < 1 || M > (bits == 8 ? W8A_ROWS : W4A_ROWS) || N < 32 || N % 32 || K < 64 || K % 64 || (bits == 8 ? w8m_bytes(N, K) : w4m_bytes(N, K)) >= (1ull << 31)) return {0, 0, 0};
-    const int units = N / 16, groups = K / 64, steps = (groups + 7) / 8;
-    if (bits == 4 && M > 8 && units < 1024) return {0, 0, 0};
-    const int halves = units >= 2048 ? 8 : (units + 255) / 256;
-    if (units >= 1024 || !may_split) return {halves, 1, 8 * steps};
-    const int wgs = (units + 3) / 4;
+    const int strips = N / 32, groups = K / 64, steps = (groups + 7) / 8;
+    const int each = strips >= 1024 ? 4 : (strips + 255) / 256;
+    if (strips >= 512 || !may_split) return {each, 1, 8 * steps};
+    const int wgs = (strips + 1) / 2;
     int S = 1;
     for (int n = 2; n <= 8 && n * wgs <= 256; ++n)
         if (steps % n == 0 && steps / n >= 2) S = n;
-    if (S == 1) return {halves, 1, 8 * steps};
-    return {4, S, 8 * (steps / S)};
+    if (S == 1) return {each, 1, 8 * steps};
+    return {2, S, 8 * (steps / S)};
 }
-bool w4a_serves(int M, int N, int K, int bits) { return pie_knob(PIE_KNOB_W4R) != 0 && w4a_plan(M, N, K, false, bits).halves != 0; }
+bool w4a_serves(int M, int N, int K, int bits) { return pie_knob(PIE_KNOB_W4R) != 0 && w4a_plan(M, N, K, false, bits).strips != 0; }
 int w4a_splits(int M, int N, int K, int bits) { return w4a_plan(M, N, K, true, bits).S; }
 size_t w4a_workspace_bytes(int M, int N, int K, int bits) {
     const int s = w4a_splits(M, N, K, bits);
     return s > 1 ? (size_t)s * M * N * sizeof(float) : 0;
 }
-template <class T, int MT>
+template <class T, int MT, int BITS>
 static void w4a_go(const W4aArgs &a, int S, hipStream_t st, const W4mRope &r) {
-    const dim3 grid((unsigned)((a.N / 16 + a.halves - 1) / a.halves), (unsigned)S), block(512);
-    switch ((a.halves + 1) / 2) {  // (rings of two steps and more: 8 KB and more of weights per wave)
-    case 1: hipLaunchKernelGGL((k_w4a_gemm<T, MT, 1, 5>), grid, block, 0, st, a, r); break;
-    case 2: hipLaunchKernelGGL((k_w4a_gemm<T, MT, 2, 4>), grid, block, 0, st, a, r); break;
-    case 3: hipLaunchKernelGGL((k_w4a_gemm<T, MT, 3, 3>), grid, block, 0, st, a, r); break;
-    default: hipLaunchKernelGGL((k_w4a_gemm<T, MT, 4, 2>), grid, block, 0, st, a, r); break;
-    }
-}
-template <class T, int MT>
-static void w8a_go(const W4aArgs &a, int S, hipStream_t st, const W4mRope &r) {
-    const dim3 grid((unsigned)((a.N / 16 + a.halves - 1) / a.halves), (unsigned)S), block(512);
-    switch ((a.halves + 1) / 2) {  // (half as many steps in flight as int4's: as many bytes)
-    case 1: hipLaunchKernelGGL((k_w4a_gemm<T, MT, 1, 4, 8>), grid, block, 0, st, a, r); break;
-    case 2: hipLaunchKernelGGL((k_w4a_gemm<T, MT, 2, 3, 8>), grid, block, 0, st, a, r); break;
-    case 3: hipLaunchKernelGGL((k_w4a_gemm<T, MT, 3, 2, 8>), grid, block, 0, st, a, r); break;
-    default: hipLaunchKernelGGL((k_w4a_gemm<T, MT, 4, 2, 8>), grid, block, 0, st, a, r); break;
+    const dim3 grid((unsigned)((a.N / 32 + a.strips - 1) / a.strips), (unsigned)S), block(512);
+    switch (a.strips) {
+    case 1: hipLaunchKernelGGL((k_w4a_gemm<T, MT, 1, 2, BITS>), grid, block, 0, st, a, r); break;
+    case 2: hipLaunchKernelGGL((k_w4a_gemm<T, MT, 2, 2, BITS>), grid, block, 0, st, a, r); break;
+    case 3: hipLaunchKernelGGL((k_w4a_gemm<T, MT, 3, 2, BITS>), grid, block, 0, st, a, r); break;
+    default: hipLaunchKernelGGL((k_w4a_gemm<T, MT, 4, 2, BITS>), grid, block, 0, st, a, r); break;
     }
 }
 // epi, rope, slabs, bias_done: as for w4r_gemm_launch; a matrix with wide scales stays there (bias - 128 scale has to be finite)
@@ -865,15 +853,21 @@ int w4a_gemm_launch(int dtype, const void *w4m, const void *x, int M, int N, int
     PIE_REQUIRE((epi == W4R_ROPE) == (rope != nullptr), PIE_E_ARG, "W4A GEMM: the q|k|v epilogue needs its arguments");
     const bool may_split = epi == W4R_STORE && workspace != nullptr && slabs != nullptr;  // (the caller's consumer sums them)
     const W4aPlan pl = w4a_plan(M, N, K, may_split, bits);
-    PIE_REQUIRE(pl.halves != 0, PIE_E_SHAPE, "W4A GEMM: 1..16 rows (32 of int8 codes), N a multiple of 32, K of 64");
+    PIE_REQUIRE(pl.strips != 0, PIE_E_SHAPE, "W4A GEMM: 1..16 rows (32 of int8 codes), N a multiple of 32, K of 64");
     PIE_REQUIRE(pie_aligned(w4m, 16) && pie_aligned(x, 16) && pie_aligned(y, 16) && pie_aligned(bias, 16), PIE_E_ALIGN, "W4A GEMM: 16-byte alignment required");
-    const W4aArgs a = {(const char *)w4m, (const u16 *)x, M, N, K, pl.halves, pl.groups, (u16 *)y, pl.S > 1 ? (float *)workspace : nullptr, pl.S > 1 ? nullptr : (const u16 *)bias,
+    const W4aArgs a = {(const char *)w4m, (const u16 *)x, M, N, K, pl.strips, pl.groups, (u16 *)y, pl.S > 1 ? (float *)workspace : nullptr, pl.S > 1 ? nullptr : (const u16 *)bias,
                        pl.S > 1 ? W4R_SLAB : epi};
     const W4mRope r = rope ? *rope : W4mRope{};
-    if (bits == 8 && dtype == PIE_BF16) M <= 8 ? w8a_go<BF16, 8>(a, pl.S, st, r) : M <= 16 ? w8a_go<BF16, 16>(a, pl.S, st, r) : w8a_go<BF16, 32>(a, pl.S, st, r);
-    else if (bits == 8) M <= 8 ? w8a_go<F16, 8>(a, pl.S, st, r) : M <= 16 ? w8a_go<F16, 16>(a, pl.S, st, r) : w8a_go<F16, 32>(a, pl.S, st, r);
-    else if (dtype == PIE_BF16) M <= 8 ? w4a_go<BF16, 8>(a, pl.S, st, r) : w4a_go<BF16, 16>(a, pl.S, st, r);
-    else M <= 8 ? w4a_go<F16, 8>(a, pl.S, st, r) : w4a_go<F16, 16>(a, pl.S, st, r);
+    auto rows = [&](auto t, auto width) {
+        using T = decltype(t);
+        constexpr int BITS = decltype(width)::value;
+        if (M <= 8) w4a_go<T, 8, BITS>(a, pl.S, st, r);
+        else if (M <= 16) w4a_go<T, 16, BITS>(a, pl.S, st, r);
+        else if constexpr (BITS == 8) w4a_go<T, 32, BITS>(a, pl.S, st, r);
+    };
+    auto go = [&](auto width) { dtype == PIE_BF16 ? rows(BF16{}, width) : rows(F16{}, width); };
+    if (bits == 8) go(std::integral_constant<int, 8>{});
+    else go(std::integral_constant<int, 4>{});
     PIE_LAUNCH_CHECK();
     if (pl.S > 1) *slabs = pl.S;
     else if (bias_done) *bias_done = true;

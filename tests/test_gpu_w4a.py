@@ -1,5 +1,5 @@
-"""k_w4a_gemm through steps of several sequences and short prompts: fewer groups of K than waves, groups that are no multiple of eight, splits of K, every count of half strips per workgroup (odd ones begin
-in the middle of a strip), a last workgroup that is not full, eight rows and sixteen, biases."""
+"""k_w4a_gemm through steps of several sequences and short prompts: fewer groups of K than waves, groups that are no multiple of eight, splits of K, every count of strips per workgroup,
+a last workgroup that is not full, eight rows and sixteen, biases."""
 import numpy as np
 import pytest
 import torch
@@ -9,8 +9,8 @@ from _util import assert_vec_close
 pytestmark = pytest.mark.gpu
 
 
-# [N, K] in half strips of 16 and groups of 64: hidden 192: 3 groups; 1088: 17, q|k|v in two half strips; 2048: gate|up in three, vocab in five, o_proj and down split; 512: gate|up in seven, vocab
-# in eight, in 268 workgroups; 4096: q|k|v, o_proj and down in four, split
+# [N, K] in strips of 32 and groups of 64: hidden 192: 3 groups; 1088: 17, every matrix strip by strip; 2048: gate|up in twos, vocab in threes, o_proj and down split; 512: gate|up in fours, vocab too, in
+# 268 workgroups; 4096: q|k|v, o_proj and down in twos, split
 @pytest.mark.parametrize("hidden,inter,vocab,heads,kv,dim,bias", [(192, 448, 96, 4, 2, 64, True), (1088, 1472, 5216, 17, 17, 64, False), (2048, 5632, 16896, 16, 4, 128, True),
                                                                   (512, 14336, 34240, 8, 2, 64, False), (4096, 4096, 12320, 32, 8, 128, False)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
