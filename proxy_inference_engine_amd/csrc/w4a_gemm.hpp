@@ -10,11 +10,11 @@
 //   * a wave's K-phase is its own: it loads the x of its groups straight into the operand's lanes (a group of eight rows is one load) and waits for nothing but its loads, all of them ordinary
 //     ones, so that the compiler's waits are exact; the scales of a step's four strips are one load.
 // Bound by the stream, a launch (3 us) and the conversion, of which 1.7 us are not hidden.  us, weights from HBM, k_w4r_gemm / the form before (32 x 32 products, x by LDS-DMA, which the compiler's
-// waits do not count: rings shallower than written) / this, 8 rows: gate|up [28672, 4096] 18.0 / 17.0 / 14.0, down [4096, 14336] 11.1 / 10.6 / 8.9, q|k|v [6144, 4096] 7.2 / 6.7 / 6.1, o [4096, 4096]
-// 5.6 / 5.3 / 4.7, head [32768, 4096] 18.3 / 17.6 / 14.7; [16384, 3072] 9.8 / 9.9 / 8.1, [3072, 8192] 7.2 / 6.7 / 6.1.  16 rows: 17.9 / 18.4 / 15.2, 11.4 / 11.2 / 9.4, 7.3 / 7.6 / 6.4,
-// 5.6 / 6.0 / 4.8, 19.8 / 19.5 / 15.7.  32 rows of int4: 18.5 / 19.8 / 21.4, 11.6 / - / 13.0: k_w4r_gemm's.  Without the conversion gate|up takes 12.8 us, without any arithmetic 11.9 to 12.8.
-// Two steps in flight per wave are enough (eight waves of 4.6 KB each); three and four cost 0.3 to 1 us, since the loads past a wave's last step, which return nothing, take their issue slots too (a
-// loop that leaves them out makes the compiler move registers about or wait for all of them: 17.8).
+// waits do not count: rings shallower than written) / this, 8 rows: gate|up [28672, 4096] 18.0 / 17.0 / 14.0, down [4096, 14336] 11.1 / 10.6 / 8.9, q|k|v [6144, 4096] 7.2 / 6.7 / 6.0, o [4096, 4096]
+// 5.6 / 5.3 / 4.6, head [32768, 4096] 18.3 / 17.6 / 14.6; [16384, 3072] 9.8 / 9.9 / 8.0, [3072, 8192] 7.2 / 6.7 / 6.0.  16 rows: 17.9 / 18.4 / 15.1, 11.4 / 11.2 / 9.2, 7.3 / 7.6 / 6.2,
+// 5.6 / 6.0 / 4.6, 19.8 / 19.5 / 15.6.  32 rows of int4: 18.5 / 19.8 / 21.4, 11.6 / - / 13.0: k_w4r_gemm's.  Without the conversion gate|up takes 12.8 us, without any arithmetic 11.9 to 12.8.
+// Two steps in flight per wave are enough (eight waves of 4.6 KB each): three and four cost 1 and 2 us of gate|up's.  The last round issues no loads (loads past a wave's end return nothing but take their
+// slots: q|k|v 6.1 / 6.0, o 4.7 / 4.6, int8 down 12.7 / 12.3); both loops need the ring as whole vectors, see there.
 // Error (2-norm, before the rounding to T) against 64 bits: 9e-7; of weights rounded to bf16 1.7e-3.
 #pragma once
 
@@ -43,8 +43,8 @@ constexpr float w4a_offset() { return std::is_same<T, F16>::value ? 0.0f : 128.0
 
 // Int8 codes, W8M tiles: as W4M, 32 rows x 64 columns, two pieces of 1 KiB and the 32 {scale, bias} words: lane l = 32 kh + n holds in piece h the codes of row n of k-steps 2 h and 2 h + 1, two words
 // each, in the W8S word format (codes 0, 2, 1, 3).  Up to 255 a code is a bf16 and an f16 as it stands.
-// Bound by the stream, half the bytes of a 16-bit copy's.  us, the form with 32 x 32 products / this, 8 rows: gate|up 23.3 / 22.6, down 13.3 / 12.7, q|k|v 8.8 / 7.8, o 6.5 / 5.8, head 24.9 / 24.5; 32 rows: 27.0 / 27.5,
-// 17.1 / 17.1, 12.1 / 10.5, 8.8 / 7.6, 28.4 / 28.5.
+// Bound by the stream, half the bytes of a 16-bit copy's.  us, the form with 32 x 32 products / this, 8 rows: gate|up 23.3 / 22.1, down 13.3 / 12.3, q|k|v 8.8 / 7.5, o 6.5 / 5.6, head 24.9 / 24.0; 32 rows: 27.0 / 26.8,
+// 17.1 / 16.6, 12.1 / 10.2, 8.8 / 7.0, 28.4 / 28.0.
 template <class T>
 __device__ __forceinline__ u32 w8a_pair(u32 a, u32 b) {  // two codes as T, b in the high half
     if constexpr (std::is_same<T, F16>::value) return __builtin_bit_cast(u32, __builtin_amdgcn_cvt_pkrtz((float)a, (float)b));
@@ -112,23 +112,17 @@ __global__ void __launch_bounds__(512) k_w4a_gemm(const W4aArgs a, const W4mRope
     }
     typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
     typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
-    uint4 xv[D][XL], cw[D][SPW][PC];
+    u32x4 xv[D][XL], cw[D][SPW][PC];  // (as vectors: split into words they would be copied from round to round, waited for right behind their loads)
     u32x2 sb[D];
     auto issue = [&](int d, int j) {
         const unsigned dead = j < steps ? 0u : NOWHERE, o = (unsigned)j * (KW * TILE), xo = (unsigned)(g_lo + j * KW) * 128u;
 #pragma unroll
-        for (int t = 0; t < XL; ++t) {
-            const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(xr, (x_at[PAIR ? 0 : t >> 1] | dead) + 64u * (t & 1), xo, 0);
-            xv[d][t] = make_uint4(v.x, v.y, v.z, v.w);
-        }
+        for (int t = 0; t < XL; ++t) xv[d][t] = __builtin_amdgcn_raw_buffer_load_b128(xr, (x_at[PAIR ? 0 : t >> 1] | dead) + 64u * (t & 1), xo, 0);
         sb[d] = __builtin_amdgcn_raw_buffer_load_b64(wr, scale_at | dead, strip_at[0] + o, 2);
 #pragma unroll
         for (int s = 0; s < SPW; ++s)
 #pragma unroll
-            for (int q = 0; q < PC; ++q) {
-                const u32x4 c = __builtin_amdgcn_raw_buffer_load_b128(wr, (code_at | gone[s] | dead) + 1024u * q, strip_at[s] + o, 2);
-                cw[d][s][q] = make_uint4(c.x, c.y, c.z, c.w);
-            }
+            for (int q = 0; q < PC; ++q) cw[d][s][q] = __builtin_amdgcn_raw_buffer_load_b128(wr, (code_at | gone[s] | dead) + 1024u * q, strip_at[s] + o, 2);
         __builtin_amdgcn_sched_barrier(0);  // (the loads stay in the order that the compiler's counted waits rely on)
     };
     if (steps > 0)
@@ -142,70 +136,78 @@ __global__ void __launch_bounds__(512) k_w4a_gemm(const W4aArgs a, const W4mRope
         for (int i = 0; i < AC; ++i) acc[s][i] = zero;
     const u32 one = std::is_same<T, F16>::value ? 0x3C003C00u : 0x3F803F80u;
     const uint4 ones = make_uint4(one, one, one, one);
-    for (int base = 0; base < steps; base += D) {
+    auto words = [](const u32x4 &v) { return make_uint4(v.x, v.y, v.z, v.w); };
+    auto compute = [&](int d) {
+        uint4 xa[PAIR ? 4 : XL];  // PAIR: the group's halves as rows 0..7, as rows 8..15
+        if constexpr (PAIR) xa[0] = w4a_eight<true, 0>(words(xv[d][0])), xa[1] = w4a_eight<false, 0>(words(xv[d][0])), xa[2] = w4a_eight<true, 8>(words(xv[d][0])), xa[3] = w4a_eight<false, 8>(words(xv[d][0]));
+        else
 #pragma unroll
-        for (int d = 0; d < D; ++d) {
-            if (base + d < steps) {
-                uint4 xa[PAIR ? 4 : XL];  // PAIR: the group's halves as rows 0..7, as rows 8..15
-                if constexpr (PAIR) xa[0] = w4a_eight<true, 0>(xv[d][0]), xa[1] = w4a_eight<false, 0>(xv[d][0]), xa[2] = w4a_eight<true, 8>(xv[d][0]), xa[3] = w4a_eight<false, 8>(xv[d][0]);
-                else
+            for (int t = 0; t < XL; ++t) xa[t] = words(xv[d][t]);
+        w4a_f32x4 xs[RB];
 #pragma unroll
-                    for (int t = 0; t < XL; ++t) xa[t] = xv[d][t];
-                w4a_f32x4 xs[RB];
+        for (int t = 0; t < RB; ++t) xs[t] = w4a_mfma<T>(xa[2 * t + 1], ones, w4a_mfma<T>(xa[2 * t], ones, zero));
+        if constexpr (PAIR) xs[0] = w4a_mfma<T>(xa[3], ones, w4a_mfma<T>(xa[2], ones, xs[0]));
+        u32 sw[4][2];  // every lane's scale word of a strip's even, of its odd column; PAIR: the one of the rows that it sums
+        {
+            u32 e0 = sb[d].x, e1 = sb[d].x, o0 = sb[d].y, o1 = sb[d].y;
+            w4a_swap16(e0, e1), w4a_swap16(o0, o1);  // strips 0 0 2 2, 1 1 3 3
+            if constexpr (PAIR) {
+                w4a_swap32(e0, o0), w4a_swap32(e1, o1);
+                sw[0][0] = e0, sw[2][0] = o0, sw[1][0] = e1, sw[3][0] = o1;
+            } else {
+                sw[0][0] = sw[2][0] = e0, sw[1][0] = sw[3][0] = e1, sw[0][1] = sw[2][1] = o0, sw[1][1] = sw[3][1] = o1;
 #pragma unroll
-                for (int t = 0; t < RB; ++t) xs[t] = w4a_mfma<T>(xa[2 * t + 1], ones, w4a_mfma<T>(xa[2 * t], ones, zero));
-                if constexpr (PAIR) xs[0] = w4a_mfma<T>(xa[3], ones, w4a_mfma<T>(xa[2], ones, xs[0]));
-                u32 sw[4][2];  // every lane's scale word of a strip's even, of its odd column; PAIR: the one of the rows that it sums
-                {
-                    u32 e0 = sb[d].x, e1 = sb[d].x, o0 = sb[d].y, o1 = sb[d].y;
-                    w4a_swap16(e0, e1), w4a_swap16(o0, o1);  // strips 0 0 2 2, 1 1 3 3
-                    if constexpr (PAIR) {
-                        w4a_swap32(e0, o0), w4a_swap32(e1, o1);
-                        sw[0][0] = e0, sw[2][0] = o0, sw[1][0] = e1, sw[3][0] = o1;
-                    } else {
-                        sw[0][0] = sw[2][0] = e0, sw[1][0] = sw[3][0] = e1, sw[0][1] = sw[2][1] = o0, sw[1][1] = sw[3][1] = o1;
-#pragma unroll
-                        for (int s = 0; s < 2; ++s) w4a_swap32(sw[s][0], sw[s + 2][0]), w4a_swap32(sw[s][1], sw[s + 2][1]);
-                    }
-                }
-#pragma unroll
-                for (int s = 0; s < SPW; ++s) {
-                    float sc[2], bi[2];
-#pragma unroll
-                    for (int h = 0; h < (PAIR ? 1 : 2); ++h) sc[h] = lo_f32<T>(sw[s][h]), bi[h] = BITS == 8 ? hi_f32<T>(sw[s][h]) : fmaf(-w4a_offset<T>(), sc[h], hi_f32<T>(sw[s][h]));
-                    uint4 wf[2][2];  // [even, odd columns][half of the group]
-                    if constexpr (BITS == 8) {
-#pragma unroll
-                        for (int h = 0; h < 2; ++h) {
-                            uint4 c = cw[d][s][h];
-                            w4a_swap16(c.x, c.z), w4a_swap16(c.y, c.w);
-                            wf[0][h] = w8a_codes<T>(c.x, c.y), wf[1][h] = w8a_codes<T>(c.z, c.w);
-                        }
-                    } else {
-                        uint4 c = cw[d][s][0];
-                        w4a_swap16(c.x, c.y), w4a_swap16(c.z, c.w);
-                        wf[0][0] = w4a_codes<T>(c.x), wf[1][0] = w4a_codes<T>(c.y), wf[0][1] = w4a_codes<T>(c.z), wf[1][1] = w4a_codes<T>(c.w);
-                    }
-                    if constexpr (PAIR) {
-                        w4a_f32x4 dot = w4a_mfma<T>(xa[1], wf[0][1], w4a_mfma<T>(xa[0], wf[0][0], zero));
-                        dot = w4a_mfma<T>(xa[3], wf[1][1], w4a_mfma<T>(xa[2], wf[1][0], dot));
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) acc[s][0][i] = fmaf(bi[0], xs[0][i], fmaf(sc[0], dot[i], acc[s][0][i]));
-                    } else {
-#pragma unroll
-                        for (int t = 0; t < RB; ++t)
-#pragma unroll
-                            for (int h = 0; h < 2; ++h) {
-                                const w4a_f32x4 dot = w4a_mfma<T>(xa[2 * t + 1], wf[h][1], w4a_mfma<T>(xa[2 * t], wf[h][0], zero));
-#pragma unroll
-                                for (int i = 0; i < 4; ++i) acc[s][2 * t + h][i] = fmaf(bi[h], xs[t][i], fmaf(sc[h], dot[i], acc[s][2 * t + h][i]));
-                            }
-                    }
-                }
+                for (int s = 0; s < 2; ++s) w4a_swap32(sw[s][0], sw[s + 2][0]), w4a_swap32(sw[s][1], sw[s + 2][1]);
             }
-            __builtin_amdgcn_sched_barrier(0);
-            issue(d, base + d + D);
         }
+#pragma unroll
+        for (int s = 0; s < SPW; ++s) {
+            float sc[2], bi[2];
+#pragma unroll
+            for (int h = 0; h < (PAIR ? 1 : 2); ++h) sc[h] = lo_f32<T>(sw[s][h]), bi[h] = BITS == 8 ? hi_f32<T>(sw[s][h]) : fmaf(-w4a_offset<T>(), sc[h], hi_f32<T>(sw[s][h]));
+            uint4 wf[2][2];  // [even, odd columns][half of the group]
+            if constexpr (BITS == 8) {
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    uint4 c = words(cw[d][s][h]);
+                    w4a_swap16(c.x, c.z), w4a_swap16(c.y, c.w);
+                    wf[0][h] = w8a_codes<T>(c.x, c.y), wf[1][h] = w8a_codes<T>(c.z, c.w);
+                }
+            } else {
+                uint4 c = words(cw[d][s][0]);
+                w4a_swap16(c.x, c.y), w4a_swap16(c.z, c.w);
+                wf[0][0] = w4a_codes<T>(c.x), wf[1][0] = w4a_codes<T>(c.y), wf[0][1] = w4a_codes<T>(c.z), wf[1][1] = w4a_codes<T>(c.w);
+            }
+            if constexpr (PAIR) {
+                w4a_f32x4 dot = w4a_mfma<T>(xa[1], wf[0][1], w4a_mfma<T>(xa[0], wf[0][0], zero));
+                dot = w4a_mfma<T>(xa[3], wf[1][1], w4a_mfma<T>(xa[2], wf[1][0], dot));
+#pragma unroll
+                for (int i = 0; i < 4; ++i) acc[s][0][i] = fmaf(bi[0], xs[0][i], fmaf(sc[0], dot[i], acc[s][0][i]));
+            } else {
+#pragma unroll
+                for (int t = 0; t < RB; ++t)
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        const w4a_f32x4 dot = w4a_mfma<T>(xa[2 * t + 1], wf[h][1], w4a_mfma<T>(xa[2 * t], wf[h][0], zero));
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) acc[s][2 * t + h][i] = fmaf(bi[h], xs[t][i], fmaf(sc[h], dot[i], acc[s][2 * t + h][i]));
+                    }
+            }
+        }
+    };
+    if (steps > 0) {
+        int base = 0;
+        for (; base + D < steps; base += D) {
+#pragma unroll
+            for (int d = 0; d < D; ++d) {
+                compute(d);
+                __builtin_amdgcn_sched_barrier(0);
+                issue(d, base + d + D);
+            }
+        }
+#pragma unroll
+        for (int d = 0; d < D; ++d)
+            if (base + d < steps) compute(d);
     }
     // a product's lane: columns 2 c16 (+ 1), rows 4 r16 .. + 3
 #pragma unroll
