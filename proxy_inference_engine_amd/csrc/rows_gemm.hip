@@ -203,6 +203,7 @@ __global__ void __launch_bounds__(512) k_rows_w16m(const RowsArgs a) {
 #pragma unroll
                 for (int t = 0; t < NT; ++t) xv[u][t] = *(const mf_u32x4 *)(xp[t] + 32 * cl);
             }
+            __builtin_amdgcn_sched_barrier(0);
         };
         auto multiply = [&](int s, const mf_u32x4(&wv)[U][NN], const mf_u32x4(&xv)[U][NT]) {
 #pragma unroll
@@ -219,14 +220,24 @@ __global__ void __launch_bounds__(512) k_rows_w16m(const RowsArgs a) {
                     for (int t = 0; t < NT; ++t) acc[n][t] = rows_mfma<E>(w, xv[u][t], acc[n][t]);
                 }
         };
+        // (each half round's loads in a piece, none past the end: the compiler's waits count them exactly.  us, one row, with its own order and a last round of loads for nothing / this: [5120, 3072] 10.4 / 9.0,
+        // [16384, 3072] 19.5 / 18.1, [6144, 4096] 12.3 / 11.9, [4096, 4096] 8.0 / 8.0)
         mf_u32x4 w0[U][NN], w1[U][NN], x0[U][NT], x1[U][NT];
-        fetch(wk, w0, x0);
-        for (int s = wk; s < steps; s += 2 * U * KW) {
-            fetch(s + U * KW, w1, x1);
+        constexpr int R = U * KW;
+        int s = wk;
+        fetch(s, w0, x0);
+        for (; s + 2 * R < steps; s += 2 * R) {
+            fetch(s + R, w1, x1);
             multiply(s, w0, x0);
-            fetch(s + 2 * U * KW, w0, x0);
-            multiply(s + U * KW, w1, x1);
+            fetch(s + 2 * R, w0, x0);
+            multiply(s + R, w1, x1);
         }
+        if (s + R < steps) {
+            fetch(s + R, w1, x1);
+            multiply(s, w0, x0);
+            multiply(s + R, w1, x1);
+        } else
+            multiply(s, w0, x0);
     }
     if constexpr (NORM) {
         ss = xor32_sum(xor16_sum(ss));
@@ -267,7 +278,7 @@ __global__ void __launch_bounds__(512) k_rows_w16m(const RowsArgs a) {
 // (registers, then one of two LDS buffers; rows padded by 16 B, conflict-free both ways), each wave multiplies every WV-th 32-column step by weights that it streams two chunks ahead.
 // Loads go by descriptors whose bounds drop what lies behind a row, a matrix or K (zeros), so no load has a branch around it.  Two workgroups of eight waves share a CU (launch bounds: 128 registers),
 // one loads while the other finishes.  Sixteen features per wave and step re-read x most (NN = 1), four blocks least: NN follows from how many workgroups are left (rows_lds_pick).
-// [28672, 4096] with 8 / 16 / 32 / 64 rows: 39 / 40 / 42 / 64 us = 6.0 / 5.8 / 5.6 / 3.7 TB/s.  Experts have fewer bytes per workgroup, and workgroups of four waves (WV) fill the gaps that
+// [28672, 4096] with 8 / 16 / 32 / 64 rows: 39 / 40 / 42 / 64 us = 6.0 / 5.9 / 5.6 / 3.7 TB/s.  Experts have fewer bytes per workgroup, and workgroups of four waves (WV) fill the gaps that
 // others leave better: 60 active ones of [2816, 2048] with 3 rows each 131 (k_rows_w16m) -> 110 (eight waves) -> 103 us (6.7 TB/s), of [2048, 1408] 90 -> 58 -> 53 us.
 template <class E, int NT, int NN, int U, int WV = 8>
 __global__ void __launch_bounds__(64 * WV, 4) k_rows_lds(const RowsArgs a) {
@@ -317,6 +328,7 @@ __global__ void __launch_bounds__(64 * WV, 4) k_rows_lds(const RowsArgs a) {
             const unsigned at = xc + it * C < K8 ? (unsigned)(it * C * 2) : NOWHERE;
 #pragma unroll
             for (int j = 0; j < XJ; ++j) xv[j] = __builtin_amdgcn_raw_buffer_load_b128(xs, (int)(xo[j] | at) < 0 ? NOWHERE : xo[j] + at, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
         };
         auto store_x = [&](int buf, const mf_u32x4(&xv)[XJ]) {
 #pragma unroll
@@ -330,6 +342,7 @@ __global__ void __launch_bounds__(64 * WV, 4) k_rows_lds(const RowsArgs a) {
                 for (int n = 0; n < NN; ++n)  // non-temporal: a weight is read once, except an expert's with more than 16 NT rows
                     wv[u][n] = __builtin_amdgcn_raw_buffer_load_b128(wr, s < steps ? wlane + (unsigned)((n >> 1) * groups * 4096 + s * 2048 + (n & 1) * 256) : NOWHERE, 0, 2);
             }
+            __builtin_amdgcn_sched_barrier(0);
         };
         mf_f32x4 acc[NN][NT];
 #pragma unroll
@@ -348,7 +361,9 @@ __global__ void __launch_bounds__(64 * WV, 4) k_rows_lds(const RowsArgs a) {
                     for (int t = 0; t < NT; ++t) acc[n][t] = rows_mfma<E>(wv[u][n], xv[t], acc[n][t]);
             }
         };
-        // (x before w: waiting for the next chunk's x must not wait for the weights behind it)
+        // (x before w: waiting for the next chunk's x must not wait for the weights behind it.  The loads stay in this order, and the last two chunks load nothing: with loads that the scheduler moved, or a
+        // round left halfway by a break, the compiler waited for every load in flight in every other chunk.  us, 8 / 32 rows, that / this: [6144, 4096] 13.1 / 12.4, 16.7 / 15.9; [5120, 3072] 10.9 / 10.0,
+        // 13.9 / 13.2; [4096, 14336] 23.5 / 23.0, 33.5 / 31.4; [10752, 4096] 19.5 / 18.7, 23.2 / 22.1; [32768, 4096] 43.4 / 43.0, 47.2 / 45.8; [28672, 4096] 40.3 / 40.3, 42.9 / 42.7)
         mf_u32x4 w[2][U][NN], xv[XJ];
         load_x(0, xv);
         load_w(0, w[0]);
@@ -356,10 +371,10 @@ __global__ void __launch_bounds__(64 * WV, 4) k_rows_lds(const RowsArgs a) {
         load_x(1, xv);
         load_w(1, w[1]);
         __syncthreads();
-        for (int it = 0; it < iters; it += 2) {
+        int it = 0;
+        for (; it + 2 < iters; it += 2) {
 #pragma unroll
             for (int d = 0; d < 2; ++d) {
-                if (it + d >= iters) break;
                 multiply(d, w[d]);
                 store_x(d ^ 1, xv);
                 load_x(it + d + 2, xv);
@@ -367,6 +382,13 @@ __global__ void __launch_bounds__(64 * WV, 4) k_rows_lds(const RowsArgs a) {
                 __syncthreads();
             }
         }
+        multiply(0, w[0]);
+        if (it + 1 < iters) {
+            store_x(1, xv);
+            __syncthreads();
+            multiply(1, w[1]);
+        }
+        __syncthreads();
         // lane (kq, c) holds features 4 kq .. + 3 of row c
 #pragma unroll
         for (int n = 0; n < NN; ++n)
