@@ -712,7 +712,7 @@ bool w4r_serves(int M, int N, int K);
 int w4r_splits(int M, int N, int K);
 size_t w4r_workspace_bytes(int M, int N, int K);
 bool w4m_wide_scales(const void *w4m);
-bool w4a_serves(int M, int N, int K, int bits = 4);
+bool w4a_serves(int M, int N, int K, int bits = 4, bool step = false);
 int w4a_splits(int M, int N, int K, int bits);
 size_t w4a_workspace_bytes(int M, int N, int K, int bits);
 size_t w8m_bytes(int N, int K);
@@ -743,8 +743,8 @@ static int bias_rows(u16 *y, const void *bias, int M, int N, hipStream_t st) {
 template <class T>
 static int linear_rows(pie_decoder *d, const void *packed, int N, int K, const u16 *x, int M, u16 *y, hipStream_t st, bool keep = true,
                        const void *bias = nullptr, bool keep_w4m = false, u16 *act = nullptr, bool *used_act = nullptr, W4mRope *rope = nullptr,
-                       W4lSlabs *slabs = nullptr, int pass_rows = 0) {
-    // pass_rows (0: M): rows of the pass that these M belong to: they decide between MLX's regimes, M between the kernels of one
+                       W4lSlabs *slabs = nullptr, int pass_rows = 0, bool step = false) {
+    // step: M sequences' next rows (w4a_serves).  pass_rows (0: M): rows of the pass that these M belong to: they decide between MLX's regimes, M between the kernels of one
     // slabs: the caller's consumer takes the fp32 slabs of a K-split many-row GEMM (and the bias) instead of y; slabs->S > 1 tells whether it must
     // rope / used_act: for the packed q|k|v matrix the few-row kernel can rotate q / k and append k / v itself
     // act / used_act: for the packed gate|up matrix the few-row kernel can apply the SwiGLU itself and write act [M, N / 2]
@@ -825,8 +825,8 @@ static int linear_rows(pie_decoder *d, const void *packed, int N, int K, const u
         if (rc || !bias || bias_done) return rc;
         return bias_rows<T>(y, bias, M, N, st);
     };
-    // Three to 16 rows: the scales on the sums.  One and two go to the GEMV below, as a step's do (batch_fused), also the one that a longer pass leaves to its last layer.
-    if (is_int4 && w4a_serves(M, N, K) && M > GEMV_FUSED_ROWS) {
+    // Three to 16 rows (8 of a prompt and a narrow matrix): the scales on the sums.  One and two go to the GEMV below, as a step's do (batch_fused), also the one that a longer pass leaves to its last layer.
+    if (is_int4 && w4a_serves(M, N, K, 4, step) && M > GEMV_FUSED_ROWS) {
         void *wm = nullptr;
         const int rc = w4m_tiles(&wm);
         if (rc) return rc;
@@ -1097,7 +1097,7 @@ static bool step_tiles(const pie_decoder *d, int B) {
     const int QD = c.n_heads * c.head_dim, NQKV = QD + 2 * c.n_kv_heads * c.head_dim;
     size_t more = 0;
     auto has = [&](const void *packed, int N, int K) {
-        if (!w4a_serves(B, N, K)) return false;
+        if (!w4a_serves(B, N, K, 4, true)) return false;
         const auto it = d->prefill->resident_w4m.find(packed);
         if (it != d->prefill->resident_w4m.end()) return !it->second.wide;
         more += w4m_bytes(N, K);
@@ -1190,7 +1190,7 @@ static int decode_batch_t(pie_decoder *d, const int32_t *tokens, const int32_t *
                       D, c.rope_traditional, s->q, nullptr, i8pb};
         bool roped = false;
         W4lSlabs sq;  // q|k|v as the fp32 slabs of a K-split product (no Linear bias: RoPE takes T(x W^T + b))
-        if ((rc = linear_rows<T>(d, w.wqkv, NQKV, H, s->xn, B, s->qkv, st, true, w.bqkv, false, nullptr, &roped, &re, w.bqkv ? nullptr : &sq)))
+        if ((rc = linear_rows<T>(d, w.wqkv, NQKV, H, s->xn, B, s->qkv, st, true, w.bqkv, false, nullptr, &roped, &re, w.bqkv ? nullptr : &sq, 0, true)))
             return rc;
         const bool rope_in_attn = !roped && !d->kv_i8;  // T pages: inside the attention launch (k_attn_step)
         if (!roped && d->kv_i8) {
@@ -1208,19 +1208,19 @@ static int decode_batch_t(pie_decoder *d, const int32_t *tokens, const int32_t *
         if (rc) return rc;
         W4lSlabs so, sd;  // o_proj / down handed over as K-split fp32 slabs where the shape qualifies
         if ((rc = linear_rows<T>(d, w.wo, H, QD, s->attn, B, s->r, st, true, w.bo, false, nullptr, nullptr, nullptr,
-                                 H <= 8192 ? &so : nullptr)))
+                                 H <= 8192 ? &so : nullptr, 0, true)))
             return rc;
         if ((rc = add_rms_norm_rows<T>(s->x, s->r, w.mlp_norm, c.rms_eps, B, H, c.dtype, s->xn, st, so.S > 1 ? w.bo : nullptr, &so)))
             return rc;
         bool fused_act = false;
-        if ((rc = linear_rows<T>(d, w.wgateup, 2 * I, H, s->xn, B, s->gu, st, true, w.bgateup, false, s->act, &fused_act))) return rc;
+        if ((rc = linear_rows<T>(d, w.wgateup, 2 * I, H, s->xn, B, s->gu, st, true, w.bgateup, false, s->act, &fused_act, nullptr, nullptr, 0, true))) return rc;
         if (!fused_act) {
             const size_t n_act = (size_t)B * I;
             hipLaunchKernelGGL(k_swiglu_rows<T>, dim3((unsigned)((n_act / 4 + 255) / 256)), dim3(256), 0, st, s->gu, n_act, s->act);
             PIE_LAUNCH_CHECK();
         }
         if ((rc = linear_rows<T>(d, w.wdown, H, I, s->act, B, s->r, st, true, w.bdown, false, nullptr, nullptr, nullptr,
-                                 H <= 8192 ? &sd : nullptr)))
+                                 H <= 8192 ? &sd : nullptr, 0, true)))
             return rc;
         const void *next_norm = li + 1 < c.n_layers ? d->layers[li + 1].attn_norm : d->glob.final_norm;  // final norm: language.py:187
         if ((rc = add_rms_norm_rows<T>(s->x, s->r, next_norm, c.rms_eps, B, H, c.dtype, s->xn, st, sd.S > 1 ? w.bdown : nullptr, &sd)))
@@ -1228,7 +1228,7 @@ static int decode_batch_t(pie_decoder *d, const int32_t *tokens, const int32_t *
     }
     // the head's 16-bit tiles stay, like the layers' (int4: its W4M tiles do): laid out anew for every step they cost more than the product (268 MB: 115 us beside 42)
     const bool keep_head = d->mat_fmt(d->glob.lm_head) != PIE_W_INT4_G64;
-    if ((rc = linear_rows<T>(d, d->glob.lm_head, c.vocab, H, s->xn, B, logits, st, keep_head, nullptr, true))) return rc;
+    if ((rc = linear_rows<T>(d, d->glob.lm_head, c.vocab, H, s->xn, B, logits, st, keep_head, nullptr, true, nullptr, nullptr, nullptr, nullptr, 0, true))) return rc;
     return logits_tail_rows_launch(c.dtype, logits, c.vocab, B, tiles ? (RowStat *)s->tail_stats : nullptr, logprobs, next_tokens, st, lens);
 }
 

@@ -828,7 +828,11 @@ static W4aPlan w4a_plan(int M, int N, int K, bool may_split, int bits) {
     if (S == 1) return {each, 1, 8 * steps};
     return {2, S, 8 * (steps / S)};
 }
-bool w4a_serves(int M, int N, int K, int bits) { return pie_knob(PIE_KNOB_W4R) != 0 && w4a_plan(M, N, K, false, bits).strips != 0; }
+// step: a batch's step, whose rows are single sequences' in the one-row arithmetic.  A prompt of 9 to 16 rows keeps weights rounded to T, as mx.quantized_matmul's matrix kernels have them from six rows on, in
+// its narrow products (k_w4r_gemm).
+bool w4a_serves(int M, int N, int K, int bits, bool step) {
+    return pie_knob(PIE_KNOB_W4R) != 0 && w4a_plan(M, N, K, false, bits).strips != 0 && (step || bits == 8 || M <= 8 || N >= 512 * 32);
+}
 int w4a_splits(int M, int N, int K, int bits) { return w4a_plan(M, N, K, true, bits).S; }
 size_t w4a_workspace_bytes(int M, int N, int K, int bits) {
     const int s = w4a_splits(M, N, K, bits);
