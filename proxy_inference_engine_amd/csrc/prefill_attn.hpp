@@ -50,6 +50,8 @@ struct PrefillAttnArgs {
     int before;                          // keys in front of the first row, as far as the host knows (plans the launch; the device's position decides)
     int splits;                          // SPLIT instantiation: workgroups along the keys (gridDim.y); their partial sums meet in k_prefill_combine
     float *part;                         //   [M, Hq, splits] x {[D] weighted sums}, then [M, Hq, splits] x {running max, sum}
+    const u16 *rot_bias;                 // ROT instantiation: q = the qkv Linear's rows [M, 3, Hq, DR], without its bias; the bias
+    const float *rot_cos, *rot_sin;      //   rotate-half angles, fp32 [M, DR / 2]
 };
 
 template <class T> struct MfmaT;
@@ -98,16 +100,25 @@ __device__ __forceinline__ int pa_off(int row, int ch) {
 // SHORT: blocks of 32 keys, for prompts that fill few of 64 (prefill_attn_short).
 // KG = 2: two waves per head and tile, which take a staged block's first and second 64 keys and meet in LDS at the end: half the serial blocks, and a wave's softmax beside the other's
 // products (prefill_attn_pairs says when).
-template <class T, int D, int REP, int QT, bool SEG = false, bool SPLIT = false, bool SHORT = false, int KG = 1>
-__global__ void __launch_bounds__(REP * QT * KG * 64, 2) k_prefill_attn(const PrefillAttnArgs a) {
+// DR: a head's columns, side by side in memory (D: what a row takes in LDS).  Heads of 80 need five steps of 16 columns for their scores and three tiles of 32 for their sums, not the eight and four of 128,
+// and no padding.  The 7B vision tower's widths, 1024 patches, us: windows of 64 7.9 -> 6.6, whole image 54 -> 46.
+// ROT: windows straight from the qkv Linear's rows: bias and rotation on the way into LDS, by twice the waves (the second half of them does nothing else), queries and the first 64 keys asked for before anything
+// waits; with the blocks of 32 keys of the others, so that the sums are theirs bit for bit.  Bound by the chain bounds -> rows -> LDS -> scores of one round of workgroups.  A window's keys are rotated once
+// per 64 query rows that see them; rotated in a launch of their own, as a whole image's still are (32 tiles would each rotate all keys), they cost 8 us beside the attention's 6.6, here 10.1 in all (12.0 with
+// as many waves as tiles and no early queries).
+template <class T, int D, int REP, int QT, bool SEG = false, bool SPLIT = false, bool SHORT = false, int KG = 1, int DR = D, bool ROT = false>
+__global__ void __launch_bounds__(REP * QT * KG * 64 * (ROT ? 2 : 1), 2) k_prefill_attn(const PrefillAttnArgs a) {
+    static_assert(DR == D || (SEG && DR % 16 == 0 && DR < D), "narrower rows: segments");
+    static_assert(!ROT || (SEG && REP == 1), "rotation on the way in: segments of plain heads");
     static_assert(KG == 1 || (KG == 2 && QT == 1 && !SEG && !SHORT), "two waves per tile: causal, one tile");
-    constexpr int NT = REP * QT * KG * 64, NB = (NT >= 256 && !SHORT) || KG == 2 ? 2 : 1, BK = 32 * NB * KG;  // keys per block: 64 (a wave's) where enough threads share their loads
-    constexpr int CH = D / 8, KS = D / 16, DT = D / 32;                      // chunks per row, k-steps of Q.K^T, 32-dim output tiles
+    constexpr int NT = REP * QT * KG * 64 * (ROT ? 2 : 1), NB = (NT >= 256 && !SHORT && !ROT) || KG == 2 ? 2 : 1, BK = 32 * NB * KG;  // keys per block: 64 (a wave's) where enough threads share their loads
+    constexpr int CH = DR / 8, KS = DR / 16, DT = (DR + 31) / 32;              // chunks per row, k-steps of Q.K^T, 32-dim output tiles (of columns past DR nothing is stored)
     constexpr int BM = 32 * QT;
     constexpr int CPT = (BK * CH + NT - 1) / NT;                                   // 16-byte chunks per thread and tile
     __shared__ __attribute__((aligned(16))) char kv_lds[2][2][BK * 2 * D];         // [block parity][K, V]
     const int lane = threadIdx.x & 63, wave_id = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int wave = KG == 2 ? wave_id % REP : wave_id, kg = KG == 2 ? wave_id / REP : 0;  // (kg: which half of a block's keys)
+    const bool helper = ROT && wave_id >= REP * QT;  // (ROT: as many waves again, which only bring rows in)
+    const int wave = KG == 2 ? wave_id % REP : ROT ? wave_id % (REP * QT) : wave_id, kg = KG == 2 ? wave_id / REP : 0;  // (kg: which half of a block's keys)
     const int c = lane & 31, h = lane >> 5;
     // XCD-aware tile mapping: workgroups go round-robin over the 8 XCDs by linear id, so the kv-head group is the FASTEST
     // index (id % Hkv): with 8 kv-heads every XCD's L2 only ever holds one group's K/V (4 MB at 4096 tokens) instead of all
@@ -122,6 +133,24 @@ __global__ void __launch_bounds__(REP * QT * KG * 64, 2) k_prefill_attn(const Pr
     const int row_mask = paged ? 63 : 0x7FFFFFFF;
     const size_t page_elems = (size_t)2 * 64 * a.Hkv * D;
     const int r_last = (wg_r0 + BM - 1 < a.M ? wg_r0 + BM - 1 : a.M - 1);
+    // ROT: this workgroup's query rows, asked for before the bounds are known
+    constexpr int HC = DR / 16, QI = ROT ? (BM * HC + NT - 1) / NT : 1;  // 16-byte pieces of half a head; (row, piece of the lower half)s per thread
+    const size_t qkv_ld = (size_t)3 * a.Hq * DR;
+    __shared__ __attribute__((aligned(16))) char q_lds[ROT ? BM * 2 * D : 16];
+    uint4 q_half[QI][2];
+    float4 q_turn[QI][4];
+    auto turns = [&](int t, int c, float4(&o)[4]) {  // cosines, sines of piece c
+        const float4 *cp = reinterpret_cast<const float4 *>(a.rot_cos + (size_t)t * (DR / 2) + 8 * c), *sp = reinterpret_cast<const float4 *>(a.rot_sin + (size_t)t * (DR / 2) + 8 * c);
+        o[0] = cp[0], o[1] = cp[1], o[2] = sp[0], o[3] = sp[1];
+    };
+    if constexpr (ROT)
+#pragma unroll
+        for (int i = 0; i < QI; ++i) {
+            const int x = min((int)threadIdx.x + i * NT, BM * HC - 1), c = x % HC, t = min(wg_r0 + x / HC, a.M - 1);
+            const u16 *row = a.q + t * qkv_ld + (size_t)g * DR + 8 * c;
+            q_half[i][0] = *reinterpret_cast<const uint4 *>(row), q_half[i][1] = *reinterpret_cast<const uint4 *>(row + DR / 2);
+            turns(t, c, q_turn[i]);
+        }
     // last / first key any row of this tile attends (segment bounds are non-decreasing in the row index)
     // (bounds clamped to the buffer: a bad segment table must not become a wild address)
     const int t_last = SEG ? max(min(a.seg_hi[r_last], a.cap), 1) - 1 : pos0 + r_last;
@@ -136,8 +165,8 @@ __global__ void __launch_bounds__(REP * QT * KG * 64, 2) k_prefill_attn(const Pr
             }
             return;
         }
-    const u16 *kbase = (a.state ? reinterpret_cast<const u16 *>(a.kv_table[a.layer]) : a.k) + (size_t)g * cap * D;
-    const u16 *vbase = (a.state ? reinterpret_cast<const u16 *>(a.kv_table[a.n_layers + a.layer]) : a.v) + (size_t)g * cap * D;
+    const u16 *kbase = (a.state ? reinterpret_cast<const u16 *>(a.kv_table[a.layer]) : a.k) + (size_t)g * cap * DR;
+    const u16 *vbase = (a.state ? reinterpret_cast<const u16 *>(a.kv_table[a.n_layers + a.layer]) : a.v) + (size_t)g * cap * DR;
 
     // staging: chunk id x = threadIdx.x + i*NT -> (row = x / CH, ch = x % CH); keys past t_last are clamped (masked later).
     // Eight NAMED register pairs, used up to CPT: as arrays (even with compile-time indices) the compiler parked them in
@@ -150,8 +179,8 @@ __global__ void __launch_bounds__(REP * QT * KG * 64, 2) k_prefill_attn(const Pr
         int t = b * BK + x / CH;                                                                 \
         t = t < t_last ? t : t_last;                                                             \
         const size_t po = KG == 2 && x >= 64 * CH ? pg_off1 : pg_off;                            \
-        kr = *reinterpret_cast<const uint4 *>(kbase + po + (size_t)(t & row_mask) * D + (x % CH) * 8); \
-        vr = *reinterpret_cast<const uint4 *>(vbase + po + (size_t)(t & row_mask) * D + (x % CH) * 8); \
+        kr = *reinterpret_cast<const uint4 *>(kbase + po + (size_t)(t & row_mask) * DR + (x % CH) * 8); \
+        vr = *reinterpret_cast<const uint4 *>(vbase + po + (size_t)(t & row_mask) * DR + (x % CH) * 8); \
     }
 #define PA_PUBLISH1(i, kr, vr)                                                                 \
     if constexpr (i < CPT) {                                                                     \
@@ -173,14 +202,72 @@ __global__ void __launch_bounds__(REP * QT * KG * 64, 2) k_prefill_attn(const Pr
     };
 #undef PA_FETCH1
 #undef PA_PUBLISH1
-    static_assert(CPT <= 8, "staging registers");
-    fetch(b_first);
+    static_assert(ROT || CPT <= 8, "staging registers");
+    // ROT: eight columns of a Linear's row with its bias, and a pair of eights turned as apply_rotary_pos_emb_vision has them: the terms and roundings of k_vision_qkv_rope
+    auto biased = [&](const uint4 &x, const u16 *bias, float(&o)[8]) {
+        const uint4 b = *reinterpret_cast<const uint4 *>(bias);
+        const u32 xw[4] = {x.x, x.y, x.z, x.w}, bw[4] = {b.x, b.y, b.z, b.w};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) o[2 * j] = round_T<T>(lo_f32<T>(xw[j]) + lo_f32<T>(bw[j])), o[2 * j + 1] = round_T<T>(hi_f32<T>(xw[j]) + hi_f32<T>(bw[j]));
+    };
+    auto packed = [&](const float(&o)[8]) { return make_uint4(pack2<T>(o[0], o[1]), pack2<T>(o[2], o[3]), pack2<T>(o[4], o[5]), pack2<T>(o[6], o[7])); };
+    auto turned = [&](char *rows, int r, int c, const uint4 &lower, const uint4 &upper, const u16 *bias, const float4(&t)[4]) {
+        float lo[8], hi[8], o[8], p[8];
+        biased(lower, bias + 8 * c, lo), biased(upper, bias + DR / 2 + 8 * c, hi);
+        const float cc[8] = {t[0].x, t[0].y, t[0].z, t[0].w, t[1].x, t[1].y, t[1].z, t[1].w}, ss[8] = {t[2].x, t[2].y, t[2].z, t[2].w, t[3].x, t[3].y, t[3].z, t[3].w};
+#pragma unroll
+        for (int j = 0; j < 8; ++j) o[j] = __fadd_rn(__fmul_rn(lo[j], cc[j]), __fmul_rn(-hi[j], ss[j])), p[j] = __fadd_rn(__fmul_rn(hi[j], cc[j]), __fmul_rn(lo[j], ss[j]));
+        *reinterpret_cast<uint4 *>(rows + pa_off<D>(r, c)) = packed(o), *reinterpret_cast<uint4 *>(rows + pa_off<D>(r, c + HC)) = packed(p);
+    };
+    auto rotate_in = [&](int b) {  // key blocks b and b + 1, into both images
+        constexpr int B2 = 2 * BK, KI = (B2 * HC + NT - 1) / NT, VI = (B2 * CH + NT - 1) / NT;
+        uint4 half[KI][2], vv[VI];
+        float4 turn[KI][4];
+#pragma unroll
+        for (int i = 0; i < KI; ++i) {
+            const int x = min((int)threadIdx.x + i * NT, B2 * HC - 1), c = x % HC, t = min(b * BK + x / HC, t_last);
+            const u16 *row = a.q + t * qkv_ld + (size_t)(a.Hq + g) * DR + 8 * c;
+            half[i][0] = *reinterpret_cast<const uint4 *>(row), half[i][1] = *reinterpret_cast<const uint4 *>(row + DR / 2);
+            turns(t, c, turn[i]);
+        }
+#pragma unroll
+        for (int i = 0; i < VI; ++i) {
+            const int x = min((int)threadIdx.x + i * NT, B2 * CH - 1), t = min(b * BK + x / CH, t_last);
+            vv[i] = *reinterpret_cast<const uint4 *>(a.q + t * qkv_ld + (size_t)(2 * a.Hq + g) * DR + 8 * (x % CH));
+        }
+        if (b == b_first)
+#pragma unroll
+            for (int i = 0; i < QI; ++i) {
+                const int x = threadIdx.x + i * NT;
+                if (x < BM * HC) turned(q_lds, x / HC, x % HC, q_half[i][0], q_half[i][1], a.rot_bias + (size_t)g * DR, q_turn[i]);
+            }
+#pragma unroll
+        for (int i = 0; i < KI; ++i) {
+            const int x = threadIdx.x + i * NT;
+            if (x < B2 * HC) turned(kv_lds[x / HC / BK][0], x / HC % BK, x % HC, half[i][0], half[i][1], a.rot_bias + (size_t)(a.Hq + g) * DR, turn[i]);
+        }
+#pragma unroll
+        for (int i = 0; i < VI; ++i) {
+            const int x = threadIdx.x + i * NT;
+            if (x >= B2 * CH) break;
+            float v[8];
+            biased(vv[i], a.rot_bias + (size_t)(2 * a.Hq + g) * DR + 8 * (x % CH), v);
+            *reinterpret_cast<uint4 *>(kv_lds[x / CH / BK][1] + pa_off<D>(x / CH % BK, x % CH)) = packed(v);
+        }
+    };
+    if constexpr (ROT) {
+        rotate_in(b_first);
+        __syncthreads();
+    }
+    if constexpr (!ROT) fetch(b_first);
 
     // Q fragments (B operand of K . Q^T): lane (row c, half h), k-step s holds Q[r0 + c][hq][16 s + 8 h .. + 8]
     const int qrow = r0 + c < a.M ? r0 + c : a.M - 1;
     uint4 qf[KS];
 #pragma unroll
-    for (int s = 0; s < KS; ++s) qf[s] = *reinterpret_cast<const uint4 *>(a.q + ((size_t)qrow * a.Hq + hq) * D + 16 * s + 8 * h);
+    for (int s = 0; s < KS; ++s)
+        if constexpr (ROT) qf[s] = *reinterpret_cast<const uint4 *>(q_lds + pa_off<D>(32 * wave + c, 2 * s + h));
+        else qf[s] = *reinterpret_cast<const uint4 *>(a.q + ((size_t)qrow * a.Hq + hq) * DR + 16 * s + 8 * h);
     // last (and, SEG, first) key this lane's query row attends (rows past M are padding: never stored)
     const int t_row = SEG ? a.seg_hi[qrow] - 1 : pos0 + r0 + c;
     const int t_lo = SEG ? a.seg_lo[qrow] : 0;
@@ -203,14 +290,17 @@ __global__ void __launch_bounds__(REP * QT * KG * 64, 2) k_prefill_attn(const Pr
     // 4-row x 16-column block; lane i of the group receives column i, row q in element q
     const int grp = lane >> 4, tq = (lane & 15) >> 2, tp = lane & 3;
 
-    publish(0);
-    __syncthreads();
+    if constexpr (!ROT) {
+        publish(0);
+        __syncthreads();
+    }
     for (int b = b_first; b < n_blocks; ++b) {
         const int buf = (b - b_first) & 1;
         const char *k_lds = kv_lds[buf][0] + kg * (64 * 2 * D), *v_lds = kv_lds[buf][1] + kg * (64 * 2 * D);
-        if (b + 1 < n_blocks) fetch(b + 1);
+        if constexpr (!ROT)
+            if (b + 1 < n_blocks) fetch(b + 1);
         const int t0 = b * BK + (KG == 2 ? 64 * kg : 0);
-        if (KG == 1 || t0 <= t_last) {
+        if ((KG == 1 || t0 <= t_last) && !helper) {
 
         // S^T = K . Q^T : rows = keys (registers), cols = query rows (lanes); the blocks of 32 keys are independent chains
         f32x16_t sc[NB];
@@ -301,11 +391,15 @@ __global__ void __launch_bounds__(REP * QT * KG * 64, 2) k_prefill_attn(const Pr
             for (int dt = 0; dt < DT; ++dt) oacc[dt] = MfmaT<T>::run(vf[dt], bl, oacc[dt]);
         }
         }
-        if (b + 1 < n_blocks) {  // (the other image: its last readers passed the barrier in front of this block)
-            publish(buf ^ 1);
+        if (b + 1 < n_blocks && (!ROT || buf)) {  // (the other image: its last readers passed the barrier in front of this block; ROT: both)
+            if constexpr (ROT) {
+                __syncthreads();
+                rotate_in(b + 1);
+            } else publish(buf ^ 1);
             __syncthreads();
         }
     }
+    if (helper) return;
     if constexpr (KG == 2) {  // the second wave's sums join the first's: 16 floats of a lane at a time, lanes side by side
         static_assert(REP * 64 * (DT * 16 + 2) * 4 <= (int)sizeof(kv_lds), "the sums fit the images");
         float *meet = reinterpret_cast<float *>(kv_lds) + wave * (64 * (DT * 16 + 2)) + lane;
@@ -344,7 +438,7 @@ __global__ void __launch_bounds__(REP * QT * KG * 64, 2) k_prefill_attn(const Pr
     // normalise: the pair (lane, lane ^ 32) shares the query row and holds the two halves of the row sum
     const float inv = 1.0f / xor32_sum(l_run);
     if (r0 + c < a.M) {
-        const int od = SEG && a.out_d ? a.out_d : D;
+        const int od = DR < D ? DR : SEG && a.out_d ? a.out_d : D;
         u16 *orow = a.out + ((size_t)(r0 + c) * a.Hq + hq) * od;
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt)
@@ -476,13 +570,22 @@ static int prefill_attn_launch_d(const PrefillAttnArgs &a, hipStream_t st) {
 }
 // block-diagonal attention (SEG): multi-head only (Hq == Hkv, the vision tower), two query tiles per workgroup while the
 // halved grid still fills the chip
-template <class T, int D>
+template <class T, int D, int DR = D>
 static int segment_attn_launch_d(const PrefillAttnArgs &a, hipStream_t st) {
     if (a.Hq != a.Hkv) return pie::fail(PIE_E_SHAPE, "segment attention: n_heads must equal n_kv_heads");
     const bool two = a.M > 32 && ((a.M + 63) / 64) * a.Hkv >= 512;
     const dim3 grid(((a.M + (two ? 63 : 31)) / (two ? 64 : 32)) * a.Hkv);
-    if (two) hipLaunchKernelGGL((k_prefill_attn<T, D, 1, 2, true>), grid, dim3(128), 0, st, a);
-    else hipLaunchKernelGGL((k_prefill_attn<T, D, 1, 1, true>), grid, dim3(64), 0, st, a);
+    if (two) hipLaunchKernelGGL((k_prefill_attn<T, D, 1, 2, true, false, false, 1, DR>), grid, dim3(128), 0, st, a);
+    else hipLaunchKernelGGL((k_prefill_attn<T, D, 1, 1, true, false, false, 1, DR>), grid, dim3(64), 0, st, a);
+    PIE_LAUNCH_CHECK();
+    return PIE_OK;
+}
+// Windows of the vision tower whose q, k and v are still the Linear's rows (ROT): the bias and the rotation on the way into LDS, keys once per 64 query rows.
+template <class T>
+static int segment_rot_launch_t(const PrefillAttnArgs &a, int D, hipStream_t st) {
+    const dim3 grid((a.M + 63) / 64 * a.Hkv);
+    if (D == 80) hipLaunchKernelGGL((k_prefill_attn<T, 128, 1, 2, true, false, false, 1, 80, true>), grid, dim3(256), 0, st, a);
+    else hipLaunchKernelGGL((k_prefill_attn<T, 64, 1, 2, true, false, false, 1, 64, true>), grid, dim3(256), 0, st, a);
     PIE_LAUNCH_CHECK();
     return PIE_OK;
 }
@@ -514,6 +617,7 @@ static int segment_attn_gqa_launch_t(const PrefillAttnArgs &a, int D, hipStream_
 
 template <class T>
 static int segment_attn_launch_t(const PrefillAttnArgs &a, int D, hipStream_t st) {
+    if (D == 80) return segment_attn_launch_d<T, 128, 80>(a, st);
     return D == 128 ? segment_attn_launch_d<T, 128>(a, st) : segment_attn_launch_d<T, 64>(a, st);
 }
 

@@ -214,23 +214,8 @@ static int by_dt(int dtype, F16F &&f16, BF16F &&bf16, const char *who) {
     return PIE_OK;
 }
 
-extern "C" {
-
-int pie_gelu(const void *x, size_t n, int dtype, void *y, void *stream) {
-    PIE_REQUIRE(x && y, PIE_E_ARG, "pie_gelu: null pointer");
-    PIE_REQUIRE(n > 0, PIE_E_SHAPE, "pie_gelu: empty input");
-    hipStream_t st = (hipStream_t)stream;
-    const dim3 grid((unsigned)((n + 255) / 256)), block(256);
-    return by_dt(
-        dtype, [&] { hipLaunchKernelGGL(k_gelu<F16>, grid, block, 0, st, (const u16 *)x, n, (u16 *)y); },
-        [&] { hipLaunchKernelGGL(k_gelu<BF16>, grid, block, 0, st, (const u16 *)x, n, (u16 *)y); }, "pie_gelu");
-}
-
-int pie_vision_qkv_rope(const void *qkv, const void *bias, const float *cos_t, const float *sin_t, int N, int H, int D, int DP, int dtype, void *q,
-                        void *k, void *v, void *stream) {
-    PIE_REQUIRE(qkv && cos_t && sin_t && q && k && v, PIE_E_ARG, "pie_vision_qkv_rope: null pointer");
-    PIE_REQUIRE(N > 0 && H > 0 && D > 0 && D % 2 == 0 && (DP == 64 || DP == 128) && D <= DP, PIE_E_SHAPE,
-                "pie_vision_qkv_rope: head_dim must be even and fit the padded size 64 or 128");
+// DP: 64, 128, or D itself (no padding)
+static int qkv_rope(const void *qkv, const void *bias, const float *cos_t, const float *sin_t, int N, int H, int D, int DP, int dtype, void *q, void *k, void *v, void *stream) {
     hipStream_t st = (hipStream_t)stream;
     if (D % 8 == 0 && pie_aligned(qkv, 8) && pie_aligned(q, 16) && pie_aligned(k, 16) && pie_aligned(v, 16) && (!bias || pie_aligned(bias, 8)) &&
         pie_aligned(cos_t, 16) && pie_aligned(sin_t, 16)) {
@@ -249,6 +234,26 @@ int pie_vision_qkv_rope(const void *qkv, const void *bias, const float *cos_t, c
         [&] { hipLaunchKernelGGL(k_vision_qkv_rope<F16>, grid, block, 0, st, (const u16 *)qkv, (const u16 *)bias, cos_t, sin_t, N, H, D, DP, (u16 *)q, (u16 *)k, (u16 *)v); },
         [&] { hipLaunchKernelGGL(k_vision_qkv_rope<BF16>, grid, block, 0, st, (const u16 *)qkv, (const u16 *)bias, cos_t, sin_t, N, H, D, DP, (u16 *)q, (u16 *)k, (u16 *)v); },
         "pie_vision_qkv_rope");
+}
+
+extern "C" {
+
+int pie_gelu(const void *x, size_t n, int dtype, void *y, void *stream) {
+    PIE_REQUIRE(x && y, PIE_E_ARG, "pie_gelu: null pointer");
+    PIE_REQUIRE(n > 0, PIE_E_SHAPE, "pie_gelu: empty input");
+    hipStream_t st = (hipStream_t)stream;
+    const dim3 grid((unsigned)((n + 255) / 256)), block(256);
+    return by_dt(
+        dtype, [&] { hipLaunchKernelGGL(k_gelu<F16>, grid, block, 0, st, (const u16 *)x, n, (u16 *)y); },
+        [&] { hipLaunchKernelGGL(k_gelu<BF16>, grid, block, 0, st, (const u16 *)x, n, (u16 *)y); }, "pie_gelu");
+}
+
+int pie_vision_qkv_rope(const void *qkv, const void *bias, const float *cos_t, const float *sin_t, int N, int H, int D, int DP, int dtype, void *q,
+                        void *k, void *v, void *stream) {
+    PIE_REQUIRE(qkv && cos_t && sin_t && q && k && v, PIE_E_ARG, "pie_vision_qkv_rope: null pointer");
+    PIE_REQUIRE(N > 0 && H > 0 && D > 0 && D % 2 == 0 && (DP == 64 || DP == 128) && D <= DP, PIE_E_SHAPE,
+                "pie_vision_qkv_rope: head_dim must be even and fit the padded size 64 or 128");
+    return qkv_rope(qkv, bias, cos_t, sin_t, N, H, D, DP, dtype, q, k, v, stream);
 }
 
 int pie_bias_silu_mul(const void *gate, const void *up, const void *bias_gate, const void *bias_up, int M, int N, int ld, int dtype, void *y,
@@ -303,10 +308,10 @@ int pie_add_bias_rms_norm(const void *x, const void *r, const void *bias, const 
 
 }  // extern "C"
 
-// out: rows of H heads of out_d columns (0: D)
+// D: 64, 128, or 80 (rows without padding); out: rows of H heads of out_d columns (0: D)
 static int segment_attn(const void *q, const void *k, const void *v, const int32_t *seg_lo, const int32_t *seg_hi, int N, int H, int D, int out_d, float scale, int dtype, void *out, void *stream) {
     PIE_REQUIRE(q && k && v && seg_lo && seg_hi && out, PIE_E_ARG, "pie_sdpa_segments: null pointer");
-    PIE_REQUIRE(N > 0 && H > 0 && (D == 64 || D == 128), PIE_E_SHAPE, "pie_sdpa_segments: head_dim must be 64 or 128");
+    PIE_REQUIRE(N > 0 && H > 0, PIE_E_SHAPE, "pie_sdpa_segments: empty input");
     PIE_REQUIRE(pie_aligned(q, 16) && pie_aligned(k, 16) && pie_aligned(v, 16) && pie_aligned(out, 8), PIE_E_ALIGN, "pie_sdpa_segments: misaligned pointer");
     PrefillAttnArgs a = {};
     a.q = (const u16 *)q, a.k = (const u16 *)k, a.v = (const u16 *)v, a.offset = 0, a.cap = N;
@@ -317,15 +322,28 @@ static int segment_attn(const void *q, const void *k, const void *v, const int32
     return pie::fail(PIE_E_ARG, "pie_sdpa_segments: dtype must be PIE_BF16 or PIE_F16");
 }
 
+// The attention of a block over windows, from the qkv Linear's rows (no bias yet): heads of 64 and 80
+static bool segment_rot_serves(int head_dim, const void *bias, const float *cos_t, const float *sin_t) {
+    return (head_dim == 64 || head_dim == 80) && pie_aligned(bias, 16) && pie_aligned(cos_t, 16) && pie_aligned(sin_t, 16);
+}
+static int segment_rot(const void *qkv, const void *bias, const float *cos_t, const float *sin_t, const int32_t *seg_lo, const int32_t *seg_hi, int N, int H, int D, float scale, int dtype, void *out, void *stream) {
+    PIE_REQUIRE(dtype == PIE_BF16 || dtype == PIE_F16, PIE_E_ARG, "segment attention: dtype must be PIE_BF16 or PIE_F16");
+    PrefillAttnArgs a = {};
+    a.q = (const u16 *)qkv, a.cap = N, a.seg_lo = seg_lo, a.seg_hi = seg_hi, a.M = N, a.Hq = H, a.Hkv = H, a.scale = scale, a.out = (u16 *)out;
+    a.rot_bias = (const u16 *)bias, a.rot_cos = cos_t, a.rot_sin = sin_t;
+    return dtype == PIE_BF16 ? segment_rot_launch_t<BF16>(a, D, (hipStream_t)stream) : segment_rot_launch_t<F16>(a, D, (hipStream_t)stream);
+}
+
 // Scratch of pie_vision_blocks, in order; every part a multiple of 256 bytes.  The qkv rows and the MLP's activation are never alive together.
 struct VisionScratch {
     size_t wide, head, out, gemm;  // bytes of: qkv / activation rows, q (k, v) rows, the products' output and the attention's rows (each), slabs of a product that splits K
     size_t total() const { return wide + 3 * head + 2 * out + gemm; }
 };
+static int vision_head_row(int head_dim) { return head_dim <= 64 ? 64 : head_dim == 80 ? 80 : 128; }  // columns of a q, k or v row between the rotation and the attention (k_prefill_attn's DR)
 static VisionScratch vision_scratch(int rows, int hidden, int inter, int heads, int head_dim) {
     auto up = [](size_t n) { return (n + 255) & ~(size_t)255; };
     auto most = [](size_t a, size_t b) { return a > b ? a : b; };
-    const int act = (inter + 63) & ~63, DP = head_dim <= 64 ? 64 : 128;
+    const int act = (inter + 63) & ~63, DP = vision_head_row(head_dim);
     const size_t slabs = most(most(pie_linear_w16m_workspace(rows, 3 * hidden, hidden), pie_linear_w16m_workspace(rows, hidden, hidden)), pie_linear_w16m_workspace(rows, hidden, inter));
     return {up((size_t)rows * (3 * hidden > act ? 3 * hidden : act) * 2), up((size_t)rows * heads * DP * 2), up((size_t)rows * hidden * 2), up(slabs)};
 }
@@ -337,6 +355,7 @@ extern "C" {
 
 int pie_sdpa_segments(const void *q, const void *k, const void *v, const int32_t *seg_lo, const int32_t *seg_hi, int N, int H, int D, float scale,
                       int dtype, void *out, void *stream) {
+    PIE_REQUIRE(D == 64 || D == 128, PIE_E_SHAPE, "pie_sdpa_segments: head_dim must be 64 or 128");
     return segment_attn(q, k, v, seg_lo, seg_hi, N, H, D, 0, scale, dtype, out, stream);
 }
 
@@ -344,7 +363,7 @@ size_t pie_vision_blocks_workspace(int rows, int hidden, int inter, int heads, i
     return vision_shape(rows, hidden, inter, heads, head_dim) ? vision_scratch(rows, hidden, inter, heads, head_dim).total() : 0;
 }
 
-// One call for all blocks: eight launches each, which a host that calls op by op starts in 12 us apiece (0.92 ms for eight blocks of the 7B tower's widths, the time of an image up to 448 x 448)
+// One call for all blocks: seven or eight launches each, which a host that calls op by op starts in 12 us apiece (0.92 ms for eight blocks of the 7B tower's widths, the time of an image up to 448 x 448)
 // and this one in 2-3.
 int pie_vision_blocks(const pie_vision_block *blocks, int n_blocks, int rows, int hidden, int inter, int heads, int head_dim, float eps, const float *cos_t, const float *sin_t, const int32_t *full_lo,
                       const int32_t *full_hi, const int32_t *win_lo, const int32_t *win_hi, int dtype, void *x, void *xn, void *workspace, size_t workspace_bytes, void *stream) {
@@ -354,7 +373,7 @@ int pie_vision_blocks(const pie_vision_block *blocks, int n_blocks, int rows, in
     PIE_REQUIRE(pie_aligned(workspace, 256), PIE_E_ALIGN, "pie_vision_blocks: the workspace needs 256-byte alignment");
     const VisionScratch z = vision_scratch(rows, hidden, inter, heads, head_dim);
     PIE_REQUIRE(workspace_bytes >= z.total(), PIE_E_ARG, "pie_vision_blocks: workspace smaller than pie_vision_blocks_workspace()");
-    const int DP = head_dim <= 64 ? 64 : 128, act_ld = (inter + 63) & ~63;
+    const int DP = vision_head_row(head_dim), act_ld = (inter + 63) & ~63;
     char *p = (char *)workspace;
     char *wide = p, *q = wide + z.wide, *k = q + z.head, *v = k + z.head, *att = v + z.head, *r = att + z.out, *slabs = r + z.out;
     const float scale = (float)(1.0 / sqrt((double)head_dim));
@@ -365,8 +384,11 @@ int pie_vision_blocks(const pie_vision_block *blocks, int n_blocks, int rows, in
         const pie_vision_block &b = blocks[i];
         PIE_REQUIRE(b.qkv_w && b.qkv_b && b.proj_w && b.proj_b && b.norm2 && b.gateup_w && b.gateup_b && b.down_w && b.down_b && b.next_norm, PIE_E_ARG, "pie_vision_blocks: null weight");
         int rc = linear(xn, hidden, b.qkv_w, 3 * hidden, hidden, wide);
-        if (!rc) rc = pie_vision_qkv_rope(wide, b.qkv_b, cos_t, sin_t, rows, heads, head_dim, DP, dtype, q, k, v, stream);
-        if (!rc) rc = segment_attn(q, k, v, b.full ? full_lo : win_lo, b.full ? full_hi : win_hi, rows, heads, DP, head_dim, scale, dtype, att, stream);
+        if (!rc && !b.full && segment_rot_serves(head_dim, b.qkv_b, cos_t, sin_t)) rc = segment_rot(wide, b.qkv_b, cos_t, sin_t, win_lo, win_hi, rows, heads, head_dim, scale, dtype, att, stream);
+        else {
+            if (!rc) rc = qkv_rope(wide, b.qkv_b, cos_t, sin_t, rows, heads, head_dim, DP, dtype, q, k, v, stream);
+            if (!rc) rc = segment_attn(q, k, v, b.full ? full_lo : win_lo, b.full ? full_hi : win_hi, rows, heads, DP, head_dim, scale, dtype, att, stream);
+        }
         if (!rc) rc = linear(att, hidden, b.proj_w, hidden, hidden, r);
         if (!rc) rc = pie_add_bias_rms_norm(x, r, b.proj_b, b.norm2, eps, rows, hidden, dtype, x, xn, stream);
         if (!rc) rc = pie_linear_w16m(xn, hidden, b.gateup_w, b.gateup_b, rows, 2 * inter, hidden, dtype, wide, act_ld, act_ld == inter ? 1 : PIE_SWIGLU_ZERO_REST, nullptr, 0, stream);

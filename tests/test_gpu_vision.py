@@ -222,6 +222,19 @@ def test_blocks_in_one_call_are_the_blocks_op_by_op(cfg, grid, dt):
     assert all(torch.equal(a, b) for a, b in zip(states, want_states))
 
 
+@pytest.mark.parametrize("head,grid", [(80, [(1, 34, 34)]), (80, [(1, 2, 6)]), (64, [(1, 40, 6)])])
+def test_windows_of_many_key_blocks_rotate_on_the_way_in(head, grid):
+    """Windows of 16 x 16 patches: up to nine blocks of 32 keys per workgroup, tiles that straddle windows, images smaller than one; the same bits as the rotation's own launch (op by op)."""
+    _, model = _tower(dict(CFG80, hidden_size=4 * head, num_heads=4, window_size=224), seed=12)
+    assert model._native is not None
+    pix = dev(po.round_T(np.random.default_rng(5).standard_normal((sum(t * h * w for t, h, w in grid), 3 * 2 * 14 * 14)), DT), DT)
+    got = model(pix, torch.tensor(grid))
+    table, model._native = model._native, None
+    want = model(pix, torch.tensor(grid))
+    model._native = table
+    assert torch.equal(got, want)
+
+
 def test_rows_of_padded_heads_are_the_projection_s_operand(monkeypatch):
     """A tower whose blocks go op by op (hidden 160): the attention's rows of 128 columns a head go into `proj` as they stand, with no copy and no padding in between."""
     from proxy_inference_engine_amd.models.intern import vision
