@@ -121,17 +121,24 @@ __device__ __forceinline__ void rows_finish(const RowsArgs &a, const RowsWork &k
 }
 
 __host__ __device__ __forceinline__ int rows_riders(const RowsArgs &a) { return (a.append.M > 0) + (a.cache.M > 0) + (a.rotate.M > 0); }
-// the last blockIdx.y: what rides along
+static void rows_slice(RowsArgs &a, unsigned x, int batches) {  // x: gridDim.x
+    const int M = std::max(a.append.M, std::max(a.cache.M, a.rotate.M));
+    a.ride_slices = M > 0 && batches < 65000 ? std::min(4, (M + (int)x - 1) / (int)x) : 1;
+}
+// the last blockIdx.y's, ride_slices each: what rides along, a row to a workgroup where rows and workgroups allow it (two rows one after the other outlast a small product: heads of [512, 128] beside 32 rows'
+// append 9.8 us, in two slices and with the norm weights asked for early 8.3)
 template <class E, int THREADS>
 __device__ __forceinline__ bool rows_ride(const RowsArgs &a, float *red) {
     int i = (int)(gridDim.y - 1 - blockIdx.y);
-    if (i >= rows_riders(a)) return false;
+    if (i >= rows_riders(a) * a.ride_slices) return false;
     if (blockIdx.z) return true;
+    const int slice = i % a.ride_slices;
+    i /= a.ride_slices;
     const bool append = a.append.M > 0 && i == 0;
     i -= a.append.M > 0;
     const bool cache = a.cache.M > 0 && i == 0;
     const int M = append ? a.append.M : cache ? a.cache.M : a.rotate.M;
-    for (int m = blockIdx.x; m < M; m += gridDim.x) {
+    for (int m = blockIdx.x + slice * gridDim.x; m < M; m += gridDim.x * a.ride_slices) {
         if (append) latent_append_row<E, ElemF32, THREADS>(a.append, m, red);
         else if (cache) latent_cache_row<E, THREADS>(a.cache, m, red);
         else rotate_row<E, THREADS>(a.rotate, m);
@@ -446,7 +453,8 @@ __global__ void __launch_bounds__(256) k_rows_f32(const RowsArgs a) {
 template <class E, int NT, int NN, int U, int WV = 8>
 int rows_lds_go(RowsArgs a, int n_max, int batches, hipStream_t st) {
     auto tiles = [](int n) { return (unsigned)((n + 16 * NN - 1) / (16 * NN)); };
-    dim3 grid(tiles(n_max), (unsigned)(batches + rows_riders(a)), (unsigned)((a.M + 16 * NT - 1) / (16 * NT)));
+    rows_slice(a, tiles(n_max), batches);
+    dim3 grid(tiles(n_max), (unsigned)(batches + rows_riders(a) * a.ride_slices), (unsigned)((a.M + 16 * NT - 1) / (16 * NT)));
     if (a.active) {  // one workgroup per tile of every expert, and it goes through all the expert's rows: most experts have few
         a.flat_batches = a.shared.w ? batches - 1 : batches, a.flat_tiles = (int)tiles(a.m.N);
         grid = dim3(a.flat_batches * a.flat_tiles + (a.shared.w ? tiles(a.shared.N) : 0));
@@ -485,13 +493,14 @@ int rows_lds_pick(const RowsArgs &a, int n_max, long blocks, int batches, hipStr
 }
 
 template <class E, int NT, int NN>
-int rows_go(const RowsArgs &a, int n_max, int k_max, int batches, hipStream_t st) {
+int rows_go(RowsArgs a, int n_max, int k_max, int batches, hipStream_t st) {
     const int steps = 2 * ((k_max + 63) / 64), tiles = (n_max + 16 * NN - 1) / (16 * NN);
     const int z = (a.M + 16 * NT - 1) / (16 * NT);  // (grouped: most experts have few rows, their later z leave at once)
     // waves along K: enough steps for each, and enough workgroups for the chip
     int kw = steps >= 32 ? 8 : steps >= 16 ? 4 : steps >= 8 ? 2 : 1;
     while (kw < 8 && steps >= 2 * kw && (size_t)((tiles + 8 / kw - 1) / (8 / kw)) * batches * z < 256) kw *= 2;
-    const dim3 grid((unsigned)((tiles + 8 / kw - 1) / (8 / kw)), (unsigned)(batches + rows_riders(a)), (unsigned)z);
+    rows_slice(a, (unsigned)((tiles + 8 / kw - 1) / (8 / kw)), batches);
+    const dim3 grid((unsigned)((tiles + 8 / kw - 1) / (8 / kw)), (unsigned)(batches + rows_riders(a) * a.ride_slices), (unsigned)z);
     auto go = [&](auto k8, auto k4, auto k2, auto k1) { hipLaunchKernelGGL((kw == 8 ? k8 : kw == 4 ? k4 : kw == 2 ? k2 : k1), grid, dim3(512), 0, st, a); };
     if constexpr (__is_same(E, ElemBF16)) {
         if (a.x_norm) go(&k_rows_w16m<E, 1, 8, 1, false, true>, &k_rows_w16m<E, 1, 4, 1, false, true>, &k_rows_w16m<E, 1, 2, 1, false, true>, &k_rows_w16m<E, 1, 1, 1, false, true>);
@@ -570,8 +579,10 @@ int rows_gemm_launch(int dtype, const RowsArgs &a, int batches, hipStream_t st) 
     }
     PIE_REQUIRE(!a.x_norm || (dtype == PIE_BF16 && a.M <= 16 && batches == 1 && !a.active && !a.shared.w && !a.rows && a.merge.splits <= 0), PIE_E_SHAPE, "row-wise Linear: too many rows to norm on the way in");
     if (dtype == PIE_F32) {
-        const dim3 grid((unsigned)((n_max + 15) / 16), (unsigned)(batches + rows_riders(a)), (unsigned)((a.M + 15) / 16));
-        hipLaunchKernelGGL(k_rows_f32, grid, dim3(256), 0, st, a);
+        RowsArgs f = a;
+        rows_slice(f, (unsigned)((n_max + 15) / 16), batches);
+        const dim3 grid((unsigned)((n_max + 15) / 16), (unsigned)(batches + rows_riders(a) * f.ride_slices), (unsigned)((a.M + 15) / 16));
+        hipLaunchKernelGGL(k_rows_f32, grid, dim3(256), 0, st, f);
         PIE_LAUNCH_CHECK();
         return PIE_OK;
     }

@@ -140,8 +140,10 @@ template <class E, class X, int THREADS>
 __device__ __forceinline__ void latent_append_row(const LatentAppend &a, int m, float *red) {  // red: THREADS / 64 floats of LDS
     const typename X::type *x = (const typename X::type *)a.c_raw + (size_t)m * a.ldc;
     const int t = a.pos[m], j = min(t / PAGE_TOKENS, a.table_width - 1);
-    float ss = 0.0f;
-    for (int r = threadIdx.x; r < a.R; r += THREADS) {
+    const bool has = (int)threadIdx.x < a.R;  // (a thread's first number and its weight are asked for before anything waits)
+    const float v0 = has ? X::load(x + threadIdx.x) : 0.0f, w0 = has ? a.w[threadIdx.x] : 0.0f;
+    float ss = v0 * v0;
+    for (int r = threadIdx.x + THREADS; r < a.R; r += THREADS) {
         const float v = X::load(x + r);
         ss = fmaf(v, v, ss);
     }
@@ -154,7 +156,8 @@ __device__ __forceinline__ void latent_append_row(const LatentAppend &a, int m, 
     for (int i = 1; i < THREADS / 64; ++i) sum += red[i];
     const float inv = 1.0f / sqrtf(sum / (float)a.R + a.eps);
     typename E::type *dst = (typename E::type *)a.slab + (page * PAGE_TOKENS + (t & (PAGE_TOKENS - 1))) * a.ldr;
-    for (int r = threadIdx.x; r < a.R; r += THREADS) dst[r] = E::pack(X::load(x + r) * inv * a.w[r]);
+    if (has) dst[threadIdx.x] = E::pack(v0 * inv * w0);
+    for (int r = threadIdx.x + THREADS; r < a.R; r += THREADS) dst[r] = E::pack(X::load(x + r) * inv * a.w[r]);
 }
 
 // rotation in halves: number i of a vector with number i + dims / 2, by position * freq[i], cos and sin times gain; what lies behind dims stays
@@ -360,6 +363,7 @@ struct RowsArgs {
     LatentAppend append;
     LatentPrepArgs cache;  // (the latent and key part only)
     RotateArgs rotate;     // (numbers of the same rows that this product does not read)
+    int ride_slices;       // blockIdx.y's that share a rider's rows (the launcher's)
 };
 // batches: blockIdx.y extent (1 for a plain Linear; heads; active experts (+ 1 with a shared expert))
 int rows_gemm_launch(int dtype, const RowsArgs &a, int batches, hipStream_t st);
