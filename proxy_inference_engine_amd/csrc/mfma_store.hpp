@@ -145,7 +145,15 @@ __global__ void __launch_bounds__(256) k_w4l_reduce(const float *part, int S, si
     const size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4;
     if (i >= MN) return;
     float4 a = *reinterpret_cast<const float4 *>(part + i);
-    for (int z = 1; z < S; ++z) {
+    int z = 1;
+    for (; z + 4 <= S; z += 4) {  // (four slabs in flight: a few rows wait for memory, slab after slab)
+        float4 b[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) b[j] = *reinterpret_cast<const float4 *>(part + (size_t)(z + j) * MN + i);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) a.x += b[j].x, a.y += b[j].y, a.z += b[j].z, a.w += b[j].w;
+    }
+    for (; z < S; ++z) {
         const float4 b = *reinterpret_cast<const float4 *>(part + (size_t)z * MN + i);
         a.x += b.x, a.y += b.y, a.z += b.z, a.w += b.w;
     }
