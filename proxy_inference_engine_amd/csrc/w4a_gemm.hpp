@@ -5,17 +5,18 @@
 // few rows that is most of its time.  Here
 //   * the codes are operands as they stand -- bf16: under the exponent of 128, one v_and_or for two, f16: less 1024 -- and a group's products are multiplied by its scale and joined by bias
 //     times the group's sum of x (another product, by ones) in fp32;
-//   * products are 16 x 16 x 32: sixteen rows and sixteen columns, the even or the odd ones of a strip (a v_permlane16_swap of two words makes two such operands of a tile's).  Up to eight
-//     rows, rows 8..15 of a product are the same rows against the odd columns (zeros in the others' place), so that no lane of the sums is idle;
-//   * a wave's K-phase is its own: it loads the x of its groups straight into the operand's lanes (a group of eight rows is one load) and waits for nothing but its loads, all of them ordinary
-//     ones, so that the compiler's waits are exact; the scales of a step's four strips are one load.
-// Bound by the stream, a launch (3 us) and the conversion, of which 1.7 us are not hidden.  us, weights from HBM, k_w4r_gemm / the form before (32 x 32 products, x by LDS-DMA, which the compiler's
-// waits do not count: rings shallower than written) / this, 8 rows: gate|up [28672, 4096] 18.0 / 17.0 / 14.0, down [4096, 14336] 11.1 / 10.6 / 8.9, q|k|v [6144, 4096] 7.2 / 6.7 / 6.0, o [4096, 4096]
-// 5.6 / 5.3 / 4.6, head [32768, 4096] 18.3 / 17.6 / 14.6; [16384, 3072] 9.8 / 9.9 / 8.0, [3072, 8192] 7.2 / 6.7 / 6.0.  16 rows: 17.9 / 18.4 / 15.1, 11.4 / 11.2 / 9.2, 7.3 / 7.6 / 6.2,
-// 5.6 / 6.0 / 4.6, 19.8 / 19.5 / 15.6.  32 rows of int4: 18.5 / 19.8 / 21.4, 11.6 / - / 13.0: k_w4r_gemm's.  Without the conversion gate|up takes 12.8 us, without any arithmetic 11.9 to 12.8.
-// Two steps in flight per wave are enough (eight waves of 4.6 KB each): three and four cost 1 and 2 us of gate|up's.  The last round issues no loads (loads past a wave's end return nothing but take their
-// slots: q|k|v 6.1 / 6.0, o 4.7 / 4.6, int8 down 12.7 / 12.3); both loops need the ring as whole vectors, see there.
-// Error (2-norm, before the rounding to T) against 64 bits: 9e-7; of weights rounded to bf16 1.7e-3.
+//   * products are 16 x 16 x 32: sixteen rows and sixteen columns, the even or the odd ones of a strip, of int8 one half of it (a v_permlane16_swap of two words makes two such operands of a
+//     tile's).  Up to eight rows, rows 8..15 of a product are the same rows against the strip's other columns (zeros in the others' place), so that no lane of the sums is idle;
+//   * a wave's K-phase is its own: it loads the x of its groups as whole lines, eight lanes to a row, turns them into operands in LDS of its own without a barrier, and waits for nothing but its
+//     loads, all of them ordinary ones, so that the compiler's waits are exact; the scales of a step's four strips are one load.  (x loaded straight into the operand's lanes: sixteen lanes side by
+//     side are sixteen rows, and each takes the load pipe a turn of its own.  Waves that share a CU with few strips and walk a long K then wait for x: us, that / this, [2048, 5632] 8 int4 rows 8.0 / 6.8, 32 int8
+//     rows 15.5 / 11.9, [10240, 8192] 8 int4 rows 13.7 / 12.6, 8 / 32 int8 rows 18.7 / 17.1, 27.0 / 24.0.  Two steps, [4096, 4096] in four splits, pay 0.1 to 0.3 us for the way through LDS: 4.5 / 4.6.)
+// Bound by the stream and a launch (3 us).  us, weights from HBM, k_w4r_gemm / 32 x 32 products with x by LDS-DMA / this, 8 rows: gate|up [28672, 4096] 17.2 / 15.4 / 13.4, down [4096, 14336] 10.2 / 9.9 / 8.3,
+// q|k|v [6144, 4096] 6.9 / 6.5 / 5.7, o [4096, 4096] 5.4 / 5.1 / 4.6, head [32768, 4096] 17.4 / 15.2 / 14.2; [16384, 3072] 9.2 / 9.3 / 7.5, [3072, 8192] 6.9 / 6.5 / 5.6, [2048, 5632] 8.6 / 7.6 / 6.8,
+// [10240, 8192] 15.5 / 14.2 / 12.6.  16 rows, k_w4r_gemm / this: 17.3 / 14.9, 10.8 / 8.9, 7.1 / 6.2, 5.6 / 4.8, 19.6 / 15.6, 9.2 / 8.2, 7.0 / 6.2, 8.8 / 8.0, 16.0 / 14.3.  32 rows of int4 are k_w4r_gemm's (gate|up 18.5 / 21.4).
+// Two steps in flight per wave are enough (three with one strip and eight rows: 256 strips of 8192 columns 10.5 / 9.7 us; three with four strips cost gate|up 1 us, sixteen waves gain nothing).  The last D
+// steps of a wave load nothing; where D does not divide the steps, the round before them still issues the loads of a step or two past the end, which return nothing.  Both loops need the ring as whole vectors, see there.
+// Error (2-norm, before the rounding to T, eight shapes, normal x) against 64 bits: 1.1e-6, that of the 32 x 32 products too; of weights rounded to bf16 1.7e-3.
 #pragma once
 
 constexpr int W4A_ROWS = 16, W8A_ROWS = 32;
@@ -24,7 +25,7 @@ struct W4aArgs {
     const char *w4m;   // W4M (W8M) tiles of the [N, K] matrix
     const u16 *x;      // [M, K]
     int M, N, K;
-    int strips;        // strips (32 columns) per workgroup
+    int halves;        // half strips (16 columns) per workgroup; int4: an even number
     int groups;        // of K (64 columns) per blockIdx.y
     u16 *y;            // STORE: [M, N]; SWIGLU: the activation [M, N / 2]
     float *part;       // SLAB: [gridDim.y][M][N] un-rounded fp32 sums
@@ -41,10 +42,12 @@ __device__ __forceinline__ uint4 w4a_codes(u32 w) {
 template <class T>
 constexpr float w4a_offset() { return std::is_same<T, F16>::value ? 0.0f : 128.0f; }
 
-// Int8 codes, W8M tiles: as W4M, 32 rows x 64 columns, two pieces of 1 KiB and the 32 {scale, bias} words: lane l = 32 kh + n holds in piece h the codes of row n of k-steps 2 h and 2 h + 1, two words
+// Int8 codes, W8M tiles: as W4M, 32 rows x 64 columns, two pieces of 1 KiB and the 32 {scale, bias} words (of rows 0, 16, 1, 17, ..): lane l = 32 kh + n holds in piece h the codes of row n of k-steps 2 h and 2 h + 1, two words
 // each, in the W8S word format (codes 0, 2, 1, 3).  Up to 255 a code is a bf16 and an f16 as it stands.
-// Bound by the stream, half the bytes of a 16-bit copy's.  us, the form with 32 x 32 products / this, 8 rows: gate|up 23.3 / 22.1, down 13.3 / 12.3, q|k|v 8.8 / 7.5, o 6.5 / 5.6, head 24.9 / 24.0; 32 rows: 27.0 / 26.8,
-// 17.1 / 16.6, 12.1 / 10.2, 8.8 / 7.0, 28.4 / 28.0.
+// The tile's halves are a product's two operands as they are read, so that a workgroup may take half strips of 16 columns and the lanes of the other half load nothing; a word of one half's scales
+// lies beside the other half's.
+// Bound by the stream, half the bytes of a 16-bit copy's.  us, the form with 32 x 32 products / this, 8 rows: gate|up 22.2 / 21.2, down 12.7 / 11.8, q|k|v 8.2 / 7.1, o 6.3 / 5.5, head 23.7 / 22.9, [2048, 5632] 7.8 / 7.6,
+// [10240, 8192] 18.5 / 17.1; 32 rows: 25.7 / 25.8, 16.2 / 15.1, 11.1 / 9.9, 8.5 / 7.0, 27.3 / 27.0, 12.6 / 11.9, 24.7 / 24.0.  Slower than that form: 17 to 32 rows of 513 to 800 strips, by 2 to 3 %.
 template <class T>
 __device__ __forceinline__ u32 w8a_pair(u32 a, u32 b) {  // two codes as T, b in the high half
     if constexpr (std::is_same<T, F16>::value) return __builtin_bit_cast(u32, __builtin_amdgcn_cvt_pkrtz((float)a, (float)b));
@@ -70,46 +73,50 @@ __device__ __forceinline__ void w4a_swap32(u32 &a, u32 &b) {  // the upper lanes
     const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
     a = r[0], b = r[1];
 }
-// lanes 0..7 of every 16 (LOW: for themselves, else 8..15) to lanes AT .. + 7, the others zero
-template <bool LOW, int AT>
-__device__ __forceinline__ u32 w4a_eight(u32 v) {
-    constexpr int from = LOW ? 0 : 8, ctrl = from == AT ? 0xE4 : 0x128;  // quad_perm 0 1 2 3 / row_ror:8
-    return (u32)__builtin_amdgcn_update_dpp(0, (int)v, ctrl, 0xF, AT ? 0xC : 0x3, false);
-}
-template <bool LOW, int AT>
-__device__ __forceinline__ uint4 w4a_eight(const uint4 &v) { return make_uint4(w4a_eight<LOW, AT>(v.x), w4a_eight<LOW, AT>(v.y), w4a_eight<LOW, AT>(v.z), w4a_eight<LOW, AT>(v.w)); }
-
 template <class T, int MT, int SPW, int D, int BITS = 4>
 __global__ void __launch_bounds__(512) k_w4a_gemm(const W4aArgs a, const W4mRope rp) {
     constexpr int PC = BITS / 4, TILE = BITS == 8 ? W8M_TILE_BYTES : W4M_TILE_BYTES;  // code pieces (16 bytes a lane) of a tile; bytes of one
     constexpr int KW = 8, RB = (MT + 15) / 16;                  // K-phases = waves; blocks of 16 rows
-    constexpr bool PAIR = MT == 8;                              // rows 8..15 of a product: the strip's odd columns
-    constexpr int XL = PAIR ? 1 : 2 * RB;                       // loads of x per step, 1 KiB each
-    constexpr int AC = PAIR ? 1 : 2 * RB;                       // accumulators of a strip: [block][even, odd columns]
+    constexpr bool PAIR = MT == 8;                              // rows 8..15 of a product: the strip's other columns
+    constexpr int XL = MT / 8, XB = MT * 128 + (PAIR ? 16 : 0); // loads of x per step, 1 KiB each; a wave's image of them
+    constexpr int AC = PAIR ? 1 : 2 * RB;                       // accumulators of a strip: [block][operand]
     constexpr int RSTR = 36, BLK = MT * RSTR * 4;               // reduction: one (phase, strip) block, rows of 32 + 4 floats
     constexpr unsigned NOWHERE = 0x80000000u;
     static_assert(SPW <= 4 && D * (XL + 1 + SPW * PC) <= 63, "a strip to 16 lanes of the scales' load; loads in flight");
-    __shared__ __attribute__((aligned(16))) char smem[KW * SPW * BLK];
+    constexpr bool APART = KW * (SPW * BLK + XB) <= 80 * 1024;  // the sums beside the images, two workgroups to a CU; else in their place
+    __shared__ __attribute__((aligned(128))) char smem[KW * (APART ? SPW * BLK + XB : SPW * BLK > XB ? SPW * BLK : XB)];
     const int lane = threadIdx.x & 63, p = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int c16 = lane & 15, r16 = lane >> 4;
     const int all_groups = a.K >> 6;
     const int g_lo = blockIdx.y * a.groups + p, g_hi = min(all_groups, ((int)blockIdx.y + 1) * a.groups);  // this wave's groups: g_lo, g_lo + 8, ..
     const int steps = g_hi > g_lo ? (g_hi - g_lo + KW - 1) / KW : 0;
-    const int strip0 = blockIdx.x * a.strips, n_strips = min(a.strips, (a.N >> 5) - strip0);
+    const int h0 = blockIdx.x * a.halves, h1 = min(h0 + a.halves, a.N >> 4), strip0 = h0 >> 1, n_strips = ((h1 + 1) >> 1) - strip0;
     const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>(a.w4m), 0, (a.N >> 5) * all_groups * TILE, 0x00020000);
     const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<u16 *>(a.x), 0, a.M * a.K * 2, 0x00020000);
-    // lanes by 16: the even and the odd columns' codes of a k-step's first eight numbers, of its other eight; the scales of strips 0 .. 3, an even and an odd column's
-    const unsigned code_at = 16u * (32 * (r16 >> 1) + 2 * c16 + (r16 & 1)), scale_at = r16 < n_strips ? (unsigned)(r16 * all_groups * TILE) + 1024u * PC + 8u * c16 : NOWHERE;
+    // lanes by 16: one and the other operand's columns (int4: the even, the odd ones; int8: the strip's halves) of a k-step's first eight numbers, of its other eight; the scales of strips 0 .. 3, a column
+    // of each operand
+    const unsigned code_at = 16u * (BITS == 8 ? lane : 32 * (r16 >> 1) + 2 * c16 + (r16 & 1)), scale_at = r16 < n_strips ? (unsigned)(r16 * all_groups * TILE) + 1024u * PC + 8u * c16 : NOWHERE;
     unsigned strip_at[SPW], gone[SPW];
 #pragma unroll
-    for (int s = 0; s < SPW; ++s) strip_at[s] = (unsigned)((strip0 + s) * all_groups + g_lo) * TILE, gone[s] = s < n_strips ? 0u : NOWHERE;
-    // A product takes 32 columns of x: runs of eight 0, 2, 1, 3 of one half of a group (as the tile's words lie), a run to 16 lanes.  PAIR: the lanes of rows 8..15 load the group's other half
-    unsigned x_at[RB];
-#pragma unroll
-    for (int t = 0; t < RB; ++t) {
-        const int r = PAIR ? c16 & 7 : 16 * t + c16;
-        x_at[t] = r < a.M ? (unsigned)(r * a.K + 16 * (r16 & 1) + 8 * (r16 >> 1) + (PAIR ? 32 * (c16 >> 3) : 0)) * 2u : NOWHERE;  // (rows past the end are zeros)
+    for (int s = 0; s < SPW; ++s) {
+        const int h = 2 * (strip0 + s) + (BITS == 8 ? r16 & 1 : 0);
+        strip_at[s] = (unsigned)((strip0 + s) * all_groups + g_lo) * TILE, gone[s] = h >= h0 && h < h1 ? 0u : NOWHERE;
     }
+    // A group of eight rows of x is one load of whole lines, eight lanes to a row; the wave's own LDS turns it into the operands: runs of eight columns 0, 2, 1, 3 of one half of a group (as the tile's
+    // words lie), a run to 16 lanes; a row's pieces rotated by the row.  PAIR: the lanes of the other rows read zeros
+    unsigned x_at[XL];
+#pragma unroll
+    for (int i = 0; i < XL; ++i) {
+        const int r = 8 * i + (lane >> 3);
+        x_at[i] = r < a.M ? (unsigned)(r * a.K + 8 * (lane & 7)) * 2u : NOWHERE;  // (rows past the end are zeros)
+    }
+    char *x_lds = smem + (APART ? KW * SPW * BLK : 0) + p * XB;
+    char *x_put = x_lds + (lane >> 3) * 128 + (((lane & 7) ^ (lane >> 3)) << 4);
+    const int run = 2 * (r16 & 1) + (r16 >> 1), xrow = PAIR ? c16 & 7 : c16;
+    const char *x_get[2];  // a half of the group each
+#pragma unroll
+    for (int h = 0; h < 2; ++h) x_get[h] = x_lds + xrow * 128 + (((4 * h + run) ^ (xrow & 7)) << 4);
+    if (PAIR && lane < 4) *reinterpret_cast<u32 *>(x_lds + MT * 128 + 4 * lane) = 0;
     typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
     typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
     u32x4 xv[D][XL], cw[D][SPW][PC];  // (as vectors: split into words they would be copied from round to round, waited for right behind their loads)
@@ -117,7 +124,7 @@ __global__ void __launch_bounds__(512) k_w4a_gemm(const W4aArgs a, const W4mRope
     auto issue = [&](int d, int j) {
         const unsigned dead = j < steps ? 0u : NOWHERE, o = (unsigned)j * (KW * TILE), xo = (unsigned)(g_lo + j * KW) * 128u;
 #pragma unroll
-        for (int t = 0; t < XL; ++t) xv[d][t] = __builtin_amdgcn_raw_buffer_load_b128(xr, (x_at[PAIR ? 0 : t >> 1] | dead) + 64u * (t & 1), xo, 0);
+        for (int t = 0; t < XL; ++t) xv[d][t] = __builtin_amdgcn_raw_buffer_load_b128(xr, x_at[t] | dead, xo, 0);
         sb[d] = __builtin_amdgcn_raw_buffer_load_b64(wr, scale_at | dead, strip_at[0] + o, 2);
 #pragma unroll
         for (int s = 0; s < SPW; ++s)
@@ -138,16 +145,22 @@ __global__ void __launch_bounds__(512) k_w4a_gemm(const W4aArgs a, const W4mRope
     const uint4 ones = make_uint4(one, one, one, one);
     auto words = [](const u32x4 &v) { return make_uint4(v.x, v.y, v.z, v.w); };
     auto compute = [&](int d) {
-        uint4 xa[PAIR ? 4 : XL];  // PAIR: the group's halves as rows 0..7, as rows 8..15
-        if constexpr (PAIR) xa[0] = w4a_eight<true, 0>(words(xv[d][0])), xa[1] = w4a_eight<false, 0>(words(xv[d][0])), xa[2] = w4a_eight<true, 8>(words(xv[d][0])), xa[3] = w4a_eight<false, 8>(words(xv[d][0]));
-        else
+        uint4 xa[PAIR ? 4 : 2 * RB];  // [block][half]; PAIR: the group's halves as rows 0..7, as rows 8..15
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // (the wave's lanes meet in LDS, whose operations go in order)
 #pragma unroll
-            for (int t = 0; t < XL; ++t) xa[t] = words(xv[d][t]);
+        for (int t = 0; t < XL; ++t) *reinterpret_cast<u32x4 *>(x_put + 1024 * t) = xv[d][t];
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int t = 0; t < (PAIR ? 4 : 2 * RB); ++t) {
+            const char *q = PAIR ? (t >> 1) == (c16 >> 3) ? x_get[t & 1] : x_lds + MT * 128 : x_get[t & 1] + 2048 * (t >> 1);
+            xa[t] = *reinterpret_cast<const uint4 *>(q);
+        }
         w4a_f32x4 xs[RB];
 #pragma unroll
         for (int t = 0; t < RB; ++t) xs[t] = w4a_mfma<T>(xa[2 * t + 1], ones, w4a_mfma<T>(xa[2 * t], ones, zero));
         if constexpr (PAIR) xs[0] = w4a_mfma<T>(xa[3], ones, w4a_mfma<T>(xa[2], ones, xs[0]));
-        u32 sw[4][2];  // every lane's scale word of a strip's even, of its odd column; PAIR: the one of the rows that it sums
+        u32 sw[4][2];  // every lane's scale word of a strip's column of one, of the other operand; PAIR: the one of the rows that it sums
         {
             u32 e0 = sb[d].x, e1 = sb[d].x, o0 = sb[d].y, o1 = sb[d].y;
             w4a_swap16(e0, e1), w4a_swap16(o0, o1);  // strips 0 0 2 2, 1 1 3 3
@@ -165,7 +178,7 @@ __global__ void __launch_bounds__(512) k_w4a_gemm(const W4aArgs a, const W4mRope
             float sc[2], bi[2];
 #pragma unroll
             for (int h = 0; h < (PAIR ? 1 : 2); ++h) sc[h] = lo_f32<T>(sw[s][h]), bi[h] = BITS == 8 ? hi_f32<T>(sw[s][h]) : fmaf(-w4a_offset<T>(), sc[h], hi_f32<T>(sw[s][h]));
-            uint4 wf[2][2];  // [even, odd columns][half of the group]
+            uint4 wf[2][2];  // [operand][half of the group]
             if constexpr (BITS == 8) {
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {
@@ -209,7 +222,8 @@ __global__ void __launch_bounds__(512) k_w4a_gemm(const W4aArgs a, const W4mRope
         for (int d = 0; d < D; ++d)
             if (base + d < steps) compute(d);
     }
-    // a product's lane: columns 2 c16 (+ 1), rows 4 r16 .. + 3
+    if (!APART) __syncthreads();
+    // a product's lane: columns 2 c16 (+ 1), int8 c16 (+ 16), rows 4 r16 .. + 3
 #pragma unroll
     for (int s = 0; s < SPW; ++s)
 #pragma unroll
@@ -218,14 +232,14 @@ __global__ void __launch_bounds__(512) k_w4a_gemm(const W4aArgs a, const W4mRope
             for (int h = 0; h < (PAIR ? 1 : 2); ++h)
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    const int row = 4 * r16 + i, m = PAIR ? row & 7 : 16 * t + row, col = 2 * c16 + (PAIR ? row >> 3 : h);
+                    const int row = 4 * r16 + i, m = PAIR ? row & 7 : 16 * t + row, o = PAIR ? row >> 3 : h, col = BITS == 8 ? c16 + 16 * o : 2 * c16 + o;
                     *reinterpret_cast<float *>(smem + (p * SPW + s) * BLK + (m * RSTR + col) * 4) = acc[s][PAIR ? 0 : 2 * t + h][i];
                 }
     __syncthreads();
     const int EPI = a.epi;
     for (int o = threadIdx.x; o < MT * SPW * 4; o += 512) {  // a row's eight columns
         const int m = o / (4 * SPW), ts = (o >> 2) % SPW, ec = o & 3, col = 32 * (strip0 + ts) + 8 * ec;
-        if (m >= a.M || ts >= n_strips) continue;
+        if (m >= a.M || col >> 4 < h0 || col >> 4 >= h1) continue;
         float v[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int ph = 0; ph < KW; ++ph) {

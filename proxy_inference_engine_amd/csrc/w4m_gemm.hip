@@ -801,7 +801,7 @@ __global__ void __launch_bounds__(256) k_w8s_to_w8m(const u32 *w8s, int N, int K
     u32 *tile = w8m + ((size_t)nt * groups + g) * (W8M_TILE_BYTES / 4);
     const uint2 a = *reinterpret_cast<const uint2 *>(unit + 512 * q + 4 * src_lane + 2 * kh), b = *reinterpret_cast<const uint2 *>(unit + 512 * q + 256 + 4 * src_lane + 2 * kh);  // k-steps 2 q, 2 q + 1
     *reinterpret_cast<uint4 *>(tile + 256 * q + 4 * lane) = make_uint4(a.x, a.y, b.x, b.y);
-    if (q == 0 && kh == 0) tile[512 + n] = unit[1024 + src_lane];
+    if (q == 0 && kh == 0) tile[512 + 2 * (n & 15) + (n >> 4)] = unit[1024 + src_lane];
 }
 int w8m_repack_launch(const void *w8s, int N, int K, void *w8m, hipStream_t st) {
     PIE_REQUIRE(N > 0 && K > 0 && N % 32 == 0 && K % 64 == 0, PIE_E_SHAPE, "W8M repack: N must be a multiple of 32 and K of 64");
@@ -810,28 +810,30 @@ int w8m_repack_launch(const void *w8s, int N, int K, void *w8m, hipStream_t st) 
     PIE_LAUNCH_CHECK();
     return PIE_OK;
 }
-// Up to 16 rows (32 of int8 codes) with the scales on the sums (k_w4a_gemm).  Workgroups of as many strips as give every CU one (at most four: 896 strips in 224 workgroups 14.0 us, two strips each 15.4,
-// three 19.1; 640 in threes 11.5, in twos 14.9, in fours 13.0; 384 in twos 9.2, one by one 10.9; 352 of 2048 columns in twos 6.3, one by one 7.2); what stays below 512 strips takes two and splits of K, in one round of
+// Up to 16 rows (32 of int8 codes) with the scales on the sums (k_w4a_gemm).  Workgroups of as many strips as give every CU one (at most four: 896 strips in 224 workgroups 13.4 us, two strips each 15.4,
+// three 19.1; 640 in threes 10.8, in twos 14.9, in fours 13.0; 384 in twos 8.3, one by one 10.9; 352 of 2048 columns in twos 5.9, one by one 7.2; just above a boundary, 4096 columns: 258 in twos 8.1, one by one 8.6,
+// 514 in threes 10.3, in fours 12.0; 256 workgroups of which some take a strip more than others are level but at 258 and 514), of half strips for int8 (whole ones / this, 8192 columns, us: 66 strips, 8 / 16 / 32 rows 10.9 / 10.1, 12.7 / 11.4,
+// 16.8 / 15.6; 258 18.0 / 16.4, 20.0 / 18.7, 24.6 / 23.4; 514 26.0 / 25.2, 28.0 / 27.2, 33.0 / 32.3); what stays below 512 strips takes two and splits of K, in one round of
 // workgroups and of at least two steps: q|k|v two splits, o_proj and down four (8 rows, two strips in splits / one strip in half as many: q|k|v 6.1 / 7.1 us, o_proj 4.7 / 5.1, [3072, 8192] 6.1 / 7.0, [8192, 4096] 6.6 / 7.4).
 struct W4aPlan {
-    int strips, S, groups;  // strips per workgroup; K splits, groups of each; strips == 0: shape not served
+    int halves, S, groups;  // half strips per workgroup (int4: whole ones); K splits, groups of each; halves == 0: shape not served
 };
 static W4aPlan w4a_plan(int M, int N, int K, bool may_split, int bits) {
     if (M < 1 || M > (bits == 8 ? W8A_ROWS : W4A_ROWS) || N < 32 || N % 32 || K < 64 || K % 64 || (bits == 8 ? w8m_bytes(N, K) : w4m_bytes(N, K)) >= (1ull << 31)) return {0, 0, 0};
     const int strips = N / 32, groups = K / 64, steps = (groups + 7) / 8;
-    const int each = strips >= 1024 ? 4 : (strips + 255) / 256;
+    const int each = strips >= 1024 ? 8 : bits == 8 ? (N / 16 + 255) / 256 : 2 * ((strips + 255) / 256);
     if (strips >= 512 || !may_split) return {each, 1, 8 * steps};
     const int wgs = (strips + 1) / 2;
     int S = 1;
     for (int n = 2; n <= 8 && n * wgs <= 256; ++n)
         if (steps % n == 0 && steps / n >= 2) S = n;
     if (S == 1) return {each, 1, 8 * steps};
-    return {2, S, 8 * (steps / S)};
+    return {4, S, 8 * (steps / S)};
 }
 // step: a batch's step, whose rows are single sequences' in the one-row arithmetic.  A prompt of 9 to 16 rows keeps weights rounded to T, as mx.quantized_matmul's matrix kernels have them from six rows on, in
 // its narrow products (k_w4r_gemm).
 bool w4a_serves(int M, int N, int K, int bits, bool step) {
-    return pie_knob(PIE_KNOB_W4R) != 0 && w4a_plan(M, N, K, false, bits).strips != 0 && (step || bits == 8 || M <= 8 || N >= 512 * 32);
+    return pie_knob(PIE_KNOB_W4R) != 0 && w4a_plan(M, N, K, false, bits).halves != 0 && (step || bits == 8 || M <= 8 || N >= 512 * 32);
 }
 int w4a_splits(int M, int N, int K, int bits) { return w4a_plan(M, N, K, true, bits).S; }
 size_t w4a_workspace_bytes(int M, int N, int K, int bits) {
@@ -840,9 +842,9 @@ size_t w4a_workspace_bytes(int M, int N, int K, int bits) {
 }
 template <class T, int MT, int BITS>
 static void w4a_go(const W4aArgs &a, int S, hipStream_t st, const W4mRope &r) {
-    const dim3 grid((unsigned)((a.N / 32 + a.strips - 1) / a.strips), (unsigned)S), block(512);
-    switch (a.strips) {
-    case 1: hipLaunchKernelGGL((k_w4a_gemm<T, MT, 1, 2, BITS>), grid, block, 0, st, a, r); break;
+    const dim3 grid((unsigned)((a.N / 16 + a.halves - 1) / a.halves), (unsigned)S), block(512);
+    switch ((a.halves + 1) / 2) {
+    case 1: hipLaunchKernelGGL((k_w4a_gemm<T, MT, 1, MT == 8 ? 3 : 2, BITS>), grid, block, 0, st, a, r); break;
     case 2: hipLaunchKernelGGL((k_w4a_gemm<T, MT, 2, 2, BITS>), grid, block, 0, st, a, r); break;
     case 3: hipLaunchKernelGGL((k_w4a_gemm<T, MT, 3, 2, BITS>), grid, block, 0, st, a, r); break;
     default: hipLaunchKernelGGL((k_w4a_gemm<T, MT, 4, 2, BITS>), grid, block, 0, st, a, r); break;
@@ -857,9 +859,9 @@ int w4a_gemm_launch(int dtype, const void *w4m, const void *x, int M, int N, int
     PIE_REQUIRE((epi == W4R_ROPE) == (rope != nullptr), PIE_E_ARG, "W4A GEMM: the q|k|v epilogue needs its arguments");
     const bool may_split = epi == W4R_STORE && workspace != nullptr && slabs != nullptr;  // (the caller's consumer sums them)
     const W4aPlan pl = w4a_plan(M, N, K, may_split, bits);
-    PIE_REQUIRE(pl.strips != 0, PIE_E_SHAPE, "W4A GEMM: 1..16 rows (32 of int8 codes), N a multiple of 32, K of 64");
+    PIE_REQUIRE(pl.halves != 0, PIE_E_SHAPE, "W4A GEMM: 1..16 rows (32 of int8 codes), N a multiple of 32, K of 64");
     PIE_REQUIRE(pie_aligned(w4m, 16) && pie_aligned(x, 16) && pie_aligned(y, 16) && pie_aligned(bias, 16), PIE_E_ALIGN, "W4A GEMM: 16-byte alignment required");
-    const W4aArgs a = {(const char *)w4m, (const u16 *)x, M, N, K, pl.strips, pl.groups, (u16 *)y, pl.S > 1 ? (float *)workspace : nullptr, pl.S > 1 ? nullptr : (const u16 *)bias,
+    const W4aArgs a = {(const char *)w4m, (const u16 *)x, M, N, K, pl.halves, pl.groups, (u16 *)y, pl.S > 1 ? (float *)workspace : nullptr, pl.S > 1 ? nullptr : (const u16 *)bias,
                        pl.S > 1 ? W4R_SLAB : epi};
     const W4mRope r = rope ? *rope : W4mRope{};
     auto rows = [&](auto t, auto width) {

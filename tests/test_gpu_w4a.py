@@ -10,9 +10,9 @@ pytestmark = pytest.mark.gpu
 
 
 # [N, K] in strips of 32 and groups of 64: hidden 192: 3 groups; 1088: 17, every matrix strip by strip; 2048: gate|up in twos, vocab in threes, o_proj and down split; 512: gate|up in fours, vocab too, in
-# 268 workgroups; 4096: q|k|v, o_proj and down in twos, split
+# 268 workgroups; 4096: q|k|v, o_proj and down in twos, split; 3136: q|k|v, o_proj and gate|up strip by strip, seven steps a wave, down two
 @pytest.mark.parametrize("hidden,inter,vocab,heads,kv,dim,bias", [(192, 448, 96, 4, 2, 64, True), (1088, 1472, 5216, 17, 17, 64, False), (2048, 5632, 16896, 16, 4, 128, True),
-                                                                  (512, 14336, 34240, 8, 2, 64, False), (4096, 4096, 12320, 32, 8, 128, False)])
+                                                                  (512, 14336, 34240, 8, 2, 64, False), (4096, 4096, 12320, 32, 8, 128, False), (3136, 1024, 96, 49, 7, 64, False)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
 def test_rows_against_single_sequences(hidden, inter, vocab, heads, kv, dim, bias, dtype):
     """One layer, every sequence's step alone (the GEMV, the same arithmetic: fp32 sums of unrounded weights, one rounding) as the reference: four ulps of the largest logit, rms four ulps, as everywhere."""

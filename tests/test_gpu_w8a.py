@@ -1,4 +1,4 @@
-"""Int8 models' steps of several sequences on the codes themselves (k_w4a_gemm, W8M tiles): fewer groups of K than waves, groups that are no multiple of eight, splits of K, every count of strips per
+"""Int8 models' steps of several sequences on the codes themselves (k_w4a_gemm, W8M tiles): fewer groups of K than waves, groups that are no multiple of eight, splits of K, every count of half strips per
 workgroup, a last workgroup that is not full, eight, sixteen and 32 rows and the 33 that go another way, biases."""
 import numpy as np
 import pytest
@@ -9,9 +9,10 @@ from _util import assert_vec_close
 pytestmark = pytest.mark.gpu
 
 
-# [N, K] in strips of 32 and groups of 64: hidden 192: 3 groups; 1088: 17, every matrix strip by strip; 2048: gate|up in twos, vocab in threes, o_proj and down split; 512: gate|up in fours, vocab too,
-# in 268 workgroups
-@pytest.mark.parametrize("hidden,inter,vocab,heads,kv,dim,bias", [(192, 448, 96, 4, 2, 64, True), (1088, 1472, 5216, 17, 17, 64, False), (2048, 5632, 16896, 16, 4, 128, True), (512, 14336, 34240, 8, 2, 64, False)])
+# [N, K] in half strips of 16 and groups of 64: hidden 192: 3 groups; 1088: 17, q|k|v in one, vocab in two; 2048: gate|up in three, vocab in five, o_proj and down split; 512: gate|up in seven, vocab
+# in eight, in 268 workgroups; 3136: q|k|v, o_proj and gate|up in one, seven steps a wave, down two
+@pytest.mark.parametrize("hidden,inter,vocab,heads,kv,dim,bias", [(192, 448, 96, 4, 2, 64, True), (1088, 1472, 5216, 17, 17, 64, False), (2048, 5632, 16896, 16, 4, 128, True), (512, 14336, 34240, 8, 2, 64, False),
+                                                                  (3136, 1024, 96, 49, 7, 64, False)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
 def test_rows_against_single_sequences(hidden, inter, vocab, heads, kv, dim, bias, dtype):
     """One layer, every sequence's step alone (the GEMV: fp32 sums of unrounded weights, one rounding) as the reference: four ulps of the largest logit, rms four ulps, as everywhere; 33 rows multiply
