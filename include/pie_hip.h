@@ -548,11 +548,11 @@ int pie_sdpa_segments(const void *q, const void *k, const void *v, const int32_t
 /* pie_vision_blocks: the tower's blocks (vision.py:203-218) one behind the other in one call: xn holds norm1 of the first block of x on entry, x and xn (T [rows, hidden], both updated in
  *   place) the residual stream and next_norm of it on return.  Weights: W16M tiles (pie_repack_w16m) of qkv [3 hidden, hidden], proj [hidden, hidden], gate | up interleaved row by row
  *   [2 inter, hidden], down [hidden, inter]; biases, gate | up's interleaved too; full: the block attends over full_lo / full_hi, else win_lo / win_hi (as pie_sdpa_segments); cos / sin as
- *   pie_vision_qkv_rope.  hidden = heads * head_dim, a multiple of 64 up to 8192; inter, head_dim multiples of 4, head_dim <= 128.  workspace: pie_vision_blocks_workspace() bytes,
+ *   pie_vision_qkv_rope.  window: rows of the longest window, 0 where that is not known (windows of up to 64 rows rotate on their way into the attention; the results are the same).  hidden = heads * head_dim, a multiple of 64 up to 8192; inter, head_dim multiples of 4, head_dim <= 128.  workspace: pie_vision_blocks_workspace() bytes,
  *   256-byte aligned (0: a shape that is not served). */
 typedef struct pie_vision_block {
     const void *qkv_w, *qkv_b, *proj_w, *proj_b, *norm2, *gateup_w, *gateup_b, *down_w, *down_b, *next_norm;
-    int full;
+    int full, window;
 } pie_vision_block;
 size_t pie_vision_blocks_workspace(int rows, int hidden, int inter, int heads, int head_dim);
 int pie_vision_blocks(const pie_vision_block *blocks, int n_blocks, int rows, int hidden, int inter, int heads, int head_dim, float eps, const float *cos_t, const float *sin_t,

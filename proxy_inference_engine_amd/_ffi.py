@@ -71,7 +71,7 @@ class pie_global_weights(C.Structure):
 
 
 class pie_vision_block(C.Structure):
-    _fields_ = [(n, C.c_void_p) for n in ("qkv_w", "qkv_b", "proj_w", "proj_b", "norm2", "gateup_w", "gateup_b", "down_w", "down_b", "next_norm")] + [("full", C.c_int)]
+    _fields_ = [(n, C.c_void_p) for n in ("qkv_w", "qkv_b", "proj_w", "proj_b", "norm2", "gateup_w", "gateup_b", "down_w", "down_b", "next_norm")] + [("full", C.c_int), ("window", C.c_int)]
 
 
 class pie_stack_norm(C.Structure):

@@ -104,7 +104,7 @@ __device__ __forceinline__ int pa_off(int row, int ch) {
 // and no padding.  The 7B vision tower's widths, 1024 patches, us: windows of 64 7.9 -> 6.6, whole image 54 -> 46.
 // ROT: windows straight from the qkv Linear's rows: bias and rotation on the way into LDS, by twice the waves (the second half of them does nothing else), queries and the first 64 keys asked for before anything
 // waits; with the blocks of 32 keys of the others, so that the sums are theirs bit for bit.  Bound by the chain bounds -> rows -> LDS -> scores of one round of workgroups.  A window's keys are rotated once
-// per 64 query rows that see them; rotated in a launch of their own, as a whole image's still are (32 tiles would each rotate all keys), they cost 8 us beside the attention's 6.6, here 10.1 in all (12.0 with
+// per 64 query rows that see them; rotated in a launch of their own, as a whole image's and long windows' still are (32 tiles would each rotate all keys), they cost 8 us beside the attention's 6.6, here 10.1 in all (12.0 with
 // as many waves as tiles and no early queries).
 template <class T, int D, int REP, int QT, bool SEG = false, bool SPLIT = false, bool SHORT = false, int KG = 1, int DR = D, bool ROT = false>
 __global__ void __launch_bounds__(REP * QT * KG * 64 * (ROT ? 2 : 1), 2) k_prefill_attn(const PrefillAttnArgs a) {

@@ -322,9 +322,12 @@ static int segment_attn(const void *q, const void *k, const void *v, const int32
     return pie::fail(PIE_E_ARG, "pie_sdpa_segments: dtype must be PIE_BF16 or PIE_F16");
 }
 
-// The attention of a block over windows, from the qkv Linear's rows (no bias yet): heads of 64 and 80
-static bool segment_rot_serves(int head_dim, const void *bias, const float *cos_t, const float *sin_t) {
-    return (head_dim == 64 || head_dim == 80) && pie_aligned(bias, 16) && pie_aligned(cos_t, 16) && pie_aligned(sin_t, 16);
+// The attention of a block over windows, from the qkv Linear's rows (no bias yet): heads of 64 and 80, windows that a tile of 64 query rows covers.  A longer one's keys are rotated again by every tile
+// of its rows, 64 at a time behind a barrier with no loads in flight.  us a block of the tower's 16 heads of 80, rotation in a launch of its own / here, 256 / 1024 / 2304 / 4096 patches: windows of 64 two / four / one /
+// six less here; of 100 level, level, 6 and 12 more; of 144 level, 1, 8 and 16 more; of 256 1, level, 11 and 10 more; of 1024 level, 12, 25 and 77 more.  Heads of 64: of 64 five to seven less here, of 100 to 256 three less
+// to five more.
+static bool segment_rot_serves(int window, int head_dim, const void *bias, const float *cos_t, const float *sin_t) {
+    return window > 0 && window <= 64 && (head_dim == 64 || head_dim == 80) && pie_aligned(bias, 16) && pie_aligned(cos_t, 16) && pie_aligned(sin_t, 16);
 }
 static int segment_rot(const void *qkv, const void *bias, const float *cos_t, const float *sin_t, const int32_t *seg_lo, const int32_t *seg_hi, int N, int H, int D, float scale, int dtype, void *out, void *stream) {
     PIE_REQUIRE(dtype == PIE_BF16 || dtype == PIE_F16, PIE_E_ARG, "segment attention: dtype must be PIE_BF16 or PIE_F16");
@@ -384,7 +387,7 @@ int pie_vision_blocks(const pie_vision_block *blocks, int n_blocks, int rows, in
         const pie_vision_block &b = blocks[i];
         PIE_REQUIRE(b.qkv_w && b.qkv_b && b.proj_w && b.proj_b && b.norm2 && b.gateup_w && b.gateup_b && b.down_w && b.down_b && b.next_norm, PIE_E_ARG, "pie_vision_blocks: null weight");
         int rc = linear(xn, hidden, b.qkv_w, 3 * hidden, hidden, wide);
-        if (!rc && !b.full && segment_rot_serves(head_dim, b.qkv_b, cos_t, sin_t)) rc = segment_rot(wide, b.qkv_b, cos_t, sin_t, win_lo, win_hi, rows, heads, head_dim, scale, dtype, att, stream);
+        if (!rc && !b.full && segment_rot_serves(b.window, head_dim, b.qkv_b, cos_t, sin_t)) rc = segment_rot(wide, b.qkv_b, cos_t, sin_t, win_lo, win_hi, rows, heads, head_dim, scale, dtype, att, stream);
         else {
             if (!rc) rc = qkv_rope(wide, b.qkv_b, cos_t, sin_t, rows, heads, head_dim, DP, dtype, q, k, v, stream);
             if (!rc) rc = segment_attn(q, k, v, b.full ? full_lo : win_lo, b.full ? full_hi : win_hi, rows, heads, DP, head_dim, scale, dtype, att, stream);

@@ -659,15 +659,16 @@ def vision_blocks_served(hidden: int, inter: int, heads: int, head_dim: int) -> 
     return _ffi.load().pie_vision_blocks_workspace(64, hidden, inter, heads, head_dim) > 0
 
 
-def vision_block_table(blocks: list[dict], after: list[torch.Tensor], full: list[int]):
-    """The blocks' weights (qkv_w, qkv_b, ..; packed Linears and tensors, which the table keeps) for vision_blocks; after[i]: the norm behind block i, full: the blocks over whole images."""
+def vision_block_table(blocks: list[dict], after: list[torch.Tensor], full: list[int], window: int = 0):
+    """The blocks' weights (qkv_w, qkv_b, ..; packed Linears and tensors, which the table keeps) for vision_blocks; after[i]: the norm behind block i, full: the blocks over whole images, window: rows of the
+    others' longest window (0: not known)."""
     def ptr(v):
         return (v.tiles if isinstance(v, PackedLinear) else v).data_ptr()
     table = (_ffi.pie_vision_block * len(blocks))()
     for i, (b, n) in enumerate(zip(blocks, after)):
         for name in ("qkv_w", "qkv_b", "proj_w", "proj_b", "norm2", "gateup_w", "gateup_b", "down_w", "down_b"):
             setattr(table[i], name, ptr(b[name]))
-        table[i].next_norm, table[i].full = ptr(n), int(i in full)
+        table[i].next_norm, table[i].full, table[i].window = ptr(n), int(i in full), window
     table.weights = [dict(b) for b in blocks], list(after)   # alive as long as the pointers
     return table
 

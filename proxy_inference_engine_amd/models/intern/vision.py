@@ -7,8 +7,8 @@ MFMA units (full-image layers and 64-patch-window layers are the same kernel wit
 pie_silu_mul, pie_add, pie_gelu.  Index bookkeeping (positions, window order, cu_seqlens) is host numpy, as it is host
 Python in the reference; the row permutations are device gathers.
 
-Layout notes: head_dim (80 for the 7B tower) is zero-padded to the attention kernel's 128 inside q / k / v; the attention of
-pie_vision_blocks stores the heads' own columns side by side.  PatchEmbed's Conv3d (stride = kernel) is a
+Layout notes: op by op, head_dim (80 for the 7B tower) is zero-padded to the attention kernel's 128 inside q / k / v; the blocks of
+pie_vision_blocks keep heads of 80 unpadded, rotate windows of up to 64 patches inside the attention, and store the heads' own columns side by side.  PatchEmbed's Conv3d (stride = kernel) is a
 GEMM over the flattened patches; its weight is flattened once at load in the pixel rows' (C, T, P, P) order."""
 from __future__ import annotations
 
@@ -99,7 +99,8 @@ class VisionModel:
         self._native = None
         if native:
             after = [b["norm1"] for b in self.blocks[1:]] + [self.merger["ln_q"]]   # the next consumer's norm
-            self._native = ops.vision_block_table(self.blocks, after, c.fullatt_block_indexes)
+            side = c.window_size // c.spatial_merge_size // c.patch_size * c.spatial_merge_size
+            self._native = ops.vision_block_table(self.blocks, after, c.fullatt_block_indexes, side * side)
 
     # ------------------------------------------------------------------ vision.py:245-279
     def rot_pos_emb(self, grid_thw) -> np.ndarray:

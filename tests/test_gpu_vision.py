@@ -224,15 +224,31 @@ def test_blocks_in_one_call_are_the_blocks_op_by_op(cfg, grid, dt):
 
 @pytest.mark.parametrize("head,grid", [(80, [(1, 34, 34)]), (80, [(1, 2, 6)]), (64, [(1, 40, 6)])])
 def test_windows_of_many_key_blocks_rotate_on_the_way_in(head, grid):
-    """Windows of 16 x 16 patches: up to nine blocks of 32 keys per workgroup, tiles that straddle windows, images smaller than one; the same bits as the rotation's own launch (op by op)."""
+    """Windows of 16 x 16 patches, announced as short ones: up to nine blocks of 32 keys per workgroup, tiles that straddle windows, images smaller than one; the same bits as the rotation's own launch (op by op)."""
     _, model = _tower(dict(CFG80, hidden_size=4 * head, num_heads=4, window_size=224), seed=12)
-    assert model._native is not None
+    for block in model._native:
+        block.window = 64
     pix = dev(po.round_T(np.random.default_rng(5).standard_normal((sum(t * h * w for t, h, w in grid), 3 * 2 * 14 * 14)), DT), DT)
     got = model(pix, torch.tensor(grid))
     table, model._native = model._native, None
     want = model(pix, torch.tensor(grid))
     model._native = table
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("window,rotations", [(112, 1), (140, 3)])
+def test_long_windows_rotate_in_a_launch_of_their_own(window, rotations):
+    """Three blocks, the second over the whole image: windows of 8 x 8 patches rotate inside the attention, of 10 x 10 in front of it, as a whole image does; the same bits as op by op."""
+    from torch.profiler import ProfilerActivity, profile
+    _, model = _tower(dict(CFG80, hidden_size=320, num_heads=4, window_size=window), seed=12)
+    pix = dev(po.round_T(np.random.default_rng(5).standard_normal((24 * 22, 3 * 2 * 14 * 14)), DT), DT)
+    got = model(pix, torch.tensor([(1, 24, 22)]))
+    with profile(activities=[ProfilerActivity.CUDA]) as p:
+        model(pix, torch.tensor([(1, 24, 22)]))
+        torch.cuda.synchronize()
+    assert sum(e.count for e in p.key_averages() if "k_vision_qkv_rope" in e.key) == rotations
+    model._native = None
+    assert torch.equal(got, model(pix, torch.tensor([(1, 24, 22)])))
 
 
 def test_rows_of_padded_heads_are_the_projection_s_operand(monkeypatch):
