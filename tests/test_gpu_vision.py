@@ -251,6 +251,17 @@ def test_long_windows_rotate_in_a_launch_of_their_own(window, rotations):
     assert torch.equal(got, model(pix, torch.tensor([(1, 24, 22)])))
 
 
+@pytest.mark.parametrize("dt", ["bfloat16", "float16"])
+def test_whole_images_of_many_tiles(dt):
+    """46 x 46 patches under 16 heads of 80: enough tiles of 64 rows that a workgroup takes two of 32, the last one four rows; the same bits as op by op, whose rows of 128 columns are padded."""
+    _, model = _tower(dict(CFG80, depth=1, hidden_size=1280, num_heads=16, fullatt_block_indexes=[0]), seed=13, dt=dt)
+    assert model._native is not None
+    pix = dev(po.round_T(np.random.default_rng(6).standard_normal((46 * 46, 3 * 2 * 14 * 14)), dt), dt)
+    got = model(pix, torch.tensor([(1, 46, 46)]))
+    model._native = None
+    assert torch.equal(got, model(pix, torch.tensor([(1, 46, 46)])))
+
+
 def test_rows_of_padded_heads_are_the_projection_s_operand(monkeypatch):
     """A tower whose blocks go op by op (hidden 160): the attention's rows of 128 columns a head go into `proj` as they stand, with no copy and no padding in between."""
     from proxy_inference_engine_amd.models.intern import vision
