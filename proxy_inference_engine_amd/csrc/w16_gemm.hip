@@ -71,9 +71,12 @@ int w16m_from_w16s_launch(const void *w16s, int N, int K, void *w16m, hipStream_
 // 3000 rows (8B, 1B and vision-tower widths, weights from HBM: a model's other matrices have passed through the caches since a matrix was last used; fitted to weights that still lie in
 // the 256 MB behind the L2s it preferred plans up to 1.4 times slower).  A K step of a (32 mb) x (128 sw) tile costs t(mb, sw) us -- larger tiles are cheaper per MFMA but quantise worse --
 // and no less than its weights take from beyond the caches, which the row tiles of a column share; workgroups run in rounds of 256, counted on the XCD that has most; all weights come
-// once through HBM (5.6 TB/s, less by fewer than 180 workgroups: 4.1 by 112, 4.2 by 128, 5.7 by 192 of one row tile; while any number counted as all, up to 64 rows took too few splits, us: 40 rows of
-// [4096, 14336] in four 34.9, in seven 26.9, of [14336, 4096] whole 35.0, in two 28.3, of [8192, 4096] in two 22.7, in three 18.8, of [5120, 3072] in three 14.3, in six 12.3); a launch costs 5.8 us of ramp, prologue and epilogue; a K split writes and re-reads its fp32 slabs and launches the reduce.  Over those products its choices
-// take 1.4 % longer than the best ones (those of the model before: 6.2 %); over 563 products of 40 matrices, most of them others, 1.9 % (6.4 %).  Up to K = 2048 the reduce's launch has little to hide behind:
+// once through HBM (5.6 TB/s; 2.2 and 0.019 for each workgroup by fewer than 165, of up to 64 rows and 2048 columns than 144: 112 workgroups of one row tile read 4.1, 128 4.2, 192 5.7, and of a handful the steps take
+// longer than the stream; while any number counted as all, up to 64 rows took too few splits, us: 40 rows of [4096, 14336] in four 34.9, in six 27.5, of [14336, 4096] whole 35.0, in two 28.3, of [8192, 4096] in
+// two 22.7, in three 18.8, of [5120, 3072] in three 14.3, in five 12.5); a launch costs 5.8 us of ramp, prologue and epilogue; a K split writes and re-reads its fp32 slabs and launches the reduce.  Up to K = 2048
+// that launch has little to hide behind, but for matrices of 30 MB and more under up to 64 rows (us, 43 / 61 rows: [8448, 2048] in three 12.5 / 13.4, in two 13.8 / 14.7, whole 16.3 / 17.2; 33 / 58 rows: [12288, 2048] in two 15.9 / 17.4, whole
+// 16.8 / 18.0).  Over 540 products of 45 matrices and 33 to 256 rows its choices take 0.9 % longer than the best ones, over 240 of 20 matrices and 40 to 2000 rows 1.6 %.  The widest of these misses, taken / best, us: [2048, 2048] 256 rows 12.6 /
+// 10.1, [5120, 5120] 509 rows 46.2 / 39.8, [4096, 14336] 1024 rows 121 / 108, [4096, 4096] 180 rows 21.8 / 19.4, [3072, 8192] 1024 rows 66.8 / 59.7.
 // The fused activation takes the same tiles (while it was built for two strips per wave alone, us: 64 / 128 / 256 / 320 rows of [28672, 4096] 68 / 67 / 76 / 102, now 48 / 55 / 70 / 99; of
 // [11264, 2048] 29 / 29 / 28 / 29, now 20 / 20 / 24 / 28; of the tower's [6840, 1280] 21 / 20 / 20 / 20, now 11 / 13 / 13 / 16).
 // [1024, 1024], 450 rows: 6.5 us, in two splits 8.8; [1280, 1280], 320 rows: 7.7, 9.5.  [4096, 14336]: 64 / 128 / 509 / 1024 rows 40 / 40 / 91 / 123 -> 34 / 34 / 67 / 113 us.
@@ -105,6 +108,7 @@ static W16Plan w16_plan(int M, int N, int K, bool no_split = false) {
     static const double t_light[4][3] = {{0, 0, 0}, {0, 0.30, 0.63}, {0, 0.43, 0.78}, {0, 0.61, 1.05}};  // [log2 mb][sw]
     static const double t_full[4][3] = {{0, 0, 0}, {0, 0.30, 0.52}, {0, 0.45, 0.82}, {0, 0.83, 1.45}};
     const double bytes = 2.0 * N * (64.0 * groups);
+    const bool few_short = M <= 64 && groups <= 32;
     for (int S = 1; S <= (no_split ? 1 : 16) && (S == 1 || 8 * S <= groups); ++S)
         for (int mb = mb_max; mb >= 2; mb >>= 1)
             for (int sw = 2; sw >= 1; --sw) {
@@ -116,9 +120,9 @@ static W16Plan w16_plan(int M, int N, int K, bool no_split = false) {
                 const int mi = mb == 8 ? 3 : (mb == 4 ? 2 : 1);
                 const double t = t_light[mi][sw] + (t_full[mi][sw] - t_light[mi][sw]) * load;
                 double us = (most + 31) / 32 * steps * (t > cold ? t : cold);
-                const double rate = 2.2 + 0.019 * wgs, stream_us = bytes / ((rate < 5.6 ? rate : 5.6) * 1e6);
+                const double stream_us = bytes / (wgs >= (few_short ? 144 : 165) ? 5.6e6 : 2.2e6 + 0.019e6 * wgs);
                 us = (us > stream_us ? us : stream_us) + 5.8;
-                if (S > 1) us += (double)M * N * 4.0 * (2 * S + 0.5) / 5.1e6 + (groups <= 32 ? 3.5 : 1.0);
+                if (S > 1) us += (double)M * N * 4.0 * (2 * S + 0.5) / 5.1e6 + (groups <= 32 && !(few_short && bytes >= 30e6) ? 3.5 : 1.0);
                 if (us < best_us) best_us = us, best = {mb, sw, S, us};
             }
     best.S = w16_even_splits(groups, best.S);
