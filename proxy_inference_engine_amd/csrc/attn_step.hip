@@ -245,8 +245,8 @@ __global__ void __launch_bounds__(STEP_WAVES * 64, REP <= 4 ? 3 : 2) k_attn_step
             }
         }
     };
-    // Between loads in flight and their use stands no branch around a load: behind one the compiler would wait for every load there is.  The last two blocks load nothing, and only they can
-    // hold the new row or tokens past the end (one loop for all, with loads past the end: 168 registers instead of 152; sixteen steps of four layers, one f16 row of TinyLlama's 2561 / 2532 us, 8 int4 rows of
+    // Between loads in flight and their use stands no branch around a load: behind one the compiler would wait for every load there is.  Behind the loop, the last two blocks, or
+    // one of an odd number, load nothing, and only they can hold the new row or tokens past the end; of an odd number the loop's last round asks for a row of the last block again (one loop for all, with loads past the end: 168 registers instead of 152; sixteen steps of four layers, one f16 row of TinyLlama's 2561 / 2532 us, 8 int4 rows of
     // Llama-3-8B's at 200 positions 4040 / 3970, 32 at 1000 6262 / 6231).
     int b0 = 0;
     for (; b0 + STEP_DEPTH < n_blk; b0 += STEP_DEPTH)

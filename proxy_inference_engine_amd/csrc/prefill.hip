@@ -1112,7 +1112,8 @@ static bool step_tiles(const pie_decoder *d, int B) {
 // unit (k_w4s_gemv_rows: RMSNorm prologues; RoPE + page append, residual, SwiGLU and logits epilogues, per row) -- 6 launches per
 // layer instead of 7, each row in MLX's row-by-row fp32 regime.  Biases, int8 pages and hidden sizes beyond 8192 take the
 // general path, and from 3 rows on every step whose matrices k_w4a_gemm takes: the GEMV's work grows with its rows (Llama-3-8B, four layers, 16 steps at 200 positions, 2 / 3 / 4 / 5 rows
-// 3823 / 4515 / 5283 / 6332 us; the general path, 3 / 4 / 5 / 6 / 8 rows 4156 / 4363 / 4415 / 4465 / 4570).
+// 3812 / 4515 / 5283 / 6332 us; the general path, 2 / 3 / 4 / 5 / 6 / 8 rows 3617 / 3672 / 3715 / 3770 / 3785 / 3897; Llama-3.2-3B, 2 rows 3172, general 2926.  Two rows, too, would gain by the general path since its
+// products are 16 x 16; the line was drawn before).
 static bool batch_fused(const pie_decoder *d, int B) {
     if (B > GEMV_ROWS_MAX || !d->uniform_int4() || d->kv_i8 || d->cfg.hidden > 8192 || w4s_gemv_waves(d->cfg.vocab, d->cfg.hidden) > TAIL_MAX_STATS) return false;
     for (const pie_layer_weights &w : d->layers)

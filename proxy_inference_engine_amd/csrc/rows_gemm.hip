@@ -227,7 +227,7 @@ __global__ void __launch_bounds__(512) k_rows_w16m(const RowsArgs a) {
                     for (int t = 0; t < NT; ++t) acc[n][t] = rows_mfma<E>(w, xv[u][t], acc[n][t]);
                 }
         };
-        // (each half round's loads in a piece, none past the end: the compiler's waits count them exactly.  us, one row, with its own order and a last round of loads for nothing / this: [5120, 3072] 10.4 / 9.0,
+        // (each half round's loads in a piece, no half round past the end (within the last one, steps past it read the last tile again): the compiler's waits count them exactly.  us, one row, with its own order and a last round of loads for nothing / this: [5120, 3072] 10.4 / 9.0,
         // [16384, 3072] 19.5 / 18.1, [6144, 4096] 12.3 / 11.9, [4096, 4096] 8.0 / 8.0)
         mf_u32x4 w0[U][NN], w1[U][NN], x0[U][NT], x1[U][NT];
         constexpr int R = U * KW;
@@ -368,7 +368,8 @@ __global__ void __launch_bounds__(64 * WV, 4) k_rows_lds(const RowsArgs a) {
                     for (int t = 0; t < NT; ++t) acc[n][t] = rows_mfma<E>(wv[u][n], xv[t], acc[n][t]);
             }
         };
-        // (x before w: waiting for the next chunk's x must not wait for the weights behind it.  The loads stay in this order, and the last two chunks load nothing: with loads that the scheduler moved, or a
+        // (x before w: waiting for the next chunk's x must not wait for the weights behind it.  The loads stay in this order, and the last two chunks, or one of an odd number, load nothing; of an odd number the round before asks for a chunk past the end, which the
+        // descriptors drop.  With loads that the scheduler moved, or a
         // round left halfway by a break, the compiler waited for every load in flight in every other chunk.  us, 8 / 32 rows, that / this: [6144, 4096] 13.1 / 12.4, 16.7 / 15.9; [5120, 3072] 10.9 / 10.0,
         // 13.9 / 13.2; [4096, 14336] 23.5 / 23.0, 33.5 / 31.4; [10752, 4096] 19.5 / 18.7, 23.2 / 22.1; [32768, 4096] 43.4 / 43.0, 47.2 / 45.8; [28672, 4096] 40.3 / 40.3, 42.9 / 42.7)
         mf_u32x4 w[2][U][NN], xv[XJ];

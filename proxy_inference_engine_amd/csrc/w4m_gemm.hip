@@ -830,8 +830,8 @@ static W4aPlan w4a_plan(int M, int N, int K, bool may_split, int bits) {
     if (S == 1) return {each, 1, 8 * steps};
     return {4, S, 8 * (steps / S)};
 }
-// step: a batch's step, whose rows are single sequences' in the one-row arithmetic.  A prompt of 9 to 16 rows keeps weights rounded to T, as mx.quantized_matmul's matrix kernels have them from six rows on, in
-// its narrow products (k_w4r_gemm).
+// step: a batch's step, whose rows are single sequences' in the one-row arithmetic.  A prompt of 9 to 16 rows has that arithmetic in its wide products; its narrow ones multiply weights rounded to T (k_w4r_gemm), as
+// mx.quantized_matmul's matrix kernels do from six rows on: with the scales on the sums there too, nine rows are closer to 64 bits, but 4.1 ulps off the oracle that rounds, where 4 are allowed.
 bool w4a_serves(int M, int N, int K, int bits, bool step) {
     return pie_knob(PIE_KNOB_W4R) != 0 && w4a_plan(M, N, K, false, bits).halves != 0 && (step || bits == 8 || M <= 8 || N >= 512 * 32);
 }
